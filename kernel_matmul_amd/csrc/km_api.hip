@@ -86,6 +86,54 @@ static const long long TARGET_WAVES = 1024;
 // Row-block items from which the workgroup-shared forward kernel is considered.
 static const long long BLOCK_VARIANT_MIN_ITEMS = 4096;
 
+// Grid form (rbf and spectral kernels): wavefronts per 128-row item.  One while that fills the SIMDs
+// (3 resident wavefronts each, 2 for the kernels with more than 32 operand columns), more to make the
+// device busy with fewer items.  Measured at ten points per unit, cutoff of 6 lengthscales, spectral
+// k = 16, wavefronts 1 / 2 / 4 / 8: 157 items 18.0 / 12.1 / 9.8 / 10.5 us (fit-like density of 700
+// points per unit: 151 / 79 / 41 / 31), 628 items 22.8 / 17.5 / 15.7 / 27.4, 782 items 23.1 / 17.8 / 19.4 /
+// 34.7, 2400 items 33.6 / 31.8 / 40.3, 3600 items 42.9 / 44.7 / 56.3.  Below 48 items the entry-wise table
+// kernels in 16-row pieces spread further (32 items: 6.1 against 9.5 us).
+// From 350 items per XCD on the last 32 of each are split between four wavefronts: without them the
+// items beyond whole rounds of resident wavefronts run alone (782 items per XCD: 66.1 against 61.4 us,
+// 391: 42.0 against 35.3; 600, the worst met: 51.4 against 52.0).  The kernels with two resident
+// wavefronts gain from it only just past a whole round (782: 103.2 against 98.3 us; 600: 79.2 against 81.2).
+static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int variant, MatmulPlan* plan) {
+    const bool automatic = variant == KM_VARIANT_AUTO &&
+                           !(opt && (opt->rows_per_wave != 0 || opt->col_splits > 1 || opt->reserved != 0));
+    if (!(automatic || variant == KM_VARIANT_GRID) || p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
+        return false;
+    }
+    const int k_chunk = p.k <= 16 ? 16 : (p.k <= 32 ? 32 : 64);
+    const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
+    const long long per_launch = row_blocks * p.num_batches;
+    const long long items = per_launch * ((p.k + k_chunk - 1) / k_chunk);
+    if (automatic && items < 48) {
+        return false;
+    }
+    plan->variant = KM_VARIANT_GRID;
+    plan->k_chunk = k_chunk;
+    plan->row_groups = 8;
+    plan->tail_balance = 0;
+    plan->group_tail_halves = 0;
+    const bool two_resident = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1) > 32;
+    if (opt && opt->rows_per_wave != 0) {
+        plan->col_splits = KM_BLOCK_SIZE / opt->rows_per_wave;
+    } else {
+        plan->col_splits = items <= 200 ? 8 : (items < 700 ? 4 : (items < 2800 ? 2 : 1));
+    }
+    if (plan->col_splits != 1) {
+        plan->group_tail = -1;
+    } else if (plan->group_tail < 0) {
+        const long long per_xcd = (per_launch + KM_NUM_XCD - 1) / KM_NUM_XCD;
+        if (two_resident) {
+            plan->group_tail = per_xcd < 1024 && per_xcd % 256 <= 24 ? 16 : -1;
+        } else {
+            plan->group_tail = per_xcd < 1500 ? 32 : -1;
+        }
+    }
+    return true;
+}
+
 static int make_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
     int variant = opt ? opt->variant : KM_VARIANT_AUTO;
     plan->phase_split = 0;
@@ -96,6 +144,16 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
         // above: 0 = the usual share of them as two halves of 64 rows, else that count + 1
         plan->group_tail = (opt->reserved - 2) & 0xffff;
         plan->group_tail_halves = ((opt->reserved - 2) >> 16) - 1;
+    }
+    if (variant == KM_VARIANT_GRID && opt->rows_per_wave != 0 && opt->rows_per_wave != 16 &&
+        opt->rows_per_wave != 32 && opt->rows_per_wave != 64 && opt->rows_per_wave != 128) {
+        return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: rows_per_wave must be 16, 32, 64 or 128");
+    }
+    if (variant == KM_VARIANT_GRID && p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
+        return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: the grid form takes rbf and spectral kernels only");
+    }
+    if (grid_plan(p, opt, variant, plan)) {
+        return KM_OK;
     }
     if (variant == KM_VARIANT_AUTO) {
         // Measured on gfx950 (n = 1e5, k = 16): for the locally periodic kernel with enough row
@@ -523,6 +581,18 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
     const char* kt = kernels[kernel_type];
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     const int G = plan.k_chunk / 16;
+    size_t used = 0;
+    if (plan.variant == KM_VARIANT_GRID) {
+        used = (size_t)snprintf(text, text_bytes, "km::fwd_grid%s<%s, G=%d, W=%d> (grid form); entry by entry it would be ",
+                                plan.group_tail > 0 ? "_grouped" : "", kt, G, plan.col_splits);
+        if (used >= text_bytes) return KM_OK;
+        km_launch_options entries;
+        memset(&entries, 0, sizeof(entries));
+        entries.variant = KM_VARIANT_MFMA_F16;
+        if (int rc = make_plan(p, &entries, &plan)) return rc;
+        text += used;
+        text_bytes -= used;
+    }
     switch (plan.variant) {
         case KM_VARIANT_VALU:
             snprintf(text, text_bytes, "km::fwd_valu<%s, KC=%d>: 128 rows per workgroup, %lld workgroups", kt,
@@ -534,6 +604,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                      kt, plan.phase_split, G);
             break;
         default: {
+            const int groups = plan.k_chunk / 16;
             const char* name = plan.variant == KM_VARIANT_MFMA_F32_DIRECT
                                    ? "km::fwd_mfma_f32"
                                    : (plan.variant == KM_VARIANT_MFMA_F32
@@ -555,7 +626,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                 break;
             }
             snprintf(text, text_bytes, "%s<%s, G=%d, R=%d>: %d rows per wavefront, %d wavefront(s) per row range%s",
-                     name, kt, G, plan.row_groups, 16 * plan.row_groups, plan.col_splits,
+                     name, kt, groups, plan.row_groups, 16 * plan.row_groups, plan.col_splits,
                      plan.tail_balance && plan.row_groups == 8 && plan.col_splits == 1 &&
                              plan.variant == KM_VARIANT_MFMA_F16_DIRECT &&
                              row_blocks * num_batches >= 2 * 128 * KM_NUM_XCD

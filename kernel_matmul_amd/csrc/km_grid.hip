@@ -1,0 +1,686 @@
+// Forward operator in the grid form (km_grid.h): rbf and spectral kernels, any number of rhs
+// columns.  A row block of 128 rows is one item, worked on by W wavefronts:
+//
+//   columns -> grid   the wavefronts take the steps of 32 columns of the block's range in turn; V is
+//                     the A operand (16 grid points x 32 columns), rhs (spectral: times cos B and
+//                     sin B, as in the phase-split table kernel) the B operand.  Grid tiles out of a
+//                     step's reach are skipped.  With W > 1 the sums meet in LDS, added in a fixed order.
+//   grid -> rows      every wavefront takes 128 / W rows; V is the A operand again (16 rows x 32 grid
+//                     points), the sums, moved between lanes into operand layout, the B operand.
+//
+// Both factors of both contractions are split into two fp16 terms as in the table kernels.  A row
+// block whose window does not fit the accumulators (points sparse against the lengthscale), whose
+// range is too short to gain, or whose coordinates or rhs are not finite is evaluated entry by entry
+// in the same launch: each wavefront its rows, tile against tile, those out of reach left out.
+#include "km_batch.h"
+#include "km_common.h"
+#include "km_fwd.h"
+#include "km_grid.h"
+#include "km_launch.h"
+
+namespace km {
+
+// Columns in a row block's range from which the grid form is taken.
+#define KM_GRID_MIN_WIDTH 160
+
+// This lane's part of a step's rhs operand: byte offsets of its 8 columns' first row (8 kk) and of its
+// rhs column in each group.  Inner strides are at most 2^22 elements (the entry point checks), so a
+// step spans less than 2^32 bytes and its row offsets come from 24-bit multiplications.
+template <int G>
+struct RhsLane {
+    unsigned row;
+    unsigned col[G];
+    bool used[G];
+};
+
+// rhs values of a step (columns c0 + 8 kk + t), zero past the end of the range.
+template <int G>
+__device__ __forceinline__ void grid_rhs(const FwdArgs& a, const float* __restrict__ rhs, int c0, int col_end,
+                                         int kk, const RhsLane<G>& lane, float (&raw)[G][8]) {
+    const buffer_rsrc ru = uniform_buffer(rhs + (long long)c0 * a.rhs_s0);
+    const unsigned s0 = (unsigned)a.rhs_s0;
+    if (c0 + 32 <= col_end) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                raw[g][t] = buffer_at(ru, lane.row + lane.col[g], 4u * (unsigned)t * s0);
+            }
+        }
+    } else {
+        const int last = col_end - 1 - c0;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const int rel = 8 * kk + t;
+            const unsigned row = 4u * __umul24((unsigned)min(rel, last), s0);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const float v = buffer_at(ru, row + lane.col[g], 0u);
+                raw[g][t] = rel <= last ? v : 0.0f;
+            }
+        }
+    }
+}
+
+// The Gaussian factor of a row against two neighbouring columns, split into fp16 halves, times
+// 2^KM_F16_KSCALE_LOG2.  (The power of two is applied to the rounded halves, exactly, and in the
+// residual: inside the exponent it would cost it four bits.)
+__device__ __forceinline__ void entry_pair_f16(float x, float ya, float yb, float scale, half2v* hi, half2v* lo) {
+    constexpr float S = (float)(1 << KM_F16_KSCALE_LOG2);
+    const float ua = (x - ya) * scale, ub = (x - yb) * scale;
+    const float ea = __builtin_amdgcn_exp2f(-ua * ua);
+    const float eb = __builtin_amdgcn_exp2f(-ub * ub);
+    const float2v kv = {ea, eb};
+    const half2v h = __builtin_convertvector(kv, half2v) * (half2v){(_Float16)S, (_Float16)S};
+    *hi = h;
+    *lo = residual_f16x2(ea, S, eb, S, h);
+}
+
+// Two powers of two split into fp16 halves.
+__device__ __forceinline__ void exp2_pair_f16(float a, float b, float one, half2v* hi, half2v* lo) {
+    const float2v kv = {__builtin_amdgcn_exp2f(a), __builtin_amdgcn_exp2f(b)};
+    const half2v h = __builtin_convertvector(kv, half2v);
+    *hi = h;
+    *lo = residual_f16x2(kv[0], one, kv[1], one, h);
+}
+
+// One step of 32 columns: scale and split the rhs operand, then for every tile of 16 points in
+// reach evaluate, split and contract.  GRID: the points are the grid's, t0 + 16 mt h; else the rows xr[].
+template <bool GRID, int G, int PARTS, int MT>
+__device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off, const float (&raw)[G][8],
+                                          const GridWindow& gw, float t0, const float* xr, const KernelConsts& kc,
+                                          int tiles, bool wide, const bool (&colmask)[G], int (&shift)[G], float (&scale)[G],
+                                          bool* rhs_finite, float4v (&acc)[MT][G * PARTS]) {
+    constexpr int CH = KM_GRID_CHUNK;
+    constexpr int GE = G * PARTS;
+    float xv[8], cb[8], sb[8];
+#pragma unroll
+    for (int t = 0; t < 8; t += 4) {
+        const float4v vx = *(const float4v*)(tab + off + t);
+        const float4v vc = *(const float4v*)(tab + CH + off + t);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            xv[t + u] = vx[u];
+            cb[t + u] = vc[u];
+        }
+        if (PARTS == 2) {
+            const float4v vs = *(const float4v*)(tab + 2 * CH + off + t);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                sb[t + u] = vs[u];
+            }
+        }
+    }
+    const float ref = tab[3 * CH + (off >> 3)];
+    const float span = tab[3 * CH + CH / 8 + (off >> 3)];
+
+    half8v bhi[GE], blo[GE];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        // The column's running power-of-two scale, as in f16_step.
+        float m = 0.0f;
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            m = fmaxf(m, fabsf(raw[g][t]));
+        }
+        m = column_max(m);
+        const bool grow = colmask[g] && !(m * scale[g] < 32768.0f);
+        if (__any(grow)) {
+            *rhs_finite = *rhs_finite && !__any(grow && !(m < __builtin_inff()));
+            if (grow) {
+                const int e = __builtin_amdgcn_frexp_expf(m);
+                const int new_shift = min(max(14 - e, -100), 100);
+                const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+                    for (int part = 0; part < PARTS; part++) {
+                        acc[mt][part * G + g] *= factor;
+                    }
+                }
+                shift[g] = new_shift;
+                scale[g] = __builtin_ldexpf(1.0f, new_shift);
+            }
+        }
+        float vc[8];
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            vc[t] = raw[g][t] * scale[g];
+        }
+        if (PARTS == 2) {
+            float vs[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                vs[t] = vc[t] * sb[t];
+            }
+            split_f16x8(vs, kc.one, &bhi[G + g], &blo[G + g]);
+        }
+        if (PARTS == 2 || GRID) {
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                vc[t] *= cb[t];
+            }
+        }
+        split_f16x8(vc, kc.one, &bhi[g], &blo[g]);
+    }
+
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        if (mt >= tiles) {
+            break;
+        }
+        const float t = GRID ? __builtin_fmaf((float)(16 * mt), gw.h, t0) : xr[mt];
+        const float av = (t - ref) * (GRID ? gw.s2 : kc.s);
+        if (!__any(!(fabsf(av) - span > KM_GRID_REACH))) {
+            continue;
+        }
+        half2v h2[4], l2[4];
+        float arg[8];
+        if (GRID) {
+            if (!wide) {
+                const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    arg[u] = __builtin_fmaf(av, xv[u], rb);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const float z = __builtin_fmaf(-0.5f, xv[u], av);
+                    arg[u] = __builtin_fmaf(-z, z, (float)KM_GRID_KS1);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (GRID) {
+                exp2_pair_f16(arg[2 * u], arg[2 * u + 1], kc.one, &h2[u], &l2[u]);
+            } else {
+                entry_pair_f16(t, xv[2 * u], xv[2 * u + 1], kc.s, &h2[u], &l2[u]);
+            }
+        }
+        const half8v ahi = join_half2x4(h2);
+        const half8v alo = join_half2x4(l2);
+#pragma unroll
+        for (int g = 0; g < GE; g++) {
+            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[g], acc[mt][g], 0, 0, 0);
+            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[g], acc[mt][g], 0, 0, 0);
+            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[g], acc[mt][g], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+// The columns of [w.range_start, w.range_end) against `tiles` groups of 16 points (GRID: of the
+// grid window; else the rows xr[]): acc in the D layout times 2^shift (per rhs column) and the scale
+// of the evaluated factor.  The wavefront takes every W-th step of 32 columns from step `wave` on.
+// Returns false if a value was met that the form cannot take (GRID; see grid_table).
+// A step's rhs values are requested a step ahead (a step is short: two or three tiles), a chunk's
+// coordinates a chunk ahead (the first chunk's, in xv, by the caller).
+template <bool GRID, int KT, int G, int MT, int W>
+__device__ __forceinline__ bool grid_columns(const FwdArgs& a, float* __restrict__ tab, const WaveView& w, int kbase,
+                                             int wave, const GridWindow& gw, const KernelConsts& kc, const float* xr,
+                                             int tiles, float (&xv)[KM_GRID_CHUNK / 64], int (&shift)[G],
+                                             float4v (&acc)[MT][G * (KT == KM_KERNEL_SPECTRAL ? 2 : 1)]) {
+    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
+    constexpr int PARTS = PHASE ? 2 : 1;
+    constexpr int CH = KM_GRID_CHUNK;
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    const float* __restrict__ rhs = w.rhs + (long long)kbase * a.rhs_s1;
+    RhsLane<G> rl;
+    float scale[G];
+    rl.row = 4u * __umul24(8u * (unsigned)kk, (unsigned)a.rhs_s0);
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int c = kbase + 16 * g + li;
+        rl.col[g] = 4u * __umul24((unsigned)(min(c, a.k - 1) - kbase), (unsigned)a.rhs_s1);
+        rl.used[g] = c < a.k;
+        shift[g] = 100;
+        scale[g] = c < a.k ? __builtin_ldexpf(1.0f, 100) : 0.0f;
+    }
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+#pragma unroll
+        for (int g = 0; g < G * PARTS; g++) {
+            acc[m][g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+    const float t0 = (gw.g_lo + (float)li) * gw.h;
+    bool fine = true;
+    for (int first = w.range_start + 32 * wave; first < w.range_end; first += CH * W) {
+        const unsigned steps = grid_table<GRID, PHASE>(xv, first, W, w.range_end, gw, kc, tab, &fine);
+        if (first + CH * W < w.range_end) {
+            grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
+        }
+        unsigned need = steps & 0xffff;
+        if (need == 0) {
+            continue;
+        }
+        float next[G][8];
+        int j = __builtin_ctz(need);
+        grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
+        do {
+            float raw[G][8];
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    raw[g][t] = next[g][t];
+                }
+            }
+            const int off = 32 * j + 8 * kk;
+            const bool wide = (steps >> (16 + j) & 1) != 0;
+            need &= need - 1;
+            if (need != 0) {
+                j = __builtin_ctz(need);
+                grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
+            }
+            // (kept as register quadruples: read element by element below, the accumulators are split
+            // up and put together again in every step otherwise)
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+#pragma unroll
+                for (int g = 0; g < G * PARTS; g++) {
+                    asm volatile("" : "+v"(acc[m][g]));
+                }
+            }
+            grid_step<GRID, G, PARTS, MT>(tab, off, raw, gw, t0, xr, kc, tiles, wide, rl.used, shift, scale, &fine, acc);
+        } while (need != 0);
+        // All reads of the table are done before the next chunk overwrites it.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    return fine;
+}
+
+// A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the
+// phase-split form combined, and the masked store.
+template <int KT, int G>
+__device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, const KernelConsts& kc, float x,
+                                           float x_ref, const float4v* res, const float* down, int row, int kbase) {
+    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    float ca[4], sa[4];
+    if (PHASE) {
+        // cos A / sin A of the row this lane holds, fetched into the accumulator layout.
+        const float th = phase_rev(kc.f, x, x_ref);
+        const float ca_own = __builtin_amdgcn_cosf(th);
+        const float sa_own = __builtin_amdgcn_sinf(th);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            ca[v] = __shfl(ca_own, 4 * kk + v, 64);
+            sa[v] = __shfl(sa_own, 4 * kk + v, 64);
+        }
+    }
+    float* __restrict__ out = a.out + w.b * (long long)a.m * a.k;
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int c = kbase + 16 * g + li;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const float value = PHASE ? ca[v] * (res[g][v] * down[g]) + sa[v] * (res[G + g][v] * down[G + g])
+                                      : res[g][v] * down[g];
+            const int r = row + 4 * kk + v;
+            if (r < a.m && c < a.k) {
+                out[(long long)r * a.k + c] = value;
+            }
+        }
+    }
+}
+
+// LDS of one item in floats: the wavefronts' tables, overlaid by the exchange of the sums, and a
+// flag per wavefront.
+template <int GE, int MT, int W>
+constexpr int grid_lds_floats() {
+    return W == 1 ? KM_GRID_TABLE_FLOATS
+                  : (W * KM_GRID_TABLE_FLOATS > W * MT * GE * 256 ? W * KM_GRID_TABLE_FLOATS : W * MT * GE * 256) + W;
+}
+
+// One item in the grid form for rhs columns [kbase, kbase + 16 G), by W wavefronts of which this is
+// number `wave`.  Returns whether it was done (the same in all W); if not, nothing was stored.
+// W > 1: synchronises the workgroup three times.
+template <int KT, int G, int MT, int W>
+__device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
+                                             int wave, const GridWindow& gw, const KernelConsts& kc,
+                                             float (&xv)[KM_GRID_CHUNK / 64]) {
+    constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
+    constexpr int GE = G * PARTS;
+    constexpr int R = 8 / W;  // groups of 16 rows of this wavefront
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+
+    int shift[G];
+    float4v acc[MT][GE];
+    bool fine = grid_columns<true, KT, G, MT, W>(a, lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, wave, gw, kc, nullptr,
+                                                 gw.tiles, xv, shift, acc);
+
+    // The sums of all W wavefronts, added in their order.
+    if (W > 1) {
+        float4v* part = (float4v*)lds;
+        int* flags = (int*)(lds + grid_lds_floats<GE, MT, W>() - W);
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1);
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+#pragma unroll
+                for (int p = 0; p < PARTS; p++) {
+                    acc[m][p * G + g] *= up;
+                }
+            }
+        }
+        __syncthreads();  // the exchange lies over the tables
+        if (lane == 0) {
+            flags[wave] = fine ? 1 : 0;
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            if (m < gw.tiles) {
+#pragma unroll
+                for (int g = 0; g < GE; g++) {
+                    part[((wave * MT + m) * GE + g) * 64 + lane] = acc[m][g];
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < W; v++) {
+            fine = fine && __builtin_amdgcn_readfirstlane(flags[v]) != 0;
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            if (m < gw.tiles) {
+#pragma unroll
+                for (int g = 0; g < GE; g++) {
+                    float4v sum = part[(m * GE + g) * 64 + lane];
+#pragma unroll
+                    for (int v = 1; v < W; v++) {
+                        sum += part[((v * MT + m) * GE + g) * 64 + lane];
+                    }
+                    acc[m][g] = sum;
+                }
+            }
+        }
+        __syncthreads();  // all reads done: the area may become tables again
+    }
+    if (!fine) {
+        return false;
+    }
+
+    // Grid -> rows.  One power-of-two scale per column over the whole window; the operands of all
+    // steps of 32 grid points replace the accumulators, so that a row group needs no more than its
+    // own accumulator at a time.
+    const float hz = gw.h * gw.s2;
+    float b2[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const float b = ((float)t - 3.5f) * hz;
+        b2[t] = uniform(b + b);
+    }
+    float fac[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        fac[t] = uniform(__builtin_amdgcn_exp2f(-0.25f * b2[t] * b2[t]));
+    }
+    const float weight = w.params[KernelTraits<KT>::SIGMA * a.params_s] * (hz * KM_GRID_WEIGHT);
+    float down[GE];
+    constexpr int KSTEPS = (MT + 1) / 2;
+    half8v bhi[KSTEPS][GE], blo[KSTEPS][GE];
+#pragma unroll
+    for (int g = 0; g < GE; g++) {
+        float m = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                m = fmaxf(m, fabsf(acc[mt][g][v]));
+            }
+        }
+        m = column_max(m);
+        const int e = min(max(14 - __builtin_amdgcn_frexp_expf(m), -100), 100);
+        const float up = __builtin_ldexpf(1.0f, e);
+        down[g] = weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 - (W > 1 ? 0 : shift[g % G] + KM_GRID_KS1));
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ks++) {
+            if (2 * ks < gw.tiles) {
+                float gv[8];
+                constexpr int LAST = MT - 1;
+                const float4v none = {0.0f, 0.0f, 0.0f, 0.0f};
+                grid_operand(acc[2 * ks][g], 2 * ks + 1 <= LAST ? acc[2 * ks + 1 <= LAST ? 2 * ks + 1 : LAST][g] : none, gv);
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    gv[t] *= up * fac[t];
+                }
+                split_f16x8(gv, kc.one, &bhi[ks][g], &blo[ks][g]);
+                __builtin_amdgcn_sched_barrier(0);  // one operand at a time (registers)
+            }
+        }
+    }
+    const float mid0 = (gw.g_lo + (float)(8 * kk) + 3.5f) * gw.h;
+    const float mid_step = 32.0f * gw.h;
+#pragma unroll 2
+    for (int r = 0; r < R; r++) {
+        const int row = row0 + 16 * (wave * R + r);
+        const float x = w.x1[(long long)min(row + li, a.m - 1) * a.x1_s];
+        float4v res[GE];
+#pragma unroll
+        for (int g = 0; g < GE; g++) {
+            res[g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ks++) {
+            if (2 * ks >= gw.tiles) {
+                break;
+            }
+            const float av = ((x - gw.x_ref) - __builtin_fmaf((float)ks, mid_step, mid0)) * gw.s2;
+            if (!__any(fabsf(av) - 3.5f * hz < KM_GRID_REACH)) {
+                continue;
+            }
+            half2v h2[4], l2[4];
+            const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS2);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                separable_pair_f16(av, rb, b2[2 * u], b2[2 * u + 1], kc.one, &h2[u], &l2[u]);
+            }
+            const half8v ahi = join_half2x4(h2);
+            const half8v alo = join_half2x4(l2);
+#pragma unroll
+            for (int g = 0; g < GE; g++) {
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[ks][g], res[g], 0, 0, 0);
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[ks][g], res[g], 0, 0, 0);
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[ks][g], res[g], 0, 0, 0);
+            }
+        }
+        grid_store<KT, G>(a, w, kc, x, gw.x_ref, res, down, row, kbase);
+    }
+    return true;
+}
+
+// The item entry by entry: each of the W wavefronts evaluates its rows, 32 at a time, against the
+// whole range.
+template <int KT, int G, int W>
+__device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
+                                               int wave, const GridWindow& gw, const KernelConsts& kc) {
+    constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
+    constexpr int GE = G * PARTS;
+    constexpr int R = W == 8 ? 1 : 2;
+    constexpr int PIECES = 8 / (W * R);
+    const int li = threadIdx.x & 15;
+#pragma unroll 1
+    for (int piece = 0; piece < PIECES; piece++) {
+        const int base = row0 + 16 * R * (wave * PIECES + piece);
+        float xr[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            xr[r] = w.x1[(long long)min(base + 16 * r + li, a.m - 1) * a.x1_s];
+        }
+        // the columns within reach of these rows
+        GridWindow rows = gw;
+        float lo = xr[0] - gw.x_ref, hi = lo;
+        bool finite = true;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const float y = xr[r] - gw.x_ref;
+            lo = fminf(lo, y);
+            hi = fmaxf(hi, y);
+            finite = finite && fabsf(y) < 1e30f;
+        }
+        wave_min_max(&lo, &hi);
+        finite = __all(finite);
+        const float reach = KM_GRID_REACH / kc.s;
+        rows.col_lo = uniform(finite ? lo - reach : -__builtin_inff());
+        rows.col_hi = uniform(finite ? hi + reach : __builtin_inff());
+        float xv[KM_GRID_CHUNK / 64];
+        if (w.range_start < w.range_end) {
+            grid_load(w.x2, a.x2_s, w.range_start, 1, w.range_end, xv);
+        }
+        int shift[G];
+        float4v acc[R][GE];
+        grid_columns<false, KT, G, R, 1>(a, lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr, R, xv, shift, acc);
+        const float sigma = w.params[KernelTraits<KT>::SIGMA * a.params_s];
+        float down[GE];
+#pragma unroll
+        for (int g = 0; g < GE; g++) {
+            down[g] = __builtin_ldexpf(sigma, -shift[g % G] - KM_F16_KSCALE_LOG2);
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            grid_store<KT, G>(a, w, kc, xr[r], gw.x_ref, acc[r], down, base + 16 * r, kbase);
+        }
+    }
+}
+
+// rhs column groups (of 16) that one pass takes, and the grid form's largest window.
+template <int KT, int G>
+struct GridShape {
+    static constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
+    static constexpr int GP = G * PARTS > 4 ? 4 / PARTS : G;
+    static constexpr int GE = GP * PARTS;
+    static constexpr int MT = GE >= 4 ? 4 : 5;
+};
+
+// One item by W wavefronts (this one is number `wave`): the grid form, or entry by entry.
+template <int KT, int G, int W>
+__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int wave) {
+    using S = GridShape<KT, G>;
+    int unused;
+    const WaveView w = wave_view<true>(a, item, 1, &unused);
+    const int row0 = w.row_block * KM_BLOCK_SIZE;
+    // The rows are requested first, then the first columns (which wait for the range), then the
+    // window is computed.
+    const BlockRows rows = block_rows(w.x1, a.x1_s, row0, a.m);
+    KernelConsts kc = make_consts<KT>(w.params, a.params_s, false);
+    kc.s = uniform(kc.s);
+    __builtin_amdgcn_sched_barrier(0);
+    float xv[KM_GRID_CHUNK / 64];
+    if (w.range_start + 32 * wave < w.range_end) {
+        grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
+    }
+    const GridWindow gw = grid_window<S::MT>(rows, kc);
+    // (the same in every lane, and said so: the barriers inside depend on it)
+    bool grid = __builtin_amdgcn_readfirstlane(gw.ok && w.range_end - w.range_start >= KM_GRID_MIN_WIDTH) != 0;
+#pragma unroll 1
+    for (int pass = 0; pass < G / S::GP; pass++) {
+        const int kbase = (blockIdx.y * G + pass * S::GP) * 16;
+        if (kbase < a.k) {
+            if (pass > 0 && w.range_start + 32 * wave < w.range_end) {
+                grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
+            }
+            grid = grid && grid_forward<KT, S::GP, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv);
+            if (!grid) {
+                grid_entrywise<KT, S::GP, W>(a, lds, w, row0, kbase, wave, gw, kc);
+            }
+        }
+    }
+}
+
+template <int KT, int G, int W>
+__global__ void __launch_bounds__(64 * W, (GridShape<KT, G>::GE >= 4 ? 2 : 3)) fwd_grid(const FwdArgs a) {
+    extern __shared__ float lds[];
+    const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
+    if (item >= a.total_items) {
+        return;
+    }
+    grid_item<KT, G, W>(a, lds, item, W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+}
+
+// Large launches: workgroups of four wavefronts.  The first items of every XCD go one per wavefront;
+// its last `tail_items` are dispatched last, one per workgroup, so that these quarter-length pieces
+// fill the SIMDs that would otherwise idle while others finish a last full item.
+template <int KT, int G>
+__global__ void __launch_bounds__(256, (GridShape<KT, G>::GE >= 4 ? 2 : 3)) fwd_grid_grouped(const FwdArgs a) {
+    extern __shared__ float lds[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned xcd = blockIdx.x % KM_NUM_XCD;
+    const long long slot = blockIdx.x / KM_NUM_XCD;
+    const long long main_items = a.items_per_xcd - a.tail_items;
+    const long long main_groups = (main_items + 3) / 4;
+    const bool split = slot >= main_groups;
+    const long long local = split ? main_items + (slot - main_groups) : slot * 4 + wave;
+    const long long item = (long long)xcd * a.items_per_xcd + local;
+    if ((!split && local >= main_items) || item >= a.total_items) {
+        return;  // (uniform for the workgroup of a split item)
+    }
+    if (split) {
+        grid_item<KT, G, 4>(a, lds, item, wave);
+    } else {
+        grid_item<KT, G, 1>(a, lds + wave * KM_GRID_TABLE_FLOATS, item, 0);
+    }
+}
+
+template <int KT, int G, int W>
+static hipError_t launch_grid_as(const FwdArgs& a, dim3 grid, hipStream_t stream) {
+    using S = GridShape<KT, G>;
+    hipLaunchKernelGGL((fwd_grid<KT, G, W>), grid, dim3(64 * W, 1, 1),
+                       (sizeof(float) * grid_lds_floats<S::GE, S::MT, W>()), stream, a);
+    return hipGetLastError();
+}
+
+template <int KT, int G>
+static hipError_t launch_grid_w(const FwdArgs& a, int waves, dim3 grid, hipStream_t stream) {
+    if (a.tail_items > 0) {
+        using S = GridShape<KT, G>;
+        const long long main_groups = (a.items_per_xcd - a.tail_items + 3) / 4;
+        grid.x = (unsigned)((main_groups + a.tail_items) * KM_NUM_XCD);
+        hipLaunchKernelGGL((fwd_grid_grouped<KT, G>), grid, dim3(256, 1, 1),
+                           (sizeof(float) * grid_lds_floats<S::GE, S::MT, 4>()), stream, a);
+        return hipGetLastError();
+    }
+    switch (waves) {
+        case 1: return launch_grid_as<KT, G, 1>(a, grid, stream);
+        case 2: return launch_grid_as<KT, G, 2>(a, grid, stream);
+        case 4: return launch_grid_as<KT, G, 4>(a, grid, stream);
+        default: return launch_grid_as<KT, G, 8>(a, grid, stream);
+    }
+}
+
+template <int KT>
+static hipError_t launch_grid_g(const FwdArgs& a, int G, int waves, dim3 grid, hipStream_t stream) {
+    switch (G) {
+        case 1: return launch_grid_w<KT, 1>(a, waves, grid, stream);
+        case 2: return launch_grid_w<KT, 2>(a, waves, grid, stream);
+        default: return launch_grid_w<KT, 4>(a, waves, grid, stream);
+    }
+}
+
+hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream) {
+    FwdArgs a;
+    fill_fwd_args(p, &a);
+    const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
+    a.chunks_per_block = 1;
+    a.total_items = row_blocks * p.num_batches;
+    a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
+    a.tail_items = (int)(plan.group_tail < 0 ? 0 : (plan.group_tail < a.items_per_xcd ? plan.group_tail : a.items_per_xcd));
+    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD), (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk), 1);
+    if (p.kernel_type == KM_KERNEL_SPECTRAL) {
+        return launch_grid_g<KM_KERNEL_SPECTRAL>(a, plan.k_chunk / 16, plan.col_splits, grid, stream);
+    }
+    return launch_grid_g<KM_KERNEL_RBF>(a, plan.k_chunk / 16, plan.col_splits, grid, stream);
+}
+
+}  // namespace km

@@ -1322,6 +1322,9 @@ hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStre
     if (plan.variant == KM_VARIANT_BLOCK) {
         return launch_matmul_block(p, plan, stream);
     }
+    if (plan.variant == KM_VARIANT_GRID) {
+        return launch_matmul_grid(p, plan, stream);
+    }
     FwdArgs a;
     fill_fwd_args(p, &a);
 

@@ -1,0 +1,181 @@
+"""The grid form of the forward operator (a Gaussian as a sum over an equidistant grid) at the places
+where it can go wrong: windows of every size up to the largest and beyond, ranges that end anywhere,
+row blocks and ranges that are cut off, gaps in the data, points next to the origin and unsorted
+ones, every number of wavefronts per item, rhs widths on both sides of its groups.
+
+Tolerance per element, against float64: 3e-6 (|envelope| @ |rhs|) + 2^-36 sigma sum |rhs|.  An entry is a
+sum of products of two factors; each is rounded by its exponent (|exponent| < 16: two roundings of
+half an fp32 ulp, 6.6e-7 together), the hardware exponential (1.2e-7) and its split into two fp16
+values (2^-22), i.e. 1e-6 each; the trapezoid rule adds 6e-8 and phases 3e-8 revolutions each.  The
+floor is what both factors drop below 2^-37."""
+import numpy as np
+import pytest
+import torch
+
+from kernel_matmul_amd.compile import load_native
+from kernel_matmul_amd.configurations import MatmulSingleConfiguration
+from oracle import kernels as oracle
+
+pytestmark = pytest.mark.gpu
+
+DEVICE = torch.device("cuda:0")
+
+
+def _run(kt, x1, x2, rhs, params, start, end, rows=None, tail=None):
+    args = tuple(t.to(DEVICE) for t in (x1, x2, rhs, params, start, end))
+    defines = MatmulSingleConfiguration(kt).make_config(args)
+    defines["MATMUL_VARIANT"] = "grid"
+    if rows:
+        defines["MATMUL_ROWS_PER_WAVE"] = rows
+    if tail is not None:
+        defines["MATMUL_GROUP_TAIL"] = tail
+    op = load_native("matmul", defines)
+    out = op.call(*args)
+    assert torch.equal(out, op.call(*args))  # sums in a fixed order
+    return out.cpu().double().numpy()
+
+
+def _check(kt, x1, x2, rhs, params, start, end, **launch):
+    out = _run(kt, x1, x2, rhs, params, start, end, **launch)
+    a = [t.numpy() for t in (x1, x2, rhs, params, start, end)]
+    expected = oracle.matmul(kt, a[0], a[1], a[2], a[3], a[4], a[5])
+    envelope = np.abs(oracle.dense("rbf", a[0], a[1], a[3][..., [0, -1]], a[4], a[5]))
+    mask = oracle.range_mask(a[4], a[5], x1.shape[-1], x2.shape[-1]).astype(np.float64)
+    size = np.abs(a[2].astype(np.float64))
+    tol = 3e-6 * (envelope @ size) + 2.0 ** -36 * np.abs(a[3][..., -1, None, None]) * (mask @ size) + 1e-30
+    err = np.abs(out - expected)
+    assert np.all(err <= tol), float((err / tol).max())
+
+
+def _params(kt, lengthscale):
+    ls = torch.as_tensor(lengthscale, dtype=torch.float32)
+    f, s = torch.full_like(ls, 0.31), torch.full_like(ls, 1.3)
+    return torch.stack([ls, f, s] if kt == "spectral" else [ls, s], dim=-1)
+
+
+def _ranges(m, n, width, seed=0):
+    """Ranges around the block's position that start and end anywhere."""
+    g = torch.Generator().manual_seed(seed)
+    rows = (m + 127) // 128
+    mid = (torch.arange(rows) * 128 + 64) * n // max(m, 1)
+    lo = mid - width // 2 - torch.randint(0, 40, (rows,), generator=g)
+    hi = mid + width // 2 + torch.randint(0, 40, (rows,), generator=g)
+    return lo.clamp(0, n).int(), hi.clamp(0, n).int()
+
+
+def _points(n, extent, seed, batch=()):
+    g = torch.Generator().manual_seed(seed)
+    return torch.sort(torch.rand(*batch, n, generator=g) * extent, dim=-1)[0]
+
+
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("kt,k", [("spectral", 1), ("spectral", 16), ("spectral", 17), ("spectral", 33), ("spectral", 70),
+                                  ("rbf", 3), ("rbf", 17), ("rbf", 64), ("rbf", 65)])
+def test_rhs_widths_and_wavefronts(kt, k, rows):
+    n = 1000
+    x = _points(n, n / 10.0, 1).expand(2, n)
+    rhs = torch.randn(2, n, k, generator=torch.Generator().manual_seed(2))
+    start, end = (t.expand(2, -1) for t in _ranges(n, n, 500))
+    _check(kt, x, x, rhs, _params(kt, [1.0, 0.6]), start, end, rows=rows)
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("lengthscale", [0.1, 0.25, 0.3, 0.36, 0.45, 0.6, 0.9, 2.0, 30.0, 1e4])
+def test_window_sizes(kt, lengthscale):
+    """Ten points per unit: a 128-row block spans 12.8 / lengthscale lengthscales, windows of two to
+    five tiles of the grid, and row blocks it does not fit (evaluated entry by entry), mixed."""
+    n = 1300
+    x = _points(n, n / 10.0, 3)
+    rhs = torch.randn(n, 5, generator=torch.Generator().manual_seed(4))
+    start, end = _ranges(n, n, 600)
+    _check(kt, x, x, rhs, _params(kt, lengthscale), start, end)
+
+
+@pytest.mark.parametrize("m,n", [(1, 400), (129, 161), (128, 159), (255, 160), (300, 1), (640, 257)])
+@pytest.mark.parametrize("rows", [32, 128])
+def test_cut_off_blocks_and_ranges(m, n, rows):
+    """Rectangular matrices, last row blocks of one row, ranges on both sides of the width from
+    which the form is taken (160), empty ranges and ranges beyond the matrix."""
+    x1, x2 = _points(m, 20.0, 5), _points(n, 20.0, 6)
+    blocks = (m + 127) // 128
+    start = torch.zeros(blocks, dtype=torch.int32)
+    end = torch.full((blocks,), n, dtype=torch.int32)
+    end[-1] = min(n, 37) if blocks > 1 else n
+    if blocks > 2:
+        start[0] = end[0]
+    rhs = torch.randn(n, 16, generator=torch.Generator().manual_seed(7))
+    _check("spectral", x1, x2, rhs, _params("spectral", 1.5), start, end, rows=rows)
+
+
+@pytest.mark.parametrize("kind", ["gaps", "origin", "negative", "far", "unsorted", "equal"])
+@pytest.mark.parametrize("rows", [32, 128])
+def test_coordinates(kind, rows):
+    n = 900
+    x = _points(n, 30.0, 8)
+    if kind == "gaps":      # groups of neighbouring columns on both sides of gaps of every size
+        x = x + torch.cumsum((torch.arange(n) % 97 == 5).float() * torch.linspace(0.5, 12.0, n), dim=0)
+    elif kind == "origin":
+        x = x * 0.3 - 2.0
+    elif kind == "negative":
+        x = x - 500.0
+    elif kind == "far":
+        x = x + 30000.0     # ulp 2^-9
+    elif kind == "unsorted":
+        x = x[torch.randperm(n, generator=torch.Generator().manual_seed(9))]
+    else:
+        x = torch.full((n,), 3.25)
+    rhs = torch.randn(n, 4, generator=torch.Generator().manual_seed(10))
+    start, end = _ranges(n, n, 700)
+    for kt in ("spectral", "rbf"):
+        _check(kt, x, x, rhs, _params(kt, 1.1), start, end, rows=rows)
+
+
+@pytest.mark.parametrize("tail", [1, 3, 16])
+def test_split_tail(tail):
+    """The last items of every XCD split between four wavefronts, the rest one per wavefront."""
+    n, batch = 128 * 24 + 5, 3
+    x = _points(n, n / 10.0, 11).expand(batch, n)
+    rhs = torch.randn(batch, n, 16, generator=torch.Generator().manual_seed(12))
+    start, end = (t.expand(batch, -1) for t in _ranges(n, n, 400))
+    _check("spectral", x, x, rhs, _params("spectral", [0.2, 0.8, 1.7]), start, end, rows=128, tail=tail)
+
+
+@pytest.mark.parametrize("rows", [32, 128])
+def test_values_that_are_not_finite(rows):
+    """A NaN or an infinity in the coordinates or in rhs reaches the rows whose reach it is in, as in
+    the entry-wise kernels, and no others."""
+    n = 1024
+    x = _points(n, n / 10.0, 13)
+    rhs = torch.randn(n, 2, generator=torch.Generator().manual_seed(14))
+    start, end = _ranges(n, n, 400)
+    params = _params("rbf", 1.0)
+    clean = _run("rbf", x, x, rhs, params, start, end, rows=rows)
+    bad = rhs.clone()
+    bad[500, 1] = float("nan")
+    out = _run_nan("rbf", x, x, bad, params, start, end, rows)
+    near = (x - x[500]).abs() < 4.0
+    assert np.all(np.isnan(out[near.numpy(), 1]))
+    assert np.array_equal(out[:, 0], clean[:, 0]) or np.allclose(out[:, 0], clean[:, 0], rtol=1e-5, atol=1e-5)
+    far = np.array([not (start[i // 128] <= 500 < end[i // 128]) for i in range(n)])
+    assert np.all(np.isfinite(out[far]))
+    moved = x.clone()
+    moved[500] = float("nan")
+    out = _run_nan("rbf", moved, x, rhs, params, start, end, rows)
+    assert np.all(np.isnan(out[500])) and np.all(np.isfinite(np.delete(out, 500, axis=0)))
+
+
+def _run_nan(kt, x1, x2, rhs, params, start, end, rows):
+    args = tuple(t.to(DEVICE) for t in (x1, x2, rhs, params, start, end))
+    defines = MatmulSingleConfiguration(kt).make_config(args)
+    defines["MATMUL_VARIANT"], defines["MATMUL_ROWS_PER_WAVE"] = "grid", rows
+    return load_native("matmul", defines).call(*args).cpu().double().numpy()
+
+
+def test_variant_is_refused_for_other_kernels():
+    x = _points(300, 30.0, 15).to(DEVICE)
+    start, end = (t.to(DEVICE) for t in _ranges(300, 300, 200))
+    args = (x, x, torch.randn(300, 2, device=DEVICE), torch.ones(4, device=DEVICE), start, end)
+    defines = MatmulSingleConfiguration("locally_periodic").make_config(args)
+    defines["MATMUL_VARIANT"] = "grid"
+    with pytest.raises(RuntimeError, match="grid form"):
+        load_native("matmul", defines).call(*args)
