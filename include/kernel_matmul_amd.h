@@ -143,7 +143,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                        const km_launch_options* options, char* text, size_t text_bytes);
 
 /* Which kernels and decomposition km_param_grad would pick for contiguous operands of this
- * size (host only; nothing is launched): the feature form or the pairwise form, and the number
+ * size (host only; nothing is launched): the grid, feature or pairwise form, and the number
  * of column shares per row block.  Like km_matmul_describe, it stands in for the reference's
  * autotune report (kernel_matmul/native_function.py:56-69). */
 int km_param_grad_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t c, char* text,

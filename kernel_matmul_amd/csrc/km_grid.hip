@@ -23,276 +23,8 @@ namespace km {
 // Columns in a row block's range from which the grid form is taken.
 #define KM_GRID_MIN_WIDTH 160
 
-// This lane's part of a step's rhs operand: byte offsets of its 8 columns' first row (8 kk) and of its
-// rhs column in each group.  Inner strides are at most 2^22 elements (the entry point checks), so a
-// step spans less than 2^32 bytes and its row offsets come from 24-bit multiplications.
-template <int G>
-struct RhsLane {
-    unsigned row;
-    unsigned col[G];
-    bool used[G];
-};
-
-// rhs values of a step (columns c0 + 8 kk + t), zero past the end of the range.
-template <int G>
-__device__ __forceinline__ void grid_rhs(const FwdArgs& a, const float* __restrict__ rhs, int c0, int col_end,
-                                         int kk, const RhsLane<G>& lane, float (&raw)[G][8]) {
-    const buffer_rsrc ru = uniform_buffer(rhs + (long long)c0 * a.rhs_s0);
-    const unsigned s0 = (unsigned)a.rhs_s0;
-    if (c0 + 32 <= col_end) {
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                raw[g][t] = buffer_at(ru, lane.row + lane.col[g], 4u * (unsigned)t * s0);
-            }
-        }
-    } else {
-        const int last = col_end - 1 - c0;
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const int rel = 8 * kk + t;
-            const unsigned row = 4u * __umul24((unsigned)min(rel, last), s0);
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-                const float v = buffer_at(ru, row + lane.col[g], 0u);
-                raw[g][t] = rel <= last ? v : 0.0f;
-            }
-        }
-    }
-}
-
-// The Gaussian factor of a row against two neighbouring columns, split into fp16 halves, times
-// 2^KM_F16_KSCALE_LOG2.  (The power of two is applied to the rounded halves, exactly, and in the
-// residual: inside the exponent it would cost it four bits.)
-__device__ __forceinline__ void entry_pair_f16(float x, float ya, float yb, float scale, half2v* hi, half2v* lo) {
-    constexpr float S = (float)(1 << KM_F16_KSCALE_LOG2);
-    const float ua = (x - ya) * scale, ub = (x - yb) * scale;
-    const float ea = __builtin_amdgcn_exp2f(-ua * ua);
-    const float eb = __builtin_amdgcn_exp2f(-ub * ub);
-    const float2v kv = {ea, eb};
-    const half2v h = __builtin_convertvector(kv, half2v) * (half2v){(_Float16)S, (_Float16)S};
-    *hi = h;
-    *lo = residual_f16x2(ea, S, eb, S, h);
-}
-
-// Two powers of two split into fp16 halves.
-__device__ __forceinline__ void exp2_pair_f16(float a, float b, float one, half2v* hi, half2v* lo) {
-    const float2v kv = {__builtin_amdgcn_exp2f(a), __builtin_amdgcn_exp2f(b)};
-    const half2v h = __builtin_convertvector(kv, half2v);
-    *hi = h;
-    *lo = residual_f16x2(kv[0], one, kv[1], one, h);
-}
-
-// One step of 32 columns: scale and split the rhs operand, then for every tile of 16 points in
-// reach evaluate, split and contract.  GRID: the points are the grid's, t0 + 16 mt h; else the rows xr[].
-template <bool GRID, int G, int PARTS, int MT>
-__device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off, const float (&raw)[G][8],
-                                          const GridWindow& gw, float t0, const float* xr, const KernelConsts& kc,
-                                          int tiles, bool wide, const bool (&colmask)[G], int (&shift)[G], float (&scale)[G],
-                                          bool* rhs_finite, float4v (&acc)[MT][G * PARTS]) {
-    constexpr int CH = KM_GRID_CHUNK;
-    constexpr int GE = G * PARTS;
-    float xv[8], cb[8], sb[8];
-#pragma unroll
-    for (int t = 0; t < 8; t += 4) {
-        const float4v vx = *(const float4v*)(tab + off + t);
-        const float4v vc = *(const float4v*)(tab + CH + off + t);
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            xv[t + u] = vx[u];
-            cb[t + u] = vc[u];
-        }
-        if (PARTS == 2) {
-            const float4v vs = *(const float4v*)(tab + 2 * CH + off + t);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                sb[t + u] = vs[u];
-            }
-        }
-    }
-    const float ref = tab[3 * CH + (off >> 3)];
-    const float span = tab[3 * CH + CH / 8 + (off >> 3)];
-
-    half8v bhi[GE], blo[GE];
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        // The column's running power-of-two scale, as in f16_step.
-        float m = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            m = fmaxf(m, fabsf(raw[g][t]));
-        }
-        m = column_max(m);
-        const bool grow = colmask[g] && !(m * scale[g] < 32768.0f);
-        if (__any(grow)) {
-            *rhs_finite = *rhs_finite && !__any(grow && !(m < __builtin_inff()));
-            if (grow) {
-                const int e = __builtin_amdgcn_frexp_expf(m);
-                const int new_shift = min(max(14 - e, -100), 100);
-                const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-                    for (int part = 0; part < PARTS; part++) {
-                        acc[mt][part * G + g] *= factor;
-                    }
-                }
-                shift[g] = new_shift;
-                scale[g] = __builtin_ldexpf(1.0f, new_shift);
-            }
-        }
-        float vc[8];
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            vc[t] = raw[g][t] * scale[g];
-        }
-        if (PARTS == 2) {
-            float vs[8];
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                vs[t] = vc[t] * sb[t];
-            }
-            split_f16x8(vs, kc.one, &bhi[G + g], &blo[G + g]);
-        }
-        if (PARTS == 2 || GRID) {
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                vc[t] *= cb[t];
-            }
-        }
-        split_f16x8(vc, kc.one, &bhi[g], &blo[g]);
-    }
-
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        if (mt >= tiles) {
-            break;
-        }
-        const float t = GRID ? __builtin_fmaf((float)(16 * mt), gw.h, t0) : xr[mt];
-        const float av = (t - ref) * (GRID ? gw.s2 : kc.s);
-        if (!__any(!(fabsf(av) - span > KM_GRID_REACH))) {
-            continue;
-        }
-        half2v h2[4], l2[4];
-        float arg[8];
-        if (GRID) {
-            if (!wide) {
-                const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    arg[u] = __builtin_fmaf(av, xv[u], rb);
-                }
-            } else {
-#pragma unroll
-                for (int u = 0; u < 8; u++) {
-                    const float z = __builtin_fmaf(-0.5f, xv[u], av);
-                    arg[u] = __builtin_fmaf(-z, z, (float)KM_GRID_KS1);
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (GRID) {
-                exp2_pair_f16(arg[2 * u], arg[2 * u + 1], kc.one, &h2[u], &l2[u]);
-            } else {
-                entry_pair_f16(t, xv[2 * u], xv[2 * u + 1], kc.s, &h2[u], &l2[u]);
-            }
-        }
-        const half8v ahi = join_half2x4(h2);
-        const half8v alo = join_half2x4(l2);
-#pragma unroll
-        for (int g = 0; g < GE; g++) {
-            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[g], acc[mt][g], 0, 0, 0);
-            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[g], acc[mt][g], 0, 0, 0);
-            acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[g], acc[mt][g], 0, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
-}
-
-// The columns of [w.range_start, w.range_end) against `tiles` groups of 16 points (GRID: of the
-// grid window; else the rows xr[]): acc in the D layout times 2^shift (per rhs column) and the scale
-// of the evaluated factor.  The wavefront takes every W-th step of 32 columns from step `wave` on.
-// Returns false if a value was met that the form cannot take (GRID; see grid_table).
-// A step's rhs values are requested a step ahead (a step is short: two or three tiles), a chunk's
-// coordinates a chunk ahead (the first chunk's, in xv, by the caller).
-template <bool GRID, int KT, int G, int MT, int W>
-__device__ __forceinline__ bool grid_columns(const FwdArgs& a, float* __restrict__ tab, const WaveView& w, int kbase,
-                                             int wave, const GridWindow& gw, const KernelConsts& kc, const float* xr,
-                                             int tiles, float (&xv)[KM_GRID_CHUNK / 64], int (&shift)[G],
-                                             float4v (&acc)[MT][G * (KT == KM_KERNEL_SPECTRAL ? 2 : 1)]) {
-    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
-    constexpr int PARTS = PHASE ? 2 : 1;
-    constexpr int CH = KM_GRID_CHUNK;
-    const int lane = threadIdx.x & 63;
-    const int li = lane & 15;
-    const int kk = lane >> 4;
-    const float* __restrict__ rhs = w.rhs + (long long)kbase * a.rhs_s1;
-    RhsLane<G> rl;
-    float scale[G];
-    rl.row = 4u * __umul24(8u * (unsigned)kk, (unsigned)a.rhs_s0);
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const int c = kbase + 16 * g + li;
-        rl.col[g] = 4u * __umul24((unsigned)(min(c, a.k - 1) - kbase), (unsigned)a.rhs_s1);
-        rl.used[g] = c < a.k;
-        shift[g] = 100;
-        scale[g] = c < a.k ? __builtin_ldexpf(1.0f, 100) : 0.0f;
-    }
-#pragma unroll
-    for (int m = 0; m < MT; m++) {
-#pragma unroll
-        for (int g = 0; g < G * PARTS; g++) {
-            acc[m][g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    }
-    const float t0 = (gw.g_lo + (float)li) * gw.h;
-    bool fine = true;
-    for (int first = w.range_start + 32 * wave; first < w.range_end; first += CH * W) {
-        const unsigned steps = grid_table<GRID, PHASE>(xv, first, W, w.range_end, gw, kc, tab, &fine);
-        if (first + CH * W < w.range_end) {
-            grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
-        }
-        unsigned need = steps & 0xffff;
-        if (need == 0) {
-            continue;
-        }
-        float next[G][8];
-        int j = __builtin_ctz(need);
-        grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
-        do {
-            float raw[G][8];
-#pragma unroll
-            for (int g = 0; g < G; g++) {
-#pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    raw[g][t] = next[g][t];
-                }
-            }
-            const int off = 32 * j + 8 * kk;
-            const bool wide = (steps >> (16 + j) & 1) != 0;
-            need &= need - 1;
-            if (need != 0) {
-                j = __builtin_ctz(need);
-                grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
-            }
-            // (kept as register quadruples: read element by element below, the accumulators are split
-            // up and put together again in every step otherwise)
-#pragma unroll
-            for (int m = 0; m < MT; m++) {
-#pragma unroll
-                for (int g = 0; g < G * PARTS; g++) {
-                    asm volatile("" : "+v"(acc[m][g]));
-                }
-            }
-            grid_step<GRID, G, PARTS, MT>(tab, off, raw, gw, t0, xr, kc, tiles, wide, rl.used, shift, scale, &fine, acc);
-        } while (need != 0);
-        // All reads of the table are done before the next chunk overwrites it.
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    return fine;
+__device__ __forceinline__ GridVectors vectors(const FwdArgs& a) {
+    return {a.x2_s, a.rhs_s0, a.rhs_s1, a.k};
 }
 
 // A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the
@@ -356,7 +88,7 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
 
     int shift[G];
     float4v acc[MT][GE];
-    bool fine = grid_columns<true, KT, G, MT, W>(a, lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, wave, gw, kc, nullptr,
+    bool fine = grid_columns<true, KT, G, MT, W>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, wave, gw, kc, nullptr,
                                                  gw.tiles, xv, shift, acc);
 
     // The sums of all W wavefronts, added in their order.
@@ -541,7 +273,7 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         }
         int shift[G];
         float4v acc[R][GE];
-        grid_columns<false, KT, G, R, 1>(a, lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr, R, xv, shift, acc);
+        grid_columns<false, KT, G, R, 1>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr, R, xv, shift, acc);
         const float sigma = w.params[KernelTraits<KT>::SIGMA * a.params_s];
         float down[GE];
 #pragma unroll

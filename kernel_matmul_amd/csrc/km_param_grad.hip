@@ -3,11 +3,13 @@
 // native/matmul_bwd/matmul_bwd.cu:12-221) and bilinear_derivative
 // (native/bilinear_derivative/bilinear_derivative.cu:12-183), which compute the same sum.
 //
-// Pass 1 has two forms.  Feature form (param_grad_features, rbf and spectral kernels with
-// narrow vectors; described at the kernel): the sums are polynomials in the rows' coordinate
-// times contractions of the Gaussian factor with a handful of column features, computed like
-// the forward table kernel.  Pairwise form (param_grad_partial, every kernel; also the
-// per-item fallback of the feature form): a wavefront owns 128 rows and a share of the row
+// Pass 1 has three forms.  Grid form (param_grad_grid, rbf and spectral kernels; described at the
+// kernel): columns and rows are contracted onto an equidistant grid, the sums are dot products over
+// it.  Feature form (param_grad_features, the same kernels with narrow vectors where batch shape or
+// strides do not suit the grid form's short addressing): the sums are polynomials in the rows'
+// coordinate times contractions of the Gaussian factor with a handful of column features, computed
+// like the forward table kernel.  Pairwise form (param_grad_partial, every kernel; also the
+// per-item fallback of the other two): a wavefront owns 128 rows and a share of the row
 // block's column range.  Per 16-column chunk and 16-row group the coefficient tile C (16x16) is
 // formed on the matrix pipe from left/right (v_mfma_f32_16x16x4_f32 over the vector
 // columns); its D layout gives each lane 4 (row, col) pairs, for which the lane evaluates
@@ -21,6 +23,7 @@
 #include "km_batch.h"
 #include "km_common.h"
 #include "km_fwd.h"
+#include "km_grid.h"
 #include "km_launch.h"
 
 namespace km {
@@ -62,7 +65,12 @@ struct GradArgs {
 // column share is a third of the wavefront's issue time (48 row operands against three chunks).
 #define KM_GRAD_FAST_STRIDE (1 << 21)
 
-template <int KT, int TL, int R, bool FAST = false>
+//
+// SKIP (rows sparse against the lengthscale): tiles of 16 rows by 16 columns whose entries are all
+// beyond the reach of the Gaussian (below 2^-37 of the largest, the floor of the other forms) are
+// left out.  One point per unit, lengthscales of half a unit to two: a third of the tiles remain
+// (n = 50000, batch 2, c = 8: 27.8 against 40.5 us without it, 32.7 us for the pairwise kernel).
+template <int KT, int TL, int R, bool FAST = false, bool SKIP = false>
 __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __restrict__ x1,
                                               const float* __restrict__ x2, const float* __restrict__ left,
                                               const float* __restrict__ right, const KernelConsts& kc,
@@ -163,6 +171,25 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
 
     float acc[KM_MAX_PARAMS] = {0.0f, 0.0f, 0.0f, 0.0f};
 
+    // Coordinates beyond which a column is out of the reach of a row group (everything is within
+    // reach of a group with a NaN).
+    float reach_lo[R], reach_hi[R];
+    if (SKIP) {
+        const float reach = KM_GRID_REACH / kc.s;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const bool nan = x1q[r][v] != x1q[r][v];
+                lo = fminf(lo, nan ? -__builtin_inff() : x1q[r][v]);
+                hi = fmaxf(hi, nan ? __builtin_inff() : x1q[r][v]);
+            }
+            reach_lo[r] = uniform(-column_max(-lo) - reach);
+            reach_hi[r] = uniform(column_max(hi) + reach);
+        }
+    }
+
     // Operands of a chunk of 16 columns: x2 of column n0 + li and, with the left operand in
     // registers, the right operand's values (column n0 + li, vector column 4 t + kk), zero outside
     // the range.  They are requested one chunk ahead.
@@ -231,6 +258,35 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
             load_chunk(n0 + 16, &x2_next, rv_next);
         }
 
+        if (SKIP) {
+            unsigned need = 0;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                need |= (unsigned)(__any(!(x2v < reach_lo[r] || x2v > reach_hi[r])) != 0) << r;
+            }
+            if (TL > 0 && need != (1u << R) - 1) {
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if ((need >> r & 1) == 0) {
+                        continue;
+                    }
+                    float4v c = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int t = 0; t < TLR; t++) {
+                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(lreg[r][t], rvs[t], c, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        accumulate_pair<KT>(x1q[r][v], x2v, c[v], kc, acc);
+                    }
+                }
+                continue;
+            }
+            if (need == 0) {
+                continue;
+            }
+        }
+
         float4v coef[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -285,6 +341,7 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
 struct GradItem {
     long long b, rest;
     int row0, col_begin, col_end;
+    int split, range_start;
     int width;  // columns of the row block's whole range (all shares)
     const float* x1;
     const float* x2;
@@ -359,6 +416,8 @@ __device__ __forceinline__ bool grad_item(const GradArgs& a, int rows_per_item, 
     // Column share of this wavefront, in whole steps of col_step columns.
     const int width = max(range_end - range_start, 0);
     g->width = width;
+    g->split = split;
+    g->range_start = range_start;
     const int per_split = ((width + a.col_splits - 1) / a.col_splits + col_step - 1) & ~(col_step - 1);
     g->col_begin = range_start + split * per_split;
     g->col_end = min(range_end, g->col_begin + per_split);
@@ -776,6 +835,268 @@ __global__ void __launch_bounds__(64, 2) param_grad_features(const GradArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Grid form of pass 1 (rbf and spectral kernels; the identity is described in km_grid.h).
+//
+// With p_ig = (x1_i - t_g) s2, q_jg = (x2_j - t_g) s2 and D = p - q, averaging over the position of
+// the grid leaves  D E = 2 C sum_g p V V  and  u^2 E = D^2 E / 2 = 2 C sum_g (p^2 - 1 / (4 ln 2)) V V,
+// so only the rows' factor carries a polynomial and nothing of the size of the window cancels.  With
+//     M_g  = sum_j V(x2_j, t_g) {cB, sB}_j right[j, c]                   (columns -> grid, as in the forward)
+//     La_g = sum_i V(x1_i, t_g) p^a {cA, sA}_i left[i, c], a = 0, 1 and p^2 - 1 / (4 ln 2) for a = 2
+// the sums are dot products over grid points and vector columns:
+//     sum C E cos     = C  sum L0c Mc + L0s Ms
+//     sum C E cos u^2 = 2C sum L2c Mc + L2s Ms
+//     sum C E sin d   = 2C / s2 sum L1s Mc - L1c Ms
+// (rbf: no phases, L0 and L2 only).  A column costs two or three tiles of 16 grid points instead of
+// eight of 16 rows, and the vectors' operands do not multiply with the number of features.
+//
+// The polynomial raises the trapezoid rule's error (its first harmonic meets k^2): the grid is a
+// little finer than the forward's, which leaves 1e-8.  Column shares: the moments of a share give
+// partial sums like those of any other split; every share repeats the rows' side, worth about nine
+// steps of 32 columns, so a share has at least KM_GG_SHARE columns and further wavefronts of a row
+// block write zeros.  Row blocks that the form does not suit (km_grid.hip) take the pairwise form.
+// Up to 8 spectral vector columns are packed with both phases into one group of 16 (PACK); more
+// than 16 take several passes.
+//
+// Measured: spectral n = 1e5, c = 4, 16 sets 273 -> 112 us (feature form before; bound by the VALU work
+// of exponentials and operand splits, about half of it on the columns' side); n = 7200 at 720 points
+// per unit, c = 11: 44.7 -> 20.7 us (pairwise before).
+// Resident wavefronts: three per SIMD; two with both phases in separate groups, whose operands would
+// spill 224 bytes a lane at three (29.2 against 23.0 us for the call).
+// ---------------------------------------------------------------------------------------
+#define KM_GG_STEP 0.58f
+#define KM_GG_MIN_WIDTH 96
+#define KM_GG_SHARE 256
+#define KM_GG_VARIANCE 0.36067376022224085f /* 1 / (4 ln 2): of the midpoint about the grid */
+
+// One pass of an item: the vector columns from kbase on (8 if PACK, else 16).  Adds to sums[]; false
+// if a value was met that the form cannot take (sums[] is then meaningless).
+template <int KT, bool PACK, int MT>
+__device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem& g, float* __restrict__ tab, int kbase,
+                                               const GridWindow& gw, const KernelConsts& kc, int col_begin, int col_end,
+                                               float (&sums)[3]) {
+    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
+    constexpr int GE = PHASE && !PACK ? 2 : 1;
+    constexpr int NP = PHASE ? 3 : 2;  // row factors: V, V (p^2 - variance), and V p
+    constexpr int CH = KM_GRID_CHUNK;
+    constexpr int STEPS = KM_BLOCK_SIZE / 32;
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    float xv[CH / 64];
+    grid_load(g.x2, a.x2_s, col_begin, 1, col_end, xv);
+    int shift[1];
+    float4v acc[MT][GE];
+    WaveView w;
+    w.x2 = g.x2;
+    w.rhs = g.right;
+    w.range_start = col_begin;
+    w.range_end = col_end;
+    const GridVectors right = {a.x2_s, a.right_s0, a.right_s1, a.c};
+    bool fine = grid_columns<true, KT, 1, MT, 1, PACK>(right, tab, w, kbase, 0, gw, kc, nullptr, gw.tiles, xv, shift, acc);
+
+    // The rows' operands: one power-of-two scale per vector column over the whole block.
+    const int row_end = min(g.row0 + KM_BLOCK_SIZE, a.m);
+    const GridVectors left = {a.x1_s, a.left_s0, a.left_s1, a.c};
+    const RhsLane<1> rl = rhs_lane<1, PACK>(left, kbase);
+    const float* lp = g.left + (long long)kbase * a.left_s1;
+    grid_load(g.x1, a.x1_s, g.row0, 1, row_end, xv);
+    float raw[STEPS][1][8];
+#pragma unroll
+    for (int j = 0; j < STEPS; j++) {
+        if (g.row0 + 32 * j < row_end) {
+            grid_rhs<1>(left, lp, g.row0 + 32 * j, row_end, kk, rl, raw[j]);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                raw[j][0][t] = 0.0f;
+            }
+        }
+    }
+    const unsigned steps = grid_table<true, PHASE>(xv, g.row0, 1, row_end, gw, kc, tab, &fine);
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < STEPS; j++) {
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            m = fmaxf(m, fabsf(raw[j][0][t]));
+        }
+    }
+    m = column_max(m);
+    fine = fine && __all(!rl.used[0] || m < __builtin_inff());
+    if (!fine) {
+        return false;
+    }
+    const int e = min(max(14 - __builtin_amdgcn_frexp_expf(m), -100), 100);
+    const float up = rl.used[0] ? __builtin_ldexpf(1.0f, e) : 0.0f;
+    half8v bhi[STEPS][GE], blo[STEPS][GE];
+#pragma unroll
+    for (int j = 0; j < STEPS; j++) {
+        if ((steps >> j & 1) == 0) {
+            continue;
+        }
+        const int off = 32 * j + 8 * kk;
+#pragma unroll
+        for (int part = 0; part < GE; part++) {
+            const float* weights = tab + (PACK && li >= 8 ? 2 * CH : CH * (1 + part)) + off;
+            const float4v w0 = *(const float4v*)weights;
+            const float4v w1 = *(const float4v*)(weights + 4);
+            float v[8];
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                v[t] = raw[j][0][t] * up * (t < 4 ? w0[t & 3] : w1[t & 3]);
+            }
+            split_f16x8(v, kc.one, &bhi[j][part], &blo[j][part]);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one operand at a time (registers)
+    }
+
+    const float t0 = (gw.g_lo + (float)li) * gw.h;
+    const float down_columns = __builtin_ldexpf(1.0f, -shift[0] - KM_GRID_KS1);
+    float s[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+        if (mt >= gw.tiles) {
+            break;
+        }
+        float4v rows[NP][GE];
+#pragma unroll
+        for (int p = 0; p < NP; p++) {
+#pragma unroll
+            for (int part = 0; part < GE; part++) {
+                rows[p][part] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+        const float t = __builtin_fmaf((float)(16 * mt), gw.h, t0);
+#pragma unroll
+        for (int j = 0; j < STEPS; j++) {
+            if ((steps >> j & 1) == 0) {
+                continue;
+            }
+            int off = 32 * j + 8 * kk;
+            asm volatile("" : "+v"(off));  // (read again for every tile, not kept over all of them: registers)
+            const float av = (t - tab[3 * CH + (off >> 3)]) * gw.s2;
+            if (!__any(!(fabsf(av) - tab[3 * CH + CH / 8 + (off >> 3)] > KM_GRID_REACH))) {
+                continue;
+            }
+            const float4v x0 = *(const float4v*)(tab + off);
+            const float4v x1 = *(const float4v*)(tab + off + 4);
+            const bool wide = (steps >> (16 + j) & 1) != 0;
+            const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
+            half2v hi[NP][4], lo[NP][4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float ev[2], pv[2], qv[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const float b2 = u < 2 ? x0[2 * (u & 1) + i] : x1[2 * (u & 1) + i];
+                    const float p = __builtin_fmaf(0.5f, b2, -av);
+                    ev[i] = __builtin_amdgcn_exp2f(wide ? __builtin_fmaf(-p, p, (float)KM_GRID_KS1)
+                                                        : __builtin_fmaf(av, b2, rb));
+                    pv[i] = p;
+                    qv[i] = __builtin_fmaf(p, p, -KM_GG_VARIANCE);
+                }
+                hi[0][u] = __builtin_convertvector((float2v){ev[0], ev[1]}, half2v);
+                lo[0][u] = residual_f16x2(ev[0], kc.one, ev[1], kc.one, hi[0][u]);
+                hi[1][u] = __builtin_convertvector((float2v){ev[0] * qv[0], ev[1] * qv[1]}, half2v);
+                lo[1][u] = residual_f16x2(ev[0], qv[0], ev[1], qv[1], hi[1][u]);
+                if (PHASE) {
+                    hi[NP - 1][u] = __builtin_convertvector((float2v){ev[0] * pv[0], ev[1] * pv[1]}, half2v);
+                    lo[NP - 1][u] = residual_f16x2(ev[0], pv[0], ev[1], pv[1], hi[NP - 1][u]);
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < NP; p++) {
+                const half8v ahi = join_half2x4(hi[p]);
+                const half8v alo = join_half2x4(lo[p]);
+#pragma unroll
+                for (int part = 0; part < GE; part++) {
+                    rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[j][part], rows[p][part], 0, 0, 0);
+                    rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[j][part], rows[p][part], 0, 0, 0);
+                    rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[j][part], rows[p][part], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // Both sides in the accumulators' layout: grid points 4 kk + v, vector column li (PACK: li & 7).
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            float mv[GE];
+#pragma unroll
+            for (int part = 0; part < GE; part++) {
+                mv[part] = acc[mt][part][v] * down_columns;
+                s[0] = __builtin_fmaf(rows[0][part][v], mv[part], s[0]);
+                s[1] = __builtin_fmaf(rows[1][part][v], mv[part], s[1]);
+            }
+            if (PACK) {
+                // the other phase of the same column sits eight lanes on (row_ror 8)
+                const float other = __uint_as_float(__builtin_amdgcn_update_dpp(
+                    __float_as_uint(mv[0]), __float_as_uint(mv[0]), 0x128, 0xf, 0xf, false));
+                s[2] = __builtin_fmaf(li >= 8 ? rows[NP - 1][0][v] : -rows[NP - 1][0][v], other, s[2]);
+            } else if (PHASE) {
+                s[2] = __builtin_fmaf(rows[NP - 1][GE - 1][v], mv[0], s[2]);
+                s[2] = __builtin_fmaf(-rows[NP - 1][0][v], mv[GE - 1], s[2]);
+            }
+        }
+    }
+    const float down_rows = __builtin_ldexpf(1.0f, -e - KM_GRID_KS1);
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+        sums[p] = __builtin_fmaf(s[p], down_rows, sums[p]);
+    }
+    // All reads of the table are done before the next pass overwrites it.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return true;
+}
+
+template <int KT, bool PACK, int TL>
+__global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3) param_grad_grid(const GradArgs a) {
+    static_assert(KT == KM_KERNEL_RBF || KT == KM_KERNEL_SPECTRAL, "grid form: rbf or spectral");
+    constexpr int MT = KT == KM_KERNEL_SPECTRAL && !PACK ? 5 : 6;
+    __shared__ float tab[KM_GRID_TABLE_FLOATS];
+    GradItem g;
+    if (!grad_item<true>(a, KM_BLOCK_SIZE, 16, &g)) {
+        return;
+    }
+    float* __restrict__ prow = a.partials + (g.b * a.partial_rows + g.rest) * KM_MAX_PARAMS;
+    const BlockRows rows = block_rows(g.x1, a.x1_s, g.row0, a.m);
+    KernelConsts kc = make_consts<KT>(g.params, a.params_s, false);
+    kc.s = uniform(kc.s);
+    const GridWindow gw = grid_window<MT>(rows, kc, KM_GG_STEP);
+    if (__builtin_amdgcn_readfirstlane(gw.ok && g.width >= KM_GG_MIN_WIDTH) != 0) {
+        // (fewer, longer shares than the pairwise form's: from the same split number)
+        const int shares = min(a.col_splits, max(g.width / KM_GG_SHARE, 1));
+        const int per_share = ((g.width + shares - 1) / shares + 31) & ~31;
+        const int range_end = g.range_start + g.width;
+        g.col_begin = g.split < shares ? g.range_start + g.split * per_share : range_end;
+        g.col_end = min(range_end, g.col_begin + per_share);
+        bool done = true;
+        float sums[3] = {0.0f, 0.0f, 0.0f};
+        if (g.col_begin < g.col_end) {
+            // (a loop for more than 16 vector columns only)
+#pragma unroll 1
+            for (int kbase = 0; done && kbase < (TL == 0 ? a.c : 1); kbase += 16) {
+                done = grid_grad_pass<KT, PACK, MT>(a, g, tab, kbase, gw, kc, g.col_begin, g.col_end, sums);
+            }
+        }
+        if (done) {
+            const float weight = gw.h * gw.s2 * KM_GRID_WEIGHT;
+            const float value = wave_sum(sums[0]) * weight;
+            const float squared = wave_sum(sums[1]) * (2.0f * weight);
+            const float slope = KT == KM_KERNEL_SPECTRAL ? wave_sum(sums[2]) * (2.0f * weight / gw.s2) : 0.0f;
+            if (threadIdx.x == 0) {
+                prow[0] = squared;
+                prow[1] = KT == KM_KERNEL_SPECTRAL ? slope : value;
+                prow[2] = KT == KM_KERNEL_SPECTRAL ? value : 0.0f;
+                prow[3] = 0.0f;
+            }
+            return;
+        }
+    }
+    pairwise_item<KT, TL, 8, true, true>(a, g.x1, g.x2, g.left, g.right, kc, g.row0, g.col_begin, g.col_end, prow);
+}
+
 struct ReduceArgs {
     BatchShape batch;
     long long partial_rows;
@@ -915,6 +1236,19 @@ void describe_param_grad(int kernel_type, int64_t m, long long num_batches, int6
     static const char* const kernels[] = {"rbf", "spectral", "locally_periodic"};
     const FeaturePlan f = feature_plan(kernel_type, c);
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
+    if (kernel_type != KM_KERNEL_LOCALLY_PERIODIC && c > 0) {
+        const int used = snprintf(text, text_bytes,
+                                  "km::param_grad_grid<%s%s, TL=%d> (grid form; per-item pairwise fallback), at most %d column "
+                                  "share(s) per row block; for strides or batch shapes that do not suit it: ",
+                                  kernels[kernel_type], kernel_type == KM_KERNEL_SPECTRAL && c <= 8 ? ", packed" : "",
+                                  c <= 4 ? 1 : (c <= 8 ? 2 : (c <= 16 ? 4 : 0)),
+                                  grad_col_splits(row_blocks * num_batches));
+        if (used < 0 || (size_t)used >= text_bytes) {
+            return;
+        }
+        text += used;
+        text_bytes -= (size_t)used;
+    }
     const int splits = grad_col_splits(row_blocks * num_batches, f.GE > 0);
     if (f.GE > 0) {
         snprintf(text, text_bytes,
@@ -979,6 +1313,35 @@ static hipError_t launch_partial_as(const GradArgs& a, unsigned grid_x, hipStrea
     return hipGetLastError();
 }
 
+// The grid form: rbf and spectral kernels under the conditions of the short addressing.
+static bool grid_form(int kernel_type, const GradArgs& a) {
+    return kernel_type != KM_KERNEL_LOCALLY_PERIODIC && pairwise_fast(a);
+}
+
+static hipError_t launch_grid(int kernel_type, const GradArgs& a, unsigned grid_x, hipStream_t stream) {
+    const dim3 grid(grid_x), block(64);
+    if (kernel_type == KM_KERNEL_SPECTRAL) {
+        if (a.c <= 4) {
+            hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_SPECTRAL, true, 1>), grid, block, 0, stream, a);
+        } else if (a.c <= 8) {
+            hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_SPECTRAL, true, 2>), grid, block, 0, stream, a);
+        } else if (a.c <= 16) {
+            hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_SPECTRAL, false, 4>), grid, block, 0, stream, a);
+        } else {
+            hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_SPECTRAL, false, 0>), grid, block, 0, stream, a);
+        }
+    } else if (a.c <= 4) {
+        hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_RBF, false, 1>), grid, block, 0, stream, a);
+    } else if (a.c <= 8) {
+        hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_RBF, false, 2>), grid, block, 0, stream, a);
+    } else if (a.c <= 16) {
+        hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_RBF, false, 4>), grid, block, 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((param_grad_grid<KM_KERNEL_RBF, false, 0>), grid, block, 0, stream, a);
+    }
+    return hipGetLastError();
+}
+
 template <int KT>
 static hipError_t launch_partial(const GradArgs& a, unsigned grid_x, hipStream_t stream) {
     return pairwise_fast(a) ? launch_partial_as<KT, true>(a, grid_x, stream)
@@ -1025,24 +1388,6 @@ hipError_t launch_param_grad(const ParamGradProblem& p, hipStream_t stream) {
     a.n = (int)p.n;
     a.c = (int)p.c;
     const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
-    // Feature form where it applies (its 32-bit lane offsets need moderate, non-negative strides
-    // of `right`); pairwise form otherwise.
-    FeaturePlan fplan = feature_plan(p.kernel_type, p.c);
-    {
-        const int64_t r0 = p.right_strides[r], r1 = p.right_strides[r + 1];
-        if (r0 < 0 || r1 < 0 || r0 > (1 << 24) || r1 > (1 << 24) || p.x2_strides[r] < 0 ||
-            p.x2_strides[r] > (1 << 24)) {
-            fplan.GE = 0;
-        }
-    }
-    long long chunks = row_blocks;
-    if (fplan.GE > 0) {
-        chunks = row_blocks * (8 / fplan.R);
-    }
-    a.col_splits = grad_col_splits(chunks * p.num_batches, fplan.GE > 0);
-    a.total_items = chunks * a.col_splits * p.num_batches;
-    a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    a.partial_rows = chunks * a.col_splits;
     {
         const BatchStrides* const all[7] = {&a.x1_bs, &a.x2_bs, &a.left_bs, &a.right_bs,
                                             &a.params_bs, &a.start_bs, &a.end_bs};
@@ -1068,8 +1413,36 @@ hipError_t launch_param_grad(const ParamGradProblem& p, hipStream_t stream) {
     a.start_s = p.start_strides[r];
     a.end_s = p.end_strides[r];
 
+    auto split_items = [&](bool feature_form) {
+        a.col_splits = grad_col_splits(row_blocks * p.num_batches, feature_form);
+        a.total_items = row_blocks * a.col_splits * p.num_batches;
+        a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
+        a.partial_rows = row_blocks * a.col_splits;
+    };
+    split_items(false);
+    const bool on_grid = grid_form(p.kernel_type, a);
+    // Grid form for batch shapes of one dimension and moderate strides; otherwise the feature form
+    // where it applies (its 32-bit lane offsets need moderate, non-negative strides
+    // of `right`); pairwise form otherwise.
+    FeaturePlan fplan = feature_plan(p.kernel_type, p.c);
+    {
+        const int64_t r0 = p.right_strides[r], r1 = p.right_strides[r + 1];
+        if (r0 < 0 || r1 < 0 || r0 > (1 << 24) || r1 > (1 << 24) || p.x2_strides[r] < 0 ||
+            p.x2_strides[r] > (1 << 24)) {
+            fplan.GE = 0;
+        }
+    }
+    if (!on_grid && fplan.GE > 0) {
+        split_items(true);
+    }
+
     const unsigned grid_x = (unsigned)(a.items_per_xcd * KM_NUM_XCD);
-    if (grid_x > 0 && fplan.GE > 0) {
+    if (grid_x > 0 && on_grid) {
+        const hipError_t err = launch_grid(p.kernel_type, a, grid_x, stream);
+        if (err != hipSuccess) {
+            return err;
+        }
+    } else if (grid_x > 0 && fplan.GE > 0) {
         const hipError_t err = launch_features(p.kernel_type, fplan, a, grid_x, stream);
         if (err != hipSuccess) {
             return err;
@@ -1086,7 +1459,7 @@ hipError_t launch_param_grad(const ParamGradProblem& p, hipStream_t stream) {
         }
     }
 
-    return launch_param_grad_reduce(p.kernel_type, a.batch, p.num_batches, chunks * a.col_splits,
+    return launch_param_grad_reduce(p.kernel_type, a.batch, p.num_batches, a.partial_rows,
                                     a.partials, p.params, a.params_bs, a.params_s, p.grad, stream);
 }
 

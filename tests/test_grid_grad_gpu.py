@@ -1,0 +1,154 @@
+"""The grid form of the hyper-parameter gradient at the places where it can go wrong: windows of
+every size up to the largest and beyond (pairwise), vector widths on both sides of its groups and
+passes, ranges and row blocks that are cut off, ranges on both sides of the least width and of a
+column share, gaps, unsorted and equal points, strides, scales and values that are not finite.
+
+Tolerance against float64, per parameter: 4e-6 sum |left| |right| times the size of the derivative's
+terms.  An entry is a sum over grid points of products of two factors, each 1e-6 exact (exponent,
+hardware exponential, split into two fp16 values, as in the forward), and the trapezoid rule at this
+spacing adds 4e-8.  The terms' size: the envelope E for the output scale, (u^2 + 2) E for the
+lengthscale (V V |p^2 - 1 / (4 ln 2)| averages to less) and (|d| + 2 l) E for the frequency.  What is
+dropped below 2^-37 is covered by a floor of 2^-34 on E within the range."""
+import numpy as np
+import pytest
+import torch
+
+from kernel_matmul_amd.compile import load_native
+from kernel_matmul_amd.configurations import BilinearDerivativeConfiguration
+from oracle import kernels as oracle
+
+pytestmark = pytest.mark.gpu
+
+DEVICE = torch.device("cuda:0")
+
+
+def _params(kt, lengthscale):
+    ls = torch.as_tensor(lengthscale, dtype=torch.float32)
+    f, s = torch.full_like(ls, 0.31), torch.full_like(ls, 1.3)
+    return torch.stack([ls, f, s] if kt == "spectral" else [ls, s], dim=-1)
+
+
+def _call(kt, *args):
+    op = load_native("bilinear_derivative", BilinearDerivativeConfiguration(kt).make_config(args))
+    result = op.call(*args)
+    assert torch.equal(result, op.call(*args))  # sums in a fixed order
+    return result.cpu().double().numpy()
+
+
+def _check(kt, x1, x2, left, right, params, start, end, transform=lambda t: t.to(DEVICE)):
+    result = _call(kt, *(transform(t) for t in (x1, x2, left, right, params, start, end)))
+    a = [t.numpy() for t in (x1, x2, left, right, params, start, end)]
+    expected = oracle.param_grad(kt, *a)
+    mask = oracle.range_mask(a[5], a[6], a[0].shape[-1], a[1].shape[-1])
+    d = a[0].astype(np.float64)[..., :, None] - a[1].astype(np.float64)[..., None, :]
+    p = a[4].astype(np.float64)
+    ls, sigma = (np.abs(p[..., i, None, None]) for i in (0, -1))
+    env = (np.exp(-0.5 * (d / ls) ** 2) + 2.0 ** -34) * mask
+    size = np.abs(a[2].astype(np.float64)) @ np.abs(np.swapaxes(a[3].astype(np.float64), -1, -2)) * env
+    u2 = 0.5 * (d / ls) ** 2 / np.log(2.0)
+    terms = [size * (u2 + 2.0) * sigma * 2.0 * np.log(2.0) / ls]
+    if kt == "spectral":
+        terms.append(size * (np.abs(d) + 2.0 * ls) * 2.0 * np.pi * sigma)
+    terms.append(size)
+    tol = 4e-6 * np.stack([t.sum((-2, -1)) for t in terms], axis=-1)
+    tol = tol + 1e-6 * np.abs(expected) + 1e-30
+    err = np.abs(result - expected)
+    assert np.all(err <= tol), (float((err / tol).max()), result, expected)
+
+
+def _points(n, extent, seed):
+    return torch.sort(torch.rand(n, generator=torch.Generator().manual_seed(seed)) * extent)[0]
+
+
+def _vectors(rows, c, seed, batch=()):
+    return torch.randn(*batch, rows, c, generator=torch.Generator().manual_seed(seed))
+
+
+def _ranges(m, n, width):
+    rows = (m + 127) // 128
+    g = torch.Generator().manual_seed(m + n + width)
+    mid = (torch.arange(rows) * 128 + 64) * n // max(m, 1)
+    lo = mid - width // 2 - torch.randint(0, 40, (rows,), generator=g)
+    hi = mid + width // 2 + torch.randint(0, 40, (rows,), generator=g)
+    return lo.clamp(0, n).int(), hi.clamp(0, n).int()
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("c", [1, 4, 5, 8, 9, 16, 17, 33])
+def test_vector_widths(kt, c):
+    n = 1000
+    x = _points(n, n / 10.0, 1).expand(2, n)
+    start, end = (t.expand(2, -1) for t in _ranges(n, n, 500))
+    right = _vectors(n, c, 2, (2,))
+    _check(kt, x, x, 0.5 * right + 0.1 * _vectors(n, c, 3, (2,)), right, _params(kt, [1.0, -0.6]), start, end)
+
+
+@pytest.mark.parametrize("kt,c", [("spectral", 3), ("spectral", 11), ("rbf", 6)])
+@pytest.mark.parametrize("lengthscale", [0.1, 0.25, 0.3, 0.36, 0.4, 0.45, 0.6, 0.9, 2.0, 30.0, 1e4])
+def test_window_sizes(kt, c, lengthscale):
+    n = 1300
+    x = _points(n, n / 10.0, 4)
+    start, end = _ranges(n, n, 600)
+    _check(kt, x, x, _vectors(n, c, 5), _vectors(n, c, 6), _params(kt, lengthscale), start, end)
+
+
+@pytest.mark.parametrize("m,n", [(1, 400), (129, 97), (128, 96), (128, 95), (255, 511), (300, 1), (640, 257), (130, 2100)])
+@pytest.mark.parametrize("c", [8, 12])
+def test_cut_off_blocks_and_ranges(m, n, c):
+    x1, x2 = _points(m, 20.0, 7), _points(n, 20.0, 8)
+    blocks = (m + 127) // 128
+    start = torch.zeros(blocks, dtype=torch.int32)
+    end = torch.full((blocks,), n, dtype=torch.int32)
+    end[-1] = min(n, 137) if blocks > 1 else n
+    if blocks > 2:
+        start[0] = end[0]
+    _check("spectral", x1, x2, _vectors(m, c, 9), _vectors(n, c, 10), _params("spectral", 1.5), start, end)
+
+
+@pytest.mark.parametrize("kind", ["gaps", "negative", "far", "unsorted", "equal"])
+@pytest.mark.parametrize("kt,c", [("spectral", 4), ("spectral", 10), ("rbf", 2)])
+def test_points(kt, c, kind):
+    n = 900
+    x = _points(n, 60.0, 11)
+    if kind == "gaps":
+        x = x + 9.0 * (torch.arange(n) // 100) + 2.5 * (torch.arange(n) % 100 > 53)
+    elif kind == "negative":
+        x = x - 30.0
+    elif kind == "far":
+        x = x + 3000.0
+    elif kind == "equal":
+        x = torch.sort((x / 4.0).round() * 4.0)[0]
+    x2 = x[torch.randperm(n, generator=torch.Generator().manual_seed(12))] if kind == "unsorted" else x
+    start, end = _ranges(n, n, 2 * n if kind == "unsorted" else 400)
+    _check(kt, x, x2, _vectors(n, c, 13), _vectors(n, c, 14), _params(kt, 1.1), start, end)
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1e12])
+def test_scales_and_strides(scale):
+    """Vectors far from one and of very different columns, read with strides of three."""
+    n, c = 700, 7
+    x = _points(n, 60.0, 15)
+    start, end = _ranges(n, n, 400)
+    left, right = _vectors(n, c, 16), _vectors(n, c, 17) * scale
+    right[:, 1:3] *= 1e-3
+
+    def transform(t):
+        t = t.to(DEVICE)
+        wide = torch.zeros(*t.shape, 3, device=DEVICE, dtype=t.dtype)
+        wide[..., 0] = t
+        return wide[..., 0]
+
+    _check("spectral", x, x, left, right, _params("spectral", 1.0), start, end, transform)
+
+
+@pytest.mark.parametrize("which", ["left", "right"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_values_that_are_not_finite(which, value):
+    n, c = 512, 4
+    x = _points(n, 50.0, 18)
+    start, end = _ranges(n, n, 400)
+    vectors = {"left": _vectors(n, c, 19), "right": _vectors(n, c, 20)}
+    vectors[which][200, 1] = value
+    args = [t.to(DEVICE) for t in (x, x, vectors["left"], vectors["right"], _params("spectral", 1.0), start, end)]
+    op = load_native("bilinear_derivative", BilinearDerivativeConfiguration("spectral").make_config(args))
+    assert not torch.isfinite(op.call(*args)).any()
