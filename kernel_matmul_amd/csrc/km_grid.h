@@ -28,7 +28,8 @@ namespace km {
 #define KM_GRID_STEP 0.64f          /* h s2: trapezoid error 2 exp(-7.119 / 0.64^2) = 5.7e-8 */
 #define KM_GRID_REACH 6.083f        /* V (and K / sigma) < 2^-37 beyond: the floor of the split-fp16 contraction */
 #define KM_GRID_COLUMN_REACH 8.603f /* the same for K / sigma in the coordinates of V: sqrt(2) times as far */
-#define KM_GRID_WEIGHT 0.66428247026796f /* C / (h s2) = sqrt(2 ln 2 / pi) */
+#define KM_GRID_WEIGHT_F64 0.66428247026735920 /* C / (h s2) = sqrt(2 ln 2 / pi) */
+#define KM_GRID_WEIGHT ((float)KM_GRID_WEIGHT_F64)
 #define KM_GRID_CHUNK 256           /* columns tabulated at a time, per wavefront */
 #define KM_GRID_KS1 11              /* V is evaluated times 2^11 (columns: reference within 2) ... */
 #define KM_GRID_SPAN 2.0f
@@ -302,8 +303,9 @@ __device__ __forceinline__ void exp2_pair_f16(float a, float b, float one, half2
 // One step of 32 columns: scale and split the rhs operand, then for every tile of 16 points in
 // reach evaluate, split and contract.  GRID: the points are the grid's, t0 + 16 mt h; else the rows xr[].
 // weights: which of the table's column factors this lane's rhs column takes (PARTS == 1; with two parts
-// the cosines for the first and the sines for the second).
-template <bool GRID, int G, int PARTS, int MT>
+// the cosines for the first and the sines for the second).  EXACT: the product of the low halves as well
+// (the gradient: hidden behind the VALU work there, and it halves the error of its long sums).
+template <bool GRID, int G, int PARTS, int MT, bool EXACT>
 __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off, const float (&raw)[G][8],
                                           const GridWindow& gw, float t0, const float* xr, const KernelConsts& kc,
                                           int tiles, bool wide, int weights, const bool (&colmask)[G], int (&shift)[G], float (&scale)[G],
@@ -423,6 +425,9 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
             acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[g], acc[mt][g], 0, 0, 0);
             acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[g], acc[mt][g], 0, 0, 0);
             acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[g], acc[mt][g], 0, 0, 0);
+            if (EXACT) {
+                acc[mt][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, blo[g], acc[mt][g], 0, 0, 0);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -436,7 +441,7 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
 // coordinates a chunk ahead (the first chunk's, in xv, by the caller).
 // PACK (spectral, at most 8 rhs columns): lanes 0 .. 7 of a group hold the columns' cosine parts, lanes
 // 8 .. 15 their sine parts.
-template <bool GRID, int KT, int G, int MT, int W, bool PACK = false>
+template <bool GRID, int KT, int G, int MT, int W, bool PACK = false, bool EXACT = false>
 __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __restrict__ tab, const WaveView& w, int kbase,
                                              int wave, const GridWindow& gw, const KernelConsts& kc, const float* xr,
                                              int tiles, float (&xv)[KM_GRID_CHUNK / 64], int (&shift)[G],
@@ -503,7 +508,7 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
                     asm volatile("" : "+v"(acc[m][g]));
                 }
             }
-            grid_step<GRID, G, PARTS, MT>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, rl.used, shift, scale, &fine, acc);
+            grid_step<GRID, G, PARTS, MT, EXACT>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, rl.used, shift, scale, &fine, acc);
         } while (need != 0);
         // All reads of the table are done before the next chunk overwrites it.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

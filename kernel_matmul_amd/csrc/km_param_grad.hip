@@ -51,6 +51,7 @@ struct GradArgs {
     long long x1_s, x2_s, left_s0, left_s1, right_s0, right_s1, params_s, start_s, end_s;
     BatchShape batch;
     BatchStrides x1_bs, x2_bs, left_bs, right_bs, params_bs, start_bs, end_bs;
+    int grid_min_width;  // grid form: columns in the row block's range from which it is taken
 };
 
 // One item of the pairwise form: R groups of 16 rows from row0 against the columns
@@ -69,7 +70,7 @@ struct GradArgs {
 // SKIP (rows sparse against the lengthscale): tiles of 16 rows by 16 columns whose entries are all
 // beyond the reach of the Gaussian (below 2^-37 of the largest, the floor of the other forms) are
 // left out.  One point per unit, lengthscales of half a unit to two: a third of the tiles remain
-// (n = 50000, batch 2, c = 8: 27.8 against 40.5 us without it, 32.7 us for the pairwise kernel).
+// (spectral n = 50000, batch 2, c = 8: 27.8 against 40.5 us without it).
 template <int KT, int TL, int R, bool FAST = false, bool SKIP = false>
 __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __restrict__ x1,
                                               const float* __restrict__ x2, const float* __restrict__ left,
@@ -858,7 +859,7 @@ __global__ void __launch_bounds__(64, 2) param_grad_features(const GradArgs a) {
 // Up to 8 spectral vector columns are packed with both phases into one group of 16 (PACK); more
 // than 16 take several passes.
 //
-// Measured: spectral n = 1e5, c = 4, 16 sets 273 -> 112 us (feature form before; bound by the VALU work
+// Measured: spectral n = 1e5, c = 4, 16 sets 273 -> 105 us (feature form before; bound by the VALU work
 // of exponentials and operand splits, about half of it on the columns' side); n = 7200 at 720 points
 // per unit, c = 11: 44.7 -> 20.7 us (pairwise before).
 // Resident wavefronts: three per SIMD; two with both phases in separate groups, whose operands would
@@ -866,6 +867,7 @@ __global__ void __launch_bounds__(64, 2) param_grad_features(const GradArgs a) {
 // ---------------------------------------------------------------------------------------
 #define KM_GG_STEP 0.58f
 #define KM_GG_MIN_WIDTH 96
+#define KM_GG_MIN_WIDTH_WIDE 2048 /* vectors beyond the feature form's widths */
 #define KM_GG_SHARE 256
 #define KM_GG_VARIANCE 0.36067376022224085f /* 1 / (4 ln 2): of the midpoint about the grid */
 
@@ -893,7 +895,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     w.range_start = col_begin;
     w.range_end = col_end;
     const GridVectors right = {a.x2_s, a.right_s0, a.right_s1, a.c};
-    bool fine = grid_columns<true, KT, 1, MT, 1, PACK>(right, tab, w, kbase, 0, gw, kc, nullptr, gw.tiles, xv, shift, acc);
+    bool fine = grid_columns<true, KT, 1, MT, 1, PACK, true>(right, tab, w, kbase, 0, gw, kc, nullptr, gw.tiles, xv, shift, acc);
 
     // The rows' operands: one power-of-two scale per vector column over the whole block.
     const int row_end = min(g.row0 + KM_BLOCK_SIZE, a.m);
@@ -1014,6 +1016,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
                     rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[j][part], rows[p][part], 0, 0, 0);
                     rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[j][part], rows[p][part], 0, 0, 0);
                     rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[j][part], rows[p][part], 0, 0, 0);
+                    rows[p][part] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, blo[j][part], rows[p][part], 0, 0, 0);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -1060,11 +1063,14 @@ __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3)
         return;
     }
     float* __restrict__ prow = a.partials + (g.b * a.partial_rows + g.rest) * KM_MAX_PARAMS;
-    const BlockRows rows = block_rows(g.x1, a.x1_s, g.row0, a.m);
     KernelConsts kc = make_consts<KT>(g.params, a.params_s, false);
     kc.s = uniform(kc.s);
-    const GridWindow gw = grid_window<MT>(rows, kc, KM_GG_STEP);
-    if (__builtin_amdgcn_readfirstlane(gw.ok && g.width >= KM_GG_MIN_WIDTH) != 0) {
+    GridWindow gw;
+    gw.ok = __builtin_amdgcn_readfirstlane(g.width >= a.grid_min_width) != 0;
+    if (gw.ok) {
+        gw = grid_window<MT>(block_rows(g.x1, a.x1_s, g.row0, a.m), kc, KM_GG_STEP);
+    }
+    if (__builtin_amdgcn_readfirstlane(gw.ok) != 0) {
         // (fewer, longer shares than the pairwise form's: from the same split number)
         const int shares = min(a.col_splits, max(g.width / KM_GG_SHARE, 1));
         const int per_share = ((g.width + shares - 1) / shares + 31) & ~31;
@@ -1081,10 +1087,11 @@ __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3)
             }
         }
         if (done) {
-            const float weight = gw.h * gw.s2 * KM_GRID_WEIGHT;
-            const float value = wave_sum(sums[0]) * weight;
-            const float squared = wave_sum(sums[1]) * (2.0f * weight);
-            const float slope = KT == KM_KERNEL_SPECTRAL ? wave_sum(sums[2]) * (2.0f * weight / gw.s2) : 0.0f;
+            // (a rounded factor would be off the same way in every row block: nothing averages it)
+            const double weight = (double)gw.h * (double)gw.s2 * KM_GRID_WEIGHT_F64;
+            const float value = (float)(wave_sum(sums[0]) * weight);
+            const float squared = (float)(wave_sum(sums[1]) * (2.0 * weight));
+            const float slope = KT == KM_KERNEL_SPECTRAL ? (float)(wave_sum(sums[2]) * (2.0 * weight / (double)gw.s2)) : 0.0f;
             if (threadIdx.x == 0) {
                 prow[0] = squared;
                 prow[1] = KT == KM_KERNEL_SPECTRAL ? slope : value;
@@ -1231,12 +1238,25 @@ long long param_grad_feature_partials_per_batch(int kernel_type, int64_t m, long
     return chunks * grad_col_splits(chunks * num_batches, true);
 }
 
+// The grid form: rbf and spectral kernels under the conditions of the short addressing.
+//
+// Vectors as narrow as the feature form's take it everywhere (error against float64, mean of 8 draws,
+// spectral c = 4, ten points per unit: 1.1e-7 against 2.2e-7).  For wider ones the pairwise form forms
+// its coefficients in fp32, which is the more exact way while ranges are short (spectral c = 11, 250 columns
+// per range: 5e-8 against 8e-8; 2400, c = 20: 1.1e-7 both; 10000, c = 11: 3.4e-7 against 1.7e-7): they
+// take the grid form for ranges of KM_GG_MIN_WIDTH_WIDE columns on, in launches of at most two
+// wavefronts per SIMD, where this kernel's lower occupancy costs the other row blocks nothing.
+static bool grid_form(int kernel_type, long long c, long long total_items) {
+    return kernel_type != KM_KERNEL_LOCALLY_PERIODIC && c > 0 &&
+           (feature_plan(kernel_type, c).GE > 0 || total_items <= 2048);
+}
+
 void describe_param_grad(int kernel_type, int64_t m, long long num_batches, int64_t c, char* text,
                          size_t text_bytes) {
     static const char* const kernels[] = {"rbf", "spectral", "locally_periodic"};
     const FeaturePlan f = feature_plan(kernel_type, c);
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
-    if (kernel_type != KM_KERNEL_LOCALLY_PERIODIC && c > 0) {
+    if (grid_form(kernel_type, c, row_blocks * num_batches * grad_col_splits(row_blocks * num_batches))) {
         const int used = snprintf(text, text_bytes,
                                   "km::param_grad_grid<%s%s, TL=%d> (grid form; per-item pairwise fallback), at most %d column "
                                   "share(s) per row block; for strides or batch shapes that do not suit it: ",
@@ -1311,11 +1331,6 @@ static hipError_t launch_partial_as(const GradArgs& a, unsigned grid_x, hipStrea
         hipLaunchKernelGGL((param_grad_partial<KT, 0, FAST>), dim3(grid_x), dim3(64), 0, stream, a);
     }
     return hipGetLastError();
-}
-
-// The grid form: rbf and spectral kernels under the conditions of the short addressing.
-static bool grid_form(int kernel_type, const GradArgs& a) {
-    return kernel_type != KM_KERNEL_LOCALLY_PERIODIC && pairwise_fast(a);
 }
 
 static hipError_t launch_grid(int kernel_type, const GradArgs& a, unsigned grid_x, hipStream_t stream) {
@@ -1420,7 +1435,8 @@ hipError_t launch_param_grad(const ParamGradProblem& p, hipStream_t stream) {
         a.partial_rows = row_blocks * a.col_splits;
     };
     split_items(false);
-    const bool on_grid = grid_form(p.kernel_type, a);
+    const bool on_grid = grid_form(p.kernel_type, p.c, a.total_items) && pairwise_fast(a);
+    a.grid_min_width = feature_plan(p.kernel_type, p.c).GE > 0 ? KM_GG_MIN_WIDTH : KM_GG_MIN_WIDTH_WIDE;
     // Grid form for batch shapes of one dimension and moderate strides; otherwise the feature form
     // where it applies (its 32-bit lane offsets need moderate, non-negative strides
     // of `right`); pairwise form otherwise.

@@ -105,6 +105,17 @@ def test_cut_off_blocks_and_ranges(m, n, c):
     _check("spectral", x1, x2, _vectors(m, c, 9), _vectors(n, c, 10), _params("spectral", 1.5), start, end)
 
 
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("c", [6, 8, 11, 16, 17, 33])
+@pytest.mark.parametrize("width", [1950, 2040, 2300])
+def test_wide_vectors_and_long_ranges(kt, c, width):
+    """Ranges on both sides of the width from which wide vectors take the form."""
+    n = 3000
+    x = _points(n, 50.0, 21)
+    start, end = _ranges(n, n, width)
+    _check(kt, x, x, _vectors(n, c, 22), _vectors(n, c, 23), _params(kt, 1.3), start, end)
+
+
 @pytest.mark.parametrize("kind", ["gaps", "negative", "far", "unsorted", "equal"])
 @pytest.mark.parametrize("kt,c", [("spectral", 4), ("spectral", 10), ("rbf", 2)])
 def test_points(kt, c, kind):
