@@ -118,6 +118,13 @@ int km_make_ranges_device(const float* x1, const float* x2, int64_t num_batch, i
 int km_make_ranges_symmetric_device(const float* x, int64_t num_batch, int64_t n, float cutoff,
                                     int block_size, int32_t* start, int32_t* end, void* stream);
 
+/* Whether x1[num_batch1][n1] and x2[num_batch2][n2] (x2 may be null) ascend along every row, enqueued
+ * on `stream`: all KM_SORTED_FLAGS words of `descents` are written, and one of them is not zero if a
+ * value is followed by one that is not at least as large (a NaN on either side counts). */
+#define KM_SORTED_FLAGS 128
+int km_check_sorted_device(const float* x1, int64_t num_batch1, int64_t n1, const float* x2,
+                           int64_t num_batch2, int64_t n2, int32_t* descents, void* stream);
+
 /* ------------------------------------------------------------------------------------
  * matmul.  out[b,i,c] = sum_{j in [start[b,i/128], end[b,i/128])} k(x1[b,i], x2[b,j]) rhs[b,j,c]
  * Replaces `call` of module km___matmul___* (native/matmul/matmul.cpp:6-17,

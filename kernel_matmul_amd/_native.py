@@ -75,6 +75,9 @@ def load_library():
     lib.km_make_ranges_device.argtypes = lib.km_make_ranges.argtypes + [_vp]
     lib.km_make_ranges_symmetric_device.restype = ctypes.c_int
     lib.km_make_ranges_symmetric_device.argtypes = lib.km_make_ranges_symmetric.argtypes + [_vp]
+    lib.km_check_sorted_device.restype = ctypes.c_int
+    lib.km_check_sorted_device.argtypes = [f32p, ctypes.c_int64, ctypes.c_int64, f32p, ctypes.c_int64,
+                                           ctypes.c_int64, i32p, _vp]
 
     tensor = [_vp, _i64p]
     lib.km_matmul.restype = ctypes.c_int
@@ -543,6 +546,23 @@ def dense_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: T
 
 
 # -- ranges ------------------------------------------------------------------------------
+_SORTED_FLAGS = 128  # KM_SORTED_FLAGS
+
+
+def sorted_flags(x1: Tensor, x2: Tensor | None) -> Tensor:
+    """Enqueues the check that the rows of contiguous float32 device tensors ``[batch, n]`` ascend; any
+    value of the result that is not zero means that they do not."""
+    lib = load_library()
+    flags = torch.empty(_SORTED_FLAGS, dtype=torch.int32, device=x1.device)
+    with _on_device(x1.device):
+        status = lib.km_check_sorted_device(
+            _ptr(x1), *x1.shape, _ptr(x2) if x2 is not None else None, *(x2.shape if x2 is not None else (0, 0)),
+            _ptr(flags), _stream(x1.device))
+    if status != 0:
+        _raise(lib, status)
+    return flags
+
+
 def make_ranges_2d(x1: Tensor, x2: Tensor | None, cutoff: float, block_size: int,
                    align: bool) -> tuple[Tensor, Tensor]:
     """Range builders on flattened [batch, n] inputs; result lives on x1's device.

@@ -471,6 +471,18 @@ int km_make_ranges_symmetric_device(const float* x, int64_t num_batch, int64_t n
     return err == hipSuccess ? KM_OK : fail_hip(op, err);
 }
 
+int km_check_sorted_device(const float* x1, int64_t num_batch1, int64_t n1, const float* x2, int64_t num_batch2,
+                           int64_t n2, int32_t* descents, void* stream) {
+    const char* op = "km_check_sorted_device";
+    if (num_batch1 < 0 || n1 < 0 || num_batch2 < 0 || n2 < 0) {
+        return fail(KM_ERR_INVALID_ARGUMENT, "%s: sizes out of range", op);
+    }
+    if (num_batch1 > 0 && n1 > 1) KM_REQUIRE_PTR(op, x1);
+    KM_REQUIRE_PTR(op, descents);
+    hipError_t err = launch_check_sorted(x1, num_batch1, n1, x2, num_batch2, n2, descents, (hipStream_t)stream);
+    return err == hipSuccess ? KM_OK : fail_hip(op, err);
+}
+
 // ---------------------------------------------------------------------------------------
 // matmul
 // ---------------------------------------------------------------------------------------

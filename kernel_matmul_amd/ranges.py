@@ -70,14 +70,31 @@ def make_ranges(
         start = torch.zeros(x1f.shape[0], rows, dtype=torch.int32, device=x1.device)
         end = torch.full((x1f.shape[0], rows), n2, dtype=torch.int32, device=x1.device)
     else:
-        if check_sorted and x1f.is_cuda and not (_ascending(x1f) and (x2f is None or _ascending(x2f))):
+        # On the device the check and the builder are enqueued together; their one wait is the read
+        # of the check's flags, after which the pattern of unsorted inputs is dropped.  (The
+        # builder's searches end on any data.)
+        flags = None
+        if check_sorted and x1f.is_cuda:
+            if x1f.dtype == torch.float32 and (
+                x2f is None or (x2f.dtype == torch.float32 and x2f.device == x1f.device)
+            ):
+                x1f = x1f.detach().contiguous()
+                x2f = x2f.detach().contiguous() if x2f is not None else None
+                flags = _native.sorted_flags(x1f, x2f)
+                on_host = False
+            else:
+                on_host = not (_ascending(x1f) and (x2f is None or _ascending(x2f)))
+        else:
+            on_host = False
+        if not on_host:
+            start, end = _native.make_ranges_2d(x1f, x2f, cutoff, block_size, align)
+            on_host = flags is not None and any(flags.tolist())
+        if on_host:
             device = x1f.device
             start, end = _native.make_ranges_2d(
                 x1f.cpu(), x2f.cpu() if x2f is not None else None, cutoff, block_size, align
             )
             start, end = start.to(device), end.to(device)
-        else:
-            start, end = _native.make_ranges_2d(x1f, x2f, cutoff, block_size, align)
 
     return start.reshape(*batch_shape, rows), end.reshape(*batch_shape, rows)
 
