@@ -859,9 +859,9 @@ __global__ void __launch_bounds__(64, 2) param_grad_features(const GradArgs a) {
 // Up to 8 spectral vector columns are packed with both phases into one group of 16 (PACK); more
 // than 16 take several passes.
 //
-// Measured: spectral n = 1e5, c = 4, 16 sets 273 -> 105 us (feature form before; bound by the VALU work
+// Measured: spectral n = 1e5, c = 4, 16 sets 245 -> 109 us a call (feature form before; bound by the VALU work
 // of exponentials and operand splits, about half of it on the columns' side); n = 7200 at 720 points
-// per unit, c = 11: 44.7 -> 20.7 us (pairwise before).
+// per unit, c = 11: 44.7 -> 20.7 us (kernel; pairwise before).
 // Resident wavefronts: three per SIMD; two with both phases in separate groups, whose operands would
 // spill 224 bytes a lane at three (29.2 against 23.0 us for the call).
 // ---------------------------------------------------------------------------------------
