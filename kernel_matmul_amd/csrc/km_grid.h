@@ -34,8 +34,10 @@ namespace km {
 #define KM_GRID_KS1 11              /* V is evaluated times 2^11 (columns: reference within 2) ... */
 #define KM_GRID_SPAN 2.0f
 #define KM_GRID_KS2 10              /* ... and 2^10 (rows: reference within 3.5 h s2 = 2.24) */
-// Table of a chunk: coordinate, the two column factors, and per 8 columns the reference and its span.
-#define KM_GRID_TABLE_FLOATS (3 * KM_GRID_CHUNK + 2 * KM_GRID_CHUNK / 8)
+// Table of a chunk: coordinate, the two column factors, per 8 columns the reference and its span (or the
+// two ends), and the remainder of the coordinate.
+#define KM_GRID_TABLE_REST (3 * KM_GRID_CHUNK + 2 * KM_GRID_CHUNK / 8)
+#define KM_GRID_TABLE_FLOATS (KM_GRID_TABLE_REST + KM_GRID_CHUNK)
 
 // A value that is the same in every lane, as a scalar register.
 __device__ __forceinline__ float uniform(float v) {
@@ -111,6 +113,12 @@ __device__ __forceinline__ void group8_min_max(float v, float* lo, float* hi) {
     *hi = b;
 }
 
+// What the subtraction d = x - origin rounded off.
+__device__ __forceinline__ float remainder_of(float x, float origin, float d) {
+    const float bb = d - x;
+    return (x - (d - bb)) - (origin + bb);
+}
+
 // Coordinates of this wavefront's next 8 steps of 32 columns, in the order grid_table takes them.
 __device__ __forceinline__ void grid_load(const float* __restrict__ x2, long long x2_s, int first, int stride, int end,
                                           float (&xv)[KM_GRID_CHUNK / 64]) {
@@ -129,9 +137,13 @@ __device__ __forceinline__ void grid_load(const float* __restrict__ x2, long lon
 // steps that reach the rows as a bit mask.
 //   GRID: coordinates as 2 b, b = (y - r) s2 with r in the middle of each group of 8 columns, the
 //         column factors times 2^(-b^2).  Steps of which a group spreads further than KM_GRID_SPAN
-//         (a gap in the data) come back in the upper half of the mask; their factors lack 2^(-b^2)
-//         (it would leave the fp16 range).  *fine is cleared when a coordinate is not finite.
-//   else: the coordinates themselves, spans in units of 1 / s (entry-wise evaluation).
+//         (a gap in the data) come back in the upper half of the mask: their factors lack 2^(-b^2)
+//         (it would leave the fp16 range) and their coordinates are y and its remainder, relative to
+//         the row block's origin: a reference in the middle of the gap would round them to a fraction
+//         of the gap.  *fine is cleared when a coordinate is not finite.
+//   else: the coordinates themselves (entry-wise evaluation).
+// The two values per group of 8 columns are its reference and half its extent in units of 1 / s2 where
+// there is a reference, else its smallest and largest coordinate.
 template <bool GRID, bool PHASE>
 __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK / 64], int first, int stride, int end,
                                                const GridWindow& gw, const KernelConsts& kc, float* __restrict__ tab,
@@ -140,7 +152,7 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
     constexpr int N = CH / 64;
     const int lane = threadIdx.x & 63;
     const int last = end - 1 - first;
-    float b[N], ref[N], span[N];
+    float b[N], lower[N], upper[N];
     bool wide[N];
     unsigned need = 0;
     bool ok = true;
@@ -157,19 +169,18 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
         need |= bits(rel <= last && !(y < gw.col_lo || y > gw.col_hi), i);
         float lo, hi;
         group8_min_max(GRID ? y : xv[i], &lo, &hi);
-        ref[i] = 0.5f * (lo + hi);
         if (GRID) {
-            // the difference to the origin as a sum of two terms: what the subtraction rounded off
-            const float bb = y - xv[i];
-            const float rest = (xv[i] - (y - bb)) - (gw.x_ref + bb);
-            b[i] = ((y - ref[i]) + rest) * gw.s2;
-            span[i] = 0.5f * (hi - lo) * gw.s2;
-            const unsigned w = bits(span[i] > KM_GRID_SPAN, i);
+            const float ref = 0.5f * (lo + hi), span = 0.5f * (hi - lo) * gw.s2;
+            b[i] = ((y - ref) + remainder_of(xv[i], gw.x_ref, y)) * gw.s2;
+            const unsigned w = bits(span > KM_GRID_SPAN, i);
             wide[i] = (w >> (2 * i + (lane >> 5)) & 1) != 0;
+            lower[i] = wide[i] ? lo : ref;
+            upper[i] = wide[i] ? hi : span;
             need |= w << 16;
             ok = ok && fabsf(y) < 1e30f;
         } else {
-            span[i] = 0.5f * (hi - lo) * kc.s;
+            lower[i] = lo;
+            upper[i] = hi;
         }
     }
     need = __builtin_amdgcn_readfirstlane(need);
@@ -187,6 +198,11 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
         const int q = lane + 64 * i;
         const float wgt = GRID && !wide[i] ? __builtin_amdgcn_exp2f(-b[i] * b[i]) : 1.0f;
         tab[q] = GRID ? b[i] + b[i] : xv[i];
+        if (GRID && wide[i]) {
+            const float y = xv[i] - gw.x_ref;
+            tab[q] = y;
+            tab[KM_GRID_TABLE_REST + q] = remainder_of(xv[i], gw.x_ref, y);
+        }
         if (PHASE) {
             const float th = phase_rev(kc.f, xv[i], gw.x_ref);
             tab[CH + q] = wgt * __builtin_amdgcn_cosf(th);
@@ -195,8 +211,8 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
             tab[CH + q] = wgt;
         }
         if ((lane & 7) == 0) {
-            tab[3 * CH + (q >> 3)] = ref[i];
-            tab[3 * CH + CH / 8 + (q >> 3)] = span[i];
+            tab[3 * CH + (q >> 3)] = lower[i];
+            tab[3 * CH + CH / 8 + (q >> 3)] = upper[i];
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -330,8 +346,8 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
             }
         }
     }
-    const float ref = tab[3 * CH + (off >> 3)];
-    const float span = tab[3 * CH + CH / 8 + (off >> 3)];
+    const float lower = tab[3 * CH + (off >> 3)];
+    const float upper = tab[3 * CH + CH / 8 + (off >> 3)];
 
     half8v bhi[GE], blo[GE];
 #pragma unroll
@@ -389,8 +405,14 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
             break;
         }
         const float t = GRID ? __builtin_fmaf((float)(16 * mt), gw.h, t0) : xr[mt];
-        const float av = (t - ref) * (GRID ? gw.s2 : kc.s);
-        if (!__any(!(fabsf(av) - span > KM_GRID_REACH))) {
+        const float av = (t - lower) * (GRID ? gw.s2 : kc.s);
+        float beyond;  // distance to the columns
+        if (GRID && !wide) {
+            beyond = fabsf(av) - upper;
+        } else {
+            beyond = fmaxf(-av, (t - upper) * (GRID ? gw.s2 : kc.s));
+        }
+        if (!__any(!(beyond > KM_GRID_REACH))) {
             continue;
         }
         half2v h2[4], l2[4];
@@ -403,9 +425,11 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
                     arg[u] = __builtin_fmaf(av, xv[u], rb);
                 }
             } else {
+                const float4v r0 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off);
+                const float4v r1 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off + 4);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
-                    const float z = __builtin_fmaf(-0.5f, xv[u], av);
+                    const float z = ((t - xv[u]) - (u < 4 ? r0[u & 3] : r1[u & 3])) * gw.s2;
                     arg[u] = __builtin_fmaf(-z, z, (float)KM_GRID_KS1);
                 }
             }

@@ -977,26 +977,43 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
             }
             int off = 32 * j + 8 * kk;
             asm volatile("" : "+v"(off));  // (read again for every tile, not kept over all of them: registers)
+            const bool wide = (steps >> (16 + j) & 1) != 0;
             const float av = (t - tab[3 * CH + (off >> 3)]) * gw.s2;
-            if (!__any(!(fabsf(av) - tab[3 * CH + CH / 8 + (off >> 3)] > KM_GRID_REACH))) {
+            const float upper = tab[3 * CH + CH / 8 + (off >> 3)];
+            const float beyond = wide ? fmaxf(-av, (t - upper) * gw.s2) : fabsf(av) - upper;
+            if (!__any(!(beyond > KM_GRID_REACH))) {
                 continue;
             }
             const float4v x0 = *(const float4v*)(tab + off);
             const float4v x1 = *(const float4v*)(tab + off + 4);
-            const bool wide = (steps >> (16 + j) & 1) != 0;
-            const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
+            float pr[8], arg[8];
+            if (!wide) {
+                const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const float b2 = u < 4 ? x0[u & 3] : x1[u & 3];
+                    pr[u] = __builtin_fmaf(0.5f, b2, -av);
+                    arg[u] = __builtin_fmaf(av, b2, rb);
+                }
+            } else {
+                const float4v r0 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off);
+                const float4v r1 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off + 4);
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const float y = u < 4 ? x0[u & 3] : x1[u & 3];
+                    pr[u] = ((y - t) + (u < 4 ? r0[u & 3] : r1[u & 3])) * gw.s2;
+                    arg[u] = __builtin_fmaf(-pr[u], pr[u], (float)KM_GRID_KS1);
+                }
+            }
             half2v hi[NP][4], lo[NP][4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 float ev[2], pv[2], qv[2];
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    const float b2 = u < 2 ? x0[2 * (u & 1) + i] : x1[2 * (u & 1) + i];
-                    const float p = __builtin_fmaf(0.5f, b2, -av);
-                    ev[i] = __builtin_amdgcn_exp2f(wide ? __builtin_fmaf(-p, p, (float)KM_GRID_KS1)
-                                                        : __builtin_fmaf(av, b2, rb));
-                    pv[i] = p;
-                    qv[i] = __builtin_fmaf(p, p, -KM_GG_VARIANCE);
+                    ev[i] = __builtin_amdgcn_exp2f(arg[2 * u + i]);
+                    pv[i] = pr[2 * u + i];
+                    qv[i] = __builtin_fmaf(pv[i], pv[i], -KM_GG_VARIANCE);
                 }
                 hi[0][u] = __builtin_convertvector((float2v){ev[0], ev[1]}, half2v);
                 lo[0][u] = residual_f16x2(ev[0], kc.one, ev[1], kc.one, hi[0][u]);

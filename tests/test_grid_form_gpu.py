@@ -14,6 +14,7 @@ import torch
 
 from kernel_matmul_amd.compile import load_native
 from kernel_matmul_amd.configurations import MatmulSingleConfiguration
+from kernel_matmul_amd.ranges import make_ranges
 from oracle import kernels as oracle
 
 pytestmark = pytest.mark.gpu
@@ -179,3 +180,19 @@ def test_variant_is_refused_for_other_kernels():
     defines["MATMUL_VARIANT"] = "grid"
     with pytest.raises(RuntimeError, match="grid form"):
         load_native("matmul", defines).call(*args)
+
+
+@pytest.mark.parametrize("gap", [1e2, 1e3, 1e4, 1e5, 1e6, 1e9])
+@pytest.mark.parametrize("rows", [16, 32, 128])
+def test_columns_next_to_a_wide_gap(gap, rows):
+    """Groups of 8 columns that lie on both sides of a gap of up to a billion lengthscales, in the ranges
+    of row blocks on either side of it: the near columns are as exact as any others, also where they are
+    the only ones that are not zero, and where the rows go entry by entry (the second lengthscale)."""
+    x = torch.cat([_points(1003, 10.03, 30), _points(500, 5.0, 31) + 10.03 + gap])
+    rhs = torch.randn(len(x), 4, generator=torch.Generator().manual_seed(32))
+    rhs[:1000, 2:] = 0.0
+    rhs[1003:, 2:] = 0.0
+    for kt, lengthscale in (("spectral", 1.0), ("rbf", 1.0), ("spectral", 0.03), ("rbf", 0.03)):
+        _check(kt, x, x, rhs, _params(kt, lengthscale), *make_ranges(6.0, x), rows=rows)
+        mirrored = -x.flip(0)
+        _check(kt, mirrored, mirrored, rhs.flip(0), _params(kt, lengthscale), *make_ranges(6.0, mirrored), rows=rows)

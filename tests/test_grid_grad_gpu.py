@@ -15,6 +15,7 @@ import torch
 
 from kernel_matmul_amd.compile import load_native
 from kernel_matmul_amd.configurations import BilinearDerivativeConfiguration
+from kernel_matmul_amd.ranges import make_ranges
 from oracle import kernels as oracle
 
 pytestmark = pytest.mark.gpu
@@ -163,3 +164,19 @@ def test_values_that_are_not_finite(which, value):
     args = [t.to(DEVICE) for t in (x, x, vectors["left"], vectors["right"], _params("spectral", 1.0), start, end)]
     op = load_native("bilinear_derivative", BilinearDerivativeConfiguration("spectral").make_config(args))
     assert not torch.isfinite(op.call(*args)).any()
+
+
+@pytest.mark.parametrize("gap", [1e2, 1e3, 1e4, 1e5, 1e6, 1e9])
+@pytest.mark.parametrize("kt,c,count", [("spectral", 4, 1003), ("rbf", 6, 1003), ("spectral", 11, 2603)])
+def test_columns_next_to_a_wide_gap(kt, c, count, gap):
+    """Groups of 8 columns that lie on both sides of a gap of up to a billion lengthscales: a gradient that
+    only the columns next to the gap and the rows near it make."""
+    extent = count / 100.0
+    x = torch.cat([_points(count, extent, 30), _points(500, 5.0, 31) + extent + gap])
+    start, end = make_ranges(extent if c == 11 else 6.0, x)
+    left, right = _vectors(len(x), c, 32), torch.zeros(len(x), c)
+    right[count - 3:count] = _vectors(3, c, 33)
+    _check(kt, x, x, left, right, _params(kt, 1.0), start, end)
+    mirrored = -x.flip(0)
+    _check(kt, mirrored, mirrored, left.flip(0), right.flip(0), _params(kt, 1.0),
+           *make_ranges(extent if c == 11 else 6.0, mirrored))
