@@ -14,8 +14,8 @@
 // reach of V, 20 to 60 points) instead of one entry per row and column of the pattern.  The column
 // ranges [start, end) are honoured exactly: each row block sums the columns of its own range.
 //
-// Coordinates are taken relative to the row block's middle row (exact for neighbouring points; the
-// column side carries the rounding of that difference as a second term) and h is rounded to 12
+// Coordinates are taken relative to the row block's middle row (exact for neighbouring points; rows
+// and columns carry the rounding of that difference as a second term) and h is rounded to 12
 // significant bits, so that all g h are exact.  Scaled coordinates z = x s2 (s2 = sqrt(log2 e) / l)
 // make V(x, t) = 2^-(z_x - z_t)^2.
 #pragma once

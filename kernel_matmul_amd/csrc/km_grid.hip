@@ -199,6 +199,8 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
     for (int r = 0; r < R; r++) {
         const int row = row0 + 16 * (wave * R + r);
         const float x = w.x1[(long long)min(row + li, a.m - 1) * a.x1_s];
+        const float y = x - gw.x_ref;
+        const float rest = remainder_of(x, gw.x_ref, y);  // (not zero in a block next to the origin)
         float4v res[GE];
 #pragma unroll
         for (int g = 0; g < GE; g++) {
@@ -209,7 +211,7 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
             if (2 * ks >= gw.tiles) {
                 break;
             }
-            const float av = ((x - gw.x_ref) - __builtin_fmaf((float)ks, mid_step, mid0)) * gw.s2;
+            const float av = ((y - __builtin_fmaf((float)ks, mid_step, mid0)) + rest) * gw.s2;
             if (!__any(fabsf(av) - 3.5f * hz < KM_GRID_REACH)) {
                 continue;
             }

@@ -196,3 +196,31 @@ def test_columns_next_to_a_wide_gap(gap, rows):
         _check(kt, x, x, rhs, _params(kt, lengthscale), *make_ranges(6.0, x), rows=rows)
         mirrored = -x.flip(0)
         _check(kt, mirrored, mirrored, rhs.flip(0), _params(kt, lengthscale), *make_ranges(6.0, mirrored), rows=rows)
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("rows", [32, 128])
+def test_block_around_the_origin(kt, rows):
+    """Rows on both sides of the origin, whose distances to the block's middle row are half an ulp of 4
+    (2.4e-7) off a representable value, against single columns two to four lengthscales away: without
+    what the subtraction rounded off entries are 1.2e-6 to 2.3e-6 off.  The bound is the form's own: two
+    factors, each of an exponent below 12 that is rounded twice (6.6e-7 at most together), averaged over
+    the grid points that share neither rounding; measured 4.0e-7 in the 2-norm."""
+    x1 = torch.cat([_points(64, 2.2, 33) - 6.3, torch.tensor([25000.49 * 2.0 ** -21]), _points(63, 2.2, 34) + 4.05])
+    x2 = torch.linspace(-7.5, 7.5, 320)
+    params = _params(kt, 0.42)
+    if kt == "spectral":
+        params[1] = 0.01
+    start, end = torch.zeros(1, dtype=torch.int32), torch.full((1,), 320, dtype=torch.int32)
+    relative = []
+    for first in range(5):
+        columns = torch.arange(16) * 20 + 4 * first
+        rhs = torch.zeros(320, 16)
+        rhs[columns, torch.arange(16)] = 1.0
+        out = _run(kt, x1, x2, rhs, params, start, end, rows=rows)
+        expected = oracle.matmul(kt, *(t.numpy() for t in (x1, x2, rhs, params, start, end)))
+        d = np.abs(x1.double().numpy()[:, None] - x2[columns].double().numpy()) / 0.42
+        relative.append((out / expected - 1.0)[(d > 2.0) & (d < 4.0)])
+    error = np.sqrt(np.mean(np.concatenate(relative) ** 2))
+    print(f"2-norm of the relative error: {error:.2e}")
+    assert error < 8e-7
