@@ -66,11 +66,12 @@ struct GradArgs {
 // column share is a third of the wavefront's issue time (48 row operands against three chunks).
 #define KM_GRAD_FAST_STRIDE (1 << 21)
 
-//
-// SKIP (rows sparse against the lengthscale): tiles of 16 rows by 16 columns whose entries are all
-// beyond the reach of the Gaussian (below 2^-37 of the largest, the floor of the other forms) are
-// left out.  One point per unit, lengthscales of half a unit to two: a third of the tiles remain
-// (spectral n = 50000, batch 2, c = 8: 27.8 against 40.5 us without it).
+// Distance in units of 1 / s from which the Gaussian is zero: 2^-(12.25^2) = 2^-150.06 rounds to zero
+// in fp32.
+#define KM_GRAD_REACH 12.25f
+
+// SKIP (rows sparse against the lengthscale): tiles of 16 rows by 16 columns of which every entry is
+// zero in fp32 are left out (see KM_GRAD_REACH): the sums are the same.
 template <int KT, int TL, int R, bool FAST = false, bool SKIP = false>
 __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __restrict__ x1,
                                               const float* __restrict__ x2, const float* __restrict__ left,
@@ -176,7 +177,7 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
     // reach of a group with a NaN).
     float reach_lo[R], reach_hi[R];
     if (SKIP) {
-        const float reach = KM_GRID_REACH / kc.s;
+        const float reach = KM_GRAD_REACH / kc.s;
 #pragma unroll
         for (int r = 0; r < R; r++) {
             float lo = __builtin_inff(), hi = -__builtin_inff();
@@ -186,8 +187,11 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
                 lo = fminf(lo, nan ? -__builtin_inff() : x1q[r][v]);
                 hi = fmaxf(hi, nan ? __builtin_inff() : x1q[r][v]);
             }
-            reach_lo[r] = uniform(-column_max(-lo) - reach);
-            reach_hi[r] = uniform(column_max(hi) + reach);
+            lo = -column_max(-lo);
+            hi = column_max(hi);
+            // (and half an ulp that either sum may be rounded by)
+            reach_lo[r] = uniform(lo - (reach + 1.2e-7f * fabsf(lo)));
+            reach_hi[r] = uniform(hi + (reach + 1.2e-7f * fabsf(hi)));
         }
     }
 

@@ -180,3 +180,22 @@ def test_columns_next_to_a_wide_gap(kt, c, count, gap):
     mirrored = -x.flip(0)
     _check(kt, mirrored, mirrored, left.flip(0), right.flip(0), _params(kt, 1.0),
            *make_ranges(extent if c == 11 else 6.0, mirrored))
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("c", [1, 4, 8, 11, 20])
+@pytest.mark.parametrize("i,j", [(207, 224), (64, 47)])
+@pytest.mark.parametrize("spacing", [0.5, 0.6, 0.7])
+def test_distant_entries_of_sparse_points(kt, c, i, j, spacing):
+    """Row blocks evaluated pair by pair: an entry that fp32 can represent is not dropped, whatever its
+    distance (here 2^-52, 2^-75 and 2^-102 of sigma, the only one of a coefficient that is not zero).
+    The exponent is exact to three roundings of half an ulp: 0.7 * 102 * 3 * 2^-24."""
+    n = 512
+    x = torch.arange(n) * spacing
+    start, end = torch.zeros(4, dtype=torch.int32), torch.full((4,), n, dtype=torch.int32)
+    left, right = torch.zeros(n, c), torch.zeros(n, c)
+    left[i], right[j] = 1e6, 1e9
+    params = _params(kt, 1.0)
+    result = _call(kt, *(t.to(DEVICE) for t in (x, x, left, right, params, start, end)))
+    expected = oracle.param_grad(kt, *(t.numpy() for t in (x, x, left, right, params, start, end)))
+    assert np.all(np.abs(result - expected) <= 2e-5 * np.abs(expected)), (result, expected)
