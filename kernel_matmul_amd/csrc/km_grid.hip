@@ -10,8 +10,10 @@
 //
 // Both factors of both contractions are split into two fp16 terms as in the table kernels.  A row
 // block whose window does not fit the accumulators (points sparse against the lengthscale), whose
-// range is too short to gain, or whose coordinates or rhs are not finite is evaluated entry by entry
-// in the same launch: each wavefront its rows, tile against tile, those out of reach left out.
+// range is too short to gain, or whose coordinates are not finite is evaluated entry by entry in the
+// same launch: each wavefront its rows, tile against tile, those out of reach left out.  A value of rhs
+// that is not finite makes its column's results NaN in every row whose range holds it, as does a NaN
+// among the range's column coordinates (spectral: an infinity as well) in all columns.
 #include "km_batch.h"
 #include "km_common.h"
 #include "km_fwd.h"
@@ -64,12 +66,13 @@ __device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, 
     }
 }
 
-// LDS of one item in floats: the wavefronts' tables, overlaid by the exchange of the sums, and a
-// flag per wavefront.
+// LDS of one item in floats: the wavefronts' tables, overlaid by the exchange of the sums, and the
+// flags of each wavefront.
 template <int GE, int MT, int W>
 constexpr int grid_lds_floats() {
     return W == 1 ? KM_GRID_TABLE_FLOATS
-                  : (W * KM_GRID_TABLE_FLOATS > W * MT * GE * 256 ? W * KM_GRID_TABLE_FLOATS : W * MT * GE * 256) + W;
+                  : (W * KM_GRID_TABLE_FLOATS > W * MT * GE * 256 ? W * KM_GRID_TABLE_FLOATS : W * MT * GE * 256) +
+                        W * (GE + 1);
 }
 
 // One item in the grid form for rhs columns [kbase, kbase + 16 G), by W wavefronts of which this is
@@ -94,7 +97,7 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
     // The sums of all W wavefronts, added in their order.
     if (W > 1) {
         float4v* part = (float4v*)lds;
-        int* flags = (int*)(lds + grid_lds_floats<GE, MT, W>() - W);
+        unsigned* flags = (unsigned*)(lds + grid_lds_floats<GE, MT, W>() - W * (GE + 1));
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1);
@@ -107,8 +110,17 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
             }
         }
         __syncthreads();  // the exchange lies over the tables
+        unsigned mine[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            mine[g] = (unsigned)__ballot(shift[g] == KM_GRID_NOT_FINITE) & 0xffff;
+        }
         if (lane == 0) {
-            flags[wave] = fine ? 1 : 0;
+            flags[wave * (G + 1)] = fine ? 1 : 0;
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                flags[wave * (G + 1) + 1 + g] = mine[g];
+            }
         }
 #pragma unroll
         for (int m = 0; m < MT; m++) {
@@ -122,7 +134,11 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
         __syncthreads();
 #pragma unroll
         for (int v = 0; v < W; v++) {
-            fine = fine && __builtin_amdgcn_readfirstlane(flags[v]) != 0;
+            fine = fine && __builtin_amdgcn_readfirstlane(flags[v * (G + 1)]) != 0;
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                shift[g] = (flags[v * (G + 1) + 1 + g] >> li & 1) != 0 ? KM_GRID_NOT_FINITE : shift[g];
+            }
         }
 #pragma unroll
         for (int m = 0; m < MT; m++) {
@@ -176,7 +192,9 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
         m = column_max(m);
         const int e = min(max(14 - __builtin_amdgcn_frexp_expf(m), -100), 100);
         const float up = __builtin_ldexpf(1.0f, e);
-        down[g] = weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 - (W > 1 ? 0 : shift[g % G] + KM_GRID_KS1));
+        down[g] = shift[g % G] == KM_GRID_NOT_FINITE
+                      ? __builtin_nanf("")
+                      : weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 - (W > 1 ? 0 : shift[g % G] + KM_GRID_KS1));
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ks++) {
             if (2 * ks < gw.tiles) {
@@ -245,6 +263,19 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
     constexpr int R = W == 8 ? 1 : 2;
     constexpr int PIECES = 8 / (W * R);
     const int li = threadIdx.x & 15;
+    // The rhs values of the whole range, once for all rows.
+    int rhs_shift[G];
+    {
+        float rhs_scale[G];
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            rhs_shift[g] = 0;
+            rhs_scale[g] = 0.0f;
+        }
+        const int steps = (max(w.range_end - w.range_start, 0) + 31) / 32;
+        look_at_steps<G>(vectors(a), w, kbase, w.range_start, 32, {steps < 64 ? (1ull << steps) - 1 : ~0ull, 64, steps},
+                         rhs_lane<G>(vectors(a), kbase), rhs_shift, rhs_scale);
+    }
 #pragma unroll 1
     for (int piece = 0; piece < PIECES; piece++) {
         const int base = row0 + 16 * R * (wave * PIECES + piece);
@@ -266,21 +297,23 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         }
         wave_min_max(&lo, &hi);
         finite = __all(finite);
-        const float reach = KM_GRID_REACH / kc.s;
-        rows.col_lo = uniform(finite ? lo - reach : -__builtin_inff());
-        rows.col_hi = uniform(finite ? hi + reach : __builtin_inff());
+        rows.reach = uniform(KM_GRID_REACH / kc.s);
+        rows.col_lo = uniform(finite ? lo - rows.reach : -__builtin_inff());
+        rows.col_hi = uniform(finite ? hi + rows.reach : __builtin_inff());
         float xv[KM_GRID_CHUNK / 64];
         if (w.range_start < w.range_end) {
             grid_load(w.x2, a.x2_s, w.range_start, 1, w.range_end, xv);
         }
         int shift[G];
         float4v acc[R][GE];
-        grid_columns<false, KT, G, R, 1>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr, R, xv, shift, acc);
+        const bool fine = grid_columns<false, KT, G, R, 1>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
+                                                           R, xv, shift, acc);
         const float sigma = w.params[KernelTraits<KT>::SIGMA * a.params_s];
         float down[GE];
 #pragma unroll
         for (int g = 0; g < GE; g++) {
-            down[g] = __builtin_ldexpf(sigma, -shift[g % G] - KM_F16_KSCALE_LOG2);
+            down[g] = fine && rhs_shift[g % G] != KM_GRID_NOT_FINITE ? __builtin_ldexpf(sigma, -shift[g % G] - KM_F16_KSCALE_LOG2)
+                                                                     : __builtin_nanf("");
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -334,7 +367,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
 }
 
 template <int KT, int G, int W>
-__global__ void __launch_bounds__(64 * W, (GridShape<KT, G>::GE >= 4 ? 2 : 3)) fwd_grid(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * W, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid(const FwdArgs a) {
     extern __shared__ float lds[];
     const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
     if (item >= a.total_items) {
@@ -347,7 +380,7 @@ __global__ void __launch_bounds__(64 * W, (GridShape<KT, G>::GE >= 4 ? 2 : 3)) f
 // its last `tail_items` are dispatched last, one per workgroup, so that these quarter-length pieces
 // fill the SIMDs that would otherwise idle while others finish a last full item.
 template <int KT, int G>
-__global__ void __launch_bounds__(256, (GridShape<KT, G>::GE >= 4 ? 2 : 3)) fwd_grid_grouped(const FwdArgs a) {
+__global__ void __launch_bounds__(256, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid_grouped(const FwdArgs a) {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned xcd = blockIdx.x % KM_NUM_XCD;

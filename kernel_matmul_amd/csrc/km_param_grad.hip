@@ -900,6 +900,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     w.range_end = col_end;
     const GridVectors right = {a.x2_s, a.right_s0, a.right_s1, a.c};
     bool fine = grid_columns<true, KT, 1, MT, 1, PACK, true>(right, tab, w, kbase, 0, gw, kc, nullptr, gw.tiles, xv, shift, acc);
+    fine = fine && !__any(shift[0] == KM_GRID_NOT_FINITE);
 
     // The rows' operands: one power-of-two scale per vector column over the whole block.
     const int row_end = min(g.row0 + KM_BLOCK_SIZE, a.m);
@@ -929,7 +930,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
         }
     }
     m = column_max(m);
-    fine = fine && __all(!rl.used[0] || m < __builtin_inff());
+    fine = fine && __all(!rl.used[0] || is_finite(m));
     if (!fine) {
         return false;
     }
@@ -982,16 +983,16 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
             int off = 32 * j + 8 * kk;
             asm volatile("" : "+v"(off));  // (read again for every tile, not kept over all of them: registers)
             const bool wide = (steps >> (16 + j) & 1) != 0;
-            const float av = (t - tab[3 * CH + (off >> 3)]) * gw.s2;
-            const float upper = tab[3 * CH + CH / 8 + (off >> 3)];
-            const float beyond = wide ? fmaxf(-av, (t - upper) * gw.s2) : fabsf(av) - upper;
-            if (!__any(!(beyond > KM_GRID_REACH))) {
+            const float lo_x = tab[3 * CH + (off >> 3)];
+            const float hi_x = tab[3 * CH + CH / 8 + (off >> 3)];
+            if (!__any(!(fmaxf(lo_x - t, t - hi_x) > gw.reach))) {
                 continue;
             }
             const float4v x0 = *(const float4v*)(tab + off);
             const float4v x1 = *(const float4v*)(tab + off + 4);
             float pr[8], arg[8];
             if (!wide) {
+                const float av = (t - 0.5f * (lo_x + hi_x)) * gw.s2;
                 const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {

@@ -143,8 +143,7 @@ def test_split_tail(tail):
 
 @pytest.mark.parametrize("rows", [32, 128])
 def test_values_that_are_not_finite(rows):
-    """A NaN or an infinity in the coordinates or in rhs reaches the rows whose reach it is in, as in
-    the entry-wise kernels, and no others."""
+    """A NaN in rhs or in a row's coordinate: near rows, rows whose range does not hold it, other rows."""
     n = 1024
     x = _points(n, n / 10.0, 13)
     rhs = torch.randn(n, 2, generator=torch.Generator().manual_seed(14))
@@ -165,11 +164,94 @@ def test_values_that_are_not_finite(rows):
     assert np.all(np.isnan(out[500])) and np.all(np.isfinite(np.delete(out, 500, axis=0)))
 
 
-def _run_nan(kt, x1, x2, rhs, params, start, end, rows):
+def _run_nan(kt, x1, x2, rhs, params, start, end, rows, tail=None):
     args = tuple(t.to(DEVICE) for t in (x1, x2, rhs, params, start, end))
     defines = MatmulSingleConfiguration(kt).make_config(args)
     defines["MATMUL_VARIANT"], defines["MATMUL_ROWS_PER_WAVE"] = "grid", rows
+    if tail is not None:
+        defines["MATMUL_GROUP_TAIL"] = tail
     return load_native("matmul", defines).call(*args).cpu().double().numpy()
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("kt,k", [("spectral", 2), ("spectral", 40), ("rbf", 3), ("rbf", 70)])
+@pytest.mark.parametrize("rows,tail", [(16, None), (32, None), (64, None), (128, None), (128, 1)])
+@pytest.mark.parametrize("layout", ["rows", "columns", "slice"])
+def test_rhs_values_that_are_not_finite(kt, k, rows, tail, layout, value):
+    """A value of rhs that is not finite reaches every row whose range holds its column, however far
+    away, in its own rhs column and no other; everything else keeps its bits.  Columns near the rows
+    and out of their reach, in the first, a middle and the last step of a range, with rhs dense across
+    its rows, along its columns and neither."""
+    n = 2048
+    x = _points(n, n / 10.0, 40)
+    rhs = torch.randn(n, k, generator=torch.Generator().manual_seed(41))
+    start, end = _ranges(n, n, 900)
+    params = _params(kt, 1.0)
+    def laid_out(t):
+        t = t.to(DEVICE)
+        if layout == "columns":
+            return t.T.contiguous().T
+        return torch.cat([t, t], dim=1)[:, :k] if layout == "slice" else t
+
+    clean = _run_nan(kt, x, x, laid_out(rhs), params, start, end, rows, tail)
+    assert np.all(np.isfinite(clean))
+    column = k - 1
+    for j in (0, 700, 1024, int(end[5]) - 1, int(start[9]), n - 1):
+        bad = rhs.clone()
+        bad[j, column] = value
+        out = _run_nan(kt, x, x, laid_out(bad), params, start, end, rows, tail)
+        hit = np.array([bool(start[i // 128] <= j < end[i // 128]) for i in range(n)])
+        assert hit.any() and not np.isfinite(out[hit, column]).any(), j
+        assert np.array_equal(out[~hit], clean[~hit]), j
+        assert np.array_equal(np.delete(out, column, 1), np.delete(clean, column, 1)), j
+
+
+@pytest.mark.parametrize("kt,k", [("spectral", 1), ("spectral", 20), ("rbf", 5), ("rbf", 33)])
+@pytest.mark.parametrize("rows", [32, 128])
+@pytest.mark.parametrize("lengthscale", [1.0, 0.03])
+def test_rhs_values_that_are_not_finite_in_a_long_range(kt, k, rows, lengthscale):
+    """Ranges of more steps than are noted one by one, in the grid form and entry by entry."""
+    n = 9000
+    x = _points(n, n / 10.0, 48)
+    rhs = torch.randn(n, k, generator=torch.Generator().manual_seed(49))
+    blocks = (n + 127) // 128
+    start, end = torch.zeros(blocks, dtype=torch.int32), torch.full((blocks,), n, dtype=torch.int32)
+    clean = _run_nan(kt, x, x, rhs, _params(kt, lengthscale), start, end, rows)
+    for j in (0, 2047, 2048, 5000, n - 1):
+        bad = rhs.clone()
+        bad[j, k - 1] = float("nan")
+        out = _run_nan(kt, x, x, bad, _params(kt, lengthscale), start, end, rows)
+        assert not np.isfinite(out[:, k - 1]).any(), j
+        assert np.array_equal(out[:, :k - 1], clean[:, :k - 1]), j
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("kt,k", [("spectral", 2), ("spectral", 40), ("rbf", 3), ("rbf", 70)])
+@pytest.mark.parametrize("rows,tail", [(16, None), (32, None), (64, None), (128, None), (128, 1)])
+def test_column_coordinates_that_are_not_finite(kt, k, rows, tail, value):
+    """A column's NaN reaches every row whose range holds it.  An infinite coordinate does where the
+    kernel has an oscillating factor, and is out of reach of every row otherwise (exp(-inf) = 0).  The
+    rows of such a range are evaluated entry by entry, within the form's bound of the clean result."""
+    n = 2048
+    x = _points(n, n / 10.0, 42)
+    rhs = torch.randn(n, k, generator=torch.Generator().manual_seed(43))
+    start, end = _ranges(n, n, 900)
+    params = _params(kt, 1.0)
+    for j in (0, 700, 1024, int(end[5]) - 1, n - 1):
+        moved, without = x.clone(), rhs.clone()
+        moved[j] = value
+        without[j] = 0.0
+        clean = _run_nan(kt, x, x, without, params, start, end, rows, tail)
+        out = _run_nan(kt, x, moved, rhs, params, start, end, rows, tail)
+        hit = np.array([bool(start[i // 128] <= j < end[i // 128]) for i in range(n)])
+        if kt == "spectral" or value != value:
+            assert not np.isfinite(out[hit]).any(), j
+        else:
+            size = np.abs(without.double().numpy())
+            bound = 4e-6 * (np.abs(oracle.dense("rbf", x.numpy(), x.numpy(), params.numpy(), start.numpy(), end.numpy()))
+                            @ size) + 2.0 ** -35 * size.sum(0)
+            assert np.all(np.abs(out - clean)[hit] <= bound[hit]), j
+        assert np.all(np.isfinite(out[~hit])), j
 
 
 def test_variant_is_refused_for_other_kernels():
