@@ -45,9 +45,10 @@ __device__ __forceinline__ float uniform(float v) {
     return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
 }
 
-// (On the bits: a vote over m < inf comes out as a vote over m != inf, true for a NaN, from this compiler.)
+// (On the bits without the sign: a vote over v < inf, or over exponent bits that are not all ones, which it
+// takes for the same, comes out of this compiler as a vote over v != inf, true for a NaN.)
 __device__ __forceinline__ bool is_finite(float v) {
-    return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u;
+    return __float_as_uint(v) << 1 < 0xff000000u;
 }
 
 // Grid window of one row block (the same in every lane).

@@ -70,8 +70,9 @@ struct GradArgs {
 // in fp32.
 #define KM_GRAD_REACH 12.25f
 
-// SKIP (rows sparse against the lengthscale): tiles of 16 rows by 16 columns of which every entry is
-// zero in fp32 are left out (see KM_GRAD_REACH): the sums are the same.
+// SKIP (rows sparse against the lengthscale; TL > 0): tiles of 16 rows by 16 columns of which every entry
+// is zero in fp32 are left out (see KM_GRAD_REACH): the sums are the same.  Rows and columns with a value
+// that is not finite are never left out (zero times it is NaN).
 template <int KT, int TL, int R, bool FAST = false, bool SKIP = false>
 __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __restrict__ x1,
                                               const float* __restrict__ x2, const float* __restrict__ left,
@@ -174,24 +175,30 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
     float acc[KM_MAX_PARAMS] = {0.0f, 0.0f, 0.0f, 0.0f};
 
     // Coordinates beyond which a column is out of the reach of a row group (everything is within
-    // reach of a group with a NaN).
+    // reach of a group with a value that is not finite).
     float reach_lo[R], reach_hi[R];
     if (SKIP) {
         const float reach = KM_GRAD_REACH / kc.s;
 #pragma unroll
         for (int r = 0; r < R; r++) {
             float lo = __builtin_inff(), hi = -__builtin_inff();
+            bool finite = true;
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const bool nan = x1q[r][v] != x1q[r][v];
-                lo = fminf(lo, nan ? -__builtin_inff() : x1q[r][v]);
-                hi = fmaxf(hi, nan ? __builtin_inff() : x1q[r][v]);
+                lo = fminf(lo, x1q[r][v]);
+                hi = fmaxf(hi, x1q[r][v]);
+                finite = finite && is_finite(x1q[r][v]);
             }
+#pragma unroll
+            for (int t = 0; t < TLR; t++) {
+                finite = finite && is_finite(lreg[r][t]);
+            }
+            finite = __all(finite);
             lo = -column_max(-lo);
             hi = column_max(hi);
             // (and half an ulp that either sum may be rounded by)
-            reach_lo[r] = uniform(lo - (reach + 1.2e-7f * fabsf(lo)));
-            reach_hi[r] = uniform(hi + (reach + 1.2e-7f * fabsf(hi)));
+            reach_lo[r] = uniform(finite ? lo - (reach + 1.2e-7f * fabsf(lo)) : -__builtin_inff());
+            reach_hi[r] = uniform(finite ? hi + (reach + 1.2e-7f * fabsf(hi)) : __builtin_inff());
         }
     }
 
@@ -269,7 +276,15 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
             for (int r = 0; r < R; r++) {
                 need |= (unsigned)(__any(!(x2v < reach_lo[r] || x2v > reach_hi[r])) != 0) << r;
             }
-            if (TL > 0 && need != (1u << R) - 1) {
+            float m = fabsf(x2v);
+#pragma unroll
+            for (int t = 0; t < TLR; t++) {
+                m = __builtin_elementwise_maximum(m, fabsf(rvs[t]));
+            }
+            if (!__all(is_finite(m))) {
+                need = (1u << R) - 1;
+            }
+            if (need != (1u << R) - 1) {
 #pragma unroll
                 for (int r = 0; r < R; r++) {
                     if ((need >> r & 1) == 0) {
@@ -285,9 +300,6 @@ __device__ __forceinline__ void pairwise_item(const GradArgs& a, const float* __
                         accumulate_pair<KT>(x1q[r][v], x2v, c[v], kc, acc);
                     }
                 }
-                continue;
-            }
-            if (need == 0) {
                 continue;
             }
         }
@@ -926,10 +938,10 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     for (int j = 0; j < STEPS; j++) {
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-            m = fmaxf(m, fabsf(raw[j][0][t]));
+            m = __builtin_elementwise_maximum(m, fabsf(raw[j][0][t]));
         }
     }
-    m = column_max(m);
+    m = column_maximum(m);
     fine = fine && __all(!rl.used[0] || is_finite(m));
     if (!fine) {
         return false;
@@ -1123,7 +1135,7 @@ __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3)
             return;
         }
     }
-    pairwise_item<KT, TL, 8, true, true>(a, g.x1, g.x2, g.left, g.right, kc, g.row0, g.col_begin, g.col_end, prow);
+    pairwise_item<KT, TL, 8, true, (TL > 0)>(a, g.x1, g.x2, g.left, g.right, kc, g.row0, g.col_begin, g.col_end, prow);
 }
 
 struct ReduceArgs {

@@ -199,3 +199,30 @@ def test_distant_entries_of_sparse_points(kt, c, i, j, spacing):
     result = _call(kt, *(t.to(DEVICE) for t in (x, x, left, right, params, start, end)))
     expected = oracle.param_grad(kt, *(t.numpy() for t in (x, x, left, right, params, start, end)))
     assert np.all(np.abs(result - expected) <= 2e-5 * np.abs(expected)), (result, expected)
+
+
+@pytest.mark.parametrize("which", ["x2", "left", "right"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("kt,c,step,n", [("spectral", 4, 0.1, 640), ("spectral", 4, 0.7, 640), ("rbf", 6, 0.1, 640),
+                                         ("rbf", 6, 0.7, 640), ("spectral", 11, 0.01, 2304), ("spectral", 11, 0.7, 640),
+                                         ("rbf", 20, 0.01, 2304), ("rbf", 20, 0.7, 640)])
+def test_values_out_of_reach_that_are_not_finite(kt, c, step, n, value, which):
+    """Also a value that only meets entries which vanish: the gradient is not finite then (zero times a
+    NaN or an infinity; an infinite coordinate of an rbf kernel makes the lengthscale's component so)."""
+    near = torch.arange(n) * step
+    x1 = torch.cat([near, near[-1] + 1000.0 + 0.01 * torch.arange(128)])
+    x2 = torch.cat([-1000.0 + 0.01 * torch.arange(75), near])
+    blocks = len(x1) // 128
+    start, end = torch.zeros(blocks, dtype=torch.int32), torch.full((blocks,), len(x2), dtype=torch.int32)
+    for place in (0, 40, 74) if which != "left" else (n, n + 100, n + 127):
+        tensors = {"x1": x1, "x2": x2.clone(), "left": _vectors(len(x1), c, 50), "right": _vectors(len(x2), c, 51)}
+        tensors[which][place] = value
+        args = [t.to(DEVICE) for t in (*tensors.values(), _params(kt, 0.5), start, end)]
+        result = _call_nan(kt, *args)
+        if kt == "rbf" and which == "x2" and value == value:
+            result = result[:1]
+        assert not np.isfinite(result).any(), (place, result)
+
+
+def _call_nan(kt, *args):
+    return load_native("bilinear_derivative", BilinearDerivativeConfiguration(kt).make_config(args)).call(*args).cpu().numpy()
