@@ -504,7 +504,7 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
                 scale[g] = 0.0f;
             } else if (grow) {
                 const int e = __builtin_amdgcn_frexp_expf(m);
-                const int new_shift = min(max(14 - e, -100), 100);
+                const int new_shift = min(14 - e, 100);
                 const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {

@@ -946,7 +946,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     if (!fine) {
         return false;
     }
-    const int e = min(max(14 - __builtin_amdgcn_frexp_expf(m), -100), 100);
+    const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 100);
     const float up = rl.used[0] ? __builtin_ldexpf(1.0f, e) : 0.0f;
     half8v bhi[STEPS][GE], blo[STEPS][GE];
 #pragma unroll
@@ -971,7 +971,6 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     }
 
     const float t0 = (gw.g_lo + (float)li) * gw.h;
-    const float down_columns = __builtin_ldexpf(1.0f, -shift[0] - KM_GRID_KS1);
     float s[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
@@ -1061,7 +1060,7 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
             float mv[GE];
 #pragma unroll
             for (int part = 0; part < GE; part++) {
-                mv[part] = acc[mt][part][v] * down_columns;
+                mv[part] = acc[mt][part][v];
                 s[0] = __builtin_fmaf(rows[0][part][v], mv[part], s[0]);
                 s[1] = __builtin_fmaf(rows[1][part][v], mv[part], s[1]);
             }
@@ -1076,10 +1075,11 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
             }
         }
     }
-    const float down_rows = __builtin_ldexpf(1.0f, -e - KM_GRID_KS1);
+    // Both sides' scales at once: a side on its own may be out of range where the product is not.
+    const int down = -shift[0] - e - 2 * KM_GRID_KS1;
 #pragma unroll
     for (int p = 0; p < 3; p++) {
-        sums[p] = __builtin_fmaf(s[p], down_rows, sums[p]);
+        sums[p] += __builtin_ldexpf(s[p], down);
     }
     // All reads of the table are done before the next pass overwrites it.
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

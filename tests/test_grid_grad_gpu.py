@@ -226,3 +226,16 @@ def test_values_out_of_reach_that_are_not_finite(kt, c, step, n, value, which):
 
 def _call_nan(kt, *args):
     return load_native("bilinear_derivative", BilinearDerivativeConfiguration(kt).make_config(args)).call(*args).cpu().numpy()
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("c", [1, 4, 6, 8, 11, 20])
+@pytest.mark.parametrize("left_scale,right_scale", [(1e-30, 1e33), (1e30, 1e-28), (1e-6, 1e37), (1e36, 1e-4)])
+def test_scales_that_cancel(kt, c, left_scale, right_scale):
+    """Vectors whose products are of ordinary size although they are not, as in a solve with a tiny or
+    huge diagonal."""
+    n = 2600
+    x = _points(n, 26.0, 52)
+    start, end = _ranges(n, n, 2 * n)
+    left, right = _vectors(n, c, 53) * left_scale, _vectors(n, c, 54) * right_scale
+    _check(kt, x, x, left, right, _params(kt, 1.3), start, end)
