@@ -24,6 +24,9 @@ namespace km {
 
 // Columns in a row block's range from which the grid form is taken.
 #define KM_GRID_MIN_WIDTH 160
+// Sums are exchanged between wavefronts times 2^-16: those over a grid point's columns can be larger than
+// any result.
+#define KM_GRID_EXCHANGE 16
 
 __device__ __forceinline__ GridVectors vectors(const FwdArgs& a) {
     return {a.x2_s, a.rhs_s0, a.rhs_s1, a.k};
@@ -100,7 +103,7 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
         unsigned* flags = (unsigned*)(lds + grid_lds_floats<GE, MT, W>() - W * (GE + 1));
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1);
+            const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1 - KM_GRID_EXCHANGE);
 #pragma unroll
             for (int m = 0; m < MT; m++) {
 #pragma unroll
@@ -190,11 +193,11 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
             }
         }
         m = column_max(m);
-        const int e = min(max(14 - __builtin_amdgcn_frexp_expf(m), -100), 100);
+        const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 100);
         const float up = __builtin_ldexpf(1.0f, e);
         down[g] = shift[g % G] == KM_GRID_NOT_FINITE
                       ? __builtin_nanf("")
-                      : weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 - (W > 1 ? 0 : shift[g % G] + KM_GRID_KS1));
+                      : weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 + (W > 1 ? KM_GRID_EXCHANGE : -shift[g % G] - KM_GRID_KS1));
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ks++) {
             if (2 * ks < gw.tiles) {

@@ -306,3 +306,21 @@ def test_block_around_the_origin(kt, rows):
     error = np.sqrt(np.mean(np.concatenate(relative) ** 2))
     print(f"2-norm of the relative error: {error:.2e}")
     assert error < 8e-7
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("scale,sigma", [(4e36, 1e-3), (1e-28, 1.0), (1e-20, 1e15)])
+def test_rhs_scales(kt, rows, scale, sigma):
+    """rhs so large that its sums over a grid point's columns are not representable although the
+    product is, and very small ones; columns of different scales beside them."""
+    n = 1000
+    x = _points(n, 10.0, 46)
+    rhs = torch.rand(n, 3, generator=torch.Generator().manual_seed(47)) * scale
+    rhs[:, 1] *= 1e-4
+    params = _params(kt, 1.0)
+    params[-1] = sigma
+    if kt == "spectral":
+        params[1] = 0.01
+    start, end = _ranges(n, n, 700)
+    _check(kt, x, x, rhs, params, start, end, rows=rows)
