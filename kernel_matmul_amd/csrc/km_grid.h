@@ -81,8 +81,15 @@ template <int MT>
 __device__ __forceinline__ GridWindow grid_window(const BlockRows& rows, const KernelConsts& kc,
                                                   float step = KM_GRID_STEP) {
     GridWindow gw;
-    gw.x_ref = uniform(rows.middle);
     const float xa = rows.xa, xb = rows.xb;
+    gw.x_ref = uniform(rows.middle);
+    if (!is_finite(gw.x_ref)) {
+        // Any row that is: the origin must not hand its value on to the others' phases.
+        const unsigned long long finite_a = __ballot(is_finite(xa)), finite_b = __ballot(is_finite(xb));
+        const float other = finite_a != 0 ? __shfl(xa, __builtin_ctzll(finite_a), 64)
+                                          : (finite_b != 0 ? __shfl(xb, __builtin_ctzll(finite_b), 64) : 0.0f);
+        gw.x_ref = uniform(other);
+    }
     float lo = fminf(xa - gw.x_ref, xb - gw.x_ref);
     float hi = fmaxf(xa - gw.x_ref, xb - gw.x_ref);
     const bool finite = __all(fabsf(xa - gw.x_ref) + fabsf(xb - gw.x_ref) < 1e30f);

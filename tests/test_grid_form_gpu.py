@@ -324,3 +324,25 @@ def test_rhs_scales(kt, rows, scale, sigma):
         params[1] = 0.01
     start, end = _ranges(n, n, 700)
     _check(kt, x, x, rhs, params, start, end, rows=rows)
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("row", [0, 63, 64, 127, 192])
+@pytest.mark.parametrize("rows", [16, 32, 128])
+def test_a_row_coordinate_that_is_not_finite_stays_in_its_row(kt, value, row, rows):
+    """Also for the block's middle row, the origin of its relative coordinates."""
+    n = 300
+    x = _points(n, 30.0, 44)
+    rhs = torch.randn(n, 2, generator=torch.Generator().manual_seed(45))
+    start, end = _ranges(n, n, 250)
+    moved = x.clone()
+    moved[row] = value
+    out = _run_nan(kt, moved, x, rhs, _params(kt, 1.0), start, end, rows)
+    clean = _run_nan(kt, x, x, rhs, _params(kt, 1.0), start, end, rows)
+    if kt == "spectral" or value != value:
+        assert not np.isfinite(out[row]).any()
+    else:
+        assert np.all(out[row] == 0.0)
+    others = np.arange(n) != row
+    assert np.allclose(out[others], clean[others], rtol=0.0, atol=2e-5)
