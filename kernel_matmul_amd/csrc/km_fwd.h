@@ -222,8 +222,9 @@ __device__ __forceinline__ WaveView wave_view(const FwdArgs& a, long long item, 
     w.params = a.params + off_params;
     // Clamped to the valid columns: a symmetric pattern over fewer points than one block
     // reports end = block size > n (native/ranges/ranges.cpp:82-93 of the reference).
-    w.range_start = max(a.start[off_start + w.row_block * a.start_s], 0);
-    w.range_end = min(a.end[off_end + w.row_block * a.end_s], a.n);
+    // An empty range ends where it starts, whatever the two values: nothing added to them overflows.
+    w.range_end = max(min(a.end[off_end + w.row_block * a.end_s], a.n), 0);
+    w.range_start = min(max(a.start[off_start + w.row_block * a.start_s], 0), w.range_end);
     return w;
 }
 

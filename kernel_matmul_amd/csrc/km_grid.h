@@ -645,16 +645,18 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
     BeyondSteps beyond = {0, 64, 0};
     int chunk = 0;
     static_assert(CH / 32 == 8, "eight steps a chunk");
-    for (int first = w.range_start + 32 * wave; first < w.range_end; first += CH * W) {
+    // (counted by what is left: a next first column may lie past the largest int)
+    for (int left = w.range_end - w.range_start - 32 * wave; left > 0; left -= CH * W) {
+        const int first = w.range_end - left;
         const unsigned steps = grid_table<GRID, PHASE>(xv, first, W, w.range_end, gw, kc, tab, &fine);
-        if (first + CH * W < w.range_end) {
+        if (left > CH * W) {
             grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
         }
         unsigned need = steps & 0xffff;
         if (!GRID) {
             // (the caller has looked at all steps)
         } else if (EACH_CHUNK) {
-            const int present = min((w.range_end - 1 - first) / (32 * W) + 1, CH / 32);
+            const int present = min((left - 1) / (32 * W) + 1, CH / 32);
             look_at_steps<G>(a, w, kbase, first, 32 * W, {~need & ((1u << present) - 1), 0, 0}, rl, shift, scale);
         } else if (chunk < 8) {
             beyond.bits |= (unsigned long long)(~need & 0xff) << (8 * chunk);
@@ -698,8 +700,9 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
         __builtin_amdgcn_wave_barrier();
     }
 
-    if (GRID && !EACH_CHUNK && w.range_start + 32 * wave < w.range_end) {
-        beyond.total = (w.range_end - 1 - (w.range_start + 32 * wave)) / (32 * W) + 1;
+    const int columns = w.range_end - w.range_start - 32 * wave;
+    if (GRID && !EACH_CHUNK && columns > 0) {
+        beyond.total = (columns - 1) / (32 * W) + 1;
         if (beyond.total < 64) {
             beyond.bits &= (1ull << beyond.total) - 1;
         }

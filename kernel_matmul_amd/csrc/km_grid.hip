@@ -275,7 +275,8 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
             rhs_shift[g] = 0;
             rhs_scale[g] = 0.0f;
         }
-        const int steps = (max(w.range_end - w.range_start, 0) + 31) / 32;
+        const int width = w.range_end - w.range_start;
+        const int steps = width > 0 ? (width - 1) / 32 + 1 : 0;
         look_at_steps<G>(vectors(a), w, kbase, w.range_start, 32, {steps < 64 ? (1ull << steps) - 1 : ~0ull, 64, steps},
                          rhs_lane<G>(vectors(a), kbase), rhs_shift, rhs_scale);
     }
@@ -348,7 +349,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     kc.s = uniform(kc.s);
     __builtin_amdgcn_sched_barrier(0);
     float xv[KM_GRID_CHUNK / 64];
-    if (w.range_start + 32 * wave < w.range_end) {
+    if (32 * wave < w.range_end - w.range_start) {
         grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
     }
     const GridWindow gw = grid_window<S::MT>(rows, kc);
@@ -358,7 +359,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     for (int pass = 0; pass < G / S::GP; pass++) {
         const int kbase = (blockIdx.y * G + pass * S::GP) * 16;
         if (kbase < a.k) {
-            if (pass > 0 && w.range_start + 32 * wave < w.range_end) {
+            if (pass > 0 && 32 * wave < w.range_end - w.range_start) {
                 grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
             }
             grid = grid && grid_forward<KT, S::GP, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv);

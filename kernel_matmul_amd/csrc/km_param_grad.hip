@@ -428,16 +428,17 @@ __device__ __forceinline__ bool grad_item(const GradArgs& a, int rows_per_item, 
     }
     int range_start = a.start[off_start + row_block * a.start_s];
     int range_end = a.end[off_end + row_block * a.end_s];
-    range_start = max(range_start, 0);
-    range_end = min(range_end, a.n);
+    range_end = max(min(range_end, a.n), 0);
+    range_start = min(max(range_start, 0), range_end);
     // Column share of this wavefront, in whole steps of col_step columns.
-    const int width = max(range_end - range_start, 0);
+    const int width = range_end - range_start;
     g->width = width;
     g->split = split;
     g->range_start = range_start;
     const int per_split = ((width + a.col_splits - 1) / a.col_splits + col_step - 1) & ~(col_step - 1);
-    g->col_begin = range_start + split * per_split;
-    g->col_end = min(range_end, g->col_begin + per_split);
+    // (shares are rounded up: the last ones may lie past the range, and past the largest int)
+    g->col_begin = (int)min(range_start + (long long)split * per_split, (long long)range_end);
+    g->col_end = g->col_begin + min(per_split, range_end - g->col_begin);
     return true;
 }
 
@@ -1109,8 +1110,8 @@ __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3)
         const int shares = min(a.col_splits, max(g.width / KM_GG_SHARE, 1));
         const int per_share = ((g.width + shares - 1) / shares + 31) & ~31;
         const int range_end = g.range_start + g.width;
-        g.col_begin = g.split < shares ? g.range_start + g.split * per_share : range_end;
-        g.col_end = min(range_end, g.col_begin + per_share);
+        g.col_begin = g.split < shares ? (int)min(g.range_start + (long long)g.split * per_share, (long long)range_end) : range_end;
+        g.col_end = g.col_begin + min(per_share, range_end - g.col_begin);
         bool done = true;
         float sums[3] = {0.0f, 0.0f, 0.0f};
         if (g.col_begin < g.col_end) {

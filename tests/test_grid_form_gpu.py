@@ -346,3 +346,27 @@ def test_a_row_coordinate_that_is_not_finite_stays_in_its_row(kt, value, row, ro
         assert np.all(out[row] == 0.0)
     others = np.arange(n) != row
     assert np.allclose(out[others], clean[others], rtol=0.0, atol=2e-5)
+
+
+@pytest.mark.parametrize("kt,k", [("spectral", 1), ("spectral", 20), ("rbf", 1), ("rbf", 40)])
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+def test_ranges_at_the_largest_sizes(kt, k, rows):
+    """The last columns of as many as the entry point takes (one point and one row, repeated), and empty
+    ranges of the largest values: nothing past the largest int is formed."""
+    n, m, width = 2**31 - 1 - 128, 300, 700
+    x1, one = _points(m, 3.0, 55), torch.ones(1)
+    rhs = torch.randn(1, k, generator=torch.Generator().manual_seed(56))
+    start = torch.tensor([n - width, 2**31 - 1, n], dtype=torch.int32)
+    end = torch.tensor([n, 2**31 - 1, -2**31], dtype=torch.int32)
+    params = _params(kt, 1.0)
+    args = [x1.to(DEVICE), one.to(DEVICE).expand(n), rhs.to(DEVICE).expand(n, k), params.to(DEVICE), start.to(DEVICE), end.to(DEVICE)]
+    defines = MatmulSingleConfiguration(kt).make_config(args)
+    defines["MATMUL_VARIANT"], defines["MATMUL_ROWS_PER_WAVE"] = "grid", rows
+    out = load_native("matmul", defines).call(*args).cpu().double().numpy()
+    column = oracle.matmul(kt, x1.numpy(), one.numpy(), rhs.numpy(), params.numpy(), np.zeros(3, np.int32), np.ones(3, np.int32))
+    expected = width * column
+    expected[128:] = 0.0
+    envelope = np.abs(oracle.dense("rbf", x1.numpy(), one.numpy(), params[[0, -1]].numpy(), np.zeros(3, np.int32), np.ones(3, np.int32)))
+    bound = 3e-6 * width * envelope @ np.abs(rhs.double().numpy())
+    bound[128:] = 0.0
+    assert np.all(np.abs(out - expected) <= bound)

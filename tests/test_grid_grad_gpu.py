@@ -239,3 +239,23 @@ def test_scales_that_cancel(kt, c, left_scale, right_scale):
     start, end = _ranges(n, n, 2 * n)
     left, right = _vectors(n, c, 53) * left_scale, _vectors(n, c, 54) * right_scale
     _check(kt, x, x, left, right, _params(kt, 1.3), start, end)
+
+
+@pytest.mark.parametrize("kt,c", [("spectral", 3), ("spectral", 12), ("rbf", 5), ("rbf", 20)])
+@pytest.mark.parametrize("width", [700, 4000])
+def test_ranges_at_the_largest_sizes(kt, c, width):
+    """The last columns of as many as the entry point takes (one point and one row, repeated), and empty
+    ranges of the largest values: nothing past the largest int is formed."""
+    n, m = 2**31 - 1 - 128, 300
+    x1, one = _points(m, 3.0, 55), torch.ones(1)
+    left, right = _vectors(m, c, 57), _vectors(1, c, 58)
+    start = torch.tensor([n - width, 2**31 - 1, n], dtype=torch.int32)
+    end = torch.tensor([n, 2**31 - 1, -2**31], dtype=torch.int32)
+    params = _params(kt, 1.0)
+    result = _call(kt, x1.to(DEVICE), one.to(DEVICE).expand(n), left.to(DEVICE), right.to(DEVICE).expand(n, c),
+                   *(t.to(DEVICE) for t in (params, start, end)))
+    first = np.array([0, 1, 1], np.int32), np.ones(3, np.int32)
+    expected = width * oracle.param_grad(kt, *(t.numpy() for t in (x1, one, left, right, params)), *first)
+    size = np.abs(left[:128].double().numpy()) @ np.abs(right.double().numpy().T)
+    # (distances up to two lengthscales: the derivatives' factors are below 15)
+    assert np.all(np.abs(result - expected) <= 4e-6 * 15.0 * width * size.sum()), (result, expected)
