@@ -81,15 +81,8 @@ template <int MT>
 __device__ __forceinline__ GridWindow grid_window(const BlockRows& rows, const KernelConsts& kc,
                                                   float step = KM_GRID_STEP) {
     GridWindow gw;
-    const float xa = rows.xa, xb = rows.xb;
     gw.x_ref = uniform(rows.middle);
-    if (!is_finite(gw.x_ref)) {
-        // Any row that is: the origin must not hand its value on to the others' phases.
-        const unsigned long long finite_a = __ballot(is_finite(xa)), finite_b = __ballot(is_finite(xb));
-        const float other = finite_a != 0 ? __shfl(xa, __builtin_ctzll(finite_a), 64)
-                                          : (finite_b != 0 ? __shfl(xb, __builtin_ctzll(finite_b), 64) : 0.0f);
-        gw.x_ref = uniform(other);
-    }
+    const float xa = rows.xa, xb = rows.xb;
     float lo = fminf(xa - gw.x_ref, xb - gw.x_ref);
     float hi = fmaxf(xa - gw.x_ref, xb - gw.x_ref);
     const bool finite = __all(fabsf(xa - gw.x_ref) + fabsf(xb - gw.x_ref) < 1e30f);
@@ -645,18 +638,18 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
     BeyondSteps beyond = {0, 64, 0};
     int chunk = 0;
     static_assert(CH / 32 == 8, "eight steps a chunk");
-    // (counted by what is left: a next first column may lie past the largest int)
-    for (int left = w.range_end - w.range_start - 32 * wave; left > 0; left -= CH * W) {
-        const int first = w.range_end - left;
+    // (unsigned: the next first column may lie past the largest int)
+    for (unsigned next_first = w.range_start + 32u * wave; next_first < (unsigned)w.range_end; next_first += CH * W) {
+        const int first = (int)next_first;
         const unsigned steps = grid_table<GRID, PHASE>(xv, first, W, w.range_end, gw, kc, tab, &fine);
-        if (left > CH * W) {
+        if (next_first + CH * W < (unsigned)w.range_end) {
             grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
         }
         unsigned need = steps & 0xffff;
         if (!GRID) {
             // (the caller has looked at all steps)
         } else if (EACH_CHUNK) {
-            const int present = min((left - 1) / (32 * W) + 1, CH / 32);
+            const int present = min((w.range_end - 1 - first) / (32 * W) + 1, CH / 32);
             look_at_steps<G>(a, w, kbase, first, 32 * W, {~need & ((1u << present) - 1), 0, 0}, rl, shift, scale);
         } else if (chunk < 8) {
             beyond.bits |= (unsigned long long)(~need & 0xff) << (8 * chunk);

@@ -266,6 +266,14 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
     constexpr int R = W == 8 ? 1 : 2;
     constexpr int PIECES = 8 / (W * R);
     const int li = threadIdx.x & 15;
+    GridWindow rows = gw;
+    if (!is_finite(rows.x_ref)) {
+        // Any row that is: the origin must not hand its value on to the other rows' phases.
+        const BlockRows block = block_rows(w.x1, a.x1_s, row0, a.m);
+        const unsigned long long in_a = __ballot(is_finite(block.xa)), in_b = __ballot(is_finite(block.xb));
+        rows.x_ref = uniform(in_a != 0 ? __shfl(block.xa, __builtin_ctzll(in_a), 64)
+                                       : (in_b != 0 ? __shfl(block.xb, __builtin_ctzll(in_b), 64) : 0.0f));
+    }
     // The rhs values of the whole range, once for all rows.
     int rhs_shift[G];
     {
@@ -289,12 +297,11 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
             xr[r] = w.x1[(long long)min(base + 16 * r + li, a.m - 1) * a.x1_s];
         }
         // the columns within reach of these rows
-        GridWindow rows = gw;
-        float lo = xr[0] - gw.x_ref, hi = lo;
+        float lo = xr[0] - rows.x_ref, hi = lo;
         bool finite = true;
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            const float y = xr[r] - gw.x_ref;
+            const float y = xr[r] - rows.x_ref;
             lo = fminf(lo, y);
             hi = fmaxf(hi, y);
             finite = finite && fabsf(y) < 1e30f;
@@ -321,7 +328,7 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            grid_store<KT, G>(a, w, kc, xr[r], gw.x_ref, acc[r], down, base + 16 * r, kbase);
+            grid_store<KT, G>(a, w, kc, xr[r], rows.x_ref, acc[r], down, base + 16 * r, kbase);
         }
     }
 }
