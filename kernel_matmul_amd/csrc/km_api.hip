@@ -149,6 +149,10 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
         opt->rows_per_wave != 32 && opt->rows_per_wave != 64 && opt->rows_per_wave != 128) {
         return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: rows_per_wave must be 16, 32, 64 or 128");
     }
+    if (variant == KM_VARIANT_GRID && opt->col_splits != 0 && opt->col_splits != 1) {
+        return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: the grid form's wavefronts per row block follow from rows_per_wave, "
+                                             "not from col_splits");
+    }
     if (variant == KM_VARIANT_GRID && p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
         return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: the grid form takes rbf and spectral kernels only");
     }

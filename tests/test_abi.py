@@ -101,6 +101,10 @@ def test_launch_descriptions_without_a_gpu():
     assert "param_grad_partial<spectral, TL=2>" in _native.describe_param_grad("spectral", 2, 50_000, 8)
     assert "param_grad_features<rbf, GE=2" in _native.describe_param_grad("rbf", 2, 50_000, 10)
     assert "param_grad_partial<locally_periodic" in _native.describe_param_grad("locally_periodic", 2, 5_000, 3)
+    # a decomposition that the asked-for kernel does not have is refused
+    options = _native.LaunchOptions(variant=7, col_splits=2)
+    with pytest.raises(RuntimeError, match="col_splits"):
+        _native.describe_matmul("rbf", 8, 100_000, 100_000, 16, options)
     lib = _native.load_library()
     buf = ctypes.create_string_buffer(16)
     assert lib.km_param_grad_describe(7, 1, 128, 4, buf, len(buf)) == -2
