@@ -597,19 +597,18 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
     const char* kt = kernels[kernel_type];
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     const int G = plan.k_chunk / 16;
-    size_t used = 0;
-    if (plan.variant == KM_VARIANT_GRID) {
-        used = (size_t)snprintf(text, text_bytes, "km::fwd_grid%s<%s, G=%d, W=%d> (grid form); entry by entry it would be ",
-                                plan.group_tail > 0 ? "_grouped" : "", kt, G, plan.col_splits);
-        if (used >= text_bytes) return KM_OK;
-        km_launch_options entries;
-        memset(&entries, 0, sizeof(entries));
-        entries.variant = KM_VARIANT_MFMA_F16;
-        if (int rc = make_plan(p, &entries, &plan)) return rc;
-        text += used;
-        text_bytes -= used;
-    }
     switch (plan.variant) {
+        case KM_VARIANT_GRID:
+            if (plan.group_tail > 0) {
+                snprintf(text, text_bytes,
+                         "km::fwd_grid_grouped<%s, G=%d>: grid form, one row block per wavefront, 4 wavefronts per workgroup, "
+                         "the last %lld row blocks of each XCD by a workgroup each",
+                         kt, G, plan.group_tail);
+            } else {
+                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefront(s) per row block", kt, G,
+                         plan.col_splits, plan.col_splits);
+            }
+            break;
         case KM_VARIANT_VALU:
             snprintf(text, text_bytes, "km::fwd_valu<%s, KC=%d>: 128 rows per workgroup, %lld workgroups", kt,
                      plan.k_chunk, row_blocks * num_batches * ((k + plan.k_chunk - 1) / plan.k_chunk));
@@ -620,7 +619,6 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                      kt, plan.phase_split, G);
             break;
         default: {
-            const int groups = plan.k_chunk / 16;
             const char* name = plan.variant == KM_VARIANT_MFMA_F32_DIRECT
                                    ? "km::fwd_mfma_f32"
                                    : (plan.variant == KM_VARIANT_MFMA_F32
@@ -642,7 +640,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                 break;
             }
             snprintf(text, text_bytes, "%s<%s, G=%d, R=%d>: %d rows per wavefront, %d wavefront(s) per row range%s",
-                     name, kt, groups, plan.row_groups, 16 * plan.row_groups, plan.col_splits,
+                     name, kt, G, plan.row_groups, 16 * plan.row_groups, plan.col_splits,
                      plan.tail_balance && plan.row_groups == 8 && plan.col_splits == 1 &&
                              plan.variant == KM_VARIANT_MFMA_F16_DIRECT &&
                              row_blocks * num_batches >= 2 * 128 * KM_NUM_XCD

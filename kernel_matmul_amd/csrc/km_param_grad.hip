@@ -1292,17 +1292,12 @@ void describe_param_grad(int kernel_type, int64_t m, long long num_batches, int6
     const FeaturePlan f = feature_plan(kernel_type, c);
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     if (grid_form(kernel_type, c, row_blocks * num_batches * grad_col_splits(row_blocks * num_batches))) {
-        const int used = snprintf(text, text_bytes,
-                                  "km::param_grad_grid<%s%s, TL=%d> (grid form; per-item pairwise fallback), at most %d column "
-                                  "share(s) per row block; for strides or batch shapes that do not suit it: ",
-                                  kernels[kernel_type], kernel_type == KM_KERNEL_SPECTRAL && c <= 8 ? ", packed" : "",
-                                  c <= 4 ? 1 : (c <= 8 ? 2 : (c <= 16 ? 4 : 0)),
-                                  grad_col_splits(row_blocks * num_batches));
-        if (used < 0 || (size_t)used >= text_bytes) {
-            return;
-        }
-        text += used;
-        text_bytes -= (size_t)used;
+        snprintf(text, text_bytes,
+                 "km::param_grad_grid<%s%s, TL=%d>: grid form (pair by pair where it does not suit a row block), at most %d "
+                 "column share(s) per row block",
+                 kernels[kernel_type], kernel_type == KM_KERNEL_SPECTRAL && c <= 8 ? ", packed" : "",
+                 c <= 4 ? 1 : (c <= 8 ? 2 : (c <= 16 ? 4 : 0)), grad_col_splits(row_blocks * num_batches));
+        return;
     }
     const int splits = grad_col_splits(row_blocks * num_batches, f.GE > 0);
     if (f.GE > 0) {

@@ -89,18 +89,31 @@ def test_missing_library_fails_loudly(monkeypatch):
 
 def test_launch_descriptions_without_a_gpu():
     """km_matmul_describe / km_param_grad_describe report the launch tables' choices (host only)."""
-    text = _native.describe_matmul("spectral", 8, 100_000, 100_000, 16, None)
+    matmul, grad = _native.describe_matmul, _native.describe_param_grad
+    # rbf and spectral kernels: the grid form from 48 row blocks on, and nothing else in the text
+    text = matmul("spectral", 8, 100_000, 100_000, 16, None)
+    assert "fwd_grid_grouped<spectral, G=1>" in text and "last 32 row blocks" in text and "fwd_table" not in text
+    assert "fwd_grid<spectral, G=2, W=1>" in matmul("spectral", 8, 1_000_000, 1_000_000, 32, None)
+    assert "fwd_grid<spectral, G=4, W=1>" in matmul("spectral", 8, 1_000_000, 1_000_000, 64, None)
+    assert "fwd_grid<rbf, G=2, W=1>" in matmul("rbf", 8, 1_000_000, 1_000_000, 32, None)
+    assert "fwd_grid<rbf, G=1, W=4>" in matmul("rbf", 1, 65_536, 65_536, 16, None)
+    assert "fwd_table_f16<rbf, G=1" in matmul("rbf", 1, 4096, 4096, 1, None)
+    assert "fwd_block<locally_periodic" in matmul("locally_periodic", 8, 1_000_000, 1_000_000, 16, None)
+    # the kernels evaluated entry by entry, where they are asked for
+    entries = _native.LaunchOptions(variant=3)
+    text = matmul("spectral", 8, 100_000, 100_000, 16, entries)
     assert "fwd_table_f16_grouped<spectral>" in text and "128 rows per wavefront" in text
-    assert "fwd_table_f16<spectral, G=2" in _native.describe_matmul("spectral", 8, 1_000_000, 1_000_000, 32, None)
-    assert "fwd_mfma_f16<spectral, G=4" in _native.describe_matmul("spectral", 8, 1_000_000, 1_000_000, 64, None)
-    assert "fwd_mfma_f16<rbf, G=2" in _native.describe_matmul("rbf", 8, 1_000_000, 1_000_000, 32, None)
-    assert "fwd_table_f16_grouped<rbf>" in _native.describe_matmul("rbf", 8, 1_000_000, 1_000_000, 16, None)
-    assert "fwd_block<locally_periodic" in _native.describe_matmul("locally_periodic", 8, 1_000_000, 1_000_000, 16, None)
-    # narrow vectors: feature form; wide ones and the locally periodic kernel: pairwise form
-    assert "param_grad_features<spectral, GE=2" in _native.describe_param_grad("spectral", 16, 100_000, 4)
-    assert "param_grad_partial<spectral, TL=2>" in _native.describe_param_grad("spectral", 2, 50_000, 8)
-    assert "param_grad_features<rbf, GE=2" in _native.describe_param_grad("rbf", 2, 50_000, 10)
-    assert "param_grad_partial<locally_periodic" in _native.describe_param_grad("locally_periodic", 2, 5_000, 3)
+    assert "fwd_table_f16<spectral, G=2" in matmul("spectral", 8, 1_000_000, 1_000_000, 32, entries)
+    assert "fwd_mfma_f16<spectral, G=4" in matmul("spectral", 8, 1_000_000, 1_000_000, 64, entries)
+    assert "fwd_mfma_f16<rbf, G=2" in matmul("rbf", 8, 1_000_000, 1_000_000, 32, entries)
+    assert "fwd_table_f16_grouped<rbf>" in matmul("rbf", 8, 1_000_000, 1_000_000, 16, entries)
+    # narrow vectors, and wide ones in small launches: grid form; else pairwise
+    assert "param_grad_grid<spectral, packed, TL=1>" in grad("spectral", 16, 100_000, 4)
+    assert "param_grad_features" not in grad("spectral", 16, 100_000, 4)
+    assert "param_grad_partial<spectral, TL=2>" in grad("spectral", 2, 50_000, 8)
+    assert "param_grad_grid<spectral, TL=4>" in grad("spectral", 1, 7200, 11)
+    assert "param_grad_grid<rbf, TL=4>" in grad("rbf", 2, 50_000, 10)
+    assert "param_grad_partial<locally_periodic" in grad("locally_periodic", 2, 5_000, 3)
     # a decomposition that the asked-for kernel does not have is refused
     options = _native.LaunchOptions(variant=7, col_splits=2)
     with pytest.raises(RuntimeError, match="col_splits"):
