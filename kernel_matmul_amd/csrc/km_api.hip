@@ -89,14 +89,16 @@ static const long long BLOCK_VARIANT_MIN_ITEMS = 4096;
 // Grid form (rbf and spectral kernels): wavefronts per 128-row item.  One while that fills the SIMDs
 // (3 resident wavefronts each, 2 for the kernels with more than 32 operand columns), more to make the
 // device busy with fewer items.  Measured at ten points per unit, cutoff of 6 lengthscales, spectral
-// k = 16, wavefronts 1 / 2 / 4 / 8: 157 items 18.0 / 12.1 / 9.8 / 10.5 us (fit-like density of 700
-// points per unit: 151 / 79 / 41 / 31), 628 items 22.8 / 17.5 / 15.7 / 27.4, 782 items 23.1 / 17.8 / 19.4 /
-// 34.7, 2400 items 33.6 / 31.8 / 40.3, 3600 items 42.9 / 44.7 / 56.3.  Below 48 items the entry-wise table
-// kernels in 16-row pieces spread further (32 items: 6.1 against 9.5 us).
+// k = 16, wavefronts 1 / 2 / 4 / 8: 157 items 19.8 / 13.4 / 11.2 / 11.9 us a call (fit-like density of 700
+// points per unit: 151 / 83 / 43 / 32), 628 items 24.2 / 18.2 / 16.1 / 31.9, 782 items 21.7 / 17.3 / 20.5 /
+// 37.7, 2346 items 36.5 / 35.0 / 43.1, 3596 items 49.5 / 50.2 / 61.2.  Below 48 items the entry-wise table
+// kernels in 16-row pieces spread further (32 items: kernels of 6.1 against 9.5 us).
 // From 350 items per XCD on the last 32 of each are split between four wavefronts: without them the
-// items beyond whole rounds of resident wavefronts run alone (782 items per XCD: 66.1 against 61.4 us,
-// 391: 42.0 against 35.3; 600, the worst met: 51.4 against 52.0).  The kernels with two resident
-// wavefronts gain from it only just past a whole round (782: 103.2 against 98.3 us; 600: 79.2 against 81.2).
+// items beyond whole rounds of resident wavefronts run alone (items per XCD 391: 46.5 against 38.6 us, 587:
+// 55.9 against 54.4, 782: 69.7 against 64.5, 978: 81.0 against 80.0, 1173: 95.0 against 90.2, 1369: 106.8
+// against 104.6).  Beyond 1500 the gain depends on how much of a round is left over and is a percent or two
+// (1955: 147.1 against 144.3, 2346: 170.8 against 169.7).  The kernels with two resident wavefronts lose by
+// it at most sizes (spectral k = 32, 489: 82.1 against 83.7, 782: 121.2 against 122.1, 1564: 205 against 226).
 static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int variant, MatmulPlan* plan) {
     const bool automatic = variant == KM_VARIANT_AUTO &&
                            !(opt && (opt->rows_per_wave != 0 || opt->col_splits > 1 || opt->reserved != 0));
@@ -125,11 +127,7 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
         plan->group_tail = -1;
     } else if (plan->group_tail < 0) {
         const long long per_xcd = (per_launch + KM_NUM_XCD - 1) / KM_NUM_XCD;
-        if (two_resident) {
-            plan->group_tail = per_xcd < 1024 && per_xcd % 256 <= 24 ? 16 : -1;
-        } else {
-            plan->group_tail = per_xcd < 1500 ? 32 : -1;
-        }
+        plan->group_tail = !two_resident && per_xcd < 1500 ? 32 : -1;
     }
     return true;
 }
@@ -196,6 +194,8 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
         plan->tail_balance = 0;
         return KM_OK;
     }
+    // From here on for what the grid form does not take: fewer than 48 row-block items, locally periodic
+    // kernels, fp32 contractions, and decompositions asked for by an option.
     // Table kernel (column tables in LDS, separable exponent): rbf and spectral kernels with up
     // to 16 rhs columns, the spectral one in phase-split form (two accumulator sets per rhs
     // column group); spectral kernels with 17 to 32 columns with the cosine per entry from
