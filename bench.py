@@ -42,7 +42,7 @@ WORKLOADS = {
                label="spectral bilinear_derivative n=100000 d=4 batch=16 cutoff=6*l_max"),
     "c5": dict(kernel="spectral", n=1_000_000, extent=100_000.0, batch=8, k=32, cutoff_l=5.0, seed=1005,
                label="spectral K@rhs n=1000000 k=32 batch=8 cutoff=5*l_max"),
-    # gradient at the headline's size with 8 vector columns (beyond the feature form's widths)
+    # gradient at the headline's size with 8 vector columns (pair by pair: wide vectors, many row blocks)
     "grad_c8": dict(kernel="spectral", n=100_000, extent=10_000.0, batch=8, k=8, cutoff_l=6.0, seed=1006, op="param_grad",
                     label="spectral bilinear_derivative n=100000 d=8 batch=8 cutoff=6*l_max"),
     # the reference's own benchmark recipe (examples/matmul.py:61-82 there)
@@ -55,23 +55,24 @@ WORKLOADS = {
 # Untimed continuous launches before a timed region, in milliseconds (clock ramp of the GPU).
 SPIN_UP_MS = 100.0
 
-TRAFFIC_SOURCE = "profiles/fwd_table_f16_grouped_headline_counters.md"
-MEASURED_TRAFFIC_BYTES = {"headline": 58609869}
+TRAFFIC_SOURCE = "profiles/grid_form_kernels_profile.md"
+MEASURED_TRAFFIC_BYTES = {"headline": 61125058}
 
 # Share of the kernel's cycles in which the SIMDs' VALU is busy (SQ_ACTIVE_INST_VALU x 4 / SIMD
 # cycles), from the offline counter runs summarised under profiles/ (not measured by this script).
 VALU_BUSY = {
-    "headline": (0.75, "profiles/fwd_table_f16_grouped_headline_counters.md"),
+    "headline": (0.66, "profiles/grid_form_kernels_profile.md"),
     "headline_fp32": (0.46, "profiles/fwd_table_f32_grouped_headline_profile.md"),
     "c1": (0.11, "profiles/fwd_table_f16_midsize_c1_c2_c3_profile.md"),
-    "c2": (0.46, "profiles/fwd_table_f16_midsize_c1_c2_c3_profile.md"),
+    "c2": (0.32, "profiles/grid_form_kernels_profile.md"),
     "c3": (0.45, "profiles/param_grad_partial_c3_and_wide_vectors_profile.md"),
-    "c3_rhs_grad": (0.47, "profiles/fwd_table_f16_midsize_c1_c2_c3_profile.md"),
-    "c4": (0.73, "profiles/param_grad_features_c4_profile.md"),
-    "c5": (0.95, "profiles/forward_c5_and_reference_recipe_profile.md"),
+    "c4": (0.81, "profiles/grid_form_kernels_profile.md"),
+    "c5": (0.70, "profiles/grid_form_kernels_profile.md"),
     "grad_c8": (0.62, "profiles/param_grad_partial_c3_and_wide_vectors_profile.md"),
-    "ref_example": (0.43, "profiles/forward_c5_and_reference_recipe_profile.md"),
+    "ref_example": (0.28, "profiles/grid_form_kernels_profile.md"),
 }
+
+EXECUTED_PER_64_PAIRS = {"valu_instructions": 5.4, "mfma_f32_16x16x32_f16": 0.23}
 
 
 def pipe_of(kernel_description: str) -> str:
@@ -333,13 +334,13 @@ def main() -> int:
     ap.add_argument("--spin-up-ms", type=float, default=SPIN_UP_MS,
                     help="untimed continuous launches after the warm-up steps (the GPU's clock ramp)")
     ap.add_argument("--workload", default="headline", choices=sorted(WORKLOADS))
-    ap.add_argument("--variant", default="auto", choices=["auto", "block", "mfma_f32", "mfma_f32_direct", "mfma_f16", "mfma_f16_direct", "valu"])
+    ap.add_argument("--variant", default="auto", choices=["auto", "grid", "block", "mfma_f32", "mfma_f32_direct", "mfma_f16", "mfma_f16_direct", "valu"])
     ap.add_argument("--rows-per-wave", type=int, default=0)
     ap.add_argument("--col-splits", type=int, default=0)
     ap.add_argument("--batch", type=int, default=None, help="override the number of batch items")
     ap.add_argument("--no-tail-balance", action="store_true")
     ap.add_argument("--group-tail", type=int, default=None,
-                    help="table kernel: grouped launch with this many column-split items per XCD")
+                    help="grouped launch with this many column-split items per XCD")
     ap.add_argument("--group-tail-halves", type=int, default=None,
                     help="with --group-tail: how many of those items also run as two halves of 64 rows")
     ap.add_argument("--no-cpu-baseline", action="store_true",
@@ -451,17 +452,17 @@ def main() -> int:
             "pipe": pipe_of(main_run.kernel),
             "valu_busy": VALU_BUSY["headline"][0] if default_run else None,
             "valu_busy_source": VALU_BUSY["headline"][1] if default_run else None,
-            # what the launched kernel executes per wavefront-wide group of 64 pairs (SQ_INSTS_VALU and
-            # SQ_INSTS_MFMA of the same counter runs over the 5.14 M groups of a launch)
-            "executed_per_64_pairs": {"valu_instructions": 8.1, "mfma_f32_16x16x32_f16": 0.75}
-                                     if default_run else None,
+            # what the launched kernel executes per wavefront-wide group of 64 pairs of the pattern
+            # (SQ_INSTS_VALU and SQ_INSTS_MFMA of the same counter runs over the 5.14 M groups of a launch)
+            "executed_per_64_pairs": EXECUTED_PER_64_PAIRS if default_run else None,
             "achieved_is": "nominal flops per pair (8 + 2k: direct evaluation, fp32 contraction) x pairs / kernel "
-                           "time; the kernel launched executes fewer VALU operations per pair (separable exponent, "
-                           "tabulated phases) and contracts on the matrix pipe named in `pipe`",
-            "note": "bound by VALU issue (kernel evaluation in fp32 + hi/lo split + MFMA issue), priced against "
-                    "the fp32 peak (157.3 TFLOP/s vector == fp32 MFMA); flops = pairs * (8 + 2k), one "
-                    "transcendental counted as 1.  The contraction itself runs as split-fp16 MFMAs, so frac is "
-                    "a figure of merit against the fp32 roofline, not a utilisation of one pipe",
+                           "time: a normalised throughput.  The grid form does not evaluate pairs: it contracts "
+                           "columns onto some 40 grid points per 128 rows and these onto the rows, so the figure may "
+                           "exceed the peak and is no utilisation of any pipe",
+            "note": "bound by VALU issue (exponentials of the two factors, hi/lo splits, address work) beside the "
+                    "fp16 MFMAs; valu_busy is the share of cycles that the VALU issues in, from the counter run "
+                    "named; flops = pairs * (8 + 2k), one transcendental counted as 1, over the fp32 peak "
+                    "(157.3 TFLOP/s vector == fp32 MFMA)",
         },
     }
 

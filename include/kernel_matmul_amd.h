@@ -68,7 +68,9 @@ typedef struct km_launch_options {
                              7 = split-fp16 MFMA with the Gaussian factor through an equidistant
                              grid (rbf and spectral kernels): columns to grid points, grid points
                              to rows; rows_per_wave chooses 1, 2, 4 or 8 wavefronts per 128 rows
-                             (col_splits must stay 0 or 1).
+                             (col_splits must stay 0 or 1).  A value of rhs or a column
+                             coordinate that is not finite reaches every row whose range holds it,
+                             as with the other variants.
                              The table picks 7 for rbf and spectral kernels from 48 row-block items
                              on, 5 for large locally periodic problems with at most 16 rhs
                              columns and 3 otherwise. */

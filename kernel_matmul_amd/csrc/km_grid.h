@@ -11,7 +11,7 @@
 //     G_g = sum_j V(y_j, t_g) rhs_j        (columns -> grid, "moments")
 //     out_i = C sum_g V(x_i, t_g) G_g      (grid -> rows)
 // and the work per column and per row is one grid window (span of the row block plus twice the
-// reach of V, 20 to 60 points) instead of one entry per row and column of the pattern.  The column
+// reach of V, 20 to 80 points, 96 at most) instead of one entry per row and column of the pattern.  The column
 // ranges [start, end) are honoured exactly: each row block sums the columns of its own range.
 //
 // Coordinates are taken relative to the row block's middle row (exact for neighbouring points; rows

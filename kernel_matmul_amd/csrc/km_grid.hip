@@ -14,6 +14,11 @@
 // same launch: each wavefront its rows, tile against tile, those out of reach left out.  A value of rhs
 // that is not finite makes its column's results NaN in every row whose range holds it, as does a NaN
 // among the range's column coordinates (spectral: an infinity as well) in all columns.
+//
+// Measured against the entry-wise kernels (a call, queued): spectral n = 1e5, k = 16, 8 sets 103.8 -> 64.8 us,
+// n = 1e6, k = 32 1085 -> 891, rbf n = 65536, k = 64 43.6 -> 21.8.  The large ones are bound by VALU issue (66
+// and 70 % of the cycles; exponentials, fma and fp16 roundings are a third of it, the rest rhs scaling,
+// maxima, tables, moves and offsets), the small ones by the latency of one wavefront's steps.
 #include "km_batch.h"
 #include "km_common.h"
 #include "km_fwd.h"

@@ -70,7 +70,8 @@ struct GradArgs {
 // in fp32.
 #define KM_GRAD_REACH 12.25f
 
-// SKIP (rows sparse against the lengthscale; TL > 0): tiles of 16 rows by 16 columns of which every entry
+// SKIP (rows sparse against the lengthscale; TL > 0; the fallback of the grid form, spectral n = 50000,
+// 8 sets, c = 4, one point per unit: 45 us a call against 115 in the feature form): tiles of 16 rows by 16 columns of which every entry
 // is zero in fp32 are left out (see KM_GRAD_REACH): the sums are the same.  Rows and columns with a value
 // that is not finite are never left out (zero times it is NaN).
 template <int KT, int TL, int R, bool FAST = false, bool SKIP = false>
@@ -869,16 +870,16 @@ __global__ void __launch_bounds__(64, 2) param_grad_features(const GradArgs a) {
 // eight of 16 rows, and the vectors' operands do not multiply with the number of features.
 //
 // The polynomial raises the trapezoid rule's error (its first harmonic meets k^2): the grid is a
-// little finer than the forward's, which leaves 1e-8.  Column shares: the moments of a share give
+// little finer than the forward's, which leaves 4e-8 of the envelope in the second moment.  Column shares: the moments of a share give
 // partial sums like those of any other split; every share repeats the rows' side, worth about nine
 // steps of 32 columns, so a share has at least KM_GG_SHARE columns and further wavefronts of a row
 // block write zeros.  Row blocks that the form does not suit (km_grid.hip) take the pairwise form.
 // Up to 8 spectral vector columns are packed with both phases into one group of 16 (PACK); more
 // than 16 take several passes.
 //
-// Measured: spectral n = 1e5, c = 4, 16 sets 245 -> 109 us a call (feature form before; bound by the VALU work
-// of exponentials and operand splits, about half of it on the columns' side); n = 7200 at 720 points
-// per unit, c = 11: 44.7 -> 20.7 us (kernel; pairwise before).
+// Measured: spectral n = 1e5, c = 4, 16 sets 245 -> 110 us a call (feature form before; bound by VALU issue,
+// busy 81 % of the cycles, of which exponentials, fma and fp16 roundings are 45 %); n = 7200 at 720 points
+// per unit, c = 11: 43.9 -> 23.6 us (pairwise before).
 // Resident wavefronts: three per SIMD; two with both phases in separate groups, whose operands would
 // spill 224 bytes a lane at three (29.2 against 23.0 us for the call).
 // ---------------------------------------------------------------------------------------
@@ -1279,8 +1280,10 @@ long long param_grad_feature_partials_per_batch(int kernel_type, int64_t m, long
 // spectral c = 4, ten points per unit: 1.1e-7 against 2.2e-7).  For wider ones the pairwise form forms
 // its coefficients in fp32, which is the more exact way while ranges are short (spectral c = 11, 250 columns
 // per range: 5e-8 against 8e-8; 2400, c = 20: 1.1e-7 both; 10000, c = 11: 3.4e-7 against 1.7e-7): they
-// take the grid form for ranges of KM_GG_MIN_WIDTH_WIDE columns on, in launches of at most two
-// wavefronts per SIMD, where this kernel's lower occupancy costs the other row blocks nothing.
+// take the grid form for ranges of KM_GG_MIN_WIDTH_WIDE columns on, in launches of at most 2048 wavefronts,
+// two per SIMD, where this kernel's lower occupancy costs the other row blocks nothing.  Column shares are
+// cut until there are 4096 or 16 per row block, so that is up to 128 row-block items, a sharp line: with
+// more of them wide vectors go pair by pair whatever their ranges.
 static bool grid_form(int kernel_type, long long c, long long total_items) {
     return kernel_type != KM_KERNEL_LOCALLY_PERIODIC && c > 0 &&
            (feature_plan(kernel_type, c).GE > 0 || total_items <= 2048);
