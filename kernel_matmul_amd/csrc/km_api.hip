@@ -86,19 +86,22 @@ static const long long TARGET_WAVES = 1024;
 // Row-block items from which the workgroup-shared forward kernel is considered.
 static const long long BLOCK_VARIANT_MIN_ITEMS = 4096;
 
-// Grid form (rbf and spectral kernels): wavefronts per 128-row item.  One while that fills the SIMDs
-// (3 resident wavefronts each, 2 for the kernels with more than 32 operand columns), more to make the
-// device busy with fewer items.  Measured at ten points per unit, cutoff of 6 lengthscales, spectral
-// k = 16, wavefronts 1 / 2 / 4 / 8: 157 items 19.8 / 13.4 / 11.2 / 11.9 us a call (fit-like density of 700
-// points per unit: 151 / 83 / 43 / 32), 628 items 24.2 / 18.2 / 16.1 / 31.9, 782 items 21.7 / 17.3 / 20.5 /
-// 37.7, 2346 items 36.5 / 35.0 / 43.1, 3596 items 49.5 / 50.2 / 61.2.  Below 48 items the entry-wise table
-// kernels in 16-row pieces spread further (32 items: kernels of 6.1 against 9.5 us).
-// From 350 items per XCD on the last 32 of each are split between four wavefronts: without them the
-// items beyond whole rounds of resident wavefronts run alone (items per XCD 391: 46.5 against 38.6 us, 587:
-// 55.9 against 54.4, 782: 69.7 against 64.5, 978: 81.0 against 80.0, 1173: 95.0 against 90.2, 1369: 106.8
-// against 104.6).  Beyond 1500 the gain depends on how much of a round is left over and is a percent or two
-// (1955: 147.1 against 144.3, 2346: 170.8 against 169.7).  The kernels with two resident wavefronts lose by
-// it at most sizes (spectral k = 32, 489: 82.1 against 83.7, 782: 121.2 against 122.1, 1564: 205 against 226).
+// Grid form (rbf and spectral kernels): wavefronts per 128-row item, more to make the device busy with few
+// items, or (col_splits 1) workgroups that take four row blocks together.  Measured at ten points per unit,
+// cutoff of 6 lengthscales, spectral k = 16, wavefronts 2 / 4 / 8: 157 items 13.4 / 11.2 / 11.9 us a call
+// (fit-like density of 700 points per unit: 83 / 43 / 32), 628 items 18.2 / 16.1 / 31.9, 782 items 17.3 / 20.5 /
+// 37.7, 2346 items 35.0 / 43.1.  Below 48 items the entry-wise table kernels in 16-row pieces spread further (32
+// items: kernels of 6.1 against 9.5 us).
+// Two wavefronts against groups of four row blocks, whose gain grows with the width of the ranges (n = 50000,
+// two batch items more each; at 10 / at 40 points per unit): spectral k = 16, 1173 items 23.6 / 36.0 against 25.6
+// / 27.9, 1564 items 29.7 / 49.6 against 28.6 / 32.0, 2346 items 34.8 / 56.3 against 35.7 / 39.1; rbf k = 32 1564
+// items 31.4 / 53.1 against 31.5 / 35.4; rbf k = 16, the lightest kernel, 1564 items 22.5 / 37.4 against 25.2 / 28.3,
+// 2346 items 30.2 / 49.0 against 31.2 / 34.0; with more than 32 operand columns two groups are resident where the
+// others have three or four: spectral k = 32 2346 items 55.5 / 87.9 against 60.8 / 64.0.
+// From 350 items per XCD on the last 32 of each get a workgroup each: without them the groups beyond whole
+// rounds run alone (n = 1e5, 8 sets: 65.4 without, 60.5 with 16 to 64, 62.7 with 128; 5 sets 50.0 without, 48.3).
+// Beyond 1500 the gain depends on how much of a round is left over and is a percent or two.  The kernels with
+// two resident groups lose by it at most sizes.
 static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int variant, MatmulPlan* plan) {
     const bool automatic = variant == KM_VARIANT_AUTO &&
                            !(opt && (opt->rows_per_wave != 0 || opt->col_splits > 1 || opt->reserved != 0));
@@ -117,11 +120,13 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     plan->row_groups = 8;
     plan->tail_balance = 0;
     plan->group_tail_halves = 0;
-    const bool two_resident = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1) > 32;
+    const int operands = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1);
+    const bool two_resident = operands > 32;
     if (opt && opt->rows_per_wave != 0) {
         plan->col_splits = KM_BLOCK_SIZE / opt->rows_per_wave;
     } else {
-        plan->col_splits = items <= 200 ? 8 : (items < 700 ? 4 : (items < 2800 ? 2 : 1));
+        const long long grouped = operands > 32 ? 2800 : (operands > 16 ? 1500 : 2300);
+        plan->col_splits = items <= 200 ? 8 : (items < 700 ? 4 : (items < grouped ? 2 : 1));
     }
     if (plan->col_splits != 1) {
         plan->group_tail = -1;
@@ -601,11 +606,13 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
         case KM_VARIANT_GRID:
             if (plan.group_tail > 0) {
                 snprintf(text, text_bytes,
-                         "km::fwd_grid_grouped<%s, G=%d>: grid form, one row block per wavefront, 4 wavefronts per workgroup, "
+                         "km::fwd_grid_grouped<%s, G=%d>: grid form, 4 row blocks per workgroup of 4 wavefronts, "
                          "the last %lld row blocks of each XCD by a workgroup each",
                          kt, G, plan.group_tail);
+            } else if (plan.col_splits == 1) {
+                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=1>: grid form, 4 row blocks per workgroup of 4 wavefronts", kt, G);
             } else {
-                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefront(s) per row block", kt, G,
+                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefronts per row block", kt, G,
                          plan.col_splits, plan.col_splits);
             }
             break;

@@ -71,6 +71,12 @@ void fill_fwd_args(const MatmulProblem& p, FwdArgs* args);
 // base-2 exponential) so that its hi and lo halves stay inside the fp16 exponent range.
 #define KM_F16_KSCALE_LOG2 14
 
+// (On the bits without the sign: a vote over v < inf, or over exponent bits that are not all ones, which it
+// takes for the same, comes out of this compiler as a vote over v != inf, true for a NaN.)
+__device__ __forceinline__ bool is_finite(float v) {
+    return __float_as_uint(v) << 1 < 0xff000000u;
+}
+
 // Phase f * (x - c) in revolutions, reduced to [-0.5, 0.5].  x - c is taken as an unevaluated
 // sum hi + lo (error-free transformation) and the product f * hi is never rounded on its own
 // (fused multiply-add), so the result carries about half an fp32 ulp of 0.5 (3e-8 revolutions) whatever the
@@ -163,6 +169,22 @@ __device__ __forceinline__ void wave_min_max(float* lo, float* hi) {
     *hi = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, b), 63));
 }
 
+// Smallest and largest value within groups of 8 lanes.
+__device__ __forceinline__ void group8_min_max(float v, float* lo, float* hi) {
+    float a = v, b = v;
+#define KM_DPP_STEP(ctrl)                                                                              \
+    a = fminf(a, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, a),     \
+                                                                       __builtin_bit_cast(int, a), ctrl, 0xf, 0xf, false))); \
+    b = fmaxf(b, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, b),     \
+                                                                       __builtin_bit_cast(int, b), ctrl, 0xf, 0xf, false)))
+    KM_DPP_STEP(0xb1);   // quad_perm [1, 0, 3, 2]
+    KM_DPP_STEP(0x4e);   // quad_perm [2, 3, 0, 1]
+    KM_DPP_STEP(0x141);  // row_half_mirror
+#undef KM_DPP_STEP
+    *lo = a;
+    *hi = b;
+}
+
 // Largest value over the 4 lanes that share an rhs column (lanes l, l+16, l+32, l+48).
 __device__ __forceinline__ float column_max(float m) {
     const unsigned bits = __float_as_uint(m);
@@ -185,6 +207,67 @@ struct WaveView {
     int range_end;
 };
 
+// The launch's arguments, to be read from memory where they are used: held in scalar registers from the
+// kernel's start on, those of a branch that is hardly ever taken make the others spill.
+__device__ __forceinline__ const FwdArgs& fresh_args() {
+    auto args = (const __attribute__((address_space(4))) FwdArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return *(const FwdArgs*)args;
+}
+
+// Element offsets of a batch item's tensors.
+struct BatchOffsets {
+    long long x1, x2, rhs, params, start, end;
+};
+
+// (the usual case after the host has collapsed the batch dimensions: one stride per tensor, no division
+// chain)
+__device__ __forceinline__ BatchOffsets batch_offsets(const FwdArgs& a, long long b) {
+    BatchOffsets o;
+    if (a.batch.rank <= 1) {
+        o.x1 = b * a.x1_bs.s[0];
+        o.x2 = b * a.x2_bs.s[0];
+        o.rhs = b * a.rhs_bs.s[0];
+        o.params = b * a.params_bs.s[0];
+        o.start = b * a.start_bs.s[0];
+        o.end = b * a.end_bs.s[0];
+    } else {
+        // One tensor per lane, in a loop over the dimensions: small, and without the strides of all
+        // tensors in scalar registers.
+        static_assert(offsetof(FwdArgs, end_bs) - offsetof(FwdArgs, x1_bs) == 5 * sizeof(BatchStrides), "in the order of BatchOffsets");
+        const FwdArgs& g = a;
+        const BatchStrides* strides = &g.x1_bs + min((int)(threadIdx.x & 63), 5);
+        unsigned flat = (unsigned)b;
+        long long off = 0;
+#pragma unroll 1
+        for (int d = g.batch.rank - 1; d >= 0; d--) {
+            const unsigned size = (unsigned)g.batch.sizes[d];
+            const unsigned rest = flat / size;
+            off += (long long)(flat - rest * size) * strides->s[d];
+            flat = rest;
+        }
+        auto of = [&](int tensor) {
+            const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)off, tensor);
+            return (long long)((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(off >> 32), tensor) << 32 | lo);
+        };
+        o.x1 = of(0);
+        o.x2 = of(1);
+        o.rhs = of(2);
+        o.params = of(3);
+        o.start = of(4);
+        o.end = of(5);
+    }
+    return o;
+}
+
+// Column range of a row block, clamped to the valid columns: a symmetric pattern over fewer points than
+// one block reports end = block size > n (native/ranges/ranges.cpp:82-93 of the reference).
+// An empty range ends where it starts, whatever the two values: nothing added to them overflows.
+__device__ __forceinline__ void block_range(const FwdArgs& a, const BatchOffsets& o, int row_block, int* start, int* end) {
+    *end = max(min(a.end[o.end + row_block * a.end_s], a.n), 0);
+    *start = min(max(a.start[o.start + row_block * a.start_s], 0), *end);
+}
+
 // FAST: take the short way when the batch shape has collapsed to at most one dimension (small
 // launches, where the scalar prologue is a visible part of a wavefront's life; the large grouped
 // launches measure 2 % slower with the extra branch and keep the general code).
@@ -196,35 +279,24 @@ __device__ __forceinline__ WaveView wave_view(const FwdArgs& a, long long item, 
     const int chunk = (int)(item / a.num_batches);
     w.row_block = chunk / chunks_per_block;
     *chunk_in_block = chunk % chunks_per_block;
-    long long off_x1, off_x2, off_rhs, off_params, off_start, off_end;
-    if (FAST && a.batch.rank <= 1) {
-        // The usual case after the host has collapsed the batch dimensions: one stride per
-        // tensor, no division chain.
-        off_x1 = w.b * a.x1_bs.s[0];
-        off_x2 = w.b * a.x2_bs.s[0];
-        off_rhs = w.b * a.rhs_bs.s[0];
-        off_params = w.b * a.params_bs.s[0];
-        off_start = w.b * a.start_bs.s[0];
-        off_end = w.b * a.end_bs.s[0];
+    BatchOffsets o;
+    if (FAST) {
+        o = batch_offsets(a, w.b);
     } else {
         int bidx[KM_MAX_BATCH_RANK];
         batch_multi_index(a.batch, w.b, bidx);
-        off_x1 = batch_offset(a.batch, a.x1_bs, bidx);
-        off_x2 = batch_offset(a.batch, a.x2_bs, bidx);
-        off_rhs = batch_offset(a.batch, a.rhs_bs, bidx);
-        off_params = batch_offset(a.batch, a.params_bs, bidx);
-        off_start = batch_offset(a.batch, a.start_bs, bidx);
-        off_end = batch_offset(a.batch, a.end_bs, bidx);
+        o.x1 = batch_offset(a.batch, a.x1_bs, bidx);
+        o.x2 = batch_offset(a.batch, a.x2_bs, bidx);
+        o.rhs = batch_offset(a.batch, a.rhs_bs, bidx);
+        o.params = batch_offset(a.batch, a.params_bs, bidx);
+        o.start = batch_offset(a.batch, a.start_bs, bidx);
+        o.end = batch_offset(a.batch, a.end_bs, bidx);
     }
-    w.x1 = a.x1 + off_x1;
-    w.x2 = a.x2 + off_x2;
-    w.rhs = a.rhs + off_rhs;
-    w.params = a.params + off_params;
-    // Clamped to the valid columns: a symmetric pattern over fewer points than one block
-    // reports end = block size > n (native/ranges/ranges.cpp:82-93 of the reference).
-    // An empty range ends where it starts, whatever the two values: nothing added to them overflows.
-    w.range_end = max(min(a.end[off_end + w.row_block * a.end_s], a.n), 0);
-    w.range_start = min(max(a.start[off_start + w.row_block * a.start_s], 0), w.range_end);
+    w.x1 = a.x1 + o.x1;
+    w.x2 = a.x2 + o.x2;
+    w.rhs = a.rhs + o.rhs;
+    w.params = a.params + o.params;
+    block_range(a, o, w.row_block, &w.range_start, &w.range_end);
     return w;
 }
 

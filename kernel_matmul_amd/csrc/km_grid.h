@@ -30,25 +30,21 @@ namespace km {
 #define KM_GRID_COLUMN_REACH 8.603f /* the same for K / sigma in the coordinates of V: sqrt(2) times as far */
 #define KM_GRID_WEIGHT_F64 0.66428247026735920 /* C / (h s2) = sqrt(2 ln 2 / pi) */
 #define KM_GRID_WEIGHT ((float)KM_GRID_WEIGHT_F64)
-#define KM_GRID_CHUNK 256           /* columns tabulated at a time, per wavefront */
+#define KM_GRID_CHUNK 256           /* columns tabulated at a time, per wavefront ... */
+#define KM_GRID_CHUNK_ONE 128       /* ... with one group of rhs columns (grid_columns) */
 #define KM_GRID_KS1 11              /* V is evaluated times 2^11 (columns: reference within 2) ... */
 #define KM_GRID_SPAN 2.0f
 #define KM_GRID_KS2 10              /* ... and 2^10 (rows: reference within 3.5 h s2 = 2.24) */
 #define KM_GRID_NOT_FINITE 1000     /* in place of a rhs column's shift: it holds a value that is not finite */
 // Table of a chunk: coordinate, the two column factors, the smallest and largest coordinate of each 8
 // columns, and the remainder of the coordinate.
-#define KM_GRID_TABLE_REST (3 * KM_GRID_CHUNK + 2 * KM_GRID_CHUNK / 8)
-#define KM_GRID_TABLE_FLOATS (KM_GRID_TABLE_REST + KM_GRID_CHUNK)
+constexpr int grid_table_rest(int chunk) { return 3 * chunk + 2 * chunk / 8; }
+constexpr int grid_table_floats(int chunk) { return grid_table_rest(chunk) + chunk; }
+#define KM_GRID_TABLE_FLOATS (grid_table_floats(KM_GRID_CHUNK))
 
 // A value that is the same in every lane, as a scalar register.
 __device__ __forceinline__ float uniform(float v) {
     return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v)));
-}
-
-// (On the bits without the sign: a vote over v < inf, or over exponent bits that are not all ones, which it
-// takes for the same, comes out of this compiler as a vote over v != inf, true for a NaN.)
-__device__ __forceinline__ bool is_finite(float v) {
-    return __float_as_uint(v) << 1 < 0xff000000u;
 }
 
 // Grid window of one row block (the same in every lane).
@@ -60,6 +56,8 @@ struct GridWindow {
     float col_lo, col_hi;  // relative coordinates beyond which columns contribute nothing
     float reach;       // distance beyond which the evaluated factor counts as zero
     int tiles;         // groups of 16 grid points
+    float first, last; // relative coordinates that no column lies beyond (where that is not known: the
+                       // largest that the form takes)
 };
 
 // The rows of a block, two per lane, and its middle row.
@@ -102,23 +100,9 @@ __device__ __forceinline__ GridWindow grid_window(const BlockRows& rows, const K
     const float cr = KM_GRID_COLUMN_REACH * inv;
     gw.col_lo = uniform(finite ? lo - cr : -__builtin_inff());
     gw.col_hi = uniform(finite ? hi + cr : __builtin_inff());
+    gw.first = -1e30f;
+    gw.last = 1e30f;
     return gw;
-}
-
-// Smallest and largest value within groups of 8 lanes.
-__device__ __forceinline__ void group8_min_max(float v, float* lo, float* hi) {
-    float a = v, b = v;
-#define KM_DPP_STEP(ctrl)                                                                              \
-    a = fminf(a, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, a),     \
-                                                                       __builtin_bit_cast(int, a), ctrl, 0xf, 0xf, false))); \
-    b = fmaxf(b, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, b),     \
-                                                                       __builtin_bit_cast(int, b), ctrl, 0xf, 0xf, false)))
-    KM_DPP_STEP(0xb1);   // quad_perm [1, 0, 3, 2]
-    KM_DPP_STEP(0x4e);   // quad_perm [2, 3, 0, 1]
-    KM_DPP_STEP(0x141);  // row_half_mirror
-#undef KM_DPP_STEP
-    *lo = a;
-    *hi = b;
 }
 
 // What the subtraction d = x - origin rounded off.
@@ -127,36 +111,36 @@ __device__ __forceinline__ float remainder_of(float x, float origin, float d) {
     return (x - (d - bb)) - (origin + bb);
 }
 
-// Coordinates of this wavefront's next 8 steps of 32 columns, in the order grid_table takes them.
+// Coordinates of this wavefront's next CH / 32 steps of 32 columns, in the order grid_table takes them.
+template <int N>
 __device__ __forceinline__ void grid_load(const float* __restrict__ x2, long long x2_s, int first, int stride, int end,
-                                          float (&xv)[KM_GRID_CHUNK / 64]) {
+                                          float (&xv)[N]) {
     const int lane = threadIdx.x & 63;
     const float* xc = x2 + (long long)first * x2_s;
     const int last = end - 1 - first;
 #pragma unroll
-    for (int i = 0; i < KM_GRID_CHUNK / 64; i++) {
+    for (int i = 0; i < N; i++) {
         const int rel = 32 * ((lane >> 5) + 2 * i) * stride + (lane & 31);
         xv[i] = xc[(unsigned long long)(unsigned)min(rel, last) * (unsigned)x2_s];
     }
 }
 
-// Tabulates this wavefront's next 8 steps of 32 columns (the steps first / 32 + j * stride of the
-// range, j = 0 .. 7: several wavefronts that share a range take its steps in turn).  Returns the
+// Tabulates this wavefront's next 2 N steps of 32 columns (the steps first / 32 + j * stride of the
+// range, j = 0 .. 2 N - 1: several wavefronts that share a range take its steps in turn).  Returns the
 // steps that reach the rows as a bit mask.
 //   GRID: coordinates as 2 b, b = (y - r) s2 with r halfway between the ends of each group of 8, the
 //         column factors times 2^(-b^2).  Steps of which a group spreads further than KM_GRID_SPAN
 //         (a gap in the data) come back in the upper half of the mask: their factors lack 2^(-b^2)
 //         (it would leave the fp16 range) and their coordinates are y and its remainder, relative to
 //         the row block's origin: a reference in the middle of the gap would round them to a fraction
-//         of the gap.  *fine is cleared when a coordinate is not finite.
+//         of the gap.  *fine is cleared when a coordinate lies beyond gw.first or gw.last or is NaN.
 //   else: the coordinates themselves (entry-wise evaluation).  *fine is cleared when a coordinate makes
 //         every entry of its column NaN: a NaN, or an infinity under an oscillating factor.
-template <bool GRID, bool PHASE>
-__device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK / 64], int first, int stride, int end,
+template <bool GRID, bool PHASE, int N>
+__device__ __forceinline__ unsigned grid_table(const float (&xv)[N], int first, int stride, int end,
                                                const GridWindow& gw, const KernelConsts& kc, float* __restrict__ tab,
                                                bool* fine) {
-    constexpr int CH = KM_GRID_CHUNK;
-    constexpr int N = CH / 64;
+    constexpr int CH = 64 * N;
     const int lane = threadIdx.x & 63;
     const int last = end - 1 - first;
     float b[N], lo[N], hi[N];
@@ -180,7 +164,7 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
             const unsigned w = bits(0.5f * (hi[i] - lo[i]) * gw.s2 > KM_GRID_SPAN, i);
             wide[i] = (w >> (2 * i + (lane >> 5)) & 1) != 0;
             need |= w << 16;
-            ok = ok && fabsf(y) < 1e30f;
+            ok = ok && y >= gw.first && y <= gw.last;
         } else {
             ok = ok && (PHASE ? is_finite(xv[i]) : xv[i] == xv[i]);
         }
@@ -201,7 +185,7 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[KM_GRID_CHUNK /
         if (GRID && wide[i]) {
             const float y = xv[i] - gw.x_ref;
             tab[q] = y;
-            tab[KM_GRID_TABLE_REST + q] = remainder_of(xv[i], gw.x_ref, y);
+            tab[grid_table_rest(CH) + q] = remainder_of(xv[i], gw.x_ref, y);
         }
         if (PHASE) {
             const float th = phase_rev(kc.f, xv[i], gw.x_ref);
@@ -459,17 +443,46 @@ __device__ __forceinline__ void look_at_steps(const GridVectors& a, const WaveVi
     } while (steps.any());
 }
 
-// One step of 32 columns: scale and split the rhs operand, then for every tile of 16 points in
-// reach evaluate, split and contract.  GRID: the points are the grid's, t0 + 16 mt h; else the rows xr[].
+// The running power-of-two scale of an rhs column, lowered when a magnitude m of its values would exceed 2^15 (NaN
+// and infinities hand themselves on).
+template <int G, int PARTS, int MT>
+__device__ __forceinline__ void lower_scale(int g, float m, bool used, int (&shift)[G], float (&scale)[G],
+                                            float4v (&acc)[MT][G * PARTS]) {
+    const bool grow = used && !(m * scale[g] < 32768.0f);
+    if (__any(grow)) {
+        if (grow && !is_finite(m)) {
+            shift[g] = KM_GRID_NOT_FINITE;
+            scale[g] = 0.0f;
+        } else if (grow) {
+            const int e = __builtin_amdgcn_frexp_expf(m);
+            const int new_shift = min(14 - e, 100);
+            if (__any(shift[g] != 100)) {  // (else these are its first values: the sums are zero)
+                const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+                    for (int part = 0; part < PARTS; part++) {
+                        acc[mt][part * G + g] *= factor;
+                    }
+                }
+            }
+            shift[g] = new_shift;
+            scale[g] = __builtin_ldexpf(1.0f, new_shift);
+        }
+    }
+}
+
+// One step of 32 columns: split the scaled rhs operand, then for every tile of 16 points in reach evaluate, split
+// and contract.  GRID: the points are the grid's, t0 + 16 mt h; else the rows xr[].
 // weights: which of the table's column factors this lane's rhs column takes (PARTS == 1; with two parts
 // the cosines for the first and the sines for the second).  EXACT: the product of the low halves as well
 // (the gradient: hidden behind the VALU work there, and it halves the error of its long sums).
-template <bool GRID, int G, int PARTS, int MT, bool EXACT>
+// WIDE: the step may be one of those whose factors lack 2^(-b^2); `wide` says whether it is.
+template <bool GRID, int G, int PARTS, int MT, bool EXACT, int CH, bool WIDE>
 __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off, const float (&raw)[G][8],
                                           const GridWindow& gw, float t0, const float* xr, const KernelConsts& kc,
-                                          int tiles, bool wide, int weights, const bool (&colmask)[G], int (&shift)[G], float (&scale)[G],
+                                          int tiles, bool wide, int weights, const float (&scale)[G],
                                           float4v (&acc)[MT][G * PARTS]) {
-    constexpr int CH = KM_GRID_CHUNK;
     constexpr int GE = G * PARTS;
     float xv[8], cb[8], sb[8];
 #pragma unroll
@@ -495,28 +508,6 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
     half8v bhi[GE], blo[GE];
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        // The column's running power-of-two scale, as in f16_step (NaN and infinities hand themselves on).
-        const float m = column_maximum(magnitude(raw[g]));
-        const bool grow = colmask[g] && !(m * scale[g] < 32768.0f);
-        if (__any(grow)) {
-            if (grow && !is_finite(m)) {
-                shift[g] = KM_GRID_NOT_FINITE;
-                scale[g] = 0.0f;
-            } else if (grow) {
-                const int e = __builtin_amdgcn_frexp_expf(m);
-                const int new_shift = min(14 - e, 100);
-                const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-                    for (int part = 0; part < PARTS; part++) {
-                        acc[mt][part * G + g] *= factor;
-                    }
-                }
-                shift[g] = new_shift;
-                scale[g] = __builtin_ldexpf(1.0f, new_shift);
-            }
-        }
         float vc[8];
 #pragma unroll
         for (int t = 0; t < 8; t++) {
@@ -551,7 +542,7 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
         half2v h2[4], l2[4];
         float arg[8];
         if (GRID) {
-            if (!wide) {
+            if (!WIDE || !wide) {
                 const float av = (t - 0.5f * (lo + hi)) * gw.s2;
                 const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
 #pragma unroll
@@ -559,8 +550,8 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
                     arg[u] = __builtin_fmaf(av, xv[u], rb);
                 }
             } else {
-                const float4v r0 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off);
-                const float4v r1 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off + 4);
+                const float4v r0 = *(const float4v*)(tab + grid_table_rest(CH) + off);
+                const float4v r1 = *(const float4v*)(tab + grid_table_rest(CH) + off + 4);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
                     const float z = ((t - xv[u]) - (u < 4 ? r0[u & 3] : r1[u & 3])) * gw.s2;
@@ -602,15 +593,14 @@ __device__ __forceinline__ void grid_step(const float* __restrict__ tab, int off
 // coordinates a chunk ahead (the first chunk's, in xv, by the caller).
 // PACK (spectral, at most 8 rhs columns): lanes 0 .. 7 of a group hold the columns' cosine parts, lanes
 // 8 .. 15 their sine parts.
-template <bool GRID, int KT, int G, int MT, int W, bool PACK = false, bool EXACT = false>
+template <bool GRID, int KT, int G, int MT, int W, bool PACK = false, bool EXACT = false, int CH = GRID && G == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK>
 __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __restrict__ tab, const WaveView& w, int kbase,
                                              int wave, const GridWindow& gw, const KernelConsts& kc, const float* xr,
-                                             int tiles, float (&xv)[KM_GRID_CHUNK / 64], int (&shift)[G],
+                                             int tiles, float (&xv)[CH / 64], int (&shift)[G],
                                              float4v (&acc)[MT][G * (KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 1)]) {
     constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
     constexpr int PARTS = PHASE && !PACK ? 2 : 1;
     static_assert(!PACK || (PHASE && G == 1 && GRID), "packed: eight rhs columns, cosine and sine part in one group");
-    constexpr int CH = KM_GRID_CHUNK;
     const int lane = threadIdx.x & 63;
     const int li = lane & 15;
     const int kk = lane >> 4;
@@ -637,10 +627,14 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
     constexpr bool EACH_CHUNK = G == 1;
     BeyondSteps beyond = {0, 64, 0};
     int chunk = 0;
-    static_assert(CH / 32 == 8, "eight steps a chunk");
+    constexpr int STEPS = CH / 32;  // of a chunk
+    static_assert(64 % STEPS == 0, "whole chunks' bits");
     // (unsigned: the next first column may lie past the largest int)
     for (unsigned next_first = w.range_start + 32u * wave; next_first < (unsigned)w.range_end; next_first += CH * W) {
         const int first = (int)next_first;
+        // (the first step's values, mostly needed, are on their way while the table is made)
+        float next[G][8];
+        grid_rhs<G>(a, rhs, first, w.range_end, kk, rl, next);
         const unsigned steps = grid_table<GRID, PHASE>(xv, first, W, w.range_end, gw, kc, tab, &fine);
         if (next_first + CH * W < (unsigned)w.range_end) {
             grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
@@ -649,18 +643,19 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
         if (!GRID) {
             // (the caller has looked at all steps)
         } else if (EACH_CHUNK) {
-            const int present = min((w.range_end - 1 - first) / (32 * W) + 1, CH / 32);
+            const int present = min((w.range_end - 1 - first) / (32 * W) + 1, STEPS);
             look_at_steps<G>(a, w, kbase, first, 32 * W, {~need & ((1u << present) - 1), 0, 0}, rl, shift, scale);
-        } else if (chunk < 8) {
-            beyond.bits |= (unsigned long long)(~need & 0xff) << (8 * chunk);
+        } else if (chunk < 64 / STEPS) {
+            beyond.bits |= (unsigned long long)(~need & ((1u << STEPS) - 1)) << (STEPS * chunk);
         }
         chunk++;
         if (need == 0) {
             continue;
         }
-        float next[G][8];
         int j = __builtin_ctz(need);
-        grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
+        if (j != 0) {
+            grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
+        }
         do {
             float raw[G][8];
 #pragma unroll
@@ -686,7 +681,11 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
                     asm volatile("" : "+v"(acc[m][g]));
                 }
             }
-            grid_step<GRID, G, PARTS, MT, EXACT>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, rl.used, shift, scale, acc);
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                lower_scale<G, PARTS, MT>(g, column_maximum(magnitude(raw[g])), rl.used[g], shift, scale, acc);
+            }
+            grid_step<GRID, G, PARTS, MT, EXACT, CH, GRID>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, scale, acc);
         } while (need != 0);
         // All reads of the table are done before the next chunk overwrites it.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

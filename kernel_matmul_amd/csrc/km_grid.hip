@@ -1,5 +1,6 @@
 // Forward operator in the grid form (km_grid.h): rbf and spectral kernels, any number of rhs
-// columns.  A row block of 128 rows is one item, worked on by W wavefronts:
+// columns.  A row block of 128 rows is one item, worked on by W wavefronts (large launches: by one, four row
+// blocks together, see group_item):
 //
 //   columns -> grid   the wavefronts take the steps of 32 columns of the block's range in turn; V is
 //                     the A operand (16 grid points x 32 columns), rhs (spectral: times cos B and
@@ -15,10 +16,8 @@
 // that is not finite makes its column's results NaN in every row whose range holds it, as does a NaN
 // among the range's column coordinates (spectral: an infinity as well) in all columns.
 //
-// Measured against the entry-wise kernels (a call, queued): spectral n = 1e5, k = 16, 8 sets 103.8 -> 64.8 us,
-// n = 1e6, k = 32 1085 -> 891, rbf n = 65536, k = 64 43.6 -> 21.8.  The large ones are bound by VALU issue (66
-// and 70 % of the cycles; exponentials, fma and fp16 roundings are a third of it, the rest rhs scaling,
-// maxima, tables, moves and offsets), the small ones by the latency of one wavefront's steps.
+// Measured against the entry-wise kernels (a call, queued): rbf n = 65536, k = 64 43.6 -> 21.2 us; the large
+// launches below, at group_item.  The small ones are bound by the latency of one wavefront's steps.
 #include "km_batch.h"
 #include "km_common.h"
 #include "km_fwd.h"
@@ -37,42 +36,206 @@ __device__ __forceinline__ GridVectors vectors(const FwdArgs& a) {
     return {a.x2_s, a.rhs_s0, a.rhs_s1, a.k};
 }
 
-// A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the
-// phase-split form combined, and the masked store.
+// A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the phase-split form
+// combined (with the cosines and sines of the rows' phases), and the masked store.
 template <int KT, int G>
-__device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, const KernelConsts& kc, float x,
-                                           float x_ref, const float4v* res, const float* down, int row, int kbase) {
+__device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, const float (&ca)[4], const float (&sa)[4],
+                                           const float4v* res, const float* down, int row, int kbase) {
     constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
     const int lane = threadIdx.x & 63;
     const int li = lane & 15;
     const int kk = lane >> 4;
-    float ca[4], sa[4];
-    if (PHASE) {
-        // cos A / sin A of the row this lane holds, fetched into the accumulator layout.
-        const float th = phase_rev(kc.f, x, x_ref);
-        const float ca_own = __builtin_amdgcn_cosf(th);
-        const float sa_own = __builtin_amdgcn_sinf(th);
+    float* __restrict__ out = a.out + (w.b * (long long)a.m + row) * a.k + kbase;
+    auto value = [&](int g, int v) {
+        return PHASE ? ca[v] * (res[g][v] * down[g]) + sa[v] * (res[G + g][v] * down[G + g]) : res[g][v] * down[g];
+    };
+    // Whole groups of rows of moderate width: a scalar base and row offset (no address arithmetic per value).
+    if (row + 16 <= a.m && a.k <= (1 << 22)) {
+        const buffer_rsrc to = uniform_buffer(out);
+        const unsigned lane_bytes = 4u * (__umul24(4u * (unsigned)kk, (unsigned)a.k) + (unsigned)li);
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-            ca[v] = __shfl(ca_own, 4 * kk + v, 64);
-            sa[v] = __shfl(sa_own, 4 * kk + v, 64);
+        for (int g = 0; g < G; g++) {
+            if (kbase + 16 * g + li < a.k) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(value(g, v)), to, (int)(lane_bytes + 64u * g),
+                                                          (int)(4u * (unsigned)v * (unsigned)a.k), 0);
+                }
+            }
         }
+        return;
     }
-    float* __restrict__ out = a.out + w.b * (long long)a.m * a.k;
 #pragma unroll
     for (int g = 0; g < G; g++) {
-        const int c = kbase + 16 * g + li;
+        const int c = 16 * g + li;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const float value = PHASE ? ca[v] * (res[g][v] * down[g]) + sa[v] * (res[G + g][v] * down[G + g])
-                                      : res[g][v] * down[g];
-            const int r = row + 4 * kk + v;
-            if (r < a.m && c < a.k) {
-                out[(long long)r * a.k + c] = value;
+            if (row + 4 * kk + v < a.m && kbase + c < a.k) {
+                out[(long long)(4 * kk + v) * a.k + c] = value(g, v);
             }
         }
     }
 }
+
+// cos A / sin A of the rows, one held by each lane, in the accumulator layout.
+__device__ __forceinline__ void row_phases(float own_cos, float own_sin, int first, float (&ca)[4], float (&sa)[4]) {
+    const int kk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        ca[v] = __shfl(own_cos, first + 4 * kk + v, 64);
+        sa[v] = __shfl(own_sin, first + 4 * kk + v, 64);
+    }
+}
+
+// Rows whose values a wavefront holds, two per lane (the layout of BlockRows).
+struct HeldRows {
+    float y[2], rest[2], cos[2], sin[2];
+};
+
+template <int KT>
+__device__ __forceinline__ HeldRows hold_rows(const BlockRows& rows, float x_ref, const KernelConsts& kc) {
+    HeldRows h;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const float x = i == 0 ? rows.xa : rows.xb;
+        h.y[i] = x - x_ref;
+        h.rest[i] = remainder_of(x, x_ref, h.y[i]);
+        const float th = KT == KM_KERNEL_SPECTRAL ? phase_rev(kc.f, x, x_ref) : 0.0f;
+        h.cos[i] = __builtin_amdgcn_cosf(th);
+        h.sin[i] = __builtin_amdgcn_sinf(th);
+    }
+    return h;
+}
+
+// Grid -> rows: `groups` groups of 16 rows from row0 from the sums of their window, in the accumulators'
+// layout.  EXCHANGED: the sums come through LDS, scaled back already; else they are times 2^shift and the scale
+// of the evaluated factor.  held: the rows, where the wavefront has all 128.
+template <int KT, int G, int MT, bool EXCHANGED, bool HELD>
+__device__ __forceinline__ void grid_rows(const FwdArgs& a, const WaveView& w, const HeldRows* held, int row0, int groups,
+                                          int kbase, const GridWindow& gw, const KernelConsts& kc, const int (&shift)[G],
+                                          float4v (&acc)[MT][G * (KT == KM_KERNEL_SPECTRAL ? 2 : 1)]) {
+    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
+    constexpr int GE = G * (PHASE ? 2 : 1);
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    // One power-of-two scale per column over the whole window; the operands of all
+    // steps of 32 grid points replace the accumulators, so that a row group needs no more than its
+    // own accumulator at a time.
+    const float hz = gw.h * gw.s2;
+    float b2[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        const float b = ((float)t - 3.5f) * hz;
+        b2[t] = uniform(b + b);
+    }
+    float fac[8];
+#pragma unroll
+    for (int t = 0; t < 8; t++) {
+        fac[t] = uniform(__builtin_amdgcn_exp2f(-0.25f * b2[t] * b2[t]));
+    }
+    const float weight = w.params[KernelTraits<KT>::SIGMA * a.params_s] * (hz * KM_GRID_WEIGHT);
+    float down[GE];
+    constexpr int KSTEPS = (MT + 1) / 2;
+    half8v bhi[KSTEPS][GE], blo[KSTEPS][GE];
+#pragma unroll
+    for (int g = 0; g < GE; g++) {
+        float m = 0.0f;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                m = fmaxf(m, fabsf(acc[mt][g][v]));
+            }
+        }
+        m = column_max(m);
+        const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 100);
+        const float up = __builtin_ldexpf(1.0f, e);
+        down[g] = shift[g % G] == KM_GRID_NOT_FINITE
+                      ? __builtin_nanf("")
+                      : weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 + (EXCHANGED ? KM_GRID_EXCHANGE : -shift[g % G] - KM_GRID_KS1));
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ks++) {
+            if (2 * ks < gw.tiles) {
+                float gv[8];
+                constexpr int LAST = MT - 1;
+                const float4v none = {0.0f, 0.0f, 0.0f, 0.0f};
+                grid_operand(acc[2 * ks][g], 2 * ks + 1 <= LAST ? acc[2 * ks + 1 <= LAST ? 2 * ks + 1 : LAST][g] : none, gv);
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    gv[t] *= up * fac[t];
+                }
+                split_f16x8(gv, kc.one, &bhi[ks][g], &blo[ks][g]);
+                __builtin_amdgcn_sched_barrier(0);  // one operand at a time (registers)
+            }
+        }
+    }
+    const float mid0 = (gw.g_lo + (float)(8 * kk) + 3.5f) * gw.h;
+    const float mid_step = 32.0f * gw.h;
+#pragma unroll 2
+    for (int r = 0; r < groups; r++) {
+        const int row = row0 + 16 * r;
+        float y, rest, ca[4], sa[4];  // (rest: not zero in a block next to the origin)
+        if (HELD) {
+            const bool upper = r >= 4;
+            const int first = 16 * (r & 3);
+            y = __shfl(upper ? held->y[1] : held->y[0], first + li, 64);
+            rest = __shfl(upper ? held->rest[1] : held->rest[0], first + li, 64);
+            if (PHASE) {
+                row_phases(upper ? held->cos[1] : held->cos[0], upper ? held->sin[1] : held->sin[0], first, ca, sa);
+            }
+        } else {
+            const float x = w.x1[(long long)min(row + li, a.m - 1) * a.x1_s];
+            y = x - gw.x_ref;
+            rest = remainder_of(x, gw.x_ref, y);
+            if (PHASE) {
+                const float th = phase_rev(kc.f, x, gw.x_ref);
+                row_phases(__builtin_amdgcn_cosf(th), __builtin_amdgcn_sinf(th), 0, ca, sa);
+            }
+        }
+        float4v res[GE];
+#pragma unroll
+        for (int g = 0; g < GE; g++) {
+            res[g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+#pragma unroll
+        for (int ks = 0; ks < KSTEPS; ks++) {
+            if (2 * ks >= gw.tiles) {
+                break;
+            }
+            const float av = ((y - __builtin_fmaf((float)ks, mid_step, mid0)) + rest) * gw.s2;
+            if (!__any(fabsf(av) - 3.5f * hz < KM_GRID_REACH)) {
+                continue;
+            }
+            half2v h2[4], l2[4];
+            const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS2);
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                separable_pair_f16(av, rb, b2[2 * u], b2[2 * u + 1], kc.one, &h2[u], &l2[u]);
+            }
+            const half8v ahi = join_half2x4(h2);
+            const half8v alo = join_half2x4(l2);
+#pragma unroll
+            for (int g = 0; g < GE; g++) {
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[ks][g], res[g], 0, 0, 0);
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[ks][g], res[g], 0, 0, 0);
+                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[ks][g], res[g], 0, 0, 0);
+            }
+        }
+        grid_store<KT, G>(a, w, ca, sa, res, down, row, kbase);
+    }
+}
+
+// rhs column groups (of 16) that one pass takes, the grid form's largest window, and the columns tabulated at a
+// time.
+template <int KT, int G>
+struct GridShape {
+    static constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
+    static constexpr int GP = G * PARTS > 4 ? 4 / PARTS : G;
+    static constexpr int GE = GP * PARTS;
+    static constexpr int MT = GE >= 4 ? 4 : 5;
+    static constexpr int CHUNK = GP == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
+};
 
 // LDS of one item in floats: the wavefronts' tables, overlaid by the exchange of the sums, and the
 // flags of each wavefront.
@@ -89,13 +252,12 @@ constexpr int grid_lds_floats() {
 template <int KT, int G, int MT, int W>
 __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
                                              int wave, const GridWindow& gw, const KernelConsts& kc,
-                                             float (&xv)[KM_GRID_CHUNK / 64]) {
+                                             float (&xv)[GridShape<KT, G>::CHUNK / 64]) {
     constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
     constexpr int GE = G * PARTS;
     constexpr int R = 8 / W;  // groups of 16 rows of this wavefront
     const int lane = threadIdx.x & 63;
     const int li = lane & 15;
-    const int kk = lane >> 4;
 
     int shift[G];
     float4v acc[MT][GE];
@@ -168,96 +330,7 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
         return false;
     }
 
-    // Grid -> rows.  One power-of-two scale per column over the whole window; the operands of all
-    // steps of 32 grid points replace the accumulators, so that a row group needs no more than its
-    // own accumulator at a time.
-    const float hz = gw.h * gw.s2;
-    float b2[8];
-#pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const float b = ((float)t - 3.5f) * hz;
-        b2[t] = uniform(b + b);
-    }
-    float fac[8];
-#pragma unroll
-    for (int t = 0; t < 8; t++) {
-        fac[t] = uniform(__builtin_amdgcn_exp2f(-0.25f * b2[t] * b2[t]));
-    }
-    const float weight = w.params[KernelTraits<KT>::SIGMA * a.params_s] * (hz * KM_GRID_WEIGHT);
-    float down[GE];
-    constexpr int KSTEPS = (MT + 1) / 2;
-    half8v bhi[KSTEPS][GE], blo[KSTEPS][GE];
-#pragma unroll
-    for (int g = 0; g < GE; g++) {
-        float m = 0.0f;
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                m = fmaxf(m, fabsf(acc[mt][g][v]));
-            }
-        }
-        m = column_max(m);
-        const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 100);
-        const float up = __builtin_ldexpf(1.0f, e);
-        down[g] = shift[g % G] == KM_GRID_NOT_FINITE
-                      ? __builtin_nanf("")
-                      : weight * __builtin_ldexpf(1.0f, -e - KM_GRID_KS2 + (W > 1 ? KM_GRID_EXCHANGE : -shift[g % G] - KM_GRID_KS1));
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ks++) {
-            if (2 * ks < gw.tiles) {
-                float gv[8];
-                constexpr int LAST = MT - 1;
-                const float4v none = {0.0f, 0.0f, 0.0f, 0.0f};
-                grid_operand(acc[2 * ks][g], 2 * ks + 1 <= LAST ? acc[2 * ks + 1 <= LAST ? 2 * ks + 1 : LAST][g] : none, gv);
-#pragma unroll
-                for (int t = 0; t < 8; t++) {
-                    gv[t] *= up * fac[t];
-                }
-                split_f16x8(gv, kc.one, &bhi[ks][g], &blo[ks][g]);
-                __builtin_amdgcn_sched_barrier(0);  // one operand at a time (registers)
-            }
-        }
-    }
-    const float mid0 = (gw.g_lo + (float)(8 * kk) + 3.5f) * gw.h;
-    const float mid_step = 32.0f * gw.h;
-#pragma unroll 2
-    for (int r = 0; r < R; r++) {
-        const int row = row0 + 16 * (wave * R + r);
-        const float x = w.x1[(long long)min(row + li, a.m - 1) * a.x1_s];
-        const float y = x - gw.x_ref;
-        const float rest = remainder_of(x, gw.x_ref, y);  // (not zero in a block next to the origin)
-        float4v res[GE];
-#pragma unroll
-        for (int g = 0; g < GE; g++) {
-            res[g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
-        }
-#pragma unroll
-        for (int ks = 0; ks < KSTEPS; ks++) {
-            if (2 * ks >= gw.tiles) {
-                break;
-            }
-            const float av = ((y - __builtin_fmaf((float)ks, mid_step, mid0)) + rest) * gw.s2;
-            if (!__any(fabsf(av) - 3.5f * hz < KM_GRID_REACH)) {
-                continue;
-            }
-            half2v h2[4], l2[4];
-            const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS2);
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                separable_pair_f16(av, rb, b2[2 * u], b2[2 * u + 1], kc.one, &h2[u], &l2[u]);
-            }
-            const half8v ahi = join_half2x4(h2);
-            const half8v alo = join_half2x4(l2);
-#pragma unroll
-            for (int g = 0; g < GE; g++) {
-                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bhi[ks][g], res[g], 0, 0, 0);
-                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, blo[ks][g], res[g], 0, 0, 0);
-                res[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bhi[ks][g], res[g], 0, 0, 0);
-            }
-        }
-        grid_store<KT, G>(a, w, kc, x, gw.x_ref, res, down, row, kbase);
-    }
+    grid_rows<KT, G, MT, (W > 1), false>(a, w, nullptr, row0 + 16 * R * wave, R, kbase, gw, kc, shift, acc);
     return true;
 }
 
@@ -333,19 +406,15 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         }
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            grid_store<KT, G>(a, w, kc, xr[r], rows.x_ref, acc[r], down, base + 16 * r, kbase);
+            float ca[4], sa[4];
+            if (PARTS == 2) {
+                const float th = phase_rev(kc.f, xr[r], rows.x_ref);
+                row_phases(__builtin_amdgcn_cosf(th), __builtin_amdgcn_sinf(th), 0, ca, sa);
+            }
+            grid_store<KT, G>(a, w, ca, sa, acc[r], down, base + 16 * r, kbase);
         }
     }
 }
-
-// rhs column groups (of 16) that one pass takes, and the grid form's largest window.
-template <int KT, int G>
-struct GridShape {
-    static constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
-    static constexpr int GP = G * PARTS > 4 ? 4 / PARTS : G;
-    static constexpr int GE = GP * PARTS;
-    static constexpr int MT = GE >= 4 ? 4 : 5;
-};
 
 // One item by W wavefronts (this one is number `wave`): the grid form, or entry by entry.
 template <int KT, int G, int W>
@@ -360,7 +429,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     KernelConsts kc = make_consts<KT>(w.params, a.params_s, false);
     kc.s = uniform(kc.s);
     __builtin_amdgcn_sched_barrier(0);
-    float xv[KM_GRID_CHUNK / 64];
+    float xv[S::CHUNK / 64];
     if (32 * wave < w.range_end - w.range_start) {
         grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
     }
@@ -382,37 +451,518 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Large launches: a workgroup of KM_GROUP wavefronts takes as many neighbouring row blocks of a batch item,
+// whose ranges consist of the same columns for the most part, and contracts every column onto the grid once
+// for all of them.
+//
+// The ends of the ranges cut the columns into cells, each of which lies inside or outside each range as a
+// whole; a row block's sums are those of its cells, so the ranges are honoured exactly and nothing is
+// subtracted.  The middle cell (the core: what all ranges have in common if they are long) is shared out to
+// the wavefronts; of the others each wavefront takes one and half of the first or the last one.  The windows of
+// these segments and of the row blocks lie on one grid and begin at multiples of four points, the unit in which
+// sums are kept in LDS.
+//
+// Windows follow from the first and the last coordinate of a cell or row block.  Coordinates beyond these
+// (unsorted ones, NaN), windows that are too wide for the accumulators or for LDS, and ranges too short to gain
+// send the row blocks through grid_item, each by its wavefront.
+//
+// Measured (a call, queued), one row block per wavefront -> four per workgroup: spectral n = 1e5, k = 16, 8 sets
+// at 10 points per unit 64.5 -> 61 us (entry by entry 103.8), at 40 115 -> 70; 4 sets at 160 182 -> 86; n = 1e6,
+// k = 32, 8 sets 850 -> 786; rbf n = 1e5, k = 64, 8 sets 135 -> 129.  A row block of the first takes 3200 VALU
+// instructions instead of 4450; a quarter of the issue slots now wait for the workgroup's latencies (start and
+// windows of a segment, the exchange), which is what bounds the narrow ranges.  Four: the sums of a group and
+// their tables are then a third of the LDS for two operand groups, so that three workgroups of four wavefronts
+// are resident, as many as the registers allow; with three row blocks for three or four wavefronts one
+// wavefront waits, or less is shared.
+// ---------------------------------------------------------------------------------------
+#define KM_GROUP 4
+#define KM_GROUP_CHUNK 128
+#define KM_GROUP_CORE_SHARED 256  /* columns of the core beyond which all wavefronts take a piece */
+// Lanes of the plan: the segments whose sums the row blocks add (the first cell in halves, two cells, the core,
+// whole or in halves, two cells, the last cell in halves), the wavefronts' pieces of a shared core, the row blocks.
+#define KM_GROUP_SEGMENTS 10
+#define KM_GROUP_CORE 4
+#define KM_GROUP_PIECE 10
+#define KM_GROUP_ROW 14
+
+// LDS in floats: a table for each wavefront, the cells' sums, and flags.
+template <int KT, int G>
+struct GroupShape {
+    using S = GridShape<KT, G>;
+    static constexpr int QUAD = S::GE * 64;  // four grid points' sums
+    static constexpr int MAX_QUADS = 4 * S::MT;  // in a wavefront's accumulators
+    static constexpr int QUADS = S::GE >= 4 ? 70 : (S::GE > 1 ? 87 : 100);
+    static constexpr int TABLE = grid_table_floats(KM_GROUP_CHUNK);
+    static constexpr int SUMS = KM_GROUP * TABLE;
+    static constexpr int FLAGS = SUMS + QUADS * QUAD;
+    static constexpr int FLOATS = FLAGS + 64;
+    static_assert(FLOATS >= grid_lds_floats<S::GE, S::MT, KM_GROUP>() && FLOATS >= KM_GROUP * KM_GRID_TABLE_FLOATS, "grid_item's LDS");
+    static_assert(KM_GROUP + (KM_GROUP_SEGMENTS + KM_GROUP) * S::GP <= 64, "flags");
+};
+
+__device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+// One segment of columns or one row block per lane.
+struct GroupPlan {
+    int start, end;         // columns
+    int rows;               // row blocks whose range holds the segment, as bits
+    float first, last;      // smallest and largest coordinate, relative to the origin
+    float row_lo, row_hi;   // of these row blocks
+    int quad, quads;        // window: first group of four points and their number
+    int place;              // of the sums in LDS, in such groups
+    bool cooperative;       // the core is in pieces (same in every lane)
+    bool ok;                // the form applies (same in every lane)
+};
+
+// The segments: ranges into cells and pieces.  False if no range is long enough to gain.
+__device__ __forceinline__ bool group_segments(const FwdArgs& a, const BatchOffsets& o, int row_block, int blocks, GroupPlan* p) {
+    static_assert(KM_GROUP == 4, "eight ends of ranges");
+    const int lane = threadIdx.x & 63;
+    // The row blocks' starts in lanes 0 .. 3, ends in 4 .. 7 (as block_range, empty past the last row block).
+    const int block = row_block + min(lane & 3, blocks - 1);
+    const bool is_end = (lane & 4) != 0;
+    const int mine = (is_end ? a.end + o.end : a.start + o.start)[block * (is_end ? a.end_s : a.start_s)];
+    const int other = __shfl_xor(mine, 4, 64);
+    const int end = max(min(is_end ? mine : other, a.n), 0);
+    const int start = min(max(is_end ? other : mine, 0), end);
+    const int length = (lane & 3) < blocks ? end - start : 0;
+    if (!__any(lane < 4 && length >= KM_GRID_MIN_WIDTH)) {
+        return false;
+    }
+    // (the ends of an empty range cut nothing)
+    const int first_start = __builtin_amdgcn_readfirstlane(start);
+    const int value = length > 0 || (lane & 3) == 0 ? (is_end ? start + length : start) : first_start;
+    int ends[2 * KM_GROUP], rank = 0;
+#pragma unroll
+    for (int i = 0; i < 2 * KM_GROUP; i++) {
+        ends[i] = lane_value(value, i);
+        rank += ends[i] < value || (ends[i] == value && i < lane) ? 1 : 0;
+    }
+    const int cut = __builtin_amdgcn_ds_permute(4 * (lane < 8 ? rank : lane), value);
+    int at[2 * KM_GROUP];
+#pragma unroll
+    for (int i = 0; i < 2 * KM_GROUP; i++) {
+        at[i] = lane_value(cut, i);
+    }
+    auto half = [](int from, int to) { return ((to - from + 1) / 2 + 31) & ~31; };  // (in whole steps)
+    const int core = at[4] - at[3];
+    p->cooperative = core > KM_GROUP_CORE_SHARED;
+    const int quarter = (core / KM_GROUP + 31) & ~31;
+    const int bounds[KM_GROUP_SEGMENTS + 1] = {
+        at[0], max(at[1] - half(at[0], at[1]), at[0]), at[1], at[2],
+        at[3], p->cooperative ? at[4] : min(at[3] + half(at[3], at[4]), at[4]), at[4], at[5],
+        at[6], min(at[6] + half(at[6], at[7]), at[7]), at[7]};
+    p->start = bounds[0];
+    p->end = bounds[0];
+#pragma unroll
+    for (int i = 0; i < KM_GROUP_SEGMENTS; i++) {
+        p->start = lane == i ? bounds[i] : p->start;
+        p->end = lane == i ? bounds[i + 1] : p->end;
+    }
+    if (p->cooperative) {
+#pragma unroll
+        for (int i = 0; i < KM_GROUP; i++) {
+            p->start = lane == KM_GROUP_PIECE + i ? at[3] + i * quarter : p->start;
+            p->end = lane == KM_GROUP_PIECE + i ? (i == KM_GROUP - 1 ? at[4] : at[3] + (i + 1) * quarter) : p->end;
+        }
+    }
+    p->rows = 0;
+#pragma unroll
+    for (int r = 0; r < KM_GROUP; r++) {
+        p->rows |= ends[r] <= p->start && p->end <= ends[KM_GROUP + r] && p->start < p->end ? 1 << r : 0;
+    }
+    // (a gap between the ranges is a cell of none)
+    p->end = p->rows != 0 ? p->end : p->start;
+    return true;
+}
+
+// The windows and their places.
+template <int KT, int G>
+__device__ __forceinline__ void group_windows(const FwdArgs& a, const WaveView& w, int row0, const GridWindow& gw, GroupPlan* plan) {
+    using P = GroupShape<KT, G>;
+    const int lane = threadIdx.x & 63;
+    GroupPlan& p = *plan;
+    // First and last coordinates: of the columns, and of the row blocks.
+    const bool is_row = lane >= KM_GROUP_ROW && lane < KM_GROUP_ROW + KM_GROUP;
+    const float* ends = is_row ? w.x1 : w.x2;
+    const long long stride = is_row ? a.x1_s : a.x2_s;
+    int at0 = min(p.start, a.n - 1), at1 = min(max(p.end, 1), a.n) - 1;
+    if (is_row) {
+        at0 = min(row0 + (lane - KM_GROUP_ROW) * KM_BLOCK_SIZE, a.m - 1);
+        at1 = min(at0 + KM_BLOCK_SIZE - 1, a.m - 1);
+        p.rows = 1 << (lane - KM_GROUP_ROW);
+    }
+    const float y0 = ends[at0 * stride] - gw.x_ref;
+    const float y1 = ends[at1 * stride] - gw.x_ref;
+    p.first = fminf(y0, y1);
+    p.last = fmaxf(y0, y1);
+    p.row_lo = __builtin_inff();
+    p.row_hi = -__builtin_inff();
+#pragma unroll
+    for (int r = 0; r < KM_GROUP; r++) {
+        const float lo = lane_value(p.first, KM_GROUP_ROW + r), hi = lane_value(p.last, KM_GROUP_ROW + r);
+        p.row_lo = (p.rows >> r & 1) != 0 ? fminf(p.row_lo, lo) : p.row_lo;
+        p.row_hi = (p.rows >> r & 1) != 0 ? fmaxf(p.row_hi, hi) : p.row_hi;
+    }
+    // Windows: the grid points within reach of both the columns and the row blocks.
+    const float per_quad = 0.25f * __builtin_amdgcn_rcpf(gw.h);
+    const float lo = floorf((fmaxf(p.first, p.row_lo) - gw.reach) * per_quad);
+    const float hi = floorf((fminf(p.last, p.row_hi) + gw.reach) * per_quad + 0.25f) + 1.0f;
+    const float count = hi - lo;  // (not positive: out of reach)
+    const bool used = is_row || p.start < p.end;
+    // (a core in pieces is in nobody's accumulators as a whole)
+    const float limit = p.cooperative && lane == KM_GROUP_CORE ? (float)P::QUADS : (float)P::MAX_QUADS;
+    const bool bad = !(fabsf(y0) + fabsf(y1) < 1e30f) || !(count <= limit) || (count > 0.0f && !(fabsf(lo) < 1000.0f));
+    p.ok = gw.h > 1e-30f && gw.h < 1e30f && !__any(used && bad);
+    const bool reached = p.ok && used && count > 0.0f;
+    p.quad = reached ? (int)lo : 0;
+    p.quads = reached ? (int)count : 0;
+    // Places: the core's, then the edges', where before them the pieces of the core lie.
+    p.place = 0;
+    const int core = lane_value(p.quads, KM_GROUP_CORE);
+    int edges = core, pieces = core;
+#pragma unroll
+    for (int c = 0; c < KM_GROUP_SEGMENTS; c++) {
+        if (c != KM_GROUP_CORE) {
+            p.place = lane == c ? edges : p.place;
+            edges += lane_value(p.quads, c);
+        }
+    }
+    if (p.cooperative) {
+#pragma unroll
+        for (int i = 0; i < KM_GROUP; i++) {
+            p.place = lane == KM_GROUP_PIECE + i ? pieces : p.place;
+            pieces += lane_value(p.quads, KM_GROUP_PIECE + i);
+        }
+    }
+    p.ok = p.ok && max(edges, pieces) <= P::QUADS;
+}
+
+// The window of one of the segments or row blocks.
+__device__ __forceinline__ GridWindow group_window(const GridWindow& common, const GroupPlan& p, int lane) {
+    GridWindow gw = common;
+    const float cr = gw.reach * (KM_GRID_COLUMN_REACH / KM_GRID_REACH);
+    gw.g_lo = uniform(4.0f * (float)lane_value(p.quad, lane));
+    gw.tiles = (lane_value(p.quads, lane) + 3) / 4;
+    gw.col_lo = uniform(lane_value(p.row_lo, lane) - cr);
+    gw.col_hi = uniform(lane_value(p.row_hi, lane) + cr);
+    gw.first = lane_value(p.first, lane);
+    gw.last = lane_value(p.last, lane);
+    return gw;
+}
+
+// The sums of a segment of columns onto its window, into LDS; bad[]: the rhs columns of each group with a value
+// that is not finite, as bits.
+template <int KT, int G>
+__device__ __forceinline__ bool group_columns(const FwdArgs& a, const WaveView& w, const GroupPlan& p, int lane_of, int kbase,
+                                              const GridWindow& common, const KernelConsts& kc, float* tab, float* sums,
+                                              float (&xv)[KM_GROUP_CHUNK / 64], unsigned (&bad)[GridShape<KT, G>::GP]) {
+    using S = GridShape<KT, G>;
+    constexpr int GP = S::GP, GE = S::GE, MT = S::MT;
+    const int lane = threadIdx.x & 63;
+    const int kk = lane >> 4;
+    WaveView seg = w;
+    seg.range_start = lane_value(p.start, lane_of);
+    seg.range_end = lane_value(p.end, lane_of);
+    const GridWindow gw = group_window(common, p, lane_of);
+    int shift[GP];
+    float4v acc[MT][GE];
+    const bool fine = grid_columns<true, KT, GP, MT, 1, false, false, KM_GROUP_CHUNK>(vectors(a), tab, seg, kbase, 0, gw, kc, nullptr,
+                                                                                     gw.tiles, xv, shift, acc);
+    const int quads = lane_value(p.quads, lane_of);
+    float4v* out = (float4v*)(sums + lane_value(p.place, lane_of) * GroupShape<KT, G>::QUAD) + (lane & 15);
+#pragma unroll
+    for (int g = 0; g < GP; g++) {
+        bad[g] = (unsigned)__ballot(shift[g] == KM_GRID_NOT_FINITE) & 0xffff;
+        const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1 - KM_GRID_EXCHANGE);
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            if (4 * m + kk < quads) {
+#pragma unroll
+                for (int part = 0; part < GE / GP; part++) {
+                    out[((4 * m + kk) * GE + part * GP + g) * 16] = acc[m][part * GP + g] * up;
+                }
+            }
+        }
+    }
+    return fine;
+}
+
+// The first coordinates of a segment.
+__device__ __forceinline__ void group_load(const FwdArgs& a, const WaveView& w, const GroupPlan& p, int segment,
+                                           float (&xv)[KM_GROUP_CHUNK / 64]) {
+    // (an empty one's lie in the matrix too)
+    const int start = min(lane_value(p.start, segment), a.n - 1);
+    grid_load(w.x2, a.x2_s, start, 1, max(lane_value(p.end, segment), start + 1), xv);
+}
+
+// The segments of a wavefront in their order: its piece of a shared core, a cell, half of a core that is
+// not shared, half of the first or last cell.  -1: none.
+__device__ __forceinline__ int group_segment(int stage, int wave, bool cooperative) {
+    static_assert(KM_GROUP == 4, "the lanes of the plan");
+    const bool outer = wave == 0 || wave == 3;
+    switch (stage) {
+        case 0: return cooperative ? KM_GROUP_PIECE + wave : -1;
+        case 1: return wave < 2 ? wave + 2 : wave + 4;
+        case 2: return outer && !cooperative ? (wave == 0 ? KM_GROUP_CORE : KM_GROUP_CORE + 1) : -1;
+        case 3: return wave < 2 ? wave : (wave == 2 ? 8 : 9);
+        default: return -1;
+    }
+}
+
+// The row blocks of a workgroup for rhs columns [kbase, kbase + 16 GP), from the coordinates xv of the first
+// segment on; false (in all wavefronts) if the form does not suit them.  Synchronises the workgroup.
+template <int KT, int G>
+__device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const WaveView& w, const BlockRows& rows,
+                                           const GroupPlan& p, int row0, int kbase, int wave, const GridWindow& common,
+                                           const KernelConsts& kc, int first_stage, float (&xv)[KM_GROUP_CHUNK / 64]) {
+    using P = GroupShape<KT, G>;
+    using S = GridShape<KT, G>;
+    constexpr int GP = S::GP, GE = S::GE, MT = S::MT;
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    float* const tab = lds + wave * P::TABLE;
+    float* const sums = lds + P::SUMS;
+    unsigned* const flags = (unsigned*)(lds + P::FLAGS);
+    unsigned* const bad_segments = flags + KM_GROUP;
+    bool fine = true;
+    const int my_row0 = row0 + wave * KM_BLOCK_SIZE;
+    if (my_row0 < a.m) {
+        const float first = lane_value(p.first, KM_GROUP_ROW + wave), last = lane_value(p.last, KM_GROUP_ROW + wave);
+        const float ya = rows.xa - common.x_ref, yb = rows.xb - common.x_ref;
+        fine = __all(ya >= first && ya <= last && yb >= first && yb <= last);
+    }
+#pragma unroll 1
+    for (int stage = 0; stage < 4; stage++) {
+        if (stage == 1 && p.cooperative) {
+            __syncthreads();
+            // The pieces' sums, added in their order.
+            const int quads = lane_value(p.quads, KM_GROUP_CORE);
+            for (int q = 4 * wave + kk; q < quads; q += 4 * KM_GROUP) {
+                float4v sum[GE];
+#pragma unroll
+                for (int g = 0; g < GE; g++) {
+                    sum[g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+                }
+#pragma unroll
+                for (int i = 0; i < KM_GROUP; i++) {
+                    const int at = q + lane_value(p.quad, KM_GROUP_CORE) - lane_value(p.quad, KM_GROUP_PIECE + i);
+                    if (at >= 0 && at < lane_value(p.quads, KM_GROUP_PIECE + i)) {
+                        const float4v* part = (const float4v*)(sums + lane_value(p.place, KM_GROUP_PIECE + i) * P::QUAD) + li;
+#pragma unroll
+                        for (int g = 0; g < GE; g++) {
+                            sum[g] += part[(at * GE + g) * 16];
+                        }
+                    }
+                }
+#pragma unroll
+                for (int g = 0; g < GE; g++) {
+                    ((float4v*)sums)[(q * GE + g) * 16 + li] = sum[g];
+                }
+            }
+            __syncthreads();
+        }
+        const int segment = group_segment(stage, wave, p.cooperative);
+        if (segment < 0) {
+            continue;
+        }
+        unsigned bad[GP];
+#pragma unroll
+        for (int g = 0; g < GP; g++) {
+            bad[g] = 0;
+        }
+        if (lane_value(p.start, segment) < lane_value(p.end, segment)) {
+            if (stage != first_stage) {
+                group_load(a, w, p, segment, xv);
+            }
+            fine = group_columns<KT, G>(a, w, p, segment, kbase, common, kc, tab, sums, xv, bad) && fine;
+        }
+        if (lane == 0) {
+            unsigned* to = bad_segments + segment * GP;
+#pragma unroll
+            for (int g = 0; g < GP; g++) {
+                to[g] = bad[g];
+            }
+        }
+    }
+    if (lane == 0) {
+        flags[wave] = fine ? 1 : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < KM_GROUP; v++) {
+        fine = fine && __builtin_amdgcn_readfirstlane(flags[v]) != 0;
+    }
+    if (!fine || my_row0 >= a.m) {
+        return fine;
+    }
+    const GridWindow gw = group_window(common, p, KM_GROUP_ROW + wave);
+    const int quad = lane_value(p.quad, KM_GROUP_ROW + wave) + kk;
+    float4v acc[MT][GE];
+    unsigned bad[GP];
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+#pragma unroll
+        for (int g = 0; g < GE; g++) {
+            acc[m][g] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < GP; g++) {
+        bad[g] = 0;
+    }
+#pragma unroll 1
+    for (int c = 0; c < KM_GROUP_SEGMENTS; c++) {
+        if ((lane_value(p.rows, c) >> wave & 1) == 0) {
+            continue;
+        }
+        const int quads = lane_value(p.quads, c);
+        const int offset = quad - lane_value(p.quad, c);
+        const float4v* part = (const float4v*)(sums + lane_value(p.place, c) * P::QUAD) + li;
+        // (kept as register quadruples, see grid_columns)
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+#pragma unroll
+            for (int g = 0; g < GE; g++) {
+                asm volatile("" : "+v"(acc[m][g]));
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++) {
+            if (m >= gw.tiles) {
+                break;
+            }
+            const int at = offset + 4 * m;
+            if (at >= 0 && at < quads) {
+#pragma unroll
+                for (int g = 0; g < GE; g++) {
+                    acc[m][g] += part[(at * GE + g) * 16];
+                }
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < GP; g++) {
+            if (c == KM_GROUP_CORE && p.cooperative) {
+#pragma unroll
+                for (int v = 0; v < KM_GROUP; v++) {
+                    bad[g] |= bad_segments[(KM_GROUP_PIECE + v) * GP + g];
+                }
+            } else {
+                bad[g] |= bad_segments[c * GP + g];
+            }
+        }
+    }
+    int shift[GP];
+#pragma unroll
+    for (int g = 0; g < GP; g++) {
+        shift[g] = (bad[g] >> li & 1) != 0 ? KM_GRID_NOT_FINITE : 0;
+    }
+    const HeldRows held = hold_rows<KT>(rows, common.x_ref, kc);
+    grid_rows<KT, GP, MT, true, true>(a, w, &held, my_row0, KM_BLOCK_SIZE / 16, kbase, gw, kc, shift, acc);
+    return true;
+}
+
+template <int KT, int G>
+__device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigned item, int wave) {
+    using S = GridShape<KT, G>;
+    WaveView w;
+    const unsigned batches = (unsigned)a.num_batches;
+    const unsigned group = item / batches;
+    w.b = item - group * batches;
+    w.row_block = (int)group * KM_GROUP;
+    const int row0 = w.row_block * KM_BLOCK_SIZE;
+    const BatchOffsets o = batch_offsets(a, w.b);
+    w.x1 = a.x1 + o.x1;
+    w.x2 = a.x2 + o.x2;
+    w.rhs = a.rhs + o.rhs;
+    w.params = a.params + o.params;
+    w.range_start = 0;
+    w.range_end = 0;
+    const int blocks = (a.m - 1) / KM_BLOCK_SIZE + 1 - w.row_block;  // in this group, if fewer than KM_GROUP
+    // (rows past the last one repeat it)
+    const BlockRows rows = block_rows(w.x1, a.x1_s, row0 + wave * KM_BLOCK_SIZE, a.m);
+    GridWindow gw;
+    gw.ok = true;
+    gw.x_ref = w.x1[(long long)min(row0 + KM_GROUP * KM_BLOCK_SIZE / 2, a.m - 1) * a.x1_s];
+    KernelConsts kc = make_consts<KT>(w.params, a.params_s, false);
+    GroupPlan p;
+    bool grouped = group_segments(a, o, w.row_block, blocks, &p);
+    if (grouped) {
+        // The first columns are requested together with the ends of all segments, which the windows need.
+        float xv[KM_GROUP_CHUNK / 64];
+        const int first = p.cooperative ? 0 : 1;
+        group_load(a, w, p, group_segment(first, wave, p.cooperative), xv);
+        kc.s = uniform(kc.s);
+        gw.x_ref = uniform(gw.x_ref);
+        gw.s2 = uniform(kc.s * 1.41421356237309504880f);
+        const float inv = __builtin_amdgcn_rcpf(gw.s2);
+        gw.h = uniform(__uint_as_float(__float_as_uint(KM_GRID_STEP * inv) & 0xfffff000u));
+        gw.reach = uniform(KM_GRID_REACH * inv);
+        group_windows<KT, G>(a, w, row0, gw, &p);
+        grouped = __builtin_amdgcn_readfirstlane(p.ok) != 0;
+#pragma unroll 1
+        for (int pass = 0; grouped && pass < G / S::GP; pass++) {
+            const int kbase = (blockIdx.y * G + pass * S::GP) * 16;
+            if (kbase < a.k) {
+                if (pass > 0) {
+                    __syncthreads();
+                    group_load(a, w, p, group_segment(first, wave, p.cooperative), xv);
+                }
+                grouped = group_pass<KT, G>(a, lds, w, rows, p, row0, kbase, wave, gw, kc, first, xv);
+            }
+        }
+        if (!grouped) {
+            __syncthreads();  // (tables of the row blocks below lie over the flags' and sums' place)
+        }
+    }
+    if (!grouped && wave < blocks) {
+        // (what a pass has stored is stored again)
+        grid_item<KT, G, 1>(fresh_args(), lds + wave * KM_GRID_TABLE_FLOATS, (long long)(w.row_block + wave) * a.num_batches + w.b, 0);
+    }
+}
+
+// W: wavefronts per row block, or 1: fewer than one, the workgroup for several row blocks.
 template <int KT, int G, int W>
-__global__ void __launch_bounds__(64 * W, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid(const FwdArgs a) {
     extern __shared__ float lds[];
     const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
     if (item >= a.total_items) {
         return;
     }
-    grid_item<KT, G, W>(a, lds, item, W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if constexpr (W == 1) {
+        group_item<KT, G>(a, lds, (unsigned)item, wave);
+    } else {
+        grid_item<KT, G, W>(a, lds, item, wave);
+    }
 }
 
-// Large launches: workgroups of four wavefronts.  The first items of every XCD go one per wavefront;
-// its last `tail_items` are dispatched last, one per workgroup, so that these quarter-length pieces
-// fill the SIMDs that would otherwise idle while others finish a last full item.
+// The grouped form with a tail: the last `tail_items` groups of every XCD come last and with a workgroup for
+// each of their row blocks, so that short pieces fill the SIMDs that would otherwise idle while others finish a
+// last group.
 template <int KT, int G>
-__global__ void __launch_bounds__(256, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid_grouped(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * KM_GROUP, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid_grouped(const FwdArgs a) {
     extern __shared__ float lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned xcd = blockIdx.x % KM_NUM_XCD;
-    const long long slot = blockIdx.x / KM_NUM_XCD;
-    const long long main_items = a.items_per_xcd - a.tail_items;
-    const long long main_groups = (main_items + 3) / 4;
-    const bool split = slot >= main_groups;
-    const long long local = split ? main_items + (slot - main_groups) : slot * 4 + wave;
-    const long long item = (long long)xcd * a.items_per_xcd + local;
-    if ((!split && local >= main_items) || item >= a.total_items) {
-        return;  // (uniform for the workgroup of a split item)
+    const unsigned slot = blockIdx.x / KM_NUM_XCD;
+    const unsigned first = xcd * (unsigned)a.items_per_xcd;
+    const unsigned main_groups = (unsigned)a.items_per_xcd - (unsigned)a.tail_items;
+    if (slot < main_groups) {
+        if (first + slot < (unsigned)a.total_items) {
+            group_item<KT, G>(a, lds, first + slot, wave);
+        }
+        return;
     }
-    if (split) {
-        grid_item<KT, G, 4>(a, lds, item, wave);
-    } else {
-        grid_item<KT, G, 1>(a, lds + wave * KM_GRID_TABLE_FLOATS, item, 0);
+    const unsigned item = first + main_groups + (slot - main_groups) / KM_GROUP;
+    const unsigned row_block = item / (unsigned)a.num_batches * KM_GROUP + (slot - main_groups) % KM_GROUP;
+    if (item < (unsigned)a.total_items && (long long)row_block * KM_BLOCK_SIZE < a.m) {
+        grid_item<KT, G, KM_GROUP>(fresh_args(), lds, (long long)row_block * a.num_batches + item % (unsigned)a.num_batches, wave);
     }
 }
 
@@ -425,17 +975,28 @@ static hipError_t launch_grid_as(const FwdArgs& a, dim3 grid, hipStream_t stream
 }
 
 template <int KT, int G>
-static hipError_t launch_grid_w(const FwdArgs& a, int waves, dim3 grid, hipStream_t stream) {
-    if (a.tail_items > 0) {
-        using S = GridShape<KT, G>;
-        const long long main_groups = (a.items_per_xcd - a.tail_items + 3) / 4;
-        grid.x = (unsigned)((main_groups + a.tail_items) * KM_NUM_XCD);
-        hipLaunchKernelGGL((fwd_grid_grouped<KT, G>), grid, dim3(256, 1, 1),
-                           (sizeof(float) * grid_lds_floats<S::GE, S::MT, 4>()), stream, a);
+static hipError_t launch_grid_w(FwdArgs& a, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
+    const long long row_blocks = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
+    if (plan.col_splits == 1) {
+        const long long groups = (row_blocks + KM_GROUP - 1) / KM_GROUP;
+        a.total_items = groups * a.num_batches;
+        a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
+        if (plan.group_tail <= 0) {
+            hipLaunchKernelGGL((fwd_grid<KT, G, 1>), dim3((unsigned)(a.items_per_xcd * KM_NUM_XCD), grid_y, 1),
+                               dim3(64 * KM_GROUP, 1, 1), (sizeof(float) * GroupShape<KT, G>::FLOATS), stream, a);
+            return hipGetLastError();
+        }
+        const long long tail = (plan.group_tail + KM_GROUP - 1) / KM_GROUP;
+        a.tail_items = (int)(tail < a.items_per_xcd ? tail : a.items_per_xcd);
+        const dim3 grid((unsigned)((a.items_per_xcd + (KM_GROUP - 1) * a.tail_items) * KM_NUM_XCD), grid_y, 1);
+        hipLaunchKernelGGL((fwd_grid_grouped<KT, G>), grid, dim3(64 * KM_GROUP, 1, 1),
+                           (sizeof(float) * GroupShape<KT, G>::FLOATS), stream, a);
         return hipGetLastError();
     }
-    switch (waves) {
-        case 1: return launch_grid_as<KT, G, 1>(a, grid, stream);
+    a.total_items = row_blocks * a.num_batches;
+    a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
+    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD), grid_y, 1);
+    switch (plan.col_splits) {
         case 2: return launch_grid_as<KT, G, 2>(a, grid, stream);
         case 4: return launch_grid_as<KT, G, 4>(a, grid, stream);
         default: return launch_grid_as<KT, G, 8>(a, grid, stream);
@@ -443,27 +1004,23 @@ static hipError_t launch_grid_w(const FwdArgs& a, int waves, dim3 grid, hipStrea
 }
 
 template <int KT>
-static hipError_t launch_grid_g(const FwdArgs& a, int G, int waves, dim3 grid, hipStream_t stream) {
-    switch (G) {
-        case 1: return launch_grid_w<KT, 1>(a, waves, grid, stream);
-        case 2: return launch_grid_w<KT, 2>(a, waves, grid, stream);
-        default: return launch_grid_w<KT, 4>(a, waves, grid, stream);
+static hipError_t launch_grid_g(FwdArgs& a, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
+    switch (plan.k_chunk / 16) {
+        case 1: return launch_grid_w<KT, 1>(a, plan, grid_y, stream);
+        case 2: return launch_grid_w<KT, 2>(a, plan, grid_y, stream);
+        default: return launch_grid_w<KT, 4>(a, plan, grid_y, stream);
     }
 }
 
 hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream) {
     FwdArgs a;
     fill_fwd_args(p, &a);
-    const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     a.chunks_per_block = 1;
-    a.total_items = row_blocks * p.num_batches;
-    a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    a.tail_items = (int)(plan.group_tail < 0 ? 0 : (plan.group_tail < a.items_per_xcd ? plan.group_tail : a.items_per_xcd));
-    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD), (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk), 1);
+    const unsigned grid_y = (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk);
     if (p.kernel_type == KM_KERNEL_SPECTRAL) {
-        return launch_grid_g<KM_KERNEL_SPECTRAL>(a, plan.k_chunk / 16, plan.col_splits, grid, stream);
+        return launch_grid_g<KM_KERNEL_SPECTRAL>(a, plan, grid_y, stream);
     }
-    return launch_grid_g<KM_KERNEL_RBF>(a, plan.k_chunk / 16, plan.col_splits, grid, stream);
+    return launch_grid_g<KM_KERNEL_RBF>(a, plan, grid_y, stream);
 }
 
 }  // namespace km

@@ -898,7 +898,8 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
     constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
     constexpr int GE = PHASE && !PACK ? 2 : 1;
     constexpr int NP = PHASE ? 3 : 2;  // row factors: V, V (p^2 - variance), and V p
-    constexpr int CH = KM_GRID_CHUNK;
+    constexpr int CH = KM_GRID_CHUNK_ONE;
+    static_assert(CH == KM_BLOCK_SIZE, "a row block is one table");
     constexpr int STEPS = KM_BLOCK_SIZE / 32;
     const int lane = threadIdx.x & 63;
     const int li = lane & 15;
@@ -1014,8 +1015,8 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
                     arg[u] = __builtin_fmaf(av, b2, rb);
                 }
             } else {
-                const float4v r0 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off);
-                const float4v r1 = *(const float4v*)(tab + KM_GRID_TABLE_REST + off + 4);
+                const float4v r0 = *(const float4v*)(tab + grid_table_rest(CH) + off);
+                const float4v r1 = *(const float4v*)(tab + grid_table_rest(CH) + off + 4);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
                     const float y = u < 4 ? x0[u & 3] : x1[u & 3];
@@ -1093,7 +1094,7 @@ template <int KT, bool PACK, int TL>
 __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3) param_grad_grid(const GradArgs a) {
     static_assert(KT == KM_KERNEL_RBF || KT == KM_KERNEL_SPECTRAL, "grid form: rbf or spectral");
     constexpr int MT = KT == KM_KERNEL_SPECTRAL && !PACK ? 5 : 6;
-    __shared__ float tab[KM_GRID_TABLE_FLOATS];
+    __shared__ float tab[grid_table_floats(KM_GRID_CHUNK_ONE)];
     GradItem g;
     if (!grad_item<true>(a, KM_BLOCK_SIZE, 16, &g)) {
         return;
