@@ -335,15 +335,48 @@ __device__ __forceinline__ void f16_load(const FwdArgs& a, const WaveView& w, in
 // column factors 2^(-b^2) come in through cb / sb).
 // PAIRCOS (with SEP): the entries also carry the spectral kernel's cosine, taken per entry from
 // the row phases pa[] and the column phases handed in through sb[] (revolutions).
+// SKIP (locally periodic): with `skip`, row groups out of reach of the step's columns are left out.
 template <int KT, int G, int R, int KS = KM_F16_KSCALE_LOG2, bool SEP = false, int PARTS = 1, bool MULT = false,
-          bool PAIRCOS = false>
+          bool PAIRCOS = false, bool SKIP = false>
 __device__ __forceinline__ void f16_step(const float (&x2v)[8], const float (&raw)[G][8],
                                          const float (&x1v)[R], const KernelConsts& kc,
                                          const bool (&colmask)[G], int (&shift)[G],
                                          float (&scale)[G], float4v (&acc)[R][G * PARTS], float ref = 0.0f,
                                          const float* cb = nullptr, const float* sb = nullptr,
-                                         const float* pa = nullptr) {
+                                         const float* pa = nullptr, bool skip = false, float reach = 0.0f) {
     constexpr int GE = G * PARTS;
+    // The row groups within reach (all of them if a value of rhs or a coordinate is not finite: zero times it is
+    // NaN).
+    unsigned need = (1u << R) - 1;
+    if (SKIP && skip) {
+        float lo = x2v[0], hi = x2v[0];
+#pragma unroll
+        for (int t = 1; t < 8; t++) {
+            lo = fminf(lo, x2v[t]);
+            hi = fmaxf(hi, x2v[t]);
+        }
+        need = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            need |= __any(!(fmaxf(lo - x1v[r], x1v[r] - hi) > reach)) ? 1u << r : 0u;
+        }
+        if (need != (1u << R) - 1) {
+            float m = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                m = __builtin_elementwise_maximum(m, fabsf(x2v[t]));
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    m = __builtin_elementwise_maximum(m, fabsf(raw[g][t]));
+                }
+            }
+            if (!__all(is_finite(m))) {
+                need = (1u << R) - 1;
+            } else if (need == 0) {
+                return;
+            }
+        }
+    }
     half8v bhi[GE], blo[GE];
 #pragma unroll
     for (int g = 0; g < G; g++) {
@@ -398,8 +431,7 @@ __device__ __forceinline__ void f16_step(const float (&x2v)[8], const float (&ra
         }
     }
 
-#pragma unroll
-    for (int r = 0; r < R; r++) {
+    auto group = [&](int r) __attribute__((always_inline)) {
         half2v h2[4], l2[4];
         if (SEP) {
             // Row constants for this lane's 8 columns (ref: their reference point).
@@ -432,6 +464,20 @@ __device__ __forceinline__ void f16_step(const float (&x2v)[8], const float (&ra
             // One row group at a time: the row constants of later groups are not formed ahead
             // of their use (registers); the MFMAs still overlap the next group's evaluation.
             __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // (without branches between them the compiler lets the row groups overlap)
+    if (!SKIP || need == (1u << R) - 1) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            group(r);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if ((need >> r & 1) != 0) {
+                group(r);
+            }
         }
     }
 }
@@ -538,6 +584,23 @@ __device__ __forceinline__ void fwd_mfma_f16_body(const FwdArgs& a, float* lds, 
         x1v[r] = w.x1[(long long)row * a.x1_s];
     }
 
+    // Row groups out of reach are looked for by wavefronts of 128 rows only: n = 50021, k = 16, 8 sets, 10 points
+    // per unit 94.6 -> 70.8 us a call, bound by VALU issue.  With fewer rows a step is too short for the branches
+    // (n = 20000, 4 sets at 40 points per unit, 32 rows: 75.9 -> 79.8 us).  (A row that is not finite has no
+    // entry of zero.)
+    constexpr bool SKIP = KT == KM_KERNEL_LOCALLY_PERIODIC && R == 8;
+    bool skip = false;
+    float reach = 0.0f;
+    if (SKIP && col_begin < col_end) {
+        bool finite = true;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            finite = finite && is_finite(x1v[r]);
+        }
+        reach = periodic_reach(kc);
+        skip = __all(finite && periodic_skip(x1v[R / 2], w.x2[(long long)col_begin * a.x2_s], w.x2[(long long)(col_end - 1) * a.x2_s], reach));
+    }
+
     // rhs columns past k read a valid column instead and are zeroed through their scale.
     bool colmask[G];
     unsigned rhs_lane[G];  // byte offset of (column 8 kk, rhs column of this lane)
@@ -563,6 +626,10 @@ __device__ __forceinline__ void fwd_mfma_f16_body(const FwdArgs& a, float* lds, 
         }
     }
 
+    auto step = [&](const float (&x2v)[8], const float (&raw)[G][8]) __attribute__((always_inline)) {
+        f16_step<KT, G, R, KM_F16_KSCALE_LOG2, false, 1, false, false, SKIP>(x2v, raw, x1v, kc, colmask, shift, scale, acc, 0.0f,
+                                                                            nullptr, nullptr, nullptr, skip, reach);
+    };
     if (col_begin < col_end) {
         float x2v[8], raw[G][8];
         f16_load<G>(a, w, col_begin, col_end, kk, x2_lane, rhs_lane, x2v, raw);
@@ -573,7 +640,7 @@ __device__ __forceinline__ void fwd_mfma_f16_body(const FwdArgs& a, float* lds, 
                 if (more) {
                     f16_load<G>(a, w, c0 + 32, col_end, kk, x2_lane, rhs_lane, x2n, rawn);
                 }
-                f16_step<KT, G, R>(x2v, raw, x1v, kc, colmask, shift, scale, acc);
+                step(x2v, raw);
                 if (more) {
 #pragma unroll
                     for (int t = 0; t < 8; t++) {
@@ -585,7 +652,7 @@ __device__ __forceinline__ void fwd_mfma_f16_body(const FwdArgs& a, float* lds, 
                     }
                 }
             } else {
-                f16_step<KT, G, R>(x2v, raw, x1v, kc, colmask, shift, scale, acc);
+                step(x2v, raw);
                 if (more) {
                     f16_load<G>(a, w, c0 + 32, col_end, kk, x2_lane, rhs_lane, x2v, raw);
                 }

@@ -154,6 +154,8 @@ struct BlockLds {
     half8v bop[KM_BLK_STEPS][GE][2][64];  // [step][group][hi, lo][lane]
     unsigned maxbuf[2][32];               // [parity][rhs column]: bits of max |rhs|
     unsigned nofold[2];                   // [parity]: nonzero if a column forbids the folded form
+    unsigned noskip[2];                   // [parity]: nonzero if a column's coordinate or rhs value is not finite
+    float ends[2][2][KM_BLK_CHUNK / 8];   // [parity][smallest, largest x2][group of 8 columns]
     unsigned x1lo, x1hi;                  // ordered keys of min / max x1 over the workgroup's rows
 };
 
@@ -201,11 +203,14 @@ __device__ __forceinline__ void block_step(BlockLds<(PHASE ? 2 : 1) * G>& lds, i
 // All steps of the current chunk for row block J: the (at most two) steps that straddle an end
 // of the block's column range go through the masked form, the others through a loop without
 // masks or branches.  Without folded coordinates (rare) every step takes the masked form.
+// Locally periodic: steps whose bit in `need` is clear are left out (n = 1e5, k = 16, 8 sets: 142 -> 125 us a call; the
+// rest of a chunk, its preparation between two barriers, stays).
 template <int KT, bool PHASE, bool FOLD, int G, int J>
 __device__ __forceinline__ void block_consume_rows(
     BlockLds<(PHASE ? 2 : 1) * G>& lds, int parity, int chunk0, int chunk_end, int range_start,
-    int range_end, const float (&x1v)[2 * KM_BLK_ROW_BLOCKS], const float (&ph1)[2 * KM_BLK_ROW_BLOCKS],
+    int range_end, unsigned need, const float (&x1v)[2 * KM_BLK_ROW_BLOCKS], const float (&ph1)[2 * KM_BLK_ROW_BLOCKS],
     const KernelConsts& kc, int kk, int lane, float4v (&acc)[2 * KM_BLK_ROW_BLOCKS][(PHASE ? 2 : 1) * G]) {
+    constexpr bool SKIP = KT == KM_KERNEL_LOCALLY_PERIODIC;
     const int lo = max(range_start, chunk0);
     const int hi = min(range_end, chunk_end);
     if (lo >= hi) {
@@ -215,6 +220,9 @@ __device__ __forceinline__ void block_consume_rows(
     int last = (hi - 1 - chunk0) >> 5;
     if (!FOLD) {
         for (int st = first; st <= last; st++) {
+            if (SKIP && (need >> st & 1) == 0) {
+                continue;
+            }
             block_step<KT, PHASE, false, true, G, J>(lds, parity, chunk0, st, range_start, range_end, x1v,
                                                      ph1, kc, kk, lane, acc);
         }
@@ -229,12 +237,15 @@ __device__ __forceinline__ void block_consume_rows(
     }
     for (int i = 0; i < 2; i++) {
         const int st = i == 0 ? partial0 : partial1;
-        if (st >= 0) {
+        if (st >= 0 && (!SKIP || (need >> st & 1) != 0)) {
             block_step<KT, PHASE, FOLD, true, G, J>(lds, parity, chunk0, st, range_start, range_end, x1v, ph1,
                                                     kc, kk, lane, acc);
         }
     }
     for (int st = first; st <= last; st++) {
+        if (SKIP && (need >> st & 1) == 0) {
+            continue;
+        }
         block_step<KT, PHASE, FOLD, false, G, J>(lds, parity, chunk0, st, range_start, range_end, x1v, ph1,
                                                  kc, kk, lane, acc);
     }
@@ -243,15 +254,15 @@ __device__ __forceinline__ void block_consume_rows(
 template <int KT, bool PHASE, bool FOLD, int G>
 __device__ __forceinline__ void block_consume(
     BlockLds<(PHASE ? 2 : 1) * G>& lds, int parity, int chunk0, int chunk_end,
-    const int (&ws)[KM_BLK_ROW_BLOCKS], const int (&we)[KM_BLK_ROW_BLOCKS],
+    const int (&ws)[KM_BLK_ROW_BLOCKS], const int (&we)[KM_BLK_ROW_BLOCKS], const unsigned (&need)[KM_BLK_ROW_BLOCKS],
     const float (&x1v)[2 * KM_BLK_ROW_BLOCKS], const float (&ph1)[2 * KM_BLK_ROW_BLOCKS],
     const KernelConsts& kc, int kk, int lane,
     float4v (&acc)[2 * KM_BLK_ROW_BLOCKS][(PHASE ? 2 : 1) * G]) {
     // Row blocks the workgroup does not have carry empty ranges.
-    block_consume_rows<KT, PHASE, FOLD, G, 0>(lds, parity, chunk0, chunk_end, ws[0], we[0], x1v, ph1, kc, kk, lane, acc);
-    block_consume_rows<KT, PHASE, FOLD, G, 1>(lds, parity, chunk0, chunk_end, ws[1], we[1], x1v, ph1, kc, kk, lane, acc);
-    block_consume_rows<KT, PHASE, FOLD, G, 2>(lds, parity, chunk0, chunk_end, ws[2], we[2], x1v, ph1, kc, kk, lane, acc);
-    block_consume_rows<KT, PHASE, FOLD, G, 3>(lds, parity, chunk0, chunk_end, ws[3], we[3], x1v, ph1, kc, kk, lane, acc);
+    block_consume_rows<KT, PHASE, FOLD, G, 0>(lds, parity, chunk0, chunk_end, ws[0], we[0], need[0], x1v, ph1, kc, kk, lane, acc);
+    block_consume_rows<KT, PHASE, FOLD, G, 1>(lds, parity, chunk0, chunk_end, ws[1], we[1], need[1], x1v, ph1, kc, kk, lane, acc);
+    block_consume_rows<KT, PHASE, FOLD, G, 2>(lds, parity, chunk0, chunk_end, ws[2], we[2], need[2], x1v, ph1, kc, kk, lane, acc);
+    block_consume_rows<KT, PHASE, FOLD, G, 3>(lds, parity, chunk0, chunk_end, ws[3], we[3], need[3], x1v, ph1, kc, kk, lane, acc);
 }
 
 template <int KT, bool PHASE, int G>
@@ -339,6 +350,7 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
     }
     if (tid < 2) {
         lds.nofold[tid] = 0u;
+        lds.noskip[tid] = 0u;
     }
     if (tid == 2) {
         lds.x1lo = 0xffffffffu;
@@ -348,18 +360,32 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
 
     // Rows of this wavefront: rows 32 wave .. 32 wave + 31 of every row block, as 2 groups of 16.
     float x1v[2 * NB], ph1[2 * NB];
+    bool rows_finite = true;
+    float row_lo[NB], row_hi[NB];  // of this wavefront's rows of each row block
     {
         float lo = __builtin_inff(), hi = -__builtin_inff();
         bool bad = false;
+        if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                row_lo[j] = __builtin_inff();
+                row_hi[j] = -__builtin_inff();
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 2 * NB; r++) {
             const int row = min((rb0 + r / 2) * KM_BLOCK_SIZE + 32 * wave + 16 * (r & 1) + li, a.m - 1);
             x1v[r] = x1[(long long)row * a.x1_s];
             ph1[r] = TWO ? phase_rev(kc.f, x1v[r], c_ref) : 0.0f;
+            if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+                row_lo[r / 2] = fminf(row_lo[r / 2], x1v[r]);
+                row_hi[r / 2] = fmaxf(row_hi[r / 2], x1v[r]);
+            }
             if (r / 2 < nblk) {
                 lo = fminf(lo, x1v[r]);
                 hi = fmaxf(hi, x1v[r]);
                 bad = bad || x1v[r] != x1v[r];
+                rows_finite = rows_finite && is_finite(x1v[r]);
             }
         }
 #pragma unroll
@@ -373,6 +399,15 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
         if (lane == 0) {
             atomicMin(&lds.x1lo, lo == lo ? float_key(lo) : 0u);
             atomicMax(&lds.x1hi, lo == lo ? float_key(hi) : 0xffffffffu);
+        }
+    }
+
+    // (a row that is not finite has no entry of zero)
+    const float reach = __all(rows_finite) ? periodic_reach(kc) : __builtin_inff();
+    if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            wave_min_max(&row_lo[j], &row_hi[j]);
         }
     }
 
@@ -429,6 +464,17 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
             } else if (TWO) {
                 lds.tab[parity][2][tid] = phase_rev(kc.f, xv, c_ref);
             }
+            if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+                float lo, hi;
+                group8_min_max(xv, &lo, &hi);
+                if ((tid & 7) == 0) {
+                    lds.ends[parity][0][tid >> 3] = lo;
+                    lds.ends[parity][1][tid >> 3] = hi;
+                }
+                if (!__all(is_finite(xv)) && lane == 0) {
+                    atomicOr(&lds.noskip[parity], 1u);
+                }
+            }
             const bool ok = err == 0.0f && fabsf(xs) <= KM_BLK_FOLD_SPAN;
             if (!__all(ok) && lane == 0) {
                 atomicOr(&lds.nofold[parity], 1u);
@@ -477,6 +523,16 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
                     m = fmaxf(m, av < __builtin_inff() ? av : 0.0f);
                 }
             }
+            if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+                float largest = 0.0f;
+#pragma unroll
+                for (int t = 0; t < 8; t++) {
+                    largest = __builtin_elementwise_maximum(largest, __builtin_elementwise_maximum(fabsf(raw[0][g][t]), fabsf(raw[1][g][t])));
+                }
+                if (!__all(is_finite(largest)) && lane == 0) {
+                    atomicOr(&lds.noskip[parity], 1u);
+                }
+            }
             m = column_max(m);
             if (kk == 0) {
                 atomicMax(&lds.maxbuf[parity][16 * g + li], __float_as_uint(m));
@@ -520,6 +576,7 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
         }
         if (tid == 32) {
             lds.nofold[parity ^ 1] = 0u;
+            lds.noskip[parity ^ 1] = 0u;
         }
         if (__any(rescale)) {
 #pragma unroll
@@ -570,10 +627,30 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
         __syncthreads();
 
         // ---- consume ---------------------------------------------------------------------
+        // Locally periodic: the steps of which a group of 8 columns is within reach of this wavefront's rows
+        // of a row block, as bits (all of them where a value is not finite: zero times it is NaN).
+        unsigned need[NB];
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            need[j] = (1u << KM_BLK_STEPS) - 1;
+        }
+        if (KT == KM_KERNEL_LOCALLY_PERIODIC && __builtin_amdgcn_readfirstlane(lds.noskip[parity]) == 0) {
+            const float lo = lds.ends[parity][0][lane & 31], hi = lds.ends[parity][1][lane & 31];
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                const unsigned groups = (unsigned)__ballot(!(fmaxf(lo - row_hi[j], row_lo[j] - hi) > reach));
+                unsigned any = groups | groups >> 1;
+                any = (any | any >> 2) & 0x11111111u;
+                // (bit 4 st -> bit st)
+                any = (any | any >> 3) & 0x03030303u;
+                any = (any | any >> 6) & 0x000f000fu;
+                need[j] = (any | any >> 12) & 0xffu;
+            }
+        }
         if (fold) {
-            block_consume<KT, PHASE, true, G>(lds, parity, chunk0, chunk_end, ws, we, x1v, ph1, kc, kk, lane, acc);
+            block_consume<KT, PHASE, true, G>(lds, parity, chunk0, chunk_end, ws, we, need, x1v, ph1, kc, kk, lane, acc);
         } else {
-            block_consume<KT, PHASE, false, G>(lds, parity, chunk0, chunk_end, ws, we, x1v, ph1, kc, kk, lane, acc);
+            block_consume<KT, PHASE, false, G>(lds, parity, chunk0, chunk_end, ws, we, need, x1v, ph1, kc, kk, lane, acc);
         }
         parity ^= 1;
     }
