@@ -193,13 +193,7 @@ _PREPARED_LIMIT = 512
 
 
 def _signature(op: str, kernel_type: str, tensors) -> tuple:
-    key = [op, kernel_type]
-    for t in tensors:
-        key.append(t.shape)
-        key.append(t.stride())
-        key.append(t.dtype)
-        key.append(t.device)
-    return tuple(key)
+    return (op, kernel_type, *[(t.shape, t.stride(), t.dtype, t.device) for t in tensors])
 
 
 def _remember(key, value):
@@ -207,6 +201,14 @@ def _remember(key, value):
         _PREPARED.clear()
     _PREPARED[key] = value
     return value
+
+
+def _marshalled(tensors, strides, nonempty) -> list:
+    """Pointer and strides of each tensor of a prepared call."""
+    call_args = []
+    for t, st, filled in zip(tensors, strides, nonempty):
+        call_args += (t.data_ptr() if filled else None, st)
+    return call_args
 
 
 # -- the checks of the reference's entry points (native/common/entrypoint.h:3-14) ----------
@@ -301,10 +303,7 @@ def matmul(kernel_type: str, x1: Tensor, x2: Tensor, rhs: Tensor, params: Tensor
     elif (tuple(out.shape) != out_shape or out.dtype != torch.float32 or out.device != device
           or not out.is_contiguous()):
         raise RuntimeError(f"out must be a contiguous float32 tensor of shape {out_shape} on {device}")
-    call_args = []
-    for t, st, filled in zip(tensors, strides, nonempty):
-        call_args.append(t.data_ptr() if filled else None)
-        call_args.append(st)
+    call_args = _marshalled(tensors, strides, nonempty)
     with _on_device(device):
         status = fn(*head, *call_args, out.data_ptr() if out.numel() > 0 else None,
                     ctypes.byref(options) if options is not None else None, _stream(device))
@@ -382,10 +381,7 @@ def param_grad(kernel_type: str, x1: Tensor, x2: Tensor, left: Tensor, right: Te
     elif (tuple(out.shape) != out_shape or out.dtype != torch.float32 or out.device != device
           or not out.is_contiguous()):
         raise RuntimeError(f"out must be a contiguous float32 tensor of shape {out_shape} on {device}")
-    call_args = []
-    for t, st, filled in zip(tensors, strides, nonempty):
-        call_args.append(t.data_ptr() if filled else None)
-        call_args.append(st)
+    call_args = _marshalled(tensors, strides, nonempty)
     out_ptr = out.data_ptr() if out.numel() > 0 else None
     if static_scratch:
         with _on_device(device):
@@ -412,40 +408,47 @@ def param_grad(kernel_type: str, x1: Tensor, x2: Tensor, left: Tensor, right: Te
 def index(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tensor, end: Tensor,
           batch_indices: Sequence[Tensor], row_index: Tensor, col_index: Tensor) -> Tensor:
     """out[q] = K[batch_indices[q]..., row_index[q], col_index[q]]   (C ABI: km_index)."""
-    kid = _kernel_id(kernel_type)
-    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
     batch_indices = tuple(batch_indices)
-    if len(batch_indices) != len(batch_shape):
-        raise RuntimeError(
-            f"expected {len(batch_shape)} batch index tensors, got {len(batch_indices)}"
-        )
-    for t in (*batch_indices, row_index, col_index):
-        check_cuda_int32(t)
-    if row_index.dim() == 0:  # scalar indices: treat as one entry
-        result = index(kernel_type, x1, x2, params, start, end,
-                       [b.reshape(1) for b in batch_indices], row_index.reshape(1),
-                       col_index.reshape(1))
-        return result.reshape(())
-    shape = tuple(row_index.shape)
-    if len(shape) < 1 or len(shape) > MAX_BATCH_RANK + 1:
-        raise RuntimeError(f"index tensors must have between 1 and {MAX_BATCH_RANK + 1} dimensions")
-    for t in (*batch_indices, col_index):
-        if tuple(t.shape) != shape:
-            raise RuntimeError("all index tensors must have the same shape")
-    lib = load_library()
-    out = torch.empty(shape, dtype=torch.float32, device=x1.device)
-    rank = len(batch_shape)
-    bi_ptrs, bi_strides, _keep = _batch_index_args(batch_indices, rank)
-    with _on_device(x1.device):
-        status = lib.km_index(
-            kid, rank, _i64(batch_shape), x1.shape[-1], x2.shape[-1],
-            *_tensor_args(x1), *_tensor_args(x2), *_tensor_args(params),
-            *_tensor_args(start), *_tensor_args(end),
-            len(shape), _i64(shape), bi_ptrs, bi_strides,
-            *_tensor_args(row_index), *_tensor_args(col_index), _ptr(out), _stream(x1.device),
-        )
+    tensors = (x1, x2, params, start, end, row_index, col_index)
+    key = _signature("index", kernel_type, tensors + batch_indices)
+    prepared = _PREPARED.get(key)
+    if prepared is None:
+        kid = _kernel_id(kernel_type)
+        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+        if len(batch_indices) != len(batch_shape):
+            raise RuntimeError(
+                f"expected {len(batch_shape)} batch index tensors, got {len(batch_indices)}"
+            )
+        for t in (*batch_indices, row_index, col_index):
+            check_cuda_int32(t)
+        if row_index.dim() == 0:  # scalar indices: treat as one entry
+            result = index(kernel_type, x1, x2, params, start, end,
+                           [b.reshape(1) for b in batch_indices], row_index.reshape(1),
+                           col_index.reshape(1))
+            return result.reshape(())
+        shape = tuple(row_index.shape)
+        if len(shape) < 1 or len(shape) > MAX_BATCH_RANK + 1:
+            raise RuntimeError(f"index tensors must have between 1 and {MAX_BATCH_RANK + 1} dimensions")
+        for t in (*batch_indices, col_index):
+            if tuple(t.shape) != shape:
+                raise RuntimeError("all index tensors must have the same shape")
+        rank = len(batch_shape)
+        stride_arrays = [_i64(t.stride()) for t in batch_indices]
+        prepared = _remember(key, (
+            load_library().km_index, (kid, rank, _i64(batch_shape), x1.shape[-1], x2.shape[-1]),
+            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors), shape, _i64(shape), rank,
+            (_i64p * max(rank, 1))(*[ctypes.cast(a, _i64p) for a in stride_arrays]), stride_arrays,
+        ))
+    fn, head, strides, nonempty, shape, sizes, rank, bi_strides, _keep = prepared
+    device = x1.device
+    out = torch.empty(shape, dtype=torch.float32, device=device)
+    call_args = _marshalled(tensors, strides, nonempty)
+    bi_ptrs = (_vp * max(rank, 1))(*[t.data_ptr() for t in batch_indices])
+    with _on_device(device):
+        status = fn(*head, *call_args[:10], len(shape), sizes, bi_ptrs, bi_strides, *call_args[10:],
+                    out.data_ptr() if out.numel() > 0 else None, _stream(device))
     if status != 0:
-        _raise(lib, status)
+        _raise(load_library(), status)
     return out
 
 
@@ -502,46 +505,59 @@ def index_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: T
 def dense(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tensor,
           end: Tensor) -> Tensor:
     """Masked kernel matrix [..., m, n]   (C ABI: km_dense)."""
-    kid = _kernel_id(kernel_type)
-    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-    lib = load_library()
-    out = torch.empty((*batch_shape, x1.shape[-1], x2.shape[-1]), dtype=torch.float32, device=x1.device)
-    with _on_device(x1.device):
-        status = lib.km_dense(
-            kid, len(batch_shape), _i64(batch_shape), x1.shape[-1], x2.shape[-1],
-            *_tensor_args(x1), *_tensor_args(x2), *_tensor_args(params),
-            *_tensor_args(start), *_tensor_args(end), _ptr(out), _stream(x1.device),
-        )
+    tensors = (x1, x2, params, start, end)
+    key = _signature("dense", kernel_type, tensors)
+    prepared = _PREPARED.get(key)
+    if prepared is None:
+        kid = _kernel_id(kernel_type)
+        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+        m, n = x1.shape[-1], x2.shape[-1]
+        prepared = _remember(key, (
+            load_library().km_dense, (kid, len(batch_shape), _i64(batch_shape), m, n),
+            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors), (*batch_shape, m, n),
+        ))
+    fn, head, strides, nonempty, out_shape = prepared
+    device = x1.device
+    out = torch.empty(out_shape, dtype=torch.float32, device=device)
+    with _on_device(device):
+        status = fn(*head, *_marshalled(tensors, strides, nonempty), out.data_ptr() if out.numel() > 0 else None,
+                    _stream(device))
     if status != 0:
-        _raise(lib, status)
+        _raise(load_library(), status)
     return out
 
 
 def dense_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tensor, end: Tensor,
               out_grad: Tensor) -> Tensor:
     """grad[..., P] of sum(out_grad * dense(...)) w.r.t. params   (C ABI: km_dense_bwd)."""
-    kid = _kernel_id(kernel_type)
-    check_cuda(out_grad)
-    check_float(out_grad)
-    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-    _check_batch("out_grad", out_grad, batch_shape, 2)
-    m, n = x1.shape[-1], x2.shape[-1]
-    if tuple(out_grad.shape[-2:]) != (m, n):
-        raise RuntimeError(f"out_grad has shape {tuple(out_grad.shape)}, expected (..., {m}, {n})")
-    lib = load_library()
-    sizes = _i64(batch_shape)
-    grad = torch.empty((*batch_shape, params.shape[-1]), dtype=torch.float32, device=x1.device)
-    need = lib.km_param_grad_workspace_size(kid, len(batch_shape), sizes, m, n, 0)
-    workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=x1.device)
-    with _on_device(x1.device):
-        status = lib.km_dense_bwd(
-            kid, len(batch_shape), sizes, m, n,
-            *_tensor_args(x1), *_tensor_args(x2), *_tensor_args(params),
-            *_tensor_args(start), *_tensor_args(end), *_tensor_args(out_grad),
-            _ptr(grad), ctypes.c_void_p(workspace.data_ptr()), need, _stream(x1.device),
-        )
+    tensors = (x1, x2, params, start, end, out_grad)
+    key = _signature("dense_bwd", kernel_type, tensors)
+    prepared = _PREPARED.get(key)
+    if prepared is None:
+        kid = _kernel_id(kernel_type)
+        check_cuda(out_grad)
+        check_float(out_grad)
+        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+        _check_batch("out_grad", out_grad, batch_shape, 2)
+        m, n = x1.shape[-1], x2.shape[-1]
+        if tuple(out_grad.shape[-2:]) != (m, n):
+            raise RuntimeError(f"out_grad has shape {tuple(out_grad.shape)}, expected (..., {m}, {n})")
+        lib = load_library()
+        sizes = _i64(batch_shape)
+        prepared = _remember(key, (
+            lib.km_dense_bwd, (kid, len(batch_shape), sizes, m, n),
+            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors),
+            (*batch_shape, params.shape[-1]), lib.km_param_grad_workspace_size(kid, len(batch_shape), sizes, m, n, 0),
+        ))
+    fn, head, strides, nonempty, out_shape, need = prepared
+    device = x1.device
+    grad = torch.empty(out_shape, dtype=torch.float32, device=device)
+    workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
+    with _on_device(device):
+        status = fn(*head, *_marshalled(tensors, strides, nonempty), grad.data_ptr() if grad.numel() > 0 else None,
+                    workspace.data_ptr(), need, _stream(device))
     if status != 0:
-        _raise(lib, status)
+        _raise(load_library(), status)
     return grad
 
 

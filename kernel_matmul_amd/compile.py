@@ -60,6 +60,11 @@ def _debug_enabled() -> bool:
     return os.environ.get("KERNEL_MATMUL_COMPILE_DEBUG", "false") == "true"
 
 
+def module_environment() -> tuple:
+    """What a module takes from the environment when it is loaded."""
+    return _debug_enabled(), os.environ.get("KERNEL_MATMUL_COMPILE_PRINT_SIZE", "false") == "true"
+
+
 class NativeModule:
     """One operator bound to a kernel type: what ``load_native`` returns.
 
@@ -82,8 +87,7 @@ class NativeModule:
         self.op = op
         self.kernel_type = kernel_types[0]
         self.defines = dict(defines)
-        self.debug = _debug_enabled()
-        self.print_size = os.environ.get("KERNEL_MATMUL_COMPILE_PRINT_SIZE", "false") == "true"
+        self.debug, self.print_size = module_environment()
         self.name = "km___" + op + "".join(
             f"___{key}" if defines[key] is None else f"___{key}__{defines[key]}"
             for key in sorted(defines)

@@ -21,6 +21,7 @@ import multiprocessing.pool
 from typing import List, Tuple
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 from torch import Size, Tensor, dtype
 
 from kernel_matmul_amd import ranges
@@ -121,6 +122,21 @@ except ImportError:
         return device, dtype_
 
 
+def _plain(differentiable: tuple) -> bool:
+    """Whether nothing records or transforms a call on these tensors, so that the native function can be called
+    itself (an autograd function costs a fifth of a small product's host time)."""
+    if torch.is_grad_enabled():
+        for t in differentiable:
+            if t.requires_grad:
+                return False
+    return (
+        forward_ad._current_level < 0  # (no dual tensors)
+        and not torch._C._are_functorch_transforms_active()
+        and torch._C._get_tracing_state() is None
+        and not torch.compiler.is_compiling()
+    )
+
+
 class _MatmulOperator(torch.autograd.Function):
     """K @ rhs with gradients for the hyper-parameters (matmul_bwd) and for rhs (K^T @ grad)."""
 
@@ -191,6 +207,34 @@ class _IndexOperator(torch.autograd.Function):
         return (None, None, grad, None, None, None, None, None, None, *[None for _ in batch_indices])
 
 
+def _widen(t: Tensor, batch_shape: Size, trailing: int) -> Tensor:
+    """``t`` as a stride-0 view of the batch shape (itself where it has it)."""
+    if t.shape[:-trailing] == batch_shape:
+        return t
+    return t.expand(*batch_shape, *t.shape[-trailing:])
+
+
+class _Native:
+    """A native function of the operator's kernel type, made when it is first used (a fit makes an operator for
+    every set of hyper-parameters and uses one or two)."""
+
+    def __init__(self, op: str, configuration, autotuned: bool = False):
+        self._op = op
+        self._configuration = configuration
+        self._autotuned = autotuned
+
+    def __set_name__(self, owner, name):
+        self._name = name
+
+    def __get__(self, operator, owner=None):
+        if operator is None:
+            return self
+        pool = {"compile_pool": operator._compile_pool} if self._autotuned else {}
+        function = NativeFunction(self._op, self._configuration(operator._kernel_type), **pool)
+        operator.__dict__[self._name] = function
+        return function
+
+
 class KernelMatmulLinearOperator(LinearOperator):
     """The (masked) kernel matrix K(x1, x2) of shape (..., M, N), never materialised.
 
@@ -203,6 +247,14 @@ class KernelMatmulLinearOperator(LinearOperator):
         symmetric: whether K equals its transpose; determined from ``x1 == x2`` if omitted.
         compile_pool: accepted for compatibility; nothing is compiled at run time.
     """
+
+    _native_matmul = _Native("matmul", MatmulAutotuneConfiguration, autotuned=True)
+    _native_matmul_bwd = _Native("matmul_bwd", MatmulBwdConfiguration)
+    _native_bilinear_derivative = _Native("bilinear_derivative", BilinearDerivativeConfiguration)
+    _native_index = _Native("index", IndexConfiguration)
+    _native_index_bwd = _Native("index_bwd", IndexBwdConfiguration)
+    _native_dense = _Native("dense", DenseConfiguration)
+    _native_dense_bwd = _Native("dense_bwd", DenseBwdConfiguration)
 
     def __init__(
         self,
@@ -226,32 +278,24 @@ class KernelMatmulLinearOperator(LinearOperator):
         if symmetric is None:
             symmetric = torch.equal(x1, x2)
 
-        batch_shape = torch.broadcast_shapes(
-            x1.shape[:-2], x2.shape[:-2], params.shape[:-1], start.shape[:-1], end.shape[:-1]
-        )
-        self._x1 = x1.expand(*batch_shape, *x1.shape[-2:])
-        self._x2 = x2.expand(*batch_shape, *x2.shape[-2:])
-        self._params = params.expand(*batch_shape, params.shape[-1])
-        self._start = start.expand(*batch_shape, start.shape[-1])
-        self._end = end.expand(*batch_shape, end.shape[-1])
+        shapes = (x1.shape[:-2], x2.shape[:-2], params.shape[:-1], start.shape[:-1], end.shape[:-1])
+        distinct = set(shapes) - {Size(())}
+        if len(distinct) > 1:
+            batch_shape = torch.broadcast_shapes(*shapes)
+        else:  # (the usual case, at a tenth of the time)
+            batch_shape = distinct.pop() if distinct else Size(())
+        self._x1 = _widen(x1, batch_shape, 2)
+        self._x2 = _widen(x2, batch_shape, 2)
+        self._params = _widen(params, batch_shape, 1)
+        self._start = _widen(start, batch_shape, 1)
+        self._end = _widen(end, batch_shape, 1)
         self._kernel_type = kernel_type
+        self._compile_pool = compile_pool
         self._batch_shape = batch_shape
         self._symmetric = symmetric
         self._ranges_t = None  # pattern of the transpose, built on first use
         self._diagonal_indices = None  # index tensors of the diagonal, built on first use
         self._native_args = None  # (batch shape, widened constructor tensors) of the last call
-
-        self._native_matmul = NativeFunction(
-            "matmul", MatmulAutotuneConfiguration(kernel_type), compile_pool=compile_pool
-        )
-        self._native_matmul_bwd = NativeFunction("matmul_bwd", MatmulBwdConfiguration(kernel_type))
-        self._native_bilinear_derivative = NativeFunction(
-            "bilinear_derivative", BilinearDerivativeConfiguration(kernel_type)
-        )
-        self._native_index = NativeFunction("index", IndexConfiguration(kernel_type))
-        self._native_index_bwd = NativeFunction("index_bwd", IndexBwdConfiguration(kernel_type))
-        self._native_dense = NativeFunction("dense", DenseConfiguration(kernel_type))
-        self._native_dense_bwd = NativeFunction("dense_bwd", DenseBwdConfiguration(kernel_type))
 
     # -- helpers -------------------------------------------------------------------------
     def _get_args_for_native(self, batch_shape) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -260,22 +304,17 @@ class KernelMatmulLinearOperator(LinearOperator):
         solvers call with the same one over and over.  ``params`` is widened on every call, so
         the view belongs to the autograd mode of that call (a view made under ``no_grad`` or
         ``inference_mode`` would cut later calls off from the hyper-parameters' gradient)."""
-        batch_shape = tuple(batch_shape)
-
-        def widen(t: Tensor, trailing: int) -> Tensor:
-            return t.expand(*batch_shape, *t.shape[-trailing:])
-
+        batch_shape = Size(batch_shape)
         if self._native_args is None or self._native_args[0] != batch_shape:
             fixed = (
-                widen(self._x1.detach().squeeze(-1), 1),
-                widen(self._x2.detach().squeeze(-1), 1),
-                widen(self._start, 1),
-                widen(self._end, 1),
+                _widen(self._x1.detach().squeeze(-1), batch_shape, 1),
+                _widen(self._x2.detach().squeeze(-1), batch_shape, 1),
+                _widen(self._start, batch_shape, 1),
+                _widen(self._end, batch_shape, 1),
             )
             self._native_args = (batch_shape, fixed)
         x1, x2, start, end = self._native_args[1]
-        params = self._params if tuple(self._params.shape[:-1]) == batch_shape else widen(self._params, 1)
-        return x1, x2, params, start, end
+        return x1, x2, _widen(self._params, batch_shape, 1), start, end
 
     def _transposed_ranges(self, batch_shape=None) -> tuple[Tensor, Tensor]:
         """Pattern of K^T, computed once per operator (the check that the pattern is block
@@ -301,11 +340,11 @@ class KernelMatmulLinearOperator(LinearOperator):
             batch_shape = broadcast[:-2]
             rhs_ = rhs.expand(*broadcast)
         x1, x2, params, start, end = self._get_args_for_native(batch_shape)
-        result = _MatmulOperator.apply(
-            x1, x2, rhs_, params, start, end, self._native_matmul, self._native_matmul_bwd,
-            self._symmetric, self._transposed_ranges,
-        )
-        return result.reshape(*batch_shape, *result.shape[-2:])
+        native = self._native_matmul
+        call = (x1, x2, rhs_, params, start, end)
+        if _plain((rhs_, params)):
+            return native(*call)
+        return _MatmulOperator.apply(*call, native, self._native_matmul_bwd, self._symmetric, self._transposed_ranges)
 
     def _size(self) -> Size:
         return Size((*self._batch_shape, self._x1.size(-2), self._x2.size(-2)))
@@ -319,10 +358,10 @@ class KernelMatmulLinearOperator(LinearOperator):
         )
 
     def to_dense(self) -> Tensor:
-        x1, x2, params, start, end = self._get_args_for_native(self._batch_shape)
-        return _DenseOperator.apply(
-            x1, x2, params, start, end, self._native_dense, self._native_dense_bwd
-        )
+        call = self._get_args_for_native(self._batch_shape)
+        if _plain((call[2],)):
+            return self._native_dense(*call)
+        return _DenseOperator.apply(*call, self._native_dense, self._native_dense_bwd)
 
     def _expand_batch(self, batch_shape: Size | List[int]) -> "KernelMatmulLinearOperator":
         return KernelMatmulLinearOperator(
@@ -348,14 +387,15 @@ class KernelMatmulLinearOperator(LinearOperator):
         return super().type(dtype)
 
     def _bilinear_derivative(self, left_vecs: Tensor, right_vecs: Tensor) -> Tuple[Tensor | None, ...]:
-        batch_shape = torch.broadcast_shapes(
-            left_vecs.shape[:-2], right_vecs.shape[:-2], self._batch_shape
-        )
-        left_vecs = left_vecs.expand(*batch_shape, *left_vecs.shape[-2:])
-        right_vecs = right_vecs.expand(*batch_shape, *right_vecs.shape[-2:])
+        batch_shape = self._batch_shape
+        if not left_vecs.shape[:-2] == right_vecs.shape[:-2] == batch_shape:
+            batch_shape = torch.broadcast_shapes(
+                left_vecs.shape[:-2], right_vecs.shape[:-2], batch_shape
+            )
+        left_vecs = _widen(left_vecs, batch_shape, 2)
+        right_vecs = _widen(right_vecs, batch_shape, 2)
         x1, x2, params, start, end = self._get_args_for_native(batch_shape)
-        result = self._native_bilinear_derivative(x1, x2, left_vecs, right_vecs, params, start, end)
-        grad = result.reshape(*batch_shape, result.shape[-1])
+        grad = self._native_bilinear_derivative(x1, x2, left_vecs, right_vecs, params, start, end)
         # one entry per constructor tensor: x1, x2, params, start, end
         return None, None, grad, None, None
 
@@ -375,10 +415,10 @@ class KernelMatmulLinearOperator(LinearOperator):
                 batch.append(torch.arange(size, dtype=torch.int32, device=device).view(view).expand(*batch_shape, n))
             self._diagonal_indices = (row, tuple(batch))
         row, batch = self._diagonal_indices
-        x1, x2, params, start, end = self._get_args_for_native(self._batch_shape)
-        return _IndexOperator.apply(
-            x1, x2, params, start, end, self._native_index, self._native_index_bwd, row, row, *batch
-        )
+        call = self._get_args_for_native(self._batch_shape)
+        if _plain((call[2],)):
+            return self._native_index(*call, batch, row, row)
+        return _IndexOperator.apply(*call, self._native_index, self._native_index_bwd, row, row, *batch)
 
     def _get_indices(self, row_index: Tensor, col_index: Tensor, *batch_indices: Tensor) -> Tensor:
         x1, x2, params, start, end = self._get_args_for_native(self._batch_shape)

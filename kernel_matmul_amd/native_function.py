@@ -11,10 +11,18 @@ from __future__ import annotations
 import multiprocessing.pool
 from typing import Any
 
-from kernel_matmul_amd.compile import Defines, find_best, load_native
+from kernel_matmul_amd import configurations
+from kernel_matmul_amd.compile import Defines, find_best, load_native, module_environment
 from kernel_matmul_amd.configurations import Configuration
 from kernel_matmul_amd.util import format_dict
 
+_SHARED_CONFIGURATIONS = frozenset({
+    configurations.MatmulAutotuneConfiguration, configurations.MatmulBwdConfiguration,
+    configurations.BilinearDerivativeConfiguration, configurations.IndexConfiguration,
+    configurations.IndexBwdConfiguration, configurations.DenseConfiguration, configurations.DenseBwdConfiguration,
+})
+_SHARED_MODULES: dict = {}
+_SHARED_LIMIT = 256
 
 class NativeFunction:
     def __init__(
@@ -57,10 +65,27 @@ class NativeFunction:
     def __call__(self, *args: Any) -> Any:
         key = self.config.cache_key(args)
         if self._module is None or key != self._cache_key:
-            self._defines = self._select(args)
-            self._module = load_native(self.name, defines=self._defines)
+            self._defines, self._module = self._bind(key, args)
             self._cache_key = key
         return self._module.call(*args)
+
+    def _bind(self, key: str, args: tuple):
+        """Define set and module for arguments of this cache key.  Operators are made anew for every set of
+        hyper-parameters, so what the configurations of this package (whose one candidate follows from kernel
+        type and cache key) lead to is shared by all functions."""
+        if type(self.config) not in _SHARED_CONFIGURATIONS:
+            defines = self._select(args)
+            return defines, load_native(self.name, defines=defines)
+        shared_key = (self.name, type(self.config), self.config.kernel_type, key, module_environment())
+        shared = _SHARED_MODULES.get(shared_key)
+        if shared is None:
+            defines = self._select(args)
+            shared = (defines, load_native(self.name, defines=defines))
+            if len(_SHARED_MODULES) >= _SHARED_LIMIT:
+                _SHARED_MODULES.clear()
+            _SHARED_MODULES[shared_key] = shared
+        defines, module = shared
+        return dict(defines), module
 
     @property
     def defines(self) -> Defines | None:
