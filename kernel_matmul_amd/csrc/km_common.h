@@ -74,6 +74,22 @@ __device__ __forceinline__ long long xcd_item(unsigned block_id, long long per_x
     return (long long)xcd * per_xcd + slot;
 }
 
+// The batch item that place b of a group of `batches` consecutive items stands for.  An XCD's workgroups go to
+// its four shader engines in turn, in order, so with an even number of batch items in the same order in every
+// group an engine gets the same few of them; hyper-parameter sets differ in their work (tiles out of reach, row
+// blocks entry by entry), and the others wait for the engine with the heaviest.  The order is therefore rotated
+// from group to group (two batch items: every other group; an odd number changes places by itself).  The rotation
+// ends below the largest power of two, which is covered without a division.
+// Measured: spectral n = 1e6, k = 32, 8 sets of which one goes entry by entry 1016 -> 832 us a call; locally
+// periodic n = 1e5, k = 16, lengthscales of 0.5 to 2 at 10 / 40 points per unit 125 -> 118 / 329 -> 307.
+__device__ __forceinline__ unsigned spread_batch(unsigned b, unsigned group, unsigned batches) {
+    if ((batches & 1) != 0) {
+        return b;
+    }
+    b += (batches == 2 ? group >> 1 : group) & ((1u << (31 - __builtin_clz(batches))) - 1);
+    return b >= batches ? b - batches : b;
+}
+
 // ---------------------------------------------------------------------------------------
 // Kernel functions.  The user-facing hyper-parameters are turned into the constants the
 // inner loop wants once per wavefront (the reference does this with ~10 ATen launches per

@@ -873,7 +873,7 @@ __device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigne
     WaveView w;
     const unsigned batches = (unsigned)a.num_batches;
     const unsigned group = item / batches;
-    w.b = item - group * batches;
+    w.b = spread_batch(item - group * batches, group, batches);
     w.row_block = (int)group * KM_GROUP;
     const int row0 = w.row_block * KM_BLOCK_SIZE;
     const BatchOffsets o = batch_offsets(a, w.b);
@@ -960,9 +960,12 @@ __global__ void __launch_bounds__(64 * KM_GROUP, (GridShape<KT, G>::GE >= 4 ? 2 
         return;
     }
     const unsigned item = first + main_groups + (slot - main_groups) / KM_GROUP;
-    const unsigned row_block = item / (unsigned)a.num_batches * KM_GROUP + (slot - main_groups) % KM_GROUP;
+    const unsigned batches = (unsigned)a.num_batches;
+    const unsigned group = item / batches;
+    const unsigned row_block = group * KM_GROUP + (slot - main_groups) % KM_GROUP;
     if (item < (unsigned)a.total_items && (long long)row_block * KM_BLOCK_SIZE < a.m) {
-        grid_item<KT, G, KM_GROUP>(fresh_args(), lds, (long long)row_block * a.num_batches + item % (unsigned)a.num_batches, wave);
+        const unsigned b = spread_batch(item - group * batches, group, batches);
+        grid_item<KT, G, KM_GROUP>(fresh_args(), lds, (long long)row_block * batches + b, wave);
     }
 }
 

@@ -679,9 +679,15 @@ __device__ __forceinline__ void fwd_mfma_f16_body(const FwdArgs& a, float* lds, 
 template <int KT, int G, int R, bool PF>
 __global__ void __launch_bounds__(512) fwd_mfma_f16(const FwdArgs a) {
     extern __shared__ float lds[];
-    const ItemRef it = decode_item(a);
+    ItemRef it = decode_item(a);
     if (!it.valid) {
         return;
+    }
+    if constexpr (KT == KM_KERNEL_LOCALLY_PERIODIC) {
+        // (tiles out of reach are left out, so the batch items differ in their work)
+        const unsigned batches = (unsigned)a.num_batches;
+        const unsigned chunk = (unsigned)it.item / batches;
+        it.item = (long long)chunk * batches + spread_batch((unsigned)it.item - chunk * batches, chunk, batches);
     }
     int chunk_in_block;
     if constexpr (R == 8) {

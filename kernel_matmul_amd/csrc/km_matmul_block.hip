@@ -294,16 +294,18 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
             if (item >= ba.main_items) {
                 return;
             }
-            b = item % a.num_batches;
-            rb0 = (int)(item / a.num_batches) * NB;
+            const unsigned group = (unsigned)(item / a.num_batches);
+            b = spread_batch((unsigned)(item % a.num_batches), group, (unsigned)a.num_batches);
+            rb0 = (int)group * NB;
             nblk = min(NB, ba.main_row_blocks - rb0);
         } else {
             const long long item = (long long)xcd * ba.tail_per_xcd + (slot - ba.main_per_xcd);
             if (item >= ba.tail_items) {
                 return;
             }
-            b = item % a.num_batches;
-            rb0 = ba.main_row_blocks + (int)(item / a.num_batches);
+            const unsigned block = (unsigned)(item / a.num_batches);
+            b = spread_batch((unsigned)(item % a.num_batches), block, (unsigned)a.num_batches);
+            rb0 = ba.main_row_blocks + (int)block;
             nblk = 1;
         }
     }

@@ -379,7 +379,7 @@ __device__ __forceinline__ bool grad_item(const GradArgs& a, int rows_per_item, 
         }
         const unsigned batches = (unsigned)a.num_batches;
         const unsigned rest = item / batches;
-        g->b = item - rest * batches;
+        g->b = spread_batch(item - rest * batches, rest, batches);
         g->rest = rest;
         chunk = (int)(rest / (unsigned)a.col_splits);
         split = (int)(rest - (unsigned)chunk * (unsigned)a.col_splits);
