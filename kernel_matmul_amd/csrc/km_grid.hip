@@ -334,14 +334,19 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
     return true;
 }
 
-// The item entry by entry: each of the W wavefronts evaluates its rows, 32 at a time, against the
-// whole range.
+// The item entry by entry: each of the W wavefronts evaluates its rows, up to 64 at a time, against the
+// whole range.  Every time the range is tabulated and its rhs operand formed anew, which is most of the work where
+// few tiles are in reach; 128 rows at a time would not leave the registers for the other paths of one wavefront
+// (37 spilled with one spectral operand group).  Measured, 32 -> 64 rows at a time, n = 1e5, 8 sets, lengthscale 0.5:
+// spectral k = 16 at 1 / 3 / 5 points per unit 70.2 -> 59.8 / 72.4 -> 59.3 / 73.8 -> 63.2 us a call, k = 32 at 10
+// 155 -> 136; rbf k = 16 at 3 56.9 -> 47.3, k = 64 at 10 251 -> 221; two wavefronts, spectral n = 1e5, 2 sets, at 2
+// 30.4 -> 25.2.  The spills in the large kernels cost dense points 1 % (spectral k = 32 98.4 -> 99.9).
 template <int KT, int G, int W>
 __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
                                                int wave, const GridWindow& gw, const KernelConsts& kc) {
     constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
     constexpr int GE = G * PARTS;
-    constexpr int R = W == 8 ? 1 : 2;
+    constexpr int R = W == 1 ? 4 : 8 / W;
     constexpr int PIECES = 8 / (W * R);
     const int li = threadIdx.x & 15;
     GridWindow rows = gw;
@@ -389,13 +394,14 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         rows.reach = uniform(KM_GRID_REACH / kc.s);
         rows.col_lo = uniform(finite ? lo - rows.reach : -__builtin_inff());
         rows.col_hi = uniform(finite ? hi + rows.reach : __builtin_inff());
-        float xv[KM_GRID_CHUNK / 64];
+        constexpr int CHUNK = G == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
+        float xv[CHUNK / 64];
         if (w.range_start < w.range_end) {
             grid_load(w.x2, a.x2_s, w.range_start, 1, w.range_end, xv);
         }
         int shift[G];
         float4v acc[R][GE];
-        const bool fine = grid_columns<false, KT, G, R, 1>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
+        const bool fine = grid_columns<false, KT, G, R, 1, false, false, CHUNK>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
                                                            R, xv, shift, acc);
         const float sigma = w.params[KernelTraits<KT>::SIGMA * a.params_s];
         float down[GE];
