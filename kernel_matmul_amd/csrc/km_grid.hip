@@ -22,6 +22,7 @@
 #include "km_common.h"
 #include "km_fwd.h"
 #include "km_grid.h"
+#include "km_group_plan.h"
 #include "km_launch.h"
 
 namespace km {
@@ -482,15 +483,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
 // are resident, as many as the registers allow; with three row blocks for three or four wavefronts one
 // wavefront waits, or less is shared.
 // ---------------------------------------------------------------------------------------
-#define KM_GROUP 4
 #define KM_GROUP_CHUNK 128
-#define KM_GROUP_CORE_SHARED 256  /* columns of the core beyond which all wavefronts take a piece */
-// Lanes of the plan: the segments whose sums the row blocks add (the first cell in halves, two cells, the core,
-// whole or in halves, two cells, the last cell in halves), the wavefronts' pieces of a shared core, the row blocks.
-#define KM_GROUP_SEGMENTS 10
-#define KM_GROUP_CORE 4
-#define KM_GROUP_PIECE 10
-#define KM_GROUP_ROW 14
 
 // LDS in floats: a table for each wavefront, the cells' sums, and flags.
 template <int KT, int G>
@@ -554,33 +547,23 @@ __device__ __forceinline__ bool group_segments(const FwdArgs& a, const BatchOffs
     for (int i = 0; i < 2 * KM_GROUP; i++) {
         at[i] = lane_value(cut, i);
     }
-    auto half = [](int from, int to) { return ((to - from + 1) / 2 + 31) & ~31; };  // (in whole steps)
-    const int core = at[4] - at[3];
-    p->cooperative = core > KM_GROUP_CORE_SHARED;
-    const int quarter = (core / KM_GROUP + 31) & ~31;
-    const int bounds[KM_GROUP_SEGMENTS + 1] = {
-        at[0], max(at[1] - half(at[0], at[1]), at[0]), at[1], at[2],
-        at[3], p->cooperative ? at[4] : min(at[3] + half(at[3], at[4]), at[4]), at[4], at[5],
-        at[6], min(at[6] + half(at[6], at[7]), at[7]), at[7]};
-    p->start = bounds[0];
-    p->end = bounds[0];
+    const GroupCut c = group_cut(at);
+    p->cooperative = c.shared;
+    p->start = c.segment[0];
+    p->end = c.segment[0];
 #pragma unroll
     for (int i = 0; i < KM_GROUP_SEGMENTS; i++) {
-        p->start = lane == i ? bounds[i] : p->start;
-        p->end = lane == i ? bounds[i + 1] : p->end;
+        p->start = lane == i ? c.segment[i] : p->start;
+        p->end = lane == i ? c.segment[i + 1] : p->end;
     }
-    if (p->cooperative) {
+    if (c.shared) {
 #pragma unroll
         for (int i = 0; i < KM_GROUP; i++) {
-            p->start = lane == KM_GROUP_PIECE + i ? at[3] + i * quarter : p->start;
-            p->end = lane == KM_GROUP_PIECE + i ? (i == KM_GROUP - 1 ? at[4] : at[3] + (i + 1) * quarter) : p->end;
+            p->start = lane == KM_GROUP_PIECE + i ? c.piece[i] : p->start;
+            p->end = lane == KM_GROUP_PIECE + i ? c.piece[i + 1] : p->end;
         }
     }
-    p->rows = 0;
-#pragma unroll
-    for (int r = 0; r < KM_GROUP; r++) {
-        p->rows |= ends[r] <= p->start && p->end <= ends[KM_GROUP + r] && p->start < p->end ? 1 << r : 0;
-    }
+    p->rows = group_rows(ends, p->start, p->end);
     // (a gap between the ranges is a cell of none)
     p->end = p->rows != 0 ? p->end : p->start;
     return true;

@@ -95,3 +95,26 @@ def test_batch_dimensions_that_do_not_collapse(kt):
     rhs = _rhs(2, 1, n, 6).expand(2, 3, n, 6)
     start, end = (t.cpu().expand(2, 3, -1) for t in make_ranges(8.0, x[0, 0].to(DEVICE)))
     _group_check(kt, x, x, rhs, params, start, end)
+
+
+@pytest.mark.parametrize("core", [257, 259, 260, 272, 287, 288, 383, 384])
+@pytest.mark.parametrize("kt,k", [("spectral", 4), ("rbf", 20)])
+@pytest.mark.parametrize("ends", ["apart", "equal", "last"])
+def test_shared_columns_that_are_no_whole_steps(core, kt, k, ends):
+    """Four shares of the core in whole steps are more than it has; behind its end the ranges go on, stop
+    together, or stop at the last column."""
+    m, n = 512, 384 + core + (0 if ends == "last" else 384)
+    x1, x2 = _points(m, 40.0, core), _points(n, 40.0, core + 1)
+    row = torch.arange(4)
+    start = row * 128
+    end = 384 + core + (row * 128 if ends == "apart" else 0 * row)
+    _group_check(kt, x1, x2, _rhs(n, k), _params(kt, 3.0), start, end)
+
+
+@pytest.mark.parametrize("density,cutoff", [(22.0, 12.0), (25.0, 25.0), (10.0, 40.0)])
+def test_rectangular_pattern(density, cutoff):
+    """make_ranges for two sets of points: ranges that start and end anywhere."""
+    m, n = 2600, 2500
+    x1, x2 = _points(m, m / density, 1), _points(n, m / density, 2)
+    start, end = make_ranges(cutoff, x1.to(DEVICE), x2.to(DEVICE))
+    _group_check("spectral", x1, x2, _rhs(n, 4), _params("spectral", 2.0), start.cpu(), end.cpu())
