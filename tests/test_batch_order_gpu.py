@@ -36,12 +36,15 @@ def _close(result, expected, rhs, start, end):
 
 
 @pytest.mark.parametrize("batch", BATCHES)
-@pytest.mark.parametrize("kt,k,variant,rows", [
-    ("spectral", 5, "grid", 128), ("spectral", 20, "grid", 128), ("rbf", 3, "grid", 128),
-    ("locally_periodic", 5, "block", None), ("locally_periodic", 5, "mfma_f16_direct", 128),
-    ("locally_periodic", 20, "mfma_f16_direct", 32),
+@pytest.mark.parametrize("kt,k,variant,rows,tail", [
+    ("spectral", 5, "grid", 128, 0), ("spectral", 20, "grid", 128, None), ("rbf", 3, "grid", 128, 0),
+    ("spectral", 5, "grid", 128, None), ("rbf", 3, "grid", 128, None), ("rbf", 3, "grid", 128, 4),
+    ("locally_periodic", 5, "block", None, None), ("locally_periodic", 5, "mfma_f16_direct", 128, None),
+    ("locally_periodic", 20, "mfma_f16_direct", 32, None),
 ])
-def test_forward(kt, k, variant, rows, batch):
+def test_forward(kt, k, variant, rows, tail, batch):
+    """tail (grid): how many row blocks of each XCD get a workgroup each; without the option all of a launch as
+    small as this."""
     n = 2000  # sixteen row blocks: some XCDs get groups of their own, others share one
     x, rhs, params, start, end = (t.to(DEVICE) for t in _inputs(kt, batch, n, k))
 
@@ -50,6 +53,8 @@ def test_forward(kt, k, variant, rows, batch):
         defines["MATMUL_VARIANT"] = variant
         if rows:
             defines["MATMUL_ROWS_PER_WAVE"] = rows
+        if tail is not None:
+            defines["MATMUL_GROUP_TAIL"] = tail
         return load_native("matmul", defines).call(*args)
 
     shared = [t.expand(batch, *t.shape) for t in (x, start, end)]
