@@ -444,9 +444,10 @@ __device__ __forceinline__ void look_at_steps(const GridVectors& a, const WaveVi
 }
 
 // The running power-of-two scale of an rhs column, lowered when a magnitude m of its values would exceed 2^15 (NaN
-// and infinities hand themselves on).
+// and infinities hand themselves on).  first: no step has added to the sums yet (a scale that is still the largest
+// does not say so: steps of values below 2^-85 leave it as it is).
 template <int G, int PARTS, int MT>
-__device__ __forceinline__ void lower_scale(int g, float m, bool used, int (&shift)[G], float (&scale)[G],
+__device__ __forceinline__ void lower_scale(int g, float m, bool used, bool first, int (&shift)[G], float (&scale)[G],
                                             float4v (&acc)[MT][G * PARTS]) {
     const bool grow = used && !(m * scale[g] < 32768.0f);
     if (__any(grow)) {
@@ -456,7 +457,7 @@ __device__ __forceinline__ void lower_scale(int g, float m, bool used, int (&shi
         } else if (grow) {
             const int e = __builtin_amdgcn_frexp_expf(m);
             const int new_shift = min(14 - e, 100);
-            if (__any(shift[g] != 100)) {  // (else these are its first values: the sums are zero)
+            if (!first) {
                 const float factor = __builtin_ldexpf(1.0f, new_shift - shift[g]);
 #pragma unroll
                 for (int mt = 0; mt < MT; mt++) {
@@ -627,6 +628,7 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
     constexpr bool EACH_CHUNK = G == 1;
     BeyondSteps beyond = {0, 64, 0};
     int chunk = 0;
+    bool first_step = true;
     constexpr int STEPS = CH / 32;  // of a chunk
     static_assert(64 % STEPS == 0, "whole chunks' bits");
     // (unsigned: the next first column may lie past the largest int)
@@ -683,8 +685,9 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
             }
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                lower_scale<G, PARTS, MT>(g, column_maximum(magnitude(raw[g])), rl.used[g], shift, scale, acc);
+                lower_scale<G, PARTS, MT>(g, column_maximum(magnitude(raw[g])), rl.used[g], first_step, shift, scale, acc);
             }
+            first_step = false;
             grid_step<GRID, G, PARTS, MT, EXACT, CH, GRID>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, scale, acc);
         } while (need != 0);
         // All reads of the table are done before the next chunk overwrites it.

@@ -376,3 +376,18 @@ def test_ranges_at_the_largest_sizes(kt, k, rows):
     bound = 3e-6 * width * envelope @ np.abs(rhs.double().numpy())
     bound[128:] = 0.0
     assert np.all(np.abs(out - expected) <= bound)
+
+
+@pytest.mark.parametrize("kt,k", [("spectral", 2), ("spectral", 20), ("spectral", 40), ("rbf", 3), ("rbf", 20), ("rbf", 50)])
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("lengthscale", [1.0, 0.03])
+@pytest.mark.parametrize("small", [1e-27, 2.5e-26, 1e-20])
+def test_rhs_that_grows_along_the_columns(kt, k, rows, lengthscale, small):
+    """Tiny values in front of ordinary ones (and behind them), whose sums follow the column's scale down."""
+    n = 1400
+    x = _points(n, n / 10.0, 59)
+    rhs = torch.randn(n, k, generator=torch.Generator().manual_seed(60))
+    rhs[:500] *= small
+    rhs[900:] *= small
+    start, end = _ranges(n, n, 900)
+    _check(kt, x, x, rhs, _params(kt, lengthscale), start, end, rows=rows)

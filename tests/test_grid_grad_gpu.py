@@ -259,3 +259,17 @@ def test_ranges_at_the_largest_sizes(kt, c, width):
     size = np.abs(left[:128].double().numpy()) @ np.abs(right.double().numpy().T)
     # (distances up to two lengthscales: the derivatives' factors are below 15)
     assert np.all(np.abs(result - expected) <= 4e-6 * 15.0 * width * size.sum()), (result, expected)
+
+
+@pytest.mark.parametrize("kt,c", [("spectral", 4), ("spectral", 12), ("rbf", 6), ("rbf", 20)])
+@pytest.mark.parametrize("small", [1e-27, 2.5e-26, 1e-20])
+def test_vectors_that_grow_along_the_columns(kt, c, small):
+    """Tiny values in front of ordinary ones (and behind them), whose sums follow the column's scale down."""
+    n = 1200
+    x = _points(n, n / 10.0, 61)
+    right = _vectors(n, c, 62)
+    right[:500] *= small
+    right[800:] *= small
+    left = _vectors(n, c, 63)
+    start, end = _ranges(n, n, 700)
+    _check(kt, x, x, left, right, _params(kt, 1.0), start, end)
