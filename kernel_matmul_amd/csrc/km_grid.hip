@@ -606,7 +606,11 @@ __device__ __forceinline__ void group_windows(const FwdArgs& a, const WaveView& 
     // (a core in pieces is in nobody's accumulators as a whole)
     const float limit = p.cooperative && lane == KM_GROUP_CORE ? (float)P::QUADS : (float)P::MAX_QUADS;
     const bool bad = !(fabsf(y0) + fabsf(y1) < 1e30f) || !(count <= limit) || (count > 0.0f && !(fabsf(lo) < 1000.0f));
-    p.ok = gw.h > 1e-30f && gw.h < 1e30f && !__any(used && bad);
+    // (the pieces of a core add to the core's window, which its first and last coordinate make)
+    const float core_first = lane_value(p.first, KM_GROUP_CORE), core_last = lane_value(p.last, KM_GROUP_CORE);
+    const bool beyond = p.cooperative && lane >= KM_GROUP_PIECE && lane < KM_GROUP_PIECE + KM_GROUP &&
+                        (p.first < core_first || p.last > core_last);
+    p.ok = gw.h > 1e-30f && gw.h < 1e30f && !__any(used && (bad || beyond));
     const bool reached = p.ok && used && count > 0.0f;
     p.quad = reached ? (int)lo : 0;
     p.quads = reached ? (int)count : 0;

@@ -118,3 +118,15 @@ def test_rectangular_pattern(density, cutoff):
     x1, x2 = _points(m, m / density, 1), _points(n, m / density, 2)
     start, end = make_ranges(cutoff, x1.to(DEVICE), x2.to(DEVICE))
     _group_check("spectral", x1, x2, _rhs(n, 4), _params("spectral", 2.0), start.cpu(), end.cpu())
+
+
+@pytest.mark.parametrize("border", [128, 256, 300, 384])
+@pytest.mark.parametrize("kt,k", [("spectral", 4), ("rbf", 20)])
+def test_ascending_runs_out_of_order(kt, k, border):
+    """Columns in two ascending runs, the upper one first: the pieces of a shared core reach further than its
+    first and last coordinate say."""
+    n = 512
+    x = _points(n, 10.0, border)
+    order = torch.cat([torch.arange(border, n), torch.arange(border)])
+    start, end = torch.zeros(4), torch.full((4,), float(n))
+    _group_check(kt, x, x[order], _rhs(n, k), _params(kt, 0.8), start, end)
