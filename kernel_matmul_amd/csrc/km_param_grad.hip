@@ -477,7 +477,8 @@ __device__ __forceinline__ bool grad_skips(const GradArgs& a, const GradItem& g,
     float covered = 0.0f;
 #pragma unroll
     for (int i = 0; i < 3; i++) {
-        const float x = g.x1[(long long)(i == 0 ? g.row0 : (i == 1 ? (g.row0 + last) / 2 : last)) * a.x1_s];
+        const int row = g.row0 + (last - g.row0) * i / 2;  // (not half the sum of both: it may lie past the largest int)
+        const float x = g.x1[(long long)row * a.x1_s];
         covered += fmaxf(fminf(hi, x + reach) - fmaxf(lo, x - reach), 0.0f);
     }
     return __builtin_amdgcn_readfirstlane(covered < 0.55f * 3.0f * (hi - lo)) != 0;

@@ -94,3 +94,27 @@ def test_ranges(ranges):
     args = _inputs("spectral", 8, 0.5)
     args[5][:], args[6][:] = ranges
     _check("spectral", args)
+
+
+@pytest.mark.parametrize("kt,c", [("locally_periodic", 8), ("rbf", 12), ("spectral", 7)])
+@pytest.mark.parametrize("m", [2**30 + 300, 2**31 - 1 - 128])
+def test_rows_at_the_largest_sizes(kt, c, m):
+    """The gradient of the last rows of as many as the entry point takes (all others' ranges are empty) is that of
+    these rows alone."""
+    n, tail = 1000, m - (m - 1) // 128 * 128 + 256  # three row blocks
+    blocks = (m + 127) // 128
+    g = torch.Generator().manual_seed(5)
+    x1 = torch.full((m,), -1e3, device=DEVICE)
+    x1[m - tail:] = torch.sort(torch.rand(tail, generator=g) * 500.0)[0].to(DEVICE)
+    x2 = torch.sort(torch.rand(n, generator=g) * 500.0)[0].to(DEVICE)
+    left = torch.randn(1, c, generator=g).to(DEVICE).expand(m, c)
+    right = torch.randn(n, c, generator=g).to(DEVICE)
+    params = torch.tensor({"rbf": [0.8, 1.2], "spectral": [0.8, 0.3, 1.2], "locally_periodic": [0.8, 0.9, 1.1, 0.9]}[kt], device=DEVICE)
+    start = torch.zeros(blocks, dtype=torch.int32, device=DEVICE)
+    end = torch.zeros(blocks, dtype=torch.int32, device=DEVICE)
+    end[-3:] = n
+    op = load_native("bilinear_derivative", BilinearDerivativeConfiguration(kt).make_config((x1, x2, left, right, params, start, end)))
+    result = op.call(x1, x2, left, right, params, start, end)
+    expected = op.call(x1[m - tail:], x2, left[m - tail:], right, params, start[-3:], end[-3:])
+    # (shorter shares of columns for fewer rows: other orders of fp32 sums, of which few terms are in reach)
+    torch.testing.assert_close(result, expected, rtol=1e-4, atol=1e-4 * float(expected.abs().max()))
