@@ -68,9 +68,11 @@ struct BlockRows {
 __device__ __forceinline__ BlockRows block_rows(const float* __restrict__ x1, long long x1_s, int row0, int m) {
     const int lane = threadIdx.x & 63;
     BlockRows r;
-    r.xa = x1[(long long)min(row0 + lane, m - 1) * x1_s];
-    r.xb = x1[(long long)min(row0 + 64 + lane, m - 1) * x1_s];
-    r.middle = x1[(long long)min(row0 + 64, m - 1) * x1_s];
+    // (unsigned: the rows of a group's last wavefronts may lie past the largest int)
+    const unsigned row = (unsigned)row0, last = (unsigned)m - 1;
+    r.xa = x1[(long long)min(row + lane, last) * x1_s];
+    r.xb = x1[(long long)min(row + 64 + lane, last) * x1_s];
+    r.middle = x1[(long long)min(row + 64, last) * x1_s];
     return r;
 }
 

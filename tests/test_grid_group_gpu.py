@@ -6,6 +6,8 @@ Tolerance as in test_grid_form_gpu."""
 import pytest
 import torch
 
+from kernel_matmul_amd.compile import load_native
+from kernel_matmul_amd.configurations import MatmulSingleConfiguration
 from kernel_matmul_amd.ranges import make_ranges
 from tests.test_grid_form_gpu import DEVICE, _check, _params, _points
 
@@ -130,3 +132,30 @@ def test_ascending_runs_out_of_order(kt, k, border):
     order = torch.cat([torch.arange(border, n), torch.arange(border)])
     start, end = torch.zeros(4), torch.full((4,), float(n))
     _group_check(kt, x, x[order], _rhs(n, k), _params(kt, 0.8), start, end)
+
+
+@pytest.mark.parametrize("kt", ["spectral", "rbf"])
+@pytest.mark.parametrize("m", [2**31 - 512 + 5, 2**31 - 1 - 128])
+@pytest.mark.parametrize("tail", [0, 4])
+def test_rows_at_the_largest_sizes(kt, m, tail):
+    """The last rows of as many as the entry point takes (all others' ranges are empty) are those of these rows
+    alone: the last group's wavefronts without a row block stay within the rows."""
+    n, last = 1000, m - (m - 1) // 512 * 512
+    x1 = torch.full((m,), -1e3, device=DEVICE)
+    x1[m - last:] = _points(last, 50.0, 1).to(DEVICE)
+    x2, rhs = _points(n, 50.0, 2).to(DEVICE), _rhs(n, 1).to(DEVICE)
+    params = _params(kt, 1.1).to(DEVICE)
+    blocks, own = (m + 127) // 128, (last + 127) // 128
+    start = torch.zeros(blocks, dtype=torch.int32, device=DEVICE)
+    end = torch.zeros(blocks, dtype=torch.int32, device=DEVICE)
+    end[blocks - own:] = n
+
+    def call(*args):
+        defines = MatmulSingleConfiguration(kt).make_config(args)
+        defines["MATMUL_VARIANT"], defines["MATMUL_ROWS_PER_WAVE"], defines["MATMUL_GROUP_TAIL"] = "grid", 128, tail
+        return load_native("matmul", defines).call(*args)
+
+    result = call(x1, x2, rhs, params, start, end)
+    alone = call(x1[m - last:], x2, rhs, params, start[blocks - own:], end[blocks - own:])
+    assert torch.equal(result[m - last:], alone)
+    assert not result[:m - last].any()
