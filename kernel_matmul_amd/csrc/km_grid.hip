@@ -150,7 +150,9 @@ __device__ __forceinline__ void grid_rows(const FwdArgs& a, const WaveView& w, c
             }
         }
         m = column_max(m);
-        const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 100);
+        // (126: the largest power of two that fp32 has both ways.  Sums of tiny values come times 2^-16 through LDS; a
+        // limit below 116 would lose bits of their halves that the contraction had.)
+        const int e = min(14 - __builtin_amdgcn_frexp_expf(m), 126);
         const float up = __builtin_ldexpf(1.0f, e);
         down[g] = shift[g % G] == KM_GRID_NOT_FINITE
                       ? __builtin_nanf("")

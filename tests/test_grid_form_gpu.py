@@ -38,14 +38,14 @@ def _run(kt, x1, x2, rhs, params, start, end, rows=None, tail=None):
     return out.cpu().double().numpy()
 
 
-def _check(kt, x1, x2, rhs, params, start, end, **launch):
+def _check(kt, x1, x2, rhs, params, start, end, floor=1e-30, **launch):
     out = _run(kt, x1, x2, rhs, params, start, end, **launch)
     a = [t.numpy() for t in (x1, x2, rhs, params, start, end)]
     expected = oracle.matmul(kt, a[0], a[1], a[2], a[3], a[4], a[5])
     envelope = np.abs(oracle.dense("rbf", a[0], a[1], a[3][..., [0, -1]], a[4], a[5]))
     mask = oracle.range_mask(a[4], a[5], x1.shape[-1], x2.shape[-1]).astype(np.float64)
     size = np.abs(a[2].astype(np.float64))
-    tol = 3e-6 * (envelope @ size) + 2.0 ** -36 * np.abs(a[3][..., -1, None, None]) * (mask @ size) + 1e-30
+    tol = 3e-6 * (envelope @ size) + 2.0 ** -36 * np.abs(a[3][..., -1, None, None]) * (mask @ size) + floor
     err = np.abs(out - expected)
     assert np.all(err <= tol), float((err / tol).max())
 
@@ -328,6 +328,19 @@ def test_rhs_scales(kt, rows, scale, sigma):
         params[1] = 0.01
     start, end = _ranges(n, n, 700)
     _check(kt, x, x, rhs, params, start, end, rows=rows)
+
+
+@pytest.mark.parametrize("kt,k", [("spectral", 3), ("spectral", 20), ("rbf", 3), ("rbf", 20), ("rbf", 40)])
+@pytest.mark.parametrize("rows", [16, 32, 64, 128])
+@pytest.mark.parametrize("scale", [1e-26, 1e-28, 1e-30])
+def test_tiny_rhs(kt, k, rows, scale):
+    """Full precision down to where the scale of rhs ends (2^100, of two fp16 halves of which the lower one takes
+    steps of 2^-24), although the wavefronts' sums are exchanged at another scale."""
+    n = 1400
+    x = _points(n, n / 20.0, 63)
+    rhs = torch.randn(n, k, generator=torch.Generator().manual_seed(64)) * scale
+    start, end = _ranges(n, n, 700)
+    _check(kt, x, x, rhs, _params(kt, 1.2), start, end, floor=0.0, rows=rows)
 
 
 @pytest.mark.parametrize("kt", ["spectral", "rbf"])
