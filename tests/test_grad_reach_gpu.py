@@ -12,8 +12,10 @@ pytestmark = pytest.mark.gpu
 
 DEVICE = torch.device("cuda:0")
 N = 1500
-# (twelve row blocks each: enough that rbf and spectral vectors of this width go pair by pair)
-BATCH = (2, 8)
+# (twelve row blocks each: enough that rbf and spectral vectors of this width go pair by pair, and that a wavefront's
+# share of a row block's columns is wide enough for the look at what is out of reach)
+BATCH = (8, 16)
+ITEMS = BATCH[0] * BATCH[1]
 
 
 def _inputs(kt, c, lengthscale, density=1.0, periodic=0.8, seed=0):
@@ -22,7 +24,7 @@ def _inputs(kt, c, lengthscale, density=1.0, periodic=0.8, seed=0):
     x2 = torch.sort(torch.rand(N, generator=g) * (N / density))[0]
     left = torch.randn(*BATCH, N, c, generator=g)
     right = torch.randn(*BATCH, N, c, generator=g)
-    ls = lengthscale * torch.linspace(1.0, 2.0, 16).reshape(BATCH)
+    ls = lengthscale * torch.linspace(1.0, 2.0, ITEMS).reshape(BATCH)
     rest = {"rbf": [1.2], "spectral": [0.3, 1.2], "locally_periodic": [periodic, 1.1, 0.9]}[kt]
     params = torch.stack([ls, *(torch.full(BATCH, v) for v in rest)], dim=-1)
     mid = torch.arange(12) * 128 + 64
@@ -32,13 +34,13 @@ def _inputs(kt, c, lengthscale, density=1.0, periodic=0.8, seed=0):
 
 def _call(kt, args):
     op = load_native("bilinear_derivative", BilinearDerivativeConfiguration(kt).make_config(args))
-    return op.call(*args).cpu().reshape(16, -1)
+    return op.call(*args).cpu().reshape(ITEMS, -1)
 
 
 def _check(kt, args):
     x1, x2, left, right, params, start, end = (t.to(DEVICE) for t in args)
     shared = [t.expand(*BATCH, *t.shape) for t in (x1, x2, start, end)]
-    flat = [t.expand(16, *t.shape) for t in (x1, x2, start, end)]
+    flat = [t.expand(ITEMS, *t.shape) for t in (x1, x2, start, end)]
     result = _call(kt, (flat[0], flat[1], left.flatten(0, 1), right.flatten(0, 1), params.flatten(0, 1), flat[2], flat[3]))
     # (a batch dimension stored the other way round)
     turned = params.transpose(0, 1).contiguous().transpose(0, 1)
