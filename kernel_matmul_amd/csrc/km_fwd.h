@@ -71,13 +71,23 @@ void fill_fwd_args(const MatmulProblem& p, FwdArgs* args);
 // base-2 exponential) so that its hi and lo halves stay inside the fp16 exponent range.
 #define KM_F16_KSCALE_LOG2 14
 
+// (On the bits without the sign: a vote over v < inf, or over exponent bits that are not all ones, which it
+// takes for the same, comes out of this compiler as a vote over v != inf, true for a NaN.)
+__device__ __forceinline__ bool is_finite(float v) {
+    return __float_as_uint(v) << 1 < 0xff000000u;
+}
+
 // Scaled distance from which a locally periodic kernel's entries are zero in the split-fp16 kernels that evaluate them
 // one by one: 2^(KM_F16_KSCALE_LOG2 - u^2) is then below half of fp16's smallest value (2^-25, with 4 % to spare for
 // roundings), the periodic factor is at most one (a negative lengthscale of it raises it to 2^-cl, cl < 0), and both
 // halves of the entry round to zero.  Tiles of 16 rows by 32 columns of which every entry is zero are left out: the
 // results are the same.
 #define KM_F16_REACH_SQUARED 39.0625f
+// Everything is within reach of a period or second lengthscale of zero or NaN, which make entries NaN.
 __device__ __forceinline__ float periodic_reach(const KernelConsts& kc) {
+    if (!is_finite(kc.f) || !is_finite(kc.cl)) {
+        return __builtin_inff();
+    }
     return __builtin_sqrtf(KM_F16_REACH_SQUARED + fmaxf(0.0f, -kc.cl)) / kc.s;
 }
 
@@ -86,12 +96,6 @@ __device__ __forceinline__ float periodic_reach(const KernelConsts& kc) {
 __device__ __forceinline__ bool periodic_skip(float middle, float first, float last, float reach) {
     const float inside = fminf(last, middle + reach) - fmaxf(first, middle - reach);
     return inside < 0.9f * (last - first);
-}
-
-// (On the bits without the sign: a vote over v < inf, or over exponent bits that are not all ones, which it
-// takes for the same, comes out of this compiler as a vote over v != inf, true for a NaN.)
-__device__ __forceinline__ bool is_finite(float v) {
-    return __float_as_uint(v) << 1 < 0xff000000u;
 }
 
 // Phase f * (x - c) in revolutions, reduced to [-0.5, 0.5].  x - c is taken as an unevaluated

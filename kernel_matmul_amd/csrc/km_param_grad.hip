@@ -73,12 +73,12 @@ struct GradArgs {
 // Distance from which every entry is zero.
 template <int KT>
 __device__ __forceinline__ float grad_reach(const KernelConsts& kc) {
-    if (KT != KM_KERNEL_RBF && !is_finite(kc.f)) {
-        return __builtin_inff();  // (every entry is NaN)
+    if (KT != KM_KERNEL_RBF && !(is_finite(kc.f) && is_finite(kc.cl))) {
+        return __builtin_inff();  // (sums are NaN)
     }
     if (KT == KM_KERNEL_LOCALLY_PERIODIC) {
-        // (a negative second lengthscale raises the entries by up to 2^-cl; NaN stays NaN: everything is in reach)
-        return __builtin_sqrtf(__builtin_fmaf(KM_GRAD_REACH, KM_GRAD_REACH, __builtin_elementwise_maximum(0.0f, -kc.cl))) / kc.s;
+        // (a negative second lengthscale raises the entries by up to 2^-cl)
+        return __builtin_sqrtf(__builtin_fmaf(KM_GRAD_REACH, KM_GRAD_REACH, fmaxf(0.0f, -kc.cl))) / kc.s;
     }
     return KM_GRAD_REACH / kc.s;
 }

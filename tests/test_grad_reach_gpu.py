@@ -120,3 +120,19 @@ def test_rows_at_the_largest_sizes(kt, c, m):
     expected = op.call(x1[m - tail:], x2, left[m - tail:], right, params, start[-3:], end[-3:])
     # (shorter shares of columns for fewer rows: other orders of fp32 sums, of which few terms are in reach)
     torch.testing.assert_close(result, expected, rtol=1e-4, atol=1e-4 * float(expected.abs().max()))
+
+
+@pytest.mark.parametrize("what,value", [(1, 0.0), (1, float("nan")), (2, 0.0), (2, float("nan"))])
+@pytest.mark.parametrize("c", [8, 16])
+def test_parameters_that_make_entries_nan(c, what, value):
+    """Where no column is in reach of a row as well (a second lengthscale of zero: entries a whole number of
+    periods apart, here every fourth)."""
+    args = _inputs("locally_periodic", c, 0.4)
+    args[0] = torch.arange(N) * 0.25 + 3000.0
+    args[1] = torch.arange(N) * 0.25
+    args[4][1, 2, 2] = 1.0
+    args[4][1, 2, what] = value
+    result = _check("locally_periodic", args)
+    item = BATCH[1] + 2
+    assert bool(result[item].isnan().all())
+    assert bool(result[:item].isfinite().all())

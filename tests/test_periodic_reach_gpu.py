@@ -76,3 +76,18 @@ def test_unsorted_coordinates():
     args[0] = args[0][torch.randperm(N, generator=g)]
     args[1] = args[1][torch.randperm(N, generator=g)]
     _check(args, 5)
+
+
+@pytest.mark.parametrize("what,value", [(0, float("nan")), (1, 0.0), (1, float("nan")), (2, 0.0), (2, float("nan"))])
+@pytest.mark.parametrize("k", [1, 20])
+@pytest.mark.parametrize("away", [0.0, 1000.0])
+def test_parameters_that_make_entries_nan(what, value, k, away):
+    """Where no column is in reach of a row as well (a second lengthscale of zero: entries a whole number of
+    periods apart, here every fourth)."""
+    args = _inputs(k, 0.5)
+    args[3][2] = 1.0
+    args[0] = torch.arange(N) * 0.25 + away
+    args[1] = torch.arange(N) * 0.25
+    args[3][what] = value
+    _check(args, k)
+    assert bool(_call(args, "mfma_f16_direct", 128).isnan().all())
