@@ -660,6 +660,9 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
         if (j != 0) {
             grid_rhs<G>(a, rhs, first + 32 * j * W, w.range_end, kk, rl, next);
         }
+        // (the first step is no code of its own: that was a fifth more instructions and 5 % of the time of rbf n = 1e5,
+        // k = 64, 2 sets entry by entry)
+#pragma nounroll
         do {
             float raw[G][8];
 #pragma unroll
