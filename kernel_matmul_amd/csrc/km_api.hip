@@ -111,7 +111,7 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     const int k_chunk = p.k <= 16 ? 16 : (p.k <= 32 ? 32 : 64);
     const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     const long long per_launch = row_blocks * p.num_batches;
-    const long long items = per_launch * ((p.k + k_chunk - 1) / k_chunk);
+    long long items = per_launch * ((p.k + k_chunk - 1) / k_chunk);
     if (automatic && items < 48) {
         return false;
     }
@@ -120,7 +120,11 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     plan->row_groups = 8;
     plan->tail_balance = 0;
     plan->group_tail_halves = 0;
-    const int operands = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1);
+    int operands = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1);
+    if (operands > 64) {  // (64 spectral columns: half of them a workgroup)
+        operands /= 2;
+        items *= 2;
+    }
     const bool two_resident = operands > 32;
     if (opt && opt->rows_per_wave != 0) {
         plan->col_splits = KM_BLOCK_SIZE / opt->rows_per_wave;
@@ -602,18 +606,20 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
     const char* kt = kernels[kernel_type];
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     const int G = plan.k_chunk / 16;
+    const char* const halves = kernel_type == KM_KERNEL_SPECTRAL && G == 4 ? ", half of 64 columns each" : "";
     switch (plan.variant) {
         case KM_VARIANT_GRID:
             if (plan.group_tail > 0) {
                 snprintf(text, text_bytes,
                          "km::fwd_grid_grouped<%s, G=%d>: grid form, 4 row blocks per workgroup of 4 wavefronts, "
-                         "the last %lld row blocks of each XCD by a workgroup each",
-                         kt, G, plan.group_tail);
+                         "the last %lld row blocks of each XCD by a workgroup each%s",
+                         kt, G, plan.group_tail, halves);
             } else if (plan.col_splits == 1) {
-                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=1>: grid form, 4 row blocks per workgroup of 4 wavefronts", kt, G);
+                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=1>: grid form, 4 row blocks per workgroup of 4 wavefronts%s", kt, G,
+                         halves);
             } else {
-                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefronts per row block", kt, G,
-                         plan.col_splits, plan.col_splits);
+                snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefronts per row block%s", kt, G,
+                         plan.col_splits, plan.col_splits, halves);
             }
             break;
         case KM_VARIANT_VALU:

@@ -229,15 +229,15 @@ __device__ __forceinline__ void grid_rows(const FwdArgs& a, const WaveView& w, c
     }
 }
 
-// rhs column groups (of 16) that one pass takes, the grid form's largest window, and the columns tabulated at a
-// time.
+// Operand groups (of 16 columns) of G groups of rhs columns, the grid form's largest window, and the columns tabulated
+// at a time.
 template <int KT, int G>
 struct GridShape {
     static constexpr int PARTS = KT == KM_KERNEL_SPECTRAL ? 2 : 1;
-    static constexpr int GP = G * PARTS > 4 ? 4 / PARTS : G;
-    static constexpr int GE = GP * PARTS;
+    static constexpr int GE = G * PARTS;
+    static_assert(GE <= 4, "what the registers hold");
     static constexpr int MT = GE >= 4 ? 4 : 5;
-    static constexpr int CHUNK = GP == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
+    static constexpr int CHUNK = G == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
 };
 
 // LDS of one item in floats: the wavefronts' tables, overlaid by the exchange of the sums, and the
@@ -425,9 +425,10 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
     }
 }
 
-// One item by W wavefronts (this one is number `wave`): the grid form, or entry by entry.
+// One item by W wavefronts (this one is number `wave`) for rhs columns [kbase, kbase + 16 G): the grid form, or
+// entry by entry.
 template <int KT, int G, int W>
-__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int wave) {
+__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int kbase, int wave) {
     using S = GridShape<KT, G>;
     int unused;
     const WaveView w = wave_view<true>(a, item, 1, &unused);
@@ -444,19 +445,9 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     }
     const GridWindow gw = grid_window<S::MT>(rows, kc);
     // (the same in every lane, and said so: the barriers inside depend on it)
-    bool grid = __builtin_amdgcn_readfirstlane(gw.ok && w.range_end - w.range_start >= KM_GRID_MIN_WIDTH) != 0;
-#pragma unroll 1
-    for (int pass = 0; pass < G / S::GP; pass++) {
-        const int kbase = (blockIdx.y * G + pass * S::GP) * 16;
-        if (kbase < a.k) {
-            if (pass > 0 && 32 * wave < w.range_end - w.range_start) {
-                grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
-            }
-            grid = grid && grid_forward<KT, S::GP, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv);
-            if (!grid) {
-                grid_entrywise<KT, S::GP, W>(a, lds, w, row0, kbase, wave, gw, kc);
-            }
-        }
+    const bool grid = __builtin_amdgcn_readfirstlane(gw.ok && w.range_end - w.range_start >= KM_GRID_MIN_WIDTH) != 0;
+    if (!grid || !grid_forward<KT, G, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv)) {
+        grid_entrywise<KT, G, W>(a, lds, w, row0, kbase, wave, gw, kc);
     }
 }
 
@@ -499,7 +490,7 @@ struct GroupShape {
     static constexpr int FLAGS = SUMS + QUADS * QUAD;
     static constexpr int FLOATS = FLAGS + 64;
     static_assert(FLOATS >= grid_lds_floats<S::GE, S::MT, KM_GROUP>() && FLOATS >= KM_GROUP * KM_GRID_TABLE_FLOATS, "grid_item's LDS");
-    static_assert(KM_GROUP + (KM_GROUP_SEGMENTS + KM_GROUP) * S::GP <= 64, "flags");
+    static_assert(KM_GROUP + (KM_GROUP_SEGMENTS + KM_GROUP) * G <= 64, "flags");
 };
 
 __device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
@@ -655,31 +646,31 @@ __device__ __forceinline__ GridWindow group_window(const GridWindow& common, con
 template <int KT, int G>
 __device__ __forceinline__ bool group_columns(const FwdArgs& a, const WaveView& w, const GroupPlan& p, int lane_of, int kbase,
                                               const GridWindow& common, const KernelConsts& kc, float* tab, float* sums,
-                                              float (&xv)[KM_GROUP_CHUNK / 64], unsigned (&bad)[GridShape<KT, G>::GP]) {
+                                              float (&xv)[KM_GROUP_CHUNK / 64], unsigned (&bad)[G]) {
     using S = GridShape<KT, G>;
-    constexpr int GP = S::GP, GE = S::GE, MT = S::MT;
+    constexpr int GE = S::GE, MT = S::MT;
     const int lane = threadIdx.x & 63;
     const int kk = lane >> 4;
     WaveView seg = w;
     seg.range_start = lane_value(p.start, lane_of);
     seg.range_end = lane_value(p.end, lane_of);
     const GridWindow gw = group_window(common, p, lane_of);
-    int shift[GP];
+    int shift[G];
     float4v acc[MT][GE];
-    const bool fine = grid_columns<true, KT, GP, MT, 1, false, false, KM_GROUP_CHUNK>(vectors(a), tab, seg, kbase, 0, gw, kc, nullptr,
+    const bool fine = grid_columns<true, KT, G, MT, 1, false, false, KM_GROUP_CHUNK>(vectors(a), tab, seg, kbase, 0, gw, kc, nullptr,
                                                                                      gw.tiles, xv, shift, acc);
     const int quads = lane_value(p.quads, lane_of);
     float4v* out = (float4v*)(sums + lane_value(p.place, lane_of) * GroupShape<KT, G>::QUAD) + (lane & 15);
 #pragma unroll
-    for (int g = 0; g < GP; g++) {
+    for (int g = 0; g < G; g++) {
         bad[g] = (unsigned)__ballot(shift[g] == KM_GRID_NOT_FINITE) & 0xffff;
         const float up = __builtin_ldexpf(1.0f, -shift[g] - KM_GRID_KS1 - KM_GRID_EXCHANGE);
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             if (4 * m + kk < quads) {
 #pragma unroll
-                for (int part = 0; part < GE / GP; part++) {
-                    out[((4 * m + kk) * GE + part * GP + g) * 16] = acc[m][part * GP + g] * up;
+                for (int part = 0; part < GE / G; part++) {
+                    out[((4 * m + kk) * GE + part * G + g) * 16] = acc[m][part * G + g] * up;
                 }
             }
         }
@@ -709,15 +700,15 @@ __device__ __forceinline__ int group_segment(int stage, int wave, bool cooperati
     }
 }
 
-// The row blocks of a workgroup for rhs columns [kbase, kbase + 16 GP), from the coordinates xv of the first
+// The row blocks of a workgroup for rhs columns [kbase, kbase + 16 G), from the coordinates xv of the first
 // segment on; false (in all wavefronts) if the form does not suit them.  Synchronises the workgroup.
 template <int KT, int G>
-__device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const WaveView& w, const BlockRows& rows,
-                                           const GroupPlan& p, int row0, int kbase, int wave, const GridWindow& common,
-                                           const KernelConsts& kc, int first_stage, float (&xv)[KM_GROUP_CHUNK / 64]) {
+__device__ __forceinline__ bool group_forward(const FwdArgs& a, float* lds, const WaveView& w, const BlockRows& rows,
+                                              const GroupPlan& p, int row0, int kbase, int wave, const GridWindow& common,
+                                              const KernelConsts& kc, int first_stage, float (&xv)[KM_GROUP_CHUNK / 64]) {
     using P = GroupShape<KT, G>;
     using S = GridShape<KT, G>;
-    constexpr int GP = S::GP, GE = S::GE, MT = S::MT;
+    constexpr int GE = S::GE, MT = S::MT;
     const int lane = threadIdx.x & 63;
     const int li = lane & 15;
     const int kk = lane >> 4;
@@ -766,9 +757,9 @@ __device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const W
         if (segment < 0) {
             continue;
         }
-        unsigned bad[GP];
+        unsigned bad[G];
 #pragma unroll
-        for (int g = 0; g < GP; g++) {
+        for (int g = 0; g < G; g++) {
             bad[g] = 0;
         }
         if (lane_value(p.start, segment) < lane_value(p.end, segment)) {
@@ -778,9 +769,9 @@ __device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const W
             fine = group_columns<KT, G>(a, w, p, segment, kbase, common, kc, tab, sums, xv, bad) && fine;
         }
         if (lane == 0) {
-            unsigned* to = bad_segments + segment * GP;
+            unsigned* to = bad_segments + segment * G;
 #pragma unroll
-            for (int g = 0; g < GP; g++) {
+            for (int g = 0; g < G; g++) {
                 to[g] = bad[g];
             }
         }
@@ -799,7 +790,7 @@ __device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const W
     const GridWindow gw = group_window(common, p, KM_GROUP_ROW + wave);
     const int quad = lane_value(p.quad, KM_GROUP_ROW + wave) + kk;
     float4v acc[MT][GE];
-    unsigned bad[GP];
+    unsigned bad[G];
 #pragma unroll
     for (int m = 0; m < MT; m++) {
 #pragma unroll
@@ -808,7 +799,7 @@ __device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const W
         }
     }
 #pragma unroll
-    for (int g = 0; g < GP; g++) {
+    for (int g = 0; g < G; g++) {
         bad[g] = 0;
     }
 #pragma unroll 1
@@ -841,30 +832,29 @@ __device__ __forceinline__ bool group_pass(const FwdArgs& a, float* lds, const W
             }
         }
 #pragma unroll
-        for (int g = 0; g < GP; g++) {
+        for (int g = 0; g < G; g++) {
             if (c == KM_GROUP_CORE && p.cooperative) {
 #pragma unroll
                 for (int v = 0; v < KM_GROUP; v++) {
-                    bad[g] |= bad_segments[(KM_GROUP_PIECE + v) * GP + g];
+                    bad[g] |= bad_segments[(KM_GROUP_PIECE + v) * G + g];
                 }
             } else {
-                bad[g] |= bad_segments[c * GP + g];
+                bad[g] |= bad_segments[c * G + g];
             }
         }
     }
-    int shift[GP];
+    int shift[G];
 #pragma unroll
-    for (int g = 0; g < GP; g++) {
+    for (int g = 0; g < G; g++) {
         shift[g] = (bad[g] >> li & 1) != 0 ? KM_GRID_NOT_FINITE : 0;
     }
     const HeldRows held = hold_rows<KT>(rows, common.x_ref, kc);
-    grid_rows<KT, GP, MT, true, true>(a, w, &held, my_row0, KM_BLOCK_SIZE / 16, kbase, gw, kc, shift, acc);
+    grid_rows<KT, G, MT, true, true>(a, w, &held, my_row0, KM_BLOCK_SIZE / 16, kbase, gw, kc, shift, acc);
     return true;
 }
 
 template <int KT, int G>
-__device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigned item, int wave) {
-    using S = GridShape<KT, G>;
+__device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigned item, int kbase, int wave) {
     WaveView w;
     const unsigned batches = (unsigned)a.num_batches;
     const unsigned group = item / batches;
@@ -899,41 +889,54 @@ __device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigne
         gw.h = uniform(__uint_as_float(__float_as_uint(KM_GRID_STEP * inv) & 0xfffff000u));
         gw.reach = uniform(KM_GRID_REACH * inv);
         group_windows<KT, G>(a, w, row0, gw, &p);
-        grouped = __builtin_amdgcn_readfirstlane(p.ok) != 0;
-#pragma unroll 1
-        for (int pass = 0; grouped && pass < G / S::GP; pass++) {
-            const int kbase = (blockIdx.y * G + pass * S::GP) * 16;
-            if (kbase < a.k) {
-                if (pass > 0) {
-                    __syncthreads();
-                    group_load(a, w, p, group_segment(first, wave, p.cooperative), xv);
-                }
-                grouped = group_pass<KT, G>(a, lds, w, rows, p, row0, kbase, wave, gw, kc, first, xv);
-            }
-        }
+        grouped = __builtin_amdgcn_readfirstlane(p.ok) != 0 &&
+                  group_forward<KT, G>(a, lds, w, rows, p, row0, kbase, wave, gw, kc, first, xv);
         if (!grouped) {
             __syncthreads();  // (tables of the row blocks below lie over the flags' and sums' place)
         }
     }
     if (!grouped && wave < blocks) {
-        // (what a pass has stored is stored again)
-        grid_item<KT, G, 1>(fresh_args(), lds + wave * KM_GRID_TABLE_FLOATS, (long long)(w.row_block + wave) * a.num_batches + w.b, 0);
+        grid_item<KT, G, 1>(fresh_args(), lds + wave * KM_GRID_TABLE_FLOATS, (long long)(w.row_block + wave) * a.num_batches + w.b, kbase, 0);
     }
 }
 
+// The rhs columns of a launch's workgroup.  64 spectral columns are more than the registers hold: two workgroups
+// take half each, neighbours on an XCD, so that both write to a row of the result at about the same time.
+// Measured, two passes of one workgroup (50 to 140 registers spilled) -> two workgroups, a call, cutoff of 6 lengthscales:
+// n = 1e5, k = 64, 2 sets at 10 / 40 points per unit 95.2 -> 62.7 / 157 -> 72.7 us, 8 sets 216 -> 187 / 239 -> 216; k = 40
+// 2 sets 95.2 -> 61.0; n = 20000, one set 30.9 -> 15.6; n = 1e6, k = 64, 8 sets 1725 -> 1596 (1720 with the second halves
+// behind all first ones); all row blocks entry by entry at 3 points per unit n = 1e5 253 -> 216, 3e5 754 -> 776, 1e6
+// 2558 -> 2527.
+template <int KT, int G>
+struct GridColumns {
+    static constexpr int HALVES = KT == KM_KERNEL_SPECTRAL && G == 4 ? 2 : 1;
+    static constexpr int GROUPS = G / HALVES;  // of a workgroup
+    using Shape = GridShape<KT, GROUPS>;
+    static constexpr int RESIDENT = Shape::GE >= 4 ? 2 : (Shape::GE > 1 ? 3 : 4);
+    unsigned block;  // number of the workgroup among those of its half
+    int kbase;
+    __device__ __forceinline__ GridColumns() {
+        const unsigned slot = blockIdx.x / KM_NUM_XCD;
+        block = blockIdx.x % KM_NUM_XCD + slot / HALVES * KM_NUM_XCD;
+        kbase = ((int)blockIdx.y * HALVES + (int)(slot % HALVES)) * GROUPS * 16;
+    }
+};
+
 // W: wavefronts per row block, or 1: fewer than one, the workgroup for several row blocks.
 template <int KT, int G, int W>
-__global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridColumns<KT, G>::RESIDENT)) fwd_grid(const FwdArgs a) {
     extern __shared__ float lds[];
-    const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
-    if (item >= a.total_items) {
+    using C = GridColumns<KT, G>;
+    const C c;
+    const long long item = xcd_item(c.block, a.items_per_xcd);
+    if (item >= a.total_items || c.kbase >= a.k) {
         return;
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if constexpr (W == 1) {
-        group_item<KT, G>(a, lds, (unsigned)item, wave);
+        group_item<KT, C::GROUPS>(a, lds, (unsigned)item, c.kbase, wave);
     } else {
-        grid_item<KT, G, W>(a, lds, item, wave);
+        grid_item<KT, C::GROUPS, W>(a, lds, item, c.kbase, wave);
     }
 }
 
@@ -941,16 +944,21 @@ __global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridShape<KT, G
 // each of their row blocks, so that short pieces fill the SIMDs that would otherwise idle while others finish a
 // last group.
 template <int KT, int G>
-__global__ void __launch_bounds__(64 * KM_GROUP, (GridShape<KT, G>::GE >= 4 ? 2 : (GridShape<KT, G>::GE > 1 ? 3 : 4))) fwd_grid_grouped(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * KM_GROUP, (GridColumns<KT, G>::RESIDENT)) fwd_grid_grouped(const FwdArgs a) {
     extern __shared__ float lds[];
+    using C = GridColumns<KT, G>;
+    const C c;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const unsigned xcd = blockIdx.x % KM_NUM_XCD;
-    const unsigned slot = blockIdx.x / KM_NUM_XCD;
+    const unsigned xcd = c.block % KM_NUM_XCD;
+    const unsigned slot = c.block / KM_NUM_XCD;
     const unsigned first = xcd * (unsigned)a.items_per_xcd;
     const unsigned main_groups = (unsigned)a.items_per_xcd - (unsigned)a.tail_items;
+    if (c.kbase >= a.k) {
+        return;
+    }
     if (slot < main_groups) {
         if (first + slot < (unsigned)a.total_items) {
-            group_item<KT, G>(a, lds, first + slot, wave);
+            group_item<KT, C::GROUPS>(a, lds, first + slot, c.kbase, wave);
         }
         return;
     }
@@ -960,13 +968,13 @@ __global__ void __launch_bounds__(64 * KM_GROUP, (GridShape<KT, G>::GE >= 4 ? 2 
     const unsigned row_block = group * KM_GROUP + (slot - main_groups) % KM_GROUP;
     if (item < (unsigned)a.total_items && (long long)row_block * KM_BLOCK_SIZE < a.m) {
         const unsigned b = spread_batch(item - group * batches, group, batches);
-        grid_item<KT, G, KM_GROUP>(fresh_args(), lds, (long long)row_block * batches + b, wave);
+        grid_item<KT, C::GROUPS, KM_GROUP>(fresh_args(), lds, (long long)row_block * batches + b, c.kbase, wave);
     }
 }
 
 template <int KT, int G, int W>
 static hipError_t launch_grid_as(const FwdArgs& a, dim3 grid, hipStream_t stream) {
-    using S = GridShape<KT, G>;
+    using S = typename GridColumns<KT, G>::Shape;
     hipLaunchKernelGGL((fwd_grid<KT, G, W>), grid, dim3(64 * W, 1, 1),
                        (sizeof(float) * grid_lds_floats<S::GE, S::MT, W>()), stream, a);
     return hipGetLastError();
@@ -974,26 +982,27 @@ static hipError_t launch_grid_as(const FwdArgs& a, dim3 grid, hipStream_t stream
 
 template <int KT, int G>
 static hipError_t launch_grid_w(FwdArgs& a, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
+    using C = GridColumns<KT, G>;
     const long long row_blocks = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     if (plan.col_splits == 1) {
         const long long groups = (row_blocks + KM_GROUP - 1) / KM_GROUP;
         a.total_items = groups * a.num_batches;
         a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
         if (plan.group_tail <= 0) {
-            hipLaunchKernelGGL((fwd_grid<KT, G, 1>), dim3((unsigned)(a.items_per_xcd * KM_NUM_XCD), grid_y, 1),
-                               dim3(64 * KM_GROUP, 1, 1), (sizeof(float) * GroupShape<KT, G>::FLOATS), stream, a);
+            hipLaunchKernelGGL((fwd_grid<KT, G, 1>), dim3((unsigned)(a.items_per_xcd * KM_NUM_XCD * C::HALVES), grid_y, 1),
+                               dim3(64 * KM_GROUP, 1, 1), (sizeof(float) * GroupShape<KT, C::GROUPS>::FLOATS), stream, a);
             return hipGetLastError();
         }
         const long long tail = (plan.group_tail + KM_GROUP - 1) / KM_GROUP;
         a.tail_items = (int)(tail < a.items_per_xcd ? tail : a.items_per_xcd);
-        const dim3 grid((unsigned)((a.items_per_xcd + (KM_GROUP - 1) * a.tail_items) * KM_NUM_XCD), grid_y, 1);
+        const dim3 grid((unsigned)((a.items_per_xcd + (KM_GROUP - 1) * a.tail_items) * KM_NUM_XCD * C::HALVES), grid_y, 1);
         hipLaunchKernelGGL((fwd_grid_grouped<KT, G>), grid, dim3(64 * KM_GROUP, 1, 1),
-                           (sizeof(float) * GroupShape<KT, G>::FLOATS), stream, a);
+                           (sizeof(float) * GroupShape<KT, C::GROUPS>::FLOATS), stream, a);
         return hipGetLastError();
     }
     a.total_items = row_blocks * a.num_batches;
     a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD), grid_y, 1);
+    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD * C::HALVES), grid_y, 1);
     switch (plan.col_splits) {
         case 2: return launch_grid_as<KT, G, 2>(a, grid, stream);
         case 4: return launch_grid_as<KT, G, 4>(a, grid, stream);
