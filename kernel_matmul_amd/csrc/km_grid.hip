@@ -343,7 +343,9 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
 // (37 spilled with one spectral operand group).  Measured, 32 -> 64 rows at a time, n = 1e5, 8 sets, lengthscale 0.5:
 // spectral k = 16 at 1 / 3 / 5 points per unit 70.2 -> 59.8 / 72.4 -> 59.3 / 73.8 -> 63.2 us a call, k = 32 at 10
 // 155 -> 136; rbf k = 16 at 3 56.9 -> 47.3, k = 64 at 10 251 -> 221; two wavefronts, spectral n = 1e5, 2 sets, at 2
-// 30.4 -> 25.2.  The spills in the large kernels cost dense points 1 % (spectral k = 32 98.4 -> 99.9).
+// 30.4 -> 25.2.  Where one or two wavefronts spill (3 to 30 registers, most of them in front of this path's loops) the
+// rows' share of the result is written to and read from scratch memory, a tenth to a quarter of it again: n = 1e6, 8 sets at
+// 3 points per unit spectral k = 32 1024 us a call with 22 spilled, 998 with 16; rbf k = 32 741 with 25, 712 with 19.
 template <int KT, int G, int W>
 __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
                                                int wave, const GridWindow& gw, const KernelConsts& kc) {
@@ -376,11 +378,13 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
     }
 #pragma unroll 1
     for (int piece = 0; piece < PIECES; piece++) {
+        // (anew for each piece: lanes' offsets formed with its strides in front of the loop would be spilled)
+        const FwdArgs& f = PIECES > 1 ? fresh_args() : a;
         const int base = row0 + 16 * R * (wave * PIECES + piece);
         float xr[R];
 #pragma unroll
         for (int r = 0; r < R; r++) {
-            xr[r] = w.x1[(long long)min(base + 16 * r + li, a.m - 1) * a.x1_s];
+            xr[r] = w.x1[(long long)min(base + 16 * r + li, f.m - 1) * f.x1_s];
         }
         // the columns within reach of these rows
         float lo = xr[0] - rows.x_ref, hi = lo;
@@ -400,13 +404,13 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         constexpr int CHUNK = G == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
         float xv[CHUNK / 64];
         if (w.range_start < w.range_end) {
-            grid_load(w.x2, a.x2_s, w.range_start, 1, w.range_end, xv);
+            grid_load(w.x2, f.x2_s, w.range_start, 1, w.range_end, xv);
         }
         int shift[G];
         float4v acc[R][GE];
-        const bool fine = grid_columns<false, KT, G, R, 1, false, false, CHUNK>(vectors(a), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
+        const bool fine = grid_columns<false, KT, G, R, 1, false, false, CHUNK>(vectors(f), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
                                                            R, xv, shift, acc);
-        const float sigma = w.params[KernelTraits<KT>::SIGMA * a.params_s];
+        const float sigma = w.params[KernelTraits<KT>::SIGMA * f.params_s];
         float down[GE];
 #pragma unroll
         for (int g = 0; g < GE; g++) {
@@ -420,7 +424,7 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
                 const float th = phase_rev(kc.f, xr[r], rows.x_ref);
                 row_phases(__builtin_amdgcn_cosf(th), __builtin_amdgcn_sinf(th), 0, ca, sa);
             }
-            grid_store<KT, G>(a, w, ca, sa, acc[r], down, base + 16 * r, kbase);
+            grid_store<KT, G>(f, w, ca, sa, acc[r], down, base + 16 * r, kbase);
         }
     }
 }
