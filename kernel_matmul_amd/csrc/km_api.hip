@@ -167,10 +167,12 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
         return KM_OK;
     }
     if (variant == KM_VARIANT_AUTO) {
-        // Measured on gfx950 (n = 1e5, k = 16): for the locally periodic kernel with enough row
-        // blocks to fill the device several times, sharing the rhs operand between four row
-        // blocks wins (batch 8: 133 against 154 us; batch 2: 52 against 49 us, hence the
-        // threshold); rbf and spectral kernels are faster through the column tables with one
+        // Locally periodic kernels with enough row blocks to fill the device several times share the rhs
+        // operand between four row blocks.  That gains by the width of the ranges, which is not known here, and
+        // is kept for its larger gains.  Measured on gfx950 with both kernels leaving tiles out (k = 16, shared
+        // against one row block per wavefront; at 2 / 10 / 40 points per unit): 1564 items 32 / 28, 55 / 53 and 135 /
+        // 147 us a call, 3128 items 41 / 37, 74 / 71 and 186 / 202, 6256 items 70 / 63, 123 / 119 and 318 / 355; 62504
+        // items at 10 880 / 798.  rbf and spectral kernels are faster through the column tables with one
         // wavefront per row block (rbf, batch 8: 77 against 86 us; batch 64: 494 against 578 us).
         const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
         const bool shared = p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC && p.k <= 16 &&

@@ -16,7 +16,7 @@
 // that is not finite makes its column's results NaN in every row whose range holds it, as does a NaN
 // among the range's column coordinates (spectral: an infinity as well) in all columns.
 //
-// Measured against the entry-wise kernels (a call, queued): rbf n = 65536, k = 64 43.6 -> 21.2 us; the large
+// Measured against the entry-wise kernels (a call, queued): rbf n = 65536, k = 64 43.6 -> 21.6 us; the large
 // launches below, at group_item.  The small ones are bound by the latency of one wavefront's steps.
 #include "km_batch.h"
 #include "km_common.h"
@@ -450,8 +450,11 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     const GridWindow gw = grid_window<S::MT>(rows, kc);
     // (the same in every lane, and said so: the barriers inside depend on it)
     const bool grid = __builtin_amdgcn_readfirstlane(gw.ok && w.range_end - w.range_start >= KM_GRID_MIN_WIDTH) != 0;
-    if (!grid || !grid_forward<KT, G, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv)) {
-        grid_entrywise<KT, G, W>(a, lds, w, row0, kbase, wave, gw, kc);
+    // (always so; without the condition the kernel came out slower, rbf n = 65536, k = 64 21.9 against 21.6 us a call)
+    if (kbase < a.k) {
+        if (!grid || !grid_forward<KT, G, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv)) {
+            grid_entrywise<KT, G, W>(a, lds, w, row0, kbase, wave, gw, kc);
+        }
     }
 }
 
@@ -473,12 +476,12 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
 //
 // Measured (a call, queued), one row block per wavefront -> four per workgroup: spectral n = 1e5, k = 16, 8 sets
 // at 10 points per unit 64.5 -> 61 us (entry by entry 103.8), at 40 115 -> 70; 4 sets at 160 182 -> 86; n = 1e6,
-// k = 32, 8 sets 850 -> 786; rbf n = 1e5, k = 64, 8 sets 135 -> 129.  A row block of the first takes 3200 VALU
-// instructions instead of 4450; a quarter of the issue slots now wait for the workgroup's latencies (start and
-// windows of a segment, the exchange), which is what bounds the narrow ranges.  Four: the sums of a group and
-// their tables are then a third of the LDS for two operand groups, so that three workgroups of four wavefronts
-// are resident, as many as the registers allow; with three row blocks for three or four wavefronts one
-// wavefront waits, or less is shared.
+// k = 32, 8 sets 850 -> 778; rbf n = 1e5, k = 64, 8 sets 130 -> 114.  A row block of the first takes 3450 VALU
+// instructions instead of 4450 and the SIMDs' VALU is busy 54 % of the cycles instead of 66: with two wavefronts
+// resident on average, what bounds the narrow ranges is the latency of a workgroup's start, windows and exchange.
+// Four: the sums of a group and their tables are then a third of the LDS for two operand groups, so that three
+// workgroups of four wavefronts are resident, as many as the registers allow; with three row blocks for three or
+// four wavefronts one wavefront waits, or less is shared.
 // ---------------------------------------------------------------------------------------
 #define KM_GROUP_CHUNK 128
 
@@ -920,9 +923,14 @@ struct GridColumns {
     unsigned block;  // number of the workgroup among those of its half
     int kbase;
     __device__ __forceinline__ GridColumns() {
-        const unsigned slot = blockIdx.x / KM_NUM_XCD;
-        block = blockIdx.x % KM_NUM_XCD + slot / HALVES * KM_NUM_XCD;
-        kbase = ((int)blockIdx.y * HALVES + (int)(slot % HALVES)) * GROUPS * 16;
+        if constexpr (HALVES == 1) {
+            block = blockIdx.x;
+            kbase = blockIdx.y * G * 16;
+        } else {
+            const unsigned slot = blockIdx.x / KM_NUM_XCD;
+            block = blockIdx.x % KM_NUM_XCD + slot / HALVES * KM_NUM_XCD;
+            kbase = ((int)blockIdx.y * HALVES + (int)(slot % HALVES)) * GROUPS * 16;
+        }
     }
 };
 
@@ -933,7 +941,7 @@ __global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridColumns<KT,
     using C = GridColumns<KT, G>;
     const C c;
     const long long item = xcd_item(c.block, a.items_per_xcd);
-    if (item >= a.total_items || c.kbase >= a.k) {
+    if (item >= a.total_items || (C::HALVES > 1 && c.kbase >= a.k)) {
         return;
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -957,7 +965,7 @@ __global__ void __launch_bounds__(64 * KM_GROUP, (GridColumns<KT, G>::RESIDENT))
     const unsigned slot = c.block / KM_NUM_XCD;
     const unsigned first = xcd * (unsigned)a.items_per_xcd;
     const unsigned main_groups = (unsigned)a.items_per_xcd - (unsigned)a.tail_items;
-    if (c.kbase >= a.k) {
+    if (C::HALVES > 1 && c.kbase >= a.k) {
         return;
     }
     if (slot < main_groups) {
