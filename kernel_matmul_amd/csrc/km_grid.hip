@@ -908,29 +908,39 @@ __device__ __forceinline__ void group_item(const FwdArgs& a, float* lds, unsigne
 }
 
 // The rhs columns of a launch's workgroup.  64 spectral columns are more than the registers hold: two workgroups
-// take half each, neighbours on an XCD, so that both write to a row of the result at about the same time.
+// take half each.  An XCD takes the two halves in turn, RUN workgroups at a time (half of what it holds): both write to
+// a row of the result before its place leaves the caches, but those that run together read the same half of rhs.
 // Measured, two passes of one workgroup (50 to 140 registers spilled) -> two workgroups, a call, cutoff of 6 lengthscales:
-// n = 1e5, k = 64, 2 sets at 10 / 40 points per unit 95.2 -> 62.7 / 157 -> 72.7 us, 8 sets 216 -> 187 / 239 -> 216; k = 40
-// 2 sets 95.2 -> 61.0; n = 20000, one set 30.9 -> 15.6; n = 1e6, k = 64, 8 sets 1725 -> 1596 (1720 with the second halves
-// behind all first ones); all row blocks entry by entry at 3 points per unit n = 1e5 253 -> 216, 3e5 754 -> 776, 1e6
-// 2558 -> 2527.
+// n = 1e5, k = 64, 2 sets at 10 / 40 points per unit 95.3 -> 63.0 / 157 -> 72.7 us, 8 sets 215 -> 188 / 239 -> 216; k = 40
+// 2 sets 94.5 -> 61.3; n = 20000, one set 30.5 -> 15.3; k = 64, 8 sets, at 10 points per unit / at 3, all row blocks entry by
+// entry: n = 3e5 583 -> 547 / 756 -> 652, 1e6 1719 -> 1638 / 2563 -> 2118.  Neighbours in turn (RUN 1): 532 / 780 and 1585 /
+// 2544; all first halves before all second ones 575 / 724 and 1721 / 2370; RUN 8 550 / 783, 64 549 / 645.
 template <int KT, int G>
 struct GridColumns {
     static constexpr int HALVES = KT == KM_KERNEL_SPECTRAL && G == 4 ? 2 : 1;
     static constexpr int GROUPS = G / HALVES;  // of a workgroup
+    static constexpr unsigned RUN = 32;
     using Shape = GridShape<KT, GROUPS>;
     static constexpr int RESIDENT = Shape::GE >= 4 ? 2 : (Shape::GE > 1 ? 3 : 4);
     unsigned block;  // number of the workgroup among those of its half
     int kbase;
-    __device__ __forceinline__ GridColumns() {
+    bool beyond;     // no columns, or no work left for the XCD
+    // per_xcd: workgroups of an XCD, of one half
+    __device__ __forceinline__ GridColumns(const FwdArgs& a, long long per_xcd) {
         if constexpr (HALVES == 1) {
             block = blockIdx.x;
             kbase = blockIdx.y * G * 16;
+            beyond = false;
         } else {
             const unsigned slot = blockIdx.x / KM_NUM_XCD;
-            block = blockIdx.x % KM_NUM_XCD + slot / HALVES * KM_NUM_XCD;
-            kbase = ((int)blockIdx.y * HALVES + (int)(slot % HALVES)) * GROUPS * 16;
+            const unsigned own = slot / (HALVES * RUN) * RUN + slot % RUN;
+            block = blockIdx.x % KM_NUM_XCD + own * KM_NUM_XCD;
+            kbase = ((int)blockIdx.y * HALVES + (int)(slot / RUN % HALVES)) * GROUPS * 16;
+            beyond = kbase >= a.k || own >= per_xcd;
         }
+    }
+    static unsigned workgroups(long long per_xcd) {
+        return (unsigned)((HALVES == 1 ? per_xcd : (per_xcd + RUN - 1) / RUN * RUN * HALVES) * KM_NUM_XCD);
     }
 };
 
@@ -939,9 +949,9 @@ template <int KT, int G, int W>
 __global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridColumns<KT, G>::RESIDENT)) fwd_grid(const FwdArgs a) {
     extern __shared__ float lds[];
     using C = GridColumns<KT, G>;
-    const C c;
+    const C c(a, a.items_per_xcd);
     const long long item = xcd_item(c.block, a.items_per_xcd);
-    if (item >= a.total_items || (C::HALVES > 1 && c.kbase >= a.k)) {
+    if (item >= a.total_items || c.beyond) {
         return;
     }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -959,13 +969,13 @@ template <int KT, int G>
 __global__ void __launch_bounds__(64 * KM_GROUP, (GridColumns<KT, G>::RESIDENT)) fwd_grid_grouped(const FwdArgs a) {
     extern __shared__ float lds[];
     using C = GridColumns<KT, G>;
-    const C c;
+    const C c(a, a.items_per_xcd + (KM_GROUP - 1) * a.tail_items);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned xcd = c.block % KM_NUM_XCD;
     const unsigned slot = c.block / KM_NUM_XCD;
     const unsigned first = xcd * (unsigned)a.items_per_xcd;
     const unsigned main_groups = (unsigned)a.items_per_xcd - (unsigned)a.tail_items;
-    if (C::HALVES > 1 && c.kbase >= a.k) {
+    if (c.beyond) {
         return;
     }
     if (slot < main_groups) {
@@ -1001,20 +1011,20 @@ static hipError_t launch_grid_w(FwdArgs& a, const MatmulPlan& plan, unsigned gri
         a.total_items = groups * a.num_batches;
         a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
         if (plan.group_tail <= 0) {
-            hipLaunchKernelGGL((fwd_grid<KT, G, 1>), dim3((unsigned)(a.items_per_xcd * KM_NUM_XCD * C::HALVES), grid_y, 1),
+            hipLaunchKernelGGL((fwd_grid<KT, G, 1>), dim3(C::workgroups(a.items_per_xcd), grid_y, 1),
                                dim3(64 * KM_GROUP, 1, 1), (sizeof(float) * GroupShape<KT, C::GROUPS>::FLOATS), stream, a);
             return hipGetLastError();
         }
         const long long tail = (plan.group_tail + KM_GROUP - 1) / KM_GROUP;
         a.tail_items = (int)(tail < a.items_per_xcd ? tail : a.items_per_xcd);
-        const dim3 grid((unsigned)((a.items_per_xcd + (KM_GROUP - 1) * a.tail_items) * KM_NUM_XCD * C::HALVES), grid_y, 1);
+        const dim3 grid(C::workgroups(a.items_per_xcd + (KM_GROUP - 1) * a.tail_items), grid_y, 1);
         hipLaunchKernelGGL((fwd_grid_grouped<KT, G>), grid, dim3(64 * KM_GROUP, 1, 1),
                            (sizeof(float) * GroupShape<KT, C::GROUPS>::FLOATS), stream, a);
         return hipGetLastError();
     }
     a.total_items = row_blocks * a.num_batches;
     a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    const dim3 grid((unsigned)(a.items_per_xcd * KM_NUM_XCD * C::HALVES), grid_y, 1);
+    const dim3 grid(C::workgroups(a.items_per_xcd), grid_y, 1);
     switch (plan.col_splits) {
         case 2: return launch_grid_as<KT, G, 2>(a, grid, stream);
         case 4: return launch_grid_as<KT, G, 4>(a, grid, stream);

@@ -86,3 +86,29 @@ def test_gradient(kt, c, batch):
     right = torch.randn(batch, n, c, generator=torch.Generator().manual_seed(1))
     shared = [t.expand(batch, *t.shape) for t in (x, start, end)]
     check_gradient(kt, shared[0], shared[0], left, right, params, shared[1], shared[2])
+
+
+@pytest.mark.parametrize("k", [33, 64, 100])
+@pytest.mark.parametrize("rows,tail", [(32, None), (64, None), (128, 0), (128, 4), (128, 37), (None, None)])
+def test_halves_of_wide_rhs(k, rows, tail):
+    """More than 32 spectral columns: an XCD's workgroups take one half of 64 columns and the other in turn, some 32 at a
+    time.  The result is that of calls with 32 columns each."""
+    n, batch = 20_000, 9
+    x, rhs, params, start, end = (t.to(DEVICE) for t in _inputs("spectral", batch, n, k))
+    shared = [t.expand(batch, *t.shape) for t in (x, start, end)]
+
+    def call(part):
+        args = (shared[0], shared[0], part, params, shared[1], shared[2])
+        defines = dict(MatmulSingleConfiguration("spectral").make_config(args))
+        if rows:
+            defines["MATMUL_VARIANT"], defines["MATMUL_ROWS_PER_WAVE"] = "grid", rows
+        if tail is not None:
+            defines["MATMUL_GROUP_TAIL"] = tail
+        return load_native("matmul", defines).call(*args)
+
+    result = call(rhs)
+    for first in range(0, k, 32):
+        part = rhs[..., first:first + 32].contiguous()
+        expected = call(part)
+        for b in range(batch):
+            _close(result[b, :, first:first + 32], expected[b], part[b], start, end)
