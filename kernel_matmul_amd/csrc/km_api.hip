@@ -120,7 +120,8 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     plan->row_groups = 8;
     plan->tail_balance = 0;
     plan->group_tail_halves = 0;
-    int operands = k_chunk * (p.kernel_type == KM_KERNEL_SPECTRAL ? 2 : 1);
+    const bool spectral = p.kernel_type == KM_KERNEL_SPECTRAL;
+    int operands = k_chunk * (spectral ? 2 : 1);
     if (operands > 64) {  // (64 spectral columns: half of them a workgroup)
         operands /= 2;
         items *= 2;
@@ -131,6 +132,10 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     } else {
         const long long grouped = operands > 32 ? 2800 : (operands > 16 ? 1500 : 2300);
         plan->col_splits = items <= 200 ? 8 : (items < 700 ? 4 : (items < grouped ? 2 : 1));
+    }
+    // (two workgroups for each row block: no more threads than a launch may have)
+    while (k_chunk == 64 && spectral && plan->col_splits > 1 && (per_launch + 512) * 2 * 64 * plan->col_splits > 0xffffffffLL) {
+        plan->col_splits /= 2;
     }
     if (plan->col_splits != 1) {
         plan->group_tail = -1;

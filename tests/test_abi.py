@@ -99,6 +99,12 @@ def test_launch_descriptions_without_a_gpu():
     assert "fwd_grid<rbf, G=1, W=4>" in matmul("rbf", 1, 65_536, 65_536, 16, None)
     assert "fwd_table_f16<rbf, G=1" in matmul("rbf", 1, 4096, 4096, 1, None)
     assert "fwd_block<locally_periodic" in matmul("locally_periodic", 8, 1_000_000, 1_000_000, 16, None)
+    # two workgroups for 64 spectral columns: as many wavefronts as asked for where a launch can have them
+    wavefronts = _native.LaunchOptions(variant=7, rows_per_wave=16)
+    assert "fwd_grid<spectral, G=4, W=8>" in matmul("spectral", 1, 100_000_000, 100_000, 64, wavefronts)
+    assert "fwd_grid<spectral, G=4, W=4>" in matmul("spectral", 1, 600_000_000, 100_000, 64, wavefronts)
+    assert "fwd_grid<spectral, G=4, W=2>" in matmul("spectral", 1, 1_500_000_000, 100_000, 64, wavefronts)
+    assert "fwd_grid<spectral, G=2, W=8>" in matmul("spectral", 1, 600_000_000, 100_000, 32, wavefronts)
     # the kernels evaluated entry by entry, where they are asked for
     entries = _native.LaunchOptions(variant=3)
     text = matmul("spectral", 8, 100_000, 100_000, 16, entries)
