@@ -189,12 +189,14 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[N], int first, 
             tab[q] = y;
             tab[grid_table_rest(CH) + q] = remainder_of(xv[i], gw.x_ref, y);
         }
+        // (zero past the end of the range, where rhs values are those of the last row again)
+        const bool inside = 32 * ((lane >> 5) + 2 * i) * stride + (lane & 31) <= last;
         if (PHASE) {
             const float th = phase_rev(kc.f, xv[i], gw.x_ref);
-            tab[CH + q] = wgt * __builtin_amdgcn_cosf(th);
-            tab[2 * CH + q] = wgt * __builtin_amdgcn_sinf(th);
+            tab[CH + q] = inside ? wgt * __builtin_amdgcn_cosf(th) : 0.0f;
+            tab[2 * CH + q] = inside ? wgt * __builtin_amdgcn_sinf(th) : 0.0f;
         } else {
-            tab[CH + q] = wgt;
+            tab[CH + q] = inside ? wgt : 0.0f;
         }
         if ((lane & 7) == 0) {
             tab[3 * CH + (q >> 3)] = lo[i];
@@ -251,7 +253,9 @@ __device__ __forceinline__ RhsLane<G> rhs_lane(const GridVectors& a, int kbase) 
     return rl;
 }
 
-// rhs values of a step (columns c0 + 8 kk + t), zero past the end of the range.
+// rhs values of a step (columns c0 + 8 kk + t).  Past the end of the range the last row's are repeated: the table's
+// factors of these columns are zero (grid_table).  Nothing here depends on a loaded value, so that all of a step's loads
+// are in flight together.
 template <int G>
 __device__ __forceinline__ void grid_rhs(const GridVectors& a, const float* __restrict__ rhs, int c0, int col_end,
                                          int kk, const RhsLane<G>& lane, float (&raw)[G][8]) {
@@ -269,12 +273,10 @@ __device__ __forceinline__ void grid_rhs(const GridVectors& a, const float* __re
         const int last = col_end - 1 - c0;
 #pragma unroll
         for (int t = 0; t < 8; t++) {
-            const int rel = 8 * kk + t;
-            const unsigned row = 4u * __umul24((unsigned)min(rel, last), s0);
+            const unsigned row = 4u * __umul24((unsigned)min(8 * kk + t, last), s0);
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                const float v = buffer_at(ru, row + lane.col[g], 0u);
-                raw[g][t] = rel <= last ? v : 0.0f;
+                raw[g][t] = buffer_at(ru, row + lane.col[g], 0u);
             }
         }
     }
@@ -445,14 +447,15 @@ __device__ __forceinline__ void look_at_steps(const GridVectors& a, const WaveVi
     } while (steps.any());
 }
 
-// The running power-of-two scale of an rhs column, lowered when a magnitude m of its values would exceed 2^15 (NaN
-// and infinities hand themselves on).  first: no step has added to the sums yet (a scale that is still the largest
+// The running power-of-two scale of an rhs column, lowered when a magnitude of its values (own: of those that this lane
+// holds) would exceed 2^15 (NaN and infinities hand themselves on).  The four lanes of a column compare theirs only then.  first: no step has added to the sums yet (a scale that is still the largest
 // does not say so: steps of values below 2^-85 leave it as it is).
 template <int G, int PARTS, int MT>
-__device__ __forceinline__ void lower_scale(int g, float m, bool used, bool first, int (&shift)[G], float (&scale)[G],
+__device__ __forceinline__ void lower_scale(int g, float own, bool used, bool first, int (&shift)[G], float (&scale)[G],
                                             float4v (&acc)[MT][G * PARTS]) {
-    const bool grow = used && !(m * scale[g] < 32768.0f);
-    if (__any(grow)) {
+    if (__any(used && !(own * scale[g] < 32768.0f))) {
+        const float m = column_maximum(own);
+        const bool grow = used && !(m * scale[g] < 32768.0f);
         if (grow && !is_finite(m)) {
             shift[g] = KM_GRID_NOT_FINITE;
             scale[g] = 0.0f;
@@ -672,6 +675,16 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
                     raw[g][t] = next[g][t];
                 }
             }
+            if (!GRID && PARTS == 1 && first + 32 * (j * W + 1) > w.range_end) {  // (no column factors to do it)
+                const int last = w.range_end - 1 - first - 32 * j * W;
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+#pragma unroll
+                    for (int t = 0; t < 8; t++) {
+                        raw[g][t] = 8 * kk + t <= last ? raw[g][t] : 0.0f;
+                    }
+                }
+            }
             const int off = 32 * j + 8 * kk;
             const bool wide = (steps >> (16 + j) & 1) != 0;
             need &= need - 1;
@@ -690,7 +703,7 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
             }
 #pragma unroll
             for (int g = 0; g < G; g++) {
-                lower_scale<G, PARTS, MT>(g, column_maximum(magnitude(raw[g])), rl.used[g], first_step, shift, scale, acc);
+                lower_scale<G, PARTS, MT>(g, magnitude(raw[g]), rl.used[g], first_step, shift, scale, acc);
             }
             first_step = false;
             grid_step<GRID, G, PARTS, MT, EXACT, CH, GRID>(tab, off, raw, gw, t0, xr, kc, tiles, wide, weights, scale, acc);
