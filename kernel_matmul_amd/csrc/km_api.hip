@@ -83,8 +83,6 @@ static int check_common(const char* op, int kernel_type, int batch_rank, const i
 // (measured: 1024 beats 2048 and 4096 from 157 to 3128 row-block items).
 // ---------------------------------------------------------------------------------------
 static const long long TARGET_WAVES = 1024;
-// Row-block items from which the workgroup-shared forward kernel is considered.
-static const long long BLOCK_VARIANT_MIN_ITEMS = 4096;
 
 // Grid form (rbf and spectral kernels): wavefronts per 128-row item, more to make the device busy with few
 // items, or (col_splits 1) workgroups that take four row blocks together.  Measured at ten points per unit,
@@ -146,6 +144,42 @@ static bool grid_plan(const MatmulProblem& p, const km_launch_options* opt, int 
     return true;
 }
 
+// Locally periodic kernels (fwd_block of km_periodic.hip): groups of 16 rows and wavefronts of a row block.  Fewer rows
+// repeat the columns' side of a step, more wavefronts add an exchange; both spread few items over the device.
+// Measured, 8 wavefronts of 32 / of 64 / of 128 rows against 4 / 2 / 1 of 128, k = 16, cutoff of 6 lengthscales: 40 items
+// at 10 points per unit 10.7 / 10.5 / 10.6 / 10.6 / 13.9 / 21 us a call, at 300 22 / 30 / 47 / 61 / 119 / 227; 314 items at
+// 10 18 / 14.6 / 17.6 / 15.4 / 23.6 / 31, at 40 29 / 23 / 30 / 33 / 57 / 78; 628 items at 10 31 / 22 / 25 / 18.8 / 24.5 / 32;
+// 3128 items at 10 137 / 87 / 96 / 51.9 / 50.2 / 53.6, at 40 226 / 153 / 181 / 119 / 130 / 148; 6256 items at 10 270 / 170 /
+// 189 / 100 / 93 / 92, at 2 245 / 146 / 159 / 74 / 60 / 55.  More rhs columns fill the device with fewer items.
+// Against fwd_mfma_f16, which took all of these (four row blocks sharing their rhs operand from 4096 items on): 314 items
+// at 10 24.0, 628 items 35.7, 3128 items 73.4, 6256 items 126.5, 62504 items 922 (614).  Below 32 items its 16-row pieces
+// spread further (16 items at 300 points per unit 11.8 against 13.9).
+static bool periodic_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
+    if (p.kernel_type != KM_KERNEL_LOCALLY_PERIODIC || (opt && (opt->rows_per_wave != 0 || opt->col_splits > 1))) {
+        return false;
+    }
+    const int k_chunk = p.k <= 16 ? 16 : (p.k <= 32 ? 32 : 64);
+    const long long items = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * p.num_batches * ((p.k + k_chunk - 1) / k_chunk);
+    if (items < 32) {
+        return false;
+    }
+    plan->variant = KM_VARIANT_PERIODIC;
+    plan->k_chunk = k_chunk;
+    plan->tail_balance = 0;
+    plan->group_tail_halves = 0;
+    if (k_chunk == 16) {
+        plan->row_groups = items <= 60 ? 2 : (items <= 450 ? 4 : 8);
+        plan->col_splits = items <= 450 ? 8 : (items < 2000 ? 4 : (items < 5000 ? 2 : 1));
+    } else if (k_chunk == 32) {
+        plan->row_groups = items <= 110 ? 4 : 8;
+        plan->col_splits = items <= 200 ? 8 : (items < 2000 ? 4 : (items < 5000 ? 2 : 1));
+    } else {
+        plan->row_groups = items <= 60 ? 2 : 4;
+        plan->col_splits = items <= 110 ? 8 : (items < 1000 ? 4 : (items < 2500 ? 2 : 1));
+    }
+    return true;
+}
+
 static int make_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
     int variant = opt ? opt->variant : KM_VARIANT_AUTO;
     plan->phase_split = 0;
@@ -171,19 +205,11 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
     if (grid_plan(p, opt, variant, plan)) {
         return KM_OK;
     }
+    if (variant == KM_VARIANT_AUTO && periodic_plan(p, opt, plan)) {
+        return KM_OK;
+    }
     if (variant == KM_VARIANT_AUTO) {
-        // Locally periodic kernels with enough row blocks to fill the device several times share the rhs
-        // operand between four row blocks.  That gains by the width of the ranges, which is not known here, and
-        // is kept for its larger gains.  Measured on gfx950 with both kernels leaving tiles out (k = 16, shared
-        // against one row block per wavefront; at 2 / 10 / 40 points per unit): 1564 items 32 / 28, 55 / 53 and 135 /
-        // 147 us a call, 3128 items 41 / 37, 74 / 71 and 186 / 202, 6256 items 70 / 63, 123 / 119 and 318 / 355; 62504
-        // items at 10 880 / 798.  rbf and spectral kernels are faster through the column tables with one
-        // wavefront per row block (rbf, batch 8: 77 against 86 us; batch 64: 494 against 578 us).
-        const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
-        const bool shared = p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC && p.k <= 16 &&
-                            row_blocks * p.num_batches >= BLOCK_VARIANT_MIN_ITEMS &&
-                            !(opt && (opt->rows_per_wave != 0 || opt->col_splits > 1));
-        variant = shared ? KM_VARIANT_BLOCK : KM_VARIANT_MFMA_F16;
+        variant = KM_VARIANT_MFMA_F16;
     }
     if (variant != KM_VARIANT_VALU && variant != KM_VARIANT_MFMA_F32 && variant != KM_VARIANT_MFMA_F16 &&
         variant != KM_VARIANT_MFMA_F16_DIRECT && variant != KM_VARIANT_BLOCK && variant != KM_VARIANT_MFMA_F32_DIRECT) {
@@ -628,6 +654,10 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
                 snprintf(text, text_bytes, "km::fwd_grid<%s, G=%d, W=%d>: grid form, %d wavefronts per row block%s", kt, G,
                          plan.col_splits, plan.col_splits, halves);
             }
+            break;
+        case KM_VARIANT_PERIODIC:
+            snprintf(text, text_bytes, "km::fwd_block<%s, G=%d, R=%d, W=%d>: tabulated phases, %d wavefront(s) per %d rows", kt, G,
+                     plan.row_groups, plan.col_splits, plan.col_splits, 16 * plan.row_groups);
             break;
         case KM_VARIANT_VALU:
             snprintf(text, text_bytes, "km::fwd_valu<%s, KC=%d>: 128 rows per workgroup, %lld workgroups", kt,

@@ -21,7 +21,7 @@
 //   fwd_valu      : one row per lane, contraction with v_fma_f32 on wave-uniform x2 / rhs
 //                   operands fetched through the scalar (read-only) path.
 //
-// (fwd_block, which prepares the rhs operand once per workgroup of four row blocks, lives in
+// (Locally periodic kernels from 32 row blocks on go through km_periodic.hip; the workgroup-shared fwd_block lives in
 // km_matmul_block.hip.)  LDS carries the column tables of fwd_table_f16 and the fixed-order
 // reduction when several wavefronts share a row range.
 #include "km_batch.h"
@@ -1397,6 +1397,9 @@ hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStre
     }
     if (plan.variant == KM_VARIANT_GRID) {
         return launch_matmul_grid(p, plan, stream);
+    }
+    if (plan.variant == KM_VARIANT_PERIODIC) {
+        return launch_matmul_periodic(p, plan, stream);
     }
     FwdArgs a;
     fill_fwd_args(p, &a);
