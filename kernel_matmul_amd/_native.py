@@ -8,6 +8,8 @@ fallback: if the library is missing, every operator raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from typing import Sequence
 
@@ -22,8 +24,10 @@ MAX_BATCH_RANK = 6
 
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libkernel_matmul_amd.so")
+TORCH_CALLS_PATH = os.path.join(_LIB_DIR, "_km_torch.so")
 
 _lib = None
+_torch_calls = None
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
 _vp = ctypes.c_void_p
@@ -139,6 +143,24 @@ def load_library():
     return lib
 
 
+def torch_calls():
+    """The native module of the calls on torch tensors (csrc/km_torch.cpp): every function returns None for a call that
+    is not its to take."""
+    global _torch_calls
+    if _torch_calls is None:
+        load_library()
+        if not os.path.exists(TORCH_CALLS_PATH):
+            raise RuntimeError(
+                f"kernel_matmul_amd: native library not found at {TORCH_CALLS_PATH}. "
+                "Build it with `make -C kernel_matmul_amd/csrc`."
+            )
+        loader = importlib.machinery.ExtensionFileLoader("_km_torch", TORCH_CALLS_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_km_torch", loader))
+        loader.exec_module(module)
+        _torch_calls = module
+    return _torch_calls
+
+
 def _raise(lib, status: int):
     # Every failed check of the reference's entry points is a TORCH_CHECK, i.e. a RuntimeError
     # (native/common/entrypoint.h:3-14).
@@ -155,6 +177,19 @@ def _ptr(t: Tensor):
 
 def _tensor_args(t: Tensor):
     return _ptr(t), _i64(t.stride())
+
+
+def _tensors_args(*tensors: Tensor) -> list:
+    return [argument for t in tensors for argument in _tensor_args(t)]
+
+
+def _result(shape: tuple, device: torch.device, out: Tensor | None) -> Tensor:
+    """A result tensor, or the caller's if it fits."""
+    if out is None:
+        return torch.empty(shape, dtype=torch.float32, device=device)
+    if tuple(out.shape) != shape or out.dtype != torch.float32 or out.device != device or not out.is_contiguous():
+        raise RuntimeError(f"out must be a contiguous float32 tensor of shape {shape} on {device}")
+    return out
 
 
 def _stream(device: torch.device):
@@ -183,32 +218,6 @@ class _on_device:
         if self._guard is not None:
             return self._guard.__exit__(*exc)
         return False
-
-
-# Validated calls, keyed by everything the validation looked at (shapes, strides, dtypes,
-# devices).  A repeated call with the same signature skips the checks and reuses the ctypes
-# stride / size arrays: only the data pointers, the output and the stream are new.
-_PREPARED: dict = {}
-_PREPARED_LIMIT = 512
-
-
-def _signature(op: str, kernel_type: str, tensors) -> tuple:
-    return (op, kernel_type, *[(t.shape, t.stride(), t.dtype, t.device) for t in tensors])
-
-
-def _remember(key, value):
-    if len(_PREPARED) >= _PREPARED_LIMIT:
-        _PREPARED.clear()
-    _PREPARED[key] = value
-    return value
-
-
-def _marshalled(tensors, strides, nonempty) -> list:
-    """Pointer and strides of each tensor of a prepared call."""
-    call_args = []
-    for t, st, filled in zip(tensors, strides, nonempty):
-        call_args += (t.data_ptr() if filled else None, st)
-    return call_args
 
 
 # -- the checks of the reference's entry points (native/common/entrypoint.h:3-14) ----------
@@ -279,36 +288,26 @@ def matmul(kernel_type: str, x1: Tensor, x2: Tensor, rhs: Tensor, params: Tensor
     """out[..., m, k] = K(x1, x2)[mask] @ rhs   (C ABI: km_matmul).
 
     ``out`` (optional) is a contiguous fp32 tensor of the result's shape to write into."""
-    tensors = (x1, x2, rhs, params, start, end)
-    key = _signature("matmul", kernel_type, tensors)
-    prepared = _PREPARED.get(key)
-    if prepared is None:
-        kid = _kernel_id(kernel_type)
-        check_cuda(rhs)
-        check_float(rhs)
-        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-        _check_batch("rhs", rhs, batch_shape, 2)
-        m, n, k = x1.shape[-1], x2.shape[-1], rhs.shape[-1]
-        if rhs.shape[-2] != n:
-            raise RuntimeError(f"rhs has {rhs.shape[-2]} rows, x2 has {n} points")
-        prepared = _remember(key, (
-            load_library().km_matmul, (kid, len(batch_shape), _i64(batch_shape), m, n, k),
-            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors),
-            (*batch_shape, m, k),
-        ))
-    fn, head, strides, nonempty, out_shape = prepared
+    result = torch_calls().matmul(KERNEL_TYPES.get(kernel_type), x1, x2, rhs, params, start, end,
+                                  ctypes.addressof(options) if options is not None else None, out)
+    if result is not None:
+        return result
+    kid = _kernel_id(kernel_type)
+    check_cuda(rhs)
+    check_float(rhs)
+    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+    _check_batch("rhs", rhs, batch_shape, 2)
+    m, n, k = x1.shape[-1], x2.shape[-1], rhs.shape[-1]
+    if rhs.shape[-2] != n:
+        raise RuntimeError(f"rhs has {rhs.shape[-2]} rows, x2 has {n} points")
     device = x1.device
-    if out is None:
-        out = torch.empty(out_shape, dtype=torch.float32, device=device)
-    elif (tuple(out.shape) != out_shape or out.dtype != torch.float32 or out.device != device
-          or not out.is_contiguous()):
-        raise RuntimeError(f"out must be a contiguous float32 tensor of shape {out_shape} on {device}")
-    call_args = _marshalled(tensors, strides, nonempty)
+    out = _result((*batch_shape, m, k), device, out)
+    lib = load_library()
     with _on_device(device):
-        status = fn(*head, *call_args, out.data_ptr() if out.numel() > 0 else None,
-                    ctypes.byref(options) if options is not None else None, _stream(device))
+        status = lib.km_matmul(kid, len(batch_shape), _i64(batch_shape), m, n, k, *_tensors_args(x1, x2, rhs, params, start, end),
+                               _ptr(out), ctypes.byref(options) if options is not None else None, _stream(device))
     if status != 0:
-        _raise(load_library(), status)
+        _raise(lib, status)
     return out
 
 
@@ -349,40 +348,28 @@ def param_grad(kernel_type: str, x1: Tensor, x2: Tensor, left: Tensor, right: Te
     allocates nothing).  Every GPU has one such array: a call on another stream than the last
     one is ordered behind it with an event; calls issued from several host threads at once, or
     through the C ABI directly, must be kept apart by the caller."""
-    tensors = (x1, x2, left, right, params, start, end)
-    key = _signature("param_grad", kernel_type, tensors)
-    prepared = _PREPARED.get(key)
-    if prepared is None:
-        kid = _kernel_id(kernel_type)
-        for t in (left, right):
-            check_cuda(t)
-            check_float(t)
-        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-        _check_batch("left", left, batch_shape, 2)
-        _check_batch("right", right, batch_shape, 2)
-        m, n, c = x1.shape[-1], x2.shape[-1], left.shape[-1]
-        if left.shape[-2] != m or right.shape[-2] != n or right.shape[-1] != c:
-            raise RuntimeError(
-                f"left {tuple(left.shape)} / right {tuple(right.shape)} do not match a {m} x {n} matrix"
-            )
-        lib = load_library()
-        sizes = _i64(batch_shape)
-        need = lib.km_param_grad_workspace_size(kid, len(batch_shape), sizes, m, n, c)
-        prepared = _remember(key, (
-            (kid, len(batch_shape), sizes, m, n, c),
-            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors),
-            (*batch_shape, params.shape[-1]), need,
-        ))
-    head, strides, nonempty, out_shape, need = prepared
+    if not static_scratch:
+        result = torch_calls().param_grad(KERNEL_TYPES.get(kernel_type), x1, x2, left, right, params, start, end, out)
+        if result is not None:
+            return result
+    kid = _kernel_id(kernel_type)
+    for t in (left, right):
+        check_cuda(t)
+        check_float(t)
+    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+    _check_batch("left", left, batch_shape, 2)
+    _check_batch("right", right, batch_shape, 2)
+    m, n, c = x1.shape[-1], x2.shape[-1], left.shape[-1]
+    if left.shape[-2] != m or right.shape[-2] != n or right.shape[-1] != c:
+        raise RuntimeError(
+            f"left {tuple(left.shape)} / right {tuple(right.shape)} do not match a {m} x {n} matrix"
+        )
     lib = load_library()
     device = x1.device
-    if out is None:
-        out = torch.empty(out_shape, dtype=torch.float32, device=device)
-    elif (tuple(out.shape) != out_shape or out.dtype != torch.float32 or out.device != device
-          or not out.is_contiguous()):
-        raise RuntimeError(f"out must be a contiguous float32 tensor of shape {out_shape} on {device}")
-    call_args = _marshalled(tensors, strides, nonempty)
-    out_ptr = out.data_ptr() if out.numel() > 0 else None
+    out = _result((*batch_shape, params.shape[-1]), device, out)
+    head = (kid, len(batch_shape), _i64(batch_shape), m, n, c)
+    call_args = _tensors_args(x1, x2, left, right, params, start, end)
+    out_ptr = _ptr(out)
     if static_scratch:
         with _on_device(device):
             stream = torch.cuda.current_stream(device)
@@ -396,6 +383,7 @@ def param_grad(kernel_type: str, x1: Tensor, x2: Tensor, left: Tensor, right: Te
             event.record(stream)
             _STATIC_SCRATCH_USE[device.index] = (stream.cuda_stream, event)
     else:
+        need = lib.km_param_grad_workspace_size(*head)
         workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
         with _on_device(device):
             status = lib.km_param_grad(*head, *call_args, out_ptr, workspace.data_ptr(), need,
@@ -409,46 +397,37 @@ def index(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tenso
           batch_indices: Sequence[Tensor], row_index: Tensor, col_index: Tensor) -> Tensor:
     """out[q] = K[batch_indices[q]..., row_index[q], col_index[q]]   (C ABI: km_index)."""
     batch_indices = tuple(batch_indices)
-    tensors = (x1, x2, params, start, end, row_index, col_index)
-    key = _signature("index", kernel_type, tensors + batch_indices)
-    prepared = _PREPARED.get(key)
-    if prepared is None:
-        kid = _kernel_id(kernel_type)
-        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-        if len(batch_indices) != len(batch_shape):
-            raise RuntimeError(
-                f"expected {len(batch_shape)} batch index tensors, got {len(batch_indices)}"
-            )
-        for t in (*batch_indices, row_index, col_index):
-            check_cuda_int32(t)
-        if row_index.dim() == 0:  # scalar indices: treat as one entry
-            result = index(kernel_type, x1, x2, params, start, end,
-                           [b.reshape(1) for b in batch_indices], row_index.reshape(1),
-                           col_index.reshape(1))
-            return result.reshape(())
-        shape = tuple(row_index.shape)
-        if len(shape) < 1 or len(shape) > MAX_BATCH_RANK + 1:
-            raise RuntimeError(f"index tensors must have between 1 and {MAX_BATCH_RANK + 1} dimensions")
-        for t in (*batch_indices, col_index):
-            if tuple(t.shape) != shape:
-                raise RuntimeError("all index tensors must have the same shape")
-        rank = len(batch_shape)
-        stride_arrays = [_i64(t.stride()) for t in batch_indices]
-        prepared = _remember(key, (
-            load_library().km_index, (kid, rank, _i64(batch_shape), x1.shape[-1], x2.shape[-1]),
-            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors), shape, _i64(shape), rank,
-            (_i64p * max(rank, 1))(*[ctypes.cast(a, _i64p) for a in stride_arrays]), stride_arrays,
-        ))
-    fn, head, strides, nonempty, shape, sizes, rank, bi_strides, _keep = prepared
-    device = x1.device
-    out = torch.empty(shape, dtype=torch.float32, device=device)
-    call_args = _marshalled(tensors, strides, nonempty)
-    bi_ptrs = (_vp * max(rank, 1))(*[t.data_ptr() for t in batch_indices])
-    with _on_device(device):
-        status = fn(*head, *call_args[:10], len(shape), sizes, bi_ptrs, bi_strides, *call_args[10:],
-                    out.data_ptr() if out.numel() > 0 else None, _stream(device))
+    result = torch_calls().index(KERNEL_TYPES.get(kernel_type), x1, x2, params, start, end, row_index, col_index, batch_indices)
+    if result is not None:
+        return result
+    kid = _kernel_id(kernel_type)
+    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+    if len(batch_indices) != len(batch_shape):
+        raise RuntimeError(
+            f"expected {len(batch_shape)} batch index tensors, got {len(batch_indices)}"
+        )
+    for t in (*batch_indices, row_index, col_index):
+        check_cuda_int32(t)
+    if row_index.dim() == 0:  # scalar indices: treat as one entry
+        result = index(kernel_type, x1, x2, params, start, end,
+                       [b.reshape(1) for b in batch_indices], row_index.reshape(1),
+                       col_index.reshape(1))
+        return result.reshape(())
+    shape = tuple(row_index.shape)
+    if len(shape) < 1 or len(shape) > MAX_BATCH_RANK + 1:
+        raise RuntimeError(f"index tensors must have between 1 and {MAX_BATCH_RANK + 1} dimensions")
+    for t in (*batch_indices, col_index):
+        if tuple(t.shape) != shape:
+            raise RuntimeError("all index tensors must have the same shape")
+    lib = load_library()
+    out = torch.empty(shape, dtype=torch.float32, device=x1.device)
+    bi_ptrs, bi_strides, _keep = _batch_index_args(batch_indices, len(batch_shape))
+    with _on_device(x1.device):
+        status = lib.km_index(kid, len(batch_shape), _i64(batch_shape), x1.shape[-1], x2.shape[-1],
+                              *_tensors_args(x1, x2, params, start, end), len(shape), _i64(shape), bi_ptrs, bi_strides,
+                              *_tensors_args(row_index, col_index), _ptr(out), _stream(x1.device))
     if status != 0:
-        _raise(load_library(), status)
+        _raise(lib, status)
     return out
 
 
@@ -463,9 +442,13 @@ def index_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: T
               batch_indices: Sequence[Tensor], row_index: Tensor, col_index: Tensor,
               out_grad: Tensor) -> Tensor:
     """grad[..., P] of sum(out_grad * index(...)) w.r.t. params   (C ABI: km_index_bwd)."""
+    batch_indices = tuple(batch_indices)
+    result = torch_calls().index_bwd(KERNEL_TYPES.get(kernel_type), x1, x2, params, start, end, row_index, col_index, out_grad,
+                                     batch_indices)
+    if result is not None:
+        return result
     kid = _kernel_id(kernel_type)
     batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-    batch_indices = tuple(batch_indices)
     if len(batch_indices) != len(batch_shape):
         raise RuntimeError(
             f"expected {len(batch_shape)} batch index tensors, got {len(batch_indices)}"
@@ -505,59 +488,48 @@ def index_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: T
 def dense(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tensor,
           end: Tensor) -> Tensor:
     """Masked kernel matrix [..., m, n]   (C ABI: km_dense)."""
-    tensors = (x1, x2, params, start, end)
-    key = _signature("dense", kernel_type, tensors)
-    prepared = _PREPARED.get(key)
-    if prepared is None:
-        kid = _kernel_id(kernel_type)
-        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-        m, n = x1.shape[-1], x2.shape[-1]
-        prepared = _remember(key, (
-            load_library().km_dense, (kid, len(batch_shape), _i64(batch_shape), m, n),
-            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors), (*batch_shape, m, n),
-        ))
-    fn, head, strides, nonempty, out_shape = prepared
+    result = torch_calls().dense(KERNEL_TYPES.get(kernel_type), x1, x2, params, start, end)
+    if result is not None:
+        return result
+    kid = _kernel_id(kernel_type)
+    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+    m, n = x1.shape[-1], x2.shape[-1]
+    lib = load_library()
     device = x1.device
-    out = torch.empty(out_shape, dtype=torch.float32, device=device)
+    out = torch.empty((*batch_shape, m, n), dtype=torch.float32, device=device)
     with _on_device(device):
-        status = fn(*head, *_marshalled(tensors, strides, nonempty), out.data_ptr() if out.numel() > 0 else None,
-                    _stream(device))
+        status = lib.km_dense(kid, len(batch_shape), _i64(batch_shape), m, n, *_tensors_args(x1, x2, params, start, end), _ptr(out),
+                              _stream(device))
     if status != 0:
-        _raise(load_library(), status)
+        _raise(lib, status)
     return out
 
 
 def dense_bwd(kernel_type: str, x1: Tensor, x2: Tensor, params: Tensor, start: Tensor, end: Tensor,
               out_grad: Tensor) -> Tensor:
     """grad[..., P] of sum(out_grad * dense(...)) w.r.t. params   (C ABI: km_dense_bwd)."""
-    tensors = (x1, x2, params, start, end, out_grad)
-    key = _signature("dense_bwd", kernel_type, tensors)
-    prepared = _PREPARED.get(key)
-    if prepared is None:
-        kid = _kernel_id(kernel_type)
-        check_cuda(out_grad)
-        check_float(out_grad)
-        batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
-        _check_batch("out_grad", out_grad, batch_shape, 2)
-        m, n = x1.shape[-1], x2.shape[-1]
-        if tuple(out_grad.shape[-2:]) != (m, n):
-            raise RuntimeError(f"out_grad has shape {tuple(out_grad.shape)}, expected (..., {m}, {n})")
-        lib = load_library()
-        sizes = _i64(batch_shape)
-        prepared = _remember(key, (
-            lib.km_dense_bwd, (kid, len(batch_shape), sizes, m, n),
-            tuple(_i64(t.stride()) for t in tensors), tuple(t.numel() > 0 for t in tensors),
-            (*batch_shape, params.shape[-1]), lib.km_param_grad_workspace_size(kid, len(batch_shape), sizes, m, n, 0),
-        ))
-    fn, head, strides, nonempty, out_shape, need = prepared
+    result = torch_calls().dense_bwd(KERNEL_TYPES.get(kernel_type), x1, x2, params, start, end, out_grad)
+    if result is not None:
+        return result
+    kid = _kernel_id(kernel_type)
+    check_cuda(out_grad)
+    check_float(out_grad)
+    batch_shape = _check_matrix_inputs(kernel_type, x1, x2, params, start, end)
+    _check_batch("out_grad", out_grad, batch_shape, 2)
+    m, n = x1.shape[-1], x2.shape[-1]
+    if tuple(out_grad.shape[-2:]) != (m, n):
+        raise RuntimeError(f"out_grad has shape {tuple(out_grad.shape)}, expected (..., {m}, {n})")
+    lib = load_library()
+    sizes = _i64(batch_shape)
+    need = lib.km_param_grad_workspace_size(kid, len(batch_shape), sizes, m, n, 0)
     device = x1.device
-    grad = torch.empty(out_shape, dtype=torch.float32, device=device)
+    grad = torch.empty((*batch_shape, params.shape[-1]), dtype=torch.float32, device=device)
     workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=device)
     with _on_device(device):
-        status = fn(*head, *_marshalled(tensors, strides, nonempty), grad.data_ptr() if grad.numel() > 0 else None,
-                    workspace.data_ptr(), need, _stream(device))
+        status = lib.km_dense_bwd(kid, len(batch_shape), sizes, m, n, *_tensors_args(x1, x2, params, start, end, out_grad), _ptr(grad),
+                                  workspace.data_ptr(), need, _stream(device))
     if status != 0:
-        _raise(load_library(), status)
+        _raise(lib, status)
     return grad
 
 

@@ -24,7 +24,7 @@ import torch
 import torch.autograd.forward_ad as forward_ad
 from torch import Size, Tensor, dtype
 
-from kernel_matmul_amd import ranges
+from kernel_matmul_amd import _native, ranges
 from kernel_matmul_amd.configurations import (
     BilinearDerivativeConfiguration,
     DenseBwdConfiguration,
@@ -122,19 +122,28 @@ except ImportError:
         return device, dtype_
 
 
-def _plain(differentiable: tuple) -> bool:
-    """Whether nothing records or transforms a call on these tensors, so that the native function can be called
-    itself (an autograd function costs a fifth of a small product's host time)."""
+def _recorded(differentiable: tuple) -> bool:
     if torch.is_grad_enabled():
         for t in differentiable:
             if t.requires_grad:
-                return False
-    return (
+                return True
+    return False
+
+
+def _transformed() -> bool:
+    return not (
         forward_ad._current_level < 0  # (no dual tensors)
         and not torch._C._are_functorch_transforms_active()
         and torch._C._get_tracing_state() is None
         and not torch.compiler.is_compiling()
     )
+
+
+def _plain(differentiable: tuple) -> bool:
+    """Whether nothing records or transforms a call on these tensors, so that the native function can be called
+    itself.  A call that is recorded but not transformed has a native node (csrc/km_torch.cpp); every other one goes
+    through the autograd functions below."""
+    return not _recorded(differentiable) and not _transformed()
 
 
 class _MatmulOperator(torch.autograd.Function):
@@ -278,18 +287,15 @@ class KernelMatmulLinearOperator(LinearOperator):
         if symmetric is None:
             symmetric = torch.equal(x1, x2)
 
+        self._given = (x1, x2, params, start, end)
         shapes = (x1.shape[:-2], x2.shape[:-2], params.shape[:-1], start.shape[:-1], end.shape[:-1])
         distinct = set(shapes) - {Size(())}
         if len(distinct) > 1:
             batch_shape = torch.broadcast_shapes(*shapes)
         else:  # (the usual case, at a tenth of the time)
             batch_shape = distinct.pop() if distinct else Size(())
-        self._x1 = _widen(x1, batch_shape, 2)
-        self._x2 = _widen(x2, batch_shape, 2)
-        self._params = _widen(params, batch_shape, 1)
-        self._start = _widen(start, batch_shape, 1)
-        self._end = _widen(end, batch_shape, 1)
         self._kernel_type = kernel_type
+        self._kernel_number = _native.KERNEL_TYPES.get(kernel_type)
         self._compile_pool = compile_pool
         self._batch_shape = batch_shape
         self._symmetric = symmetric
@@ -298,6 +304,22 @@ class KernelMatmulLinearOperator(LinearOperator):
         self._native_args = None  # (batch shape, widened constructor tensors) of the last call
 
     # -- helpers -------------------------------------------------------------------------
+    # The constructor tensors as stride-0 views of the batch shape.
+    _x1 = property(lambda self: _widen(self._given[0], self._batch_shape, 2))
+    _x2 = property(lambda self: _widen(self._given[1], self._batch_shape, 2))
+    _params = property(lambda self: _widen(self._given[2], self._batch_shape, 1))
+    _start = property(lambda self: _widen(self._given[3], self._batch_shape, 1))
+    _end = property(lambda self: _widen(self._given[4], self._batch_shape, 1))
+
+    def _calls(self, *functions: str):
+        """The native module of calls on tensors, if nothing asks for the native functions of these names: they are
+        the operator's own and nobody has taken them in hand, and their modules would watch no call."""
+        for name in functions:
+            if name in self.__dict__ or getattr(type(self), name) is not KernelMatmulLinearOperator.__dict__[name]:
+                return None
+        calls = _native.torch_calls()
+        return None if calls.watched() else calls
+
     def _get_args_for_native(self, batch_shape) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
         """The constructor tensors as stride-0 views of ``batch_shape``.  The views of the tensors
         that carry no gradient (coordinates and pattern) are kept for the last shape asked for:
@@ -306,15 +328,10 @@ class KernelMatmulLinearOperator(LinearOperator):
         ``inference_mode`` would cut later calls off from the hyper-parameters' gradient)."""
         batch_shape = Size(batch_shape)
         if self._native_args is None or self._native_args[0] != batch_shape:
-            fixed = (
-                _widen(self._x1.detach().squeeze(-1), batch_shape, 1),
-                _widen(self._x2.detach().squeeze(-1), batch_shape, 1),
-                _widen(self._start, batch_shape, 1),
-                _widen(self._end, batch_shape, 1),
-            )
-            self._native_args = (batch_shape, fixed)
+            x1, x2, _, start, end = self._given
+            self._native_args = (batch_shape, _native.torch_calls().views(x1, x2, start, end, tuple(batch_shape)))
         x1, x2, start, end = self._native_args[1]
-        return x1, x2, _widen(self._params, batch_shape, 1), start, end
+        return x1, x2, _widen(self._given[2], batch_shape, 1), start, end
 
     def _transposed_ranges(self, batch_shape=None) -> tuple[Tensor, Tensor]:
         """Pattern of K^T, computed once per operator (the check that the pattern is block
@@ -332,22 +349,31 @@ class KernelMatmulLinearOperator(LinearOperator):
 
     # -- LinearOperator hooks ------------------------------------------------------------
     def _matmul(self, rhs: Tensor) -> Tensor:
-        if rhs.shape[:-2] == self._batch_shape and rhs.size(-2) == self._x2.size(-2):
+        columns = self._given[1].size(-2)
+        if rhs.shape[:-2] == self._batch_shape and rhs.size(-2) == columns:
             batch_shape, rhs_ = self._batch_shape, rhs  # nothing to broadcast
         else:
-            expected = Size((*self._batch_shape, self._x2.size(-2), rhs.size(-1)))
+            expected = Size((*self._batch_shape, columns, rhs.size(-1)))
             broadcast = torch.broadcast_shapes(expected, rhs.shape)
             batch_shape = broadcast[:-2]
             rhs_ = rhs.expand(*broadcast)
         x1, x2, params, start, end = self._get_args_for_native(batch_shape)
-        native = self._native_matmul
         call = (x1, x2, rhs_, params, start, end)
-        if _plain((rhs_, params)):
+        recorded, transformed = _recorded((rhs_, params)), _transformed()
+        # (the transposed pattern of one that is not symmetric is the autograd function's to find)
+        if not transformed and (not recorded or self._symmetric or not rhs_.requires_grad):
+            calls = self._calls("_native_matmul", "_native_matmul_bwd")
+            if calls is not None:
+                out = calls.matmul_recorded(self._kernel_number, *call)
+                if out is not None:
+                    return out
+        native = self._native_matmul
+        if not recorded and not transformed:
             return native(*call)
         return _MatmulOperator.apply(*call, native, self._native_matmul_bwd, self._symmetric, self._transposed_ranges)
 
     def _size(self) -> Size:
-        return Size((*self._batch_shape, self._x1.size(-2), self._x2.size(-2)))
+        return Size((*self._batch_shape, self._given[0].size(-2), self._given[1].size(-2)))
 
     def _transpose_nonbatch(self) -> "KernelMatmulLinearOperator":
         if self._symmetric:
@@ -359,6 +385,12 @@ class KernelMatmulLinearOperator(LinearOperator):
 
     def to_dense(self) -> Tensor:
         call = self._get_args_for_native(self._batch_shape)
+        if not _transformed():
+            calls = self._calls("_native_dense", "_native_dense_bwd")
+            if calls is not None:
+                out = calls.dense_recorded(self._kernel_number, *call)
+                if out is not None:
+                    return out
         if _plain((call[2],)):
             return self._native_dense(*call)
         return _DenseOperator.apply(*call, self._native_dense, self._native_dense_bwd)
@@ -395,7 +427,11 @@ class KernelMatmulLinearOperator(LinearOperator):
         left_vecs = _widen(left_vecs, batch_shape, 2)
         right_vecs = _widen(right_vecs, batch_shape, 2)
         x1, x2, params, start, end = self._get_args_for_native(batch_shape)
-        grad = self._native_bilinear_derivative(x1, x2, left_vecs, right_vecs, params, start, end)
+        call = (x1, x2, left_vecs, right_vecs, params, start, end)
+        calls = self._calls("_native_bilinear_derivative")
+        grad = calls.param_grad(self._kernel_number, *call, None) if calls is not None else None
+        if grad is None:
+            grad = self._native_bilinear_derivative(*call)
         # one entry per constructor tensor: x1, x2, params, start, end
         return None, None, grad, None, None
 
@@ -415,21 +451,27 @@ class KernelMatmulLinearOperator(LinearOperator):
                 batch.append(torch.arange(size, dtype=torch.int32, device=device).view(view).expand(*batch_shape, n))
             self._diagonal_indices = (row, tuple(batch))
         row, batch = self._diagonal_indices
+        return self._entries(batch, row, row)
+
+    def _entries(self, batch: tuple, row: Tensor, col: Tensor) -> Tensor:
         call = self._get_args_for_native(self._batch_shape)
+        if not _transformed():
+            calls = self._calls("_native_index", "_native_index_bwd")
+            if calls is not None:
+                out = calls.index_recorded(self._kernel_number, *call, row, col, batch)
+                if out is not None:
+                    return out
         if _plain((call[2],)):
-            return self._native_index(*call, batch, row, row)
-        return _IndexOperator.apply(*call, self._native_index, self._native_index_bwd, row, row, *batch)
+            return self._native_index(*call, batch, row, col)
+        return _IndexOperator.apply(*call, self._native_index, self._native_index_bwd, row, col, *batch)
 
     def _get_indices(self, row_index: Tensor, col_index: Tensor, *batch_indices: Tensor) -> Tensor:
-        x1, x2, params, start, end = self._get_args_for_native(self._batch_shape)
+        device = self._given[0].device
         shape = torch.broadcast_shapes(
             row_index.shape, col_index.shape, *(b.shape for b in batch_indices)
         )
 
         def prepare(index: Tensor) -> Tensor:
-            return index.expand(*shape).to(device=x1.device, dtype=torch.int32)
+            return index.expand(*shape).to(device=device, dtype=torch.int32)
 
-        return _IndexOperator.apply(
-            x1, x2, params, start, end, self._native_index, self._native_index_bwd,
-            prepare(row_index), prepare(col_index), *(prepare(b) for b in batch_indices),
-        )
+        return self._entries(tuple(prepare(b) for b in batch_indices), prepare(row_index), prepare(col_index))

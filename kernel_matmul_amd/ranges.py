@@ -60,6 +60,10 @@ def make_ranges(
         ``(start, end)``, int32 tensors of shape ``(batch..., ceil(n1 / block_size))`` on
         ``x1``'s device.
     """
+    if check_sorted and x1.is_cuda and isinstance(cutoff, (int, float)):
+        pattern = _native.torch_calls().make_ranges(float(cutoff), x1, x2, block_size, bool(align))
+        if pattern is not None:
+            return pattern
     batch_shape = x1.shape[:-1]
     x1f = _flatten(x1)
     x2f = _flatten(x2) if x2 is not None else None
