@@ -60,13 +60,14 @@ __device__ __forceinline__ DenseView dense_view(const DenseArgs& a, long long it
     return v;
 }
 
-// One workgroup of 256 threads per (row block, column share, batch item): each wavefront writes
-// 32 of the block's rows over the share's columns, lanes run along the columns so that stores are
-// 256 B contiguous.  The column shares only exist to fill the device when row blocks x batch
-// items are few.  A wavefront keeps its 32 row coordinates one per lane and broadcasts them with
-// v_readlane (no load inside the row loop).
-template <int KT>
+// One workgroup of 256 threads per (row block, column share, batch item): each wavefront writes 32 of the block's rows
+// over the share's columns, lanes run along the columns, V of them each, so that stores are 256 V contiguous bytes
+// (V = 4: rows begin at multiples of 16 bytes).  The column shares only exist to fill the device when row blocks x
+// batch items are few.  A wavefront keeps its 32 row coordinates one per lane and broadcasts them with v_readlane (no
+// load inside the row loop).  Bound by the writes; V = 1 -> 4, spectral n = 7200 35.9 -> 31.6 us (6.5 TB/s), n = 20000 334 -> 312.
+template <int KT, int V>
 __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
+    typedef float Vec __attribute__((ext_vector_type(V)));
     const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
     if (item >= a.total_items) {
         return;
@@ -85,33 +86,48 @@ __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
     const KernelConsts kc = make_consts<KT>(v.params, a.params_s, true);
     float* __restrict__ out = a.out + v.b * (long long)a.m * a.n + (long long)row_begin * a.n;
     const int x1_bits = __float_as_int(v.x1[(long long)(row_begin + min(lane, rows - 1)) * a.x1_s]);
-    for (int col0 = col_lo; col0 < col_hi; col0 += 64) {
-        const int col = col0 + lane;
-        const bool in_matrix = col < col_hi;
-        const bool in_range = in_matrix && col >= v.range_start && col < v.range_end;
+    for (int col0 = col_lo; col0 < col_hi; col0 += 64 * V) {
+        const int col = col0 + V * lane;
+        const bool in_matrix = col < col_hi;  // (with all V: their number divides that of the columns)
         float* __restrict__ o = out + col;
         // Wave-uniform choice: column tiles fully outside the range are only cleared.
-        if (col0 < v.range_end && col0 + 64 > v.range_start) {
-            const float x2v = in_range ? v.x2[(long long)col * a.x2_s] : 0.0f;
+        if (col0 < v.range_end && col0 + 64 * V > v.range_start) {
+            float x2v[V];
+            bool in_range[V];
+#pragma unroll
+            for (int t = 0; t < V; t++) {
+                in_range[t] = in_matrix && col + t >= v.range_start && col + t < v.range_end;
+                x2v[t] = in_range[t] ? v.x2[(long long)(col + t) * a.x2_s] : 0.0f;
+            }
             for (int r = 0; r < rows; r++) {
                 const float x1v = __int_as_float(__builtin_amdgcn_readlane(x1_bits, r));
-                const float kv = kernel_value<KT>(x1v, x2v, kc) * kc.sgn;
+                Vec kv;
+#pragma unroll
+                for (int t = 0; t < V; t++) {
+                    const float k = kernel_value<KT>(x1v, x2v[t], kc) * kc.sgn;
+                    kv[t] = in_range[t] ? k : 0.0f;
+                }
                 if (in_matrix) {
-                    o[(long long)r * a.n] = in_range ? kv : 0.0f;
+                    *(Vec*)(o + (long long)r * a.n) = kv;
                 }
             }
         } else if (in_matrix) {
             for (int r = 0; r < rows; r++) {
-                o[(long long)r * a.n] = 0.0f;
+                *(Vec*)(o + (long long)r * a.n) = (Vec)(0.0f);
             }
         }
     }
 }
 
-// One wavefront per (row block, column split, batch item): lanes run along the columns,
-// the 128 rows are walked one by one (x1 is wave-uniform), weights are read 256 B contiguous.
+// One workgroup per (row block, column split, batch item), whose wavefronts take 16 rows each: lanes run along the
+// columns, weights are read 256 B contiguous, all 16 rows' together: narrow ranges are bound by that latency, wide ones by
+// memory.  Against one wavefront for all 128 rows, eight at a time (spectral, a call with its reduction): n = 7200, 290 /
+// 2500 columns a row block 17.0 -> 12.6 / 43.9 -> 24.3 us; n = 20000, all columns 385 -> 311 (5.2 TB/s).
+#define KM_DENSE_BWD_ROWS 16
+#define KM_DENSE_BWD_WAVES (KM_BLOCK_SIZE / KM_DENSE_BWD_ROWS)
 template <int KT>
-__global__ void __launch_bounds__(64) dense_bwd_partial(const DenseArgs a) {
+__global__ void __launch_bounds__(64 * KM_DENSE_BWD_WAVES) dense_bwd_partial(const DenseArgs a) {
+    __shared__ float sums[KM_DENSE_BWD_WAVES][KM_MAX_PARAMS];
     const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
     if (item >= a.total_items) {
         return;
@@ -119,53 +135,62 @@ __global__ void __launch_bounds__(64) dense_bwd_partial(const DenseArgs a) {
     int row_block, split;
     const DenseView v = dense_view(a, item, a.col_splits, &row_block, &split);
     const KernelConsts kc = make_consts<KT>(v.params, a.params_s, false);
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     const int width = max(v.range_end - v.range_start, 0);
     const int per_split = ((width + a.col_splits - 1) / a.col_splits + 63) & ~63;
     const int col_begin = v.range_start + split * per_split;
     const int col_end = min(v.range_end, col_begin + per_split);
-    const int row_begin = row_block * KM_BLOCK_SIZE;
-    const int row_end = min(row_begin + KM_BLOCK_SIZE, a.m);
+    const int row_begin = row_block * KM_BLOCK_SIZE + wave * KM_DENSE_BWD_ROWS;
+    const int rows = min(KM_DENSE_BWD_ROWS, a.m - row_begin);
 
-    // The block's 128 row coordinates, two per lane (rows past the matrix repeat the last one;
-    // their weights are zero).
-    const int x1_lo = __float_as_int(v.x1[(long long)min(row_begin + lane, a.m - 1) * a.x1_s]);
-    const int x1_hi = __float_as_int(v.x1[(long long)min(row_begin + 64 + lane, a.m - 1) * a.x1_s]);
-
+    const long long partial_rows = a.total_items / a.num_batches;
+    float* __restrict__ partial = a.partials + (v.b * partial_rows + v.rest) * KM_MAX_PARAMS;
+    if (col_begin >= col_end) {  // (the same in all wavefronts)
+        if (threadIdx.x < KM_MAX_PARAMS) {
+            partial[threadIdx.x] = 0.0f;
+        }
+        return;
+    }
     float acc[KM_MAX_PARAMS] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int col0 = col_begin; col0 < col_end; col0 += 64) {
-        const int col = col0 + lane;
-        const bool ok = col < col_end;
-        const int colc = min(col, col_end - 1);
-        const float x2v = v.x2[(long long)colc * a.x2_s];
-        const float* __restrict__ wcol = v.weights + (long long)colc * a.weights_s1;
-        // 8 rows at a time: their weights are requested together, their coordinates come from
-        // the lanes that hold them (below) by v_readlane.
-        for (int row0 = row_begin; row0 < row_end; row0 += 8) {
-            float wv[8];
+    if (rows > 0) {
+        // The row coordinates one per lane, to be read from there (rows past the matrix repeat the last one; their
+        // weights are zero).
+        const int x1_bits = __float_as_int(v.x1[(long long)(row_begin + min(lane, rows - 1)) * a.x1_s]);
+        for (int col0 = col_begin; col0 < col_end; col0 += 64) {
+            const int col = col0 + lane;
+            const bool ok = col < col_end;
+            const int colc = min(col, col_end - 1);
+            const float x2v = v.x2[(long long)colc * a.x2_s];
+            const float* __restrict__ w = v.weights + (long long)row_begin * a.weights_s0 + (long long)colc * a.weights_s1;
+            float wv[KM_DENSE_BWD_ROWS];
 #pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const int row = row0 + t;
-                wv[t] = (ok && row < row_end) ? wcol[(long long)row * a.weights_s0] : 0.0f;
+            for (int t = 0; t < KM_DENSE_BWD_ROWS; t++) {
+                wv[t] = w[(long long)min(t, rows - 1) * a.weights_s0];
             }
-            const int x1_bits = row0 - row_begin < 64 ? x1_lo : x1_hi;
-            const int first = (row0 - row_begin) & 63;
 #pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const float x1v = __int_as_float(__builtin_amdgcn_readlane(x1_bits, first + t));
-                accumulate_pair<KT>(x1v, x2v, wv[t], kc, acc);
+            for (int t = 0; t < KM_DENSE_BWD_ROWS; t++) {
+                const float x1v = __int_as_float(__builtin_amdgcn_readlane(x1_bits, t));
+                accumulate_pair<KT>(x1v, x2v, ok && t < rows ? wv[t] : 0.0f, kc, acc);
             }
         }
     }
-    const long long partial_rows = a.total_items / a.num_batches;
-    float* __restrict__ prow = a.partials + (v.b * partial_rows + v.rest) * KM_MAX_PARAMS;
 #pragma unroll
     for (int p = 0; p < KM_MAX_PARAMS; p++) {
         const float total = wave_sum(acc[p]);
         if (lane == 0) {
-            prow[p] = total;
+            sums[wave][p] = total;
         }
+    }
+    __syncthreads();
+    if (threadIdx.x < KM_MAX_PARAMS) {
+        float total = sums[0][threadIdx.x];
+#pragma unroll
+        for (int i = 1; i < KM_DENSE_BWD_WAVES; i++) {
+            total += sums[i][threadIdx.x];
+        }
+        partial[threadIdx.x] = total;
     }
 }
 
@@ -191,6 +216,22 @@ static void fill_common(DenseArgs& a, const DenseProblem& p) {
     a.weights_s1 = p.weights ? p.weights_strides[r + 1] : 0;
 }
 
+template <int V>
+static void launch_dense_as(int kernel_type, const DenseArgs& a, hipStream_t stream) {
+    const unsigned grid = (unsigned)(a.items_per_xcd * KM_NUM_XCD);
+    switch (kernel_type) {
+        case KM_KERNEL_RBF:
+            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_RBF, V>), dim3(grid), dim3(256), 0, stream, a);
+            break;
+        case KM_KERNEL_SPECTRAL:
+            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_SPECTRAL, V>), dim3(grid), dim3(256), 0, stream, a);
+            break;
+        default:
+            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_LOCALLY_PERIODIC, V>), dim3(grid), dim3(256), 0, stream, a);
+            break;
+    }
+}
+
 hipError_t launch_dense(const DenseProblem& p, hipStream_t stream) {
     DenseArgs a;
     const int64_t* const strides[5] = {p.x1_strides, p.x2_strides, p.params_strides,
@@ -212,17 +253,10 @@ hipError_t launch_dense(const DenseProblem& p, hipStream_t stream) {
     if (a.col_splits < 1) a.col_splits = 1;
     a.total_items = row_blocks * a.col_splits * p.num_batches;
     a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    const unsigned grid = (unsigned)(a.items_per_xcd * KM_NUM_XCD);
-    switch (p.kernel_type) {
-        case KM_KERNEL_RBF:
-            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_RBF>), dim3(grid), dim3(256), 0, stream, a);
-            break;
-        case KM_KERNEL_SPECTRAL:
-            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_SPECTRAL>), dim3(grid), dim3(256), 0, stream, a);
-            break;
-        default:
-            hipLaunchKernelGGL((dense_kernel<KM_KERNEL_LOCALLY_PERIODIC>), dim3(grid), dim3(256), 0, stream, a);
-            break;
+    if (p.n % 4 == 0 && (uintptr_t)p.out % 16 == 0) {
+        launch_dense_as<4>(p.kernel_type, a, stream);
+    } else {
+        launch_dense_as<1>(p.kernel_type, a, stream);
     }
     return hipGetLastError();
 }
@@ -236,6 +270,10 @@ hipError_t launch_dense_bwd(const DenseProblem& p, hipStream_t stream) {
     fill_common(a, p);
     const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     a.col_splits = (int)(param_grad_partials_per_batch(p.m, p.num_batches) / (row_blocks > 0 ? row_blocks : 1));
+    // (a share has eight wavefronts here: four workgroups a CU, no more, of which narrow ranges leave most without columns.
+    // n = 12000, 230 columns a row block, 2 sets: 24 us with sixteen shares, 20 with six)
+    const long long shares = row_blocks * p.num_batches > 0 ? (1024 + row_blocks * p.num_batches - 1) / (row_blocks * p.num_batches) : 1;
+    if (a.col_splits > shares) a.col_splits = (int)shares;
     if (a.col_splits < 1) a.col_splits = 1;
     a.total_items = row_blocks * a.col_splits * p.num_batches;
     a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
@@ -243,13 +281,13 @@ hipError_t launch_dense_bwd(const DenseProblem& p, hipStream_t stream) {
     if (grid > 0) {
         switch (p.kernel_type) {
             case KM_KERNEL_RBF:
-                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_RBF>), dim3(grid), dim3(64), 0, stream, a);
+                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_RBF>), dim3(grid), dim3(64 * KM_DENSE_BWD_WAVES), 0, stream, a);
                 break;
             case KM_KERNEL_SPECTRAL:
-                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_SPECTRAL>), dim3(grid), dim3(64), 0, stream, a);
+                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_SPECTRAL>), dim3(grid), dim3(64 * KM_DENSE_BWD_WAVES), 0, stream, a);
                 break;
             default:
-                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_LOCALLY_PERIODIC>), dim3(grid), dim3(64), 0, stream, a);
+                hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_LOCALLY_PERIODIC>), dim3(grid), dim3(64 * KM_DENSE_BWD_WAVES), 0, stream, a);
                 break;
         }
         hipError_t err = hipGetLastError();

@@ -1,0 +1,61 @@
+"""Dense matrices and their gradient at the edges of what a wavefront writes and reads: whole and ragged groups of four
+columns, shares and row groups, ranges that end inside of them, weights in any layout.
+
+The matrix against float64 closed forms: an exponent u^2 of up to 95 (lengthscales from 0.7 on, distances up to 8) and a phase
+of up to 14 turns, two roundings (2^-24 of either) each.  The gradient: the same for each term, relative to the largest, of
+which roundings of random signs add up."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from kernel_matmul_amd import _native
+from oracle import kernels as oracle
+
+pytestmark = pytest.mark.gpu
+
+DEVICE = torch.device("cuda:0")
+RELATIVE = 2.0 ** -23 * (95 * math.log(2) + 2 * math.pi * 14)
+COLUMNS = {"rbf": 2, "spectral": 3, "locally_periodic": 4}
+
+
+def _inputs(kernel, batch, m, n, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    x1 = torch.sort(torch.rand(batch, m, generator=g) * 8)[0]
+    x2 = torch.sort(torch.rand(batch, n, generator=g) * 8)[0]
+    params = 0.7 + torch.rand(batch, COLUMNS[kernel], generator=g)
+    blocks = -(-m // 128)
+    start = (torch.arange(batch * blocks).view(batch, blocks) * 37 % max(n // 2, 1)).int()
+    end = (start + n // 3 + 1 + 5 * torch.arange(blocks)).clamp(max=n).int()
+    end[:, -1] = n
+    if blocks > 2:
+        end[:, 1] = start[:, 1]
+    return x1, x2, params, start, end
+
+
+@pytest.mark.parametrize("kernel", ["rbf", "spectral", "locally_periodic"])
+@pytest.mark.parametrize("batch,m,n", [
+    (1, 1, 1), (1, 15, 4), (2, 16, 5), (1, 17, 252), (3, 31, 255), (1, 33, 256), (2, 127, 257), (1, 129, 260), (1, 300, 515),
+    (1, 385, 1028), (9, 130, 64), (40, 260, 68),
+])
+def test_tiles(kernel, batch, m, n):
+    args = _inputs(kernel, batch, m, n)
+    on = [t.to(DEVICE) for t in args]
+    dense = _native.dense(kernel, *on).cpu().double().numpy()
+    mine = np.stack([oracle.dense(kernel, *(t[b].numpy() for t in args)) for b in range(batch)])
+    assert ((dense == 0) >= (mine == 0)).all()
+    np.testing.assert_allclose(dense, mine, rtol=RELATIVE, atol=2 * RELATIVE)
+    g = torch.Generator().manual_seed(5)
+    weights = torch.randn(batch, m, n, generator=g)
+    gapped = torch.full((batch, 2 * m, 3 * n), float("nan"))
+    gapped[:, ::2, ::3] = weights
+    grads = [_native.dense_bwd(kernel, *on, w) for w in (
+        weights.to(DEVICE), weights.mT.contiguous().to(DEVICE).mT, gapped.to(DEVICE)[:, ::2, ::3])]
+    assert torch.equal(grads[0], grads[1]) and torch.equal(grads[0], grads[2])
+    for b in range(batch):
+        x1, x2, p, start, end = (t[b].numpy() for t in args)
+        terms = oracle.kernel_matrix_grad(kernel, x1, x2, p) * oracle.range_mask(start, end, m, n) * weights[b].double().numpy()
+        size = abs(terms).max(axis=(1, 2)) * np.count_nonzero(terms, axis=(1, 2)) ** 0.5  # (of a sum of random signs)
+        difference = abs(grads[0][b].cpu().double().numpy() - terms.sum(axis=(1, 2)))
+        assert (difference <= RELATIVE * size + 1e-12).all()
