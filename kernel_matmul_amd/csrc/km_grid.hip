@@ -346,6 +346,9 @@ __device__ __forceinline__ bool grid_forward(const FwdArgs& a, float* lds, const
 // 30.4 -> 25.2.  Where one or two wavefronts spill (3 to 30 registers, most of them in front of this path's loops) the
 // rows' share of the result is written to and read from scratch memory, a tenth to a quarter of it again: n = 1e6, 8 sets at
 // 3 points per unit spectral k = 32 1024 us a call with 22 spilled, 998 with 16; rbf k = 32 741 with 25, 712 with 19.
+// W > 1: synchronises the workgroup.  What bounds it then are round trips to memory, one after the other: the range's rhs
+// values looked at by each wavefront, and 128 instead of 256 columns tabulated at a time, took rbf 9973 rows with 840
+// columns each, k = 3, 4 sets 25.8 us instead of 20.7, n = 50000 at one point per unit, k = 8, 2 sets 13.8 instead of 12.5.
 template <int KT, int G, int W>
 __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, const WaveView& w, int row0, int kbase,
                                                int wave, const GridWindow& gw, const KernelConsts& kc) {
@@ -353,6 +356,7 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
     constexpr int GE = G * PARTS;
     constexpr int R = W == 1 ? 4 : 8 / W;
     constexpr int PIECES = 8 / (W * R);
+    static_assert(W == 1 || PIECES == 1, "one barrier");
     const int li = threadIdx.x & 15;
     GridWindow rows = gw;
     if (!is_finite(rows.x_ref)) {
@@ -362,8 +366,10 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         rows.x_ref = uniform(in_a != 0 ? __shfl(block.xa, __builtin_ctzll(in_a), 64)
                                        : (in_b != 0 ? __shfl(block.xb, __builtin_ctzll(in_b), 64) : 0.0f));
     }
-    // The rhs values of the whole range, once for all rows.
+    // The rhs values of the whole range, once for all rows: several wavefronts share its steps out and hand what they
+    // find on behind their rows.
     int rhs_shift[G];
+    unsigned* const flags = (unsigned*)(lds + grid_lds_floats<GE, GridShape<KT, G>::MT, W>() - W * (GE + 1));
     {
         float rhs_scale[G];
 #pragma unroll
@@ -371,10 +377,19 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
             rhs_shift[g] = 0;
             rhs_scale[g] = 0.0f;
         }
-        const int width = w.range_end - w.range_start;
-        const int steps = width > 0 ? (width - 1) / 32 + 1 : 0;
-        look_at_steps<G>(vectors(a), w, kbase, w.range_start, 32, {steps < 64 ? (1ull << steps) - 1 : ~0ull, 64, steps},
+        const int width = w.range_end - w.range_start - 32 * wave;
+        const int steps = width > 0 ? (width - 1) / (32 * W) + 1 : 0;
+        look_at_steps<G>(vectors(a), w, kbase, w.range_start + 32 * wave, 32 * W, {steps < 64 ? (1ull << steps) - 1 : ~0ull, 64, steps},
                          rhs_lane<G>(vectors(a), kbase), rhs_shift, rhs_scale);
+        if (W > 1) {
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const unsigned found = (unsigned)__ballot(rhs_shift[g] == KM_GRID_NOT_FINITE) & 0xffff;
+                if ((threadIdx.x & 63) == 0) {
+                    flags[wave * G + g] = found;
+                }
+            }
+        }
     }
 #pragma unroll 1
     for (int piece = 0; piece < PIECES; piece++) {
@@ -401,7 +416,7 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         rows.reach = uniform(KM_GRID_REACH / kc.s);
         rows.col_lo = uniform(finite ? lo - rows.reach : -__builtin_inff());
         rows.col_hi = uniform(finite ? hi + rows.reach : __builtin_inff());
-        constexpr int CHUNK = G == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
+        constexpr int CHUNK = G == 1 && W == 1 ? KM_GRID_CHUNK_ONE : KM_GRID_CHUNK;
         float xv[CHUNK / 64];
         if (w.range_start < w.range_end) {
             grid_load(w.x2, f.x2_s, w.range_start, 1, w.range_end, xv);
@@ -410,6 +425,16 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
         float4v acc[R][GE];
         const bool fine = grid_columns<false, KT, G, R, 1, false, false, CHUNK>(vectors(f), lds + wave * KM_GRID_TABLE_FLOATS, w, kbase, 0, rows, kc, xr,
                                                            R, xv, shift, acc);
+        if (W > 1) {
+            __syncthreads();
+#pragma unroll
+            for (int v = 0; v < W; v++) {
+#pragma unroll
+                for (int g = 0; g < G; g++) {
+                    rhs_shift[g] = (flags[v * G + g] >> li & 1) != 0 ? KM_GRID_NOT_FINITE : rhs_shift[g];
+                }
+            }
+        }
         const float sigma = w.params[KernelTraits<KT>::SIGMA * f.params_s];
         float down[GE];
 #pragma unroll
