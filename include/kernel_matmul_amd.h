@@ -128,6 +128,11 @@ int km_make_ranges_symmetric_device(const float* x, int64_t num_batch, int64_t n
 int km_check_sorted_device(const float* x1, int64_t num_batch1, int64_t n1, const float* x2,
                            int64_t num_batch2, int64_t n2, int32_t* descents, void* stream);
 
+/* km_make_ranges_device and km_check_sorted_device of x1[num_batch][n1] and x2[num_batch][n2] together; where a word of
+ * `descents` is not zero, the pattern is meaningless. */
+int km_make_ranges_checked_device(const float* x1, const float* x2, int64_t num_batch, int64_t n1, int64_t n2, float cutoff,
+                                  int block_size, int align, int32_t* start, int32_t* end, int32_t* descents, void* stream);
+
 /* ------------------------------------------------------------------------------------
  * matmul.  out[b,i,c] = sum_{j in [start[b,i/128], end[b,i/128])} k(x1[b,i], x2[b,j]) rhs[b,j,c]
  * Replaces `call` of module km___matmul___* (native/matmul/matmul.cpp:6-17,

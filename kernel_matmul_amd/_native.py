@@ -79,6 +79,8 @@ def load_library():
     lib.km_make_ranges_device.argtypes = lib.km_make_ranges.argtypes + [_vp]
     lib.km_make_ranges_symmetric_device.restype = ctypes.c_int
     lib.km_make_ranges_symmetric_device.argtypes = lib.km_make_ranges_symmetric.argtypes + [_vp]
+    lib.km_make_ranges_checked_device.restype = ctypes.c_int
+    lib.km_make_ranges_checked_device.argtypes = lib.km_make_ranges.argtypes + [i32p, _vp]
     lib.km_check_sorted_device.restype = ctypes.c_int
     lib.km_check_sorted_device.argtypes = [f32p, ctypes.c_int64, ctypes.c_int64, f32p, ctypes.c_int64,
                                            ctypes.c_int64, i32p, _vp]

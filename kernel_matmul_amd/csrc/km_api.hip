@@ -504,6 +504,22 @@ int km_make_ranges_device(const float* x1, const float* x2, int64_t num_batch, i
     return err == hipSuccess ? KM_OK : fail_hip(op, err);
 }
 
+int km_make_ranges_checked_device(const float* x1, const float* x2, int64_t num_batch, int64_t n1, int64_t n2, float cutoff,
+                                  int block_size, int align, int32_t* start, int32_t* end, int32_t* descents, void* stream) {
+    const char* op = "km_make_ranges_checked_device";
+    if (int rc = check_ranges(op, num_batch, n1, n2, block_size)) return rc;
+    KM_REQUIRE_PTR(op, descents);
+    if (num_batch > 0 && n1 > 0) {
+        KM_REQUIRE_PTR(op, x1);
+        KM_REQUIRE_PTR(op, start);
+        KM_REQUIRE_PTR(op, end);
+    }
+    if (num_batch > 0 && n2 > 0) KM_REQUIRE_PTR(op, x2);
+    hipError_t err = launch_make_ranges_checked(x1, x2, num_batch, n1, n2, cutoff, block_size, align, start, end, descents,
+                                                (hipStream_t)stream);
+    return err == hipSuccess ? KM_OK : fail_hip(op, err);
+}
+
 int km_make_ranges_symmetric_device(const float* x, int64_t num_batch, int64_t n, float cutoff,
                                     int block_size, int32_t* start, int32_t* end, void* stream) {
     const char* op = "km_make_ranges_symmetric_device";

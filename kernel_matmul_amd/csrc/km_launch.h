@@ -168,6 +168,9 @@ hipError_t launch_param_grad_reduce(int kernel_type, const BatchShape& batch, lo
 hipError_t launch_make_ranges(const float* x1, const float* x2, int64_t num_batch, int64_t n1,
                               int64_t n2, float cutoff, int block_size, int align, int32_t* start,
                               int32_t* end, hipStream_t stream);
+hipError_t launch_make_ranges_checked(const float* x1, const float* x2, int64_t num_batch, int64_t n1, int64_t n2, float cutoff,
+                                      int block_size, int align, int32_t* start, int32_t* end, int32_t* descents,
+                                      hipStream_t stream);
 hipError_t launch_check_sorted(const float* x1, int64_t num_batch1, int64_t n1, const float* x2, int64_t num_batch2,
                                int64_t n2, int32_t* descents, hipStream_t stream);
 hipError_t launch_make_ranges_symmetric(const float* x, int64_t num_batch, int64_t n, float cutoff,

@@ -131,6 +131,59 @@ struct RangeArgs {
     int* end;
 };
 
+// Row blocks up to which a wavefront searches for each.
+#define KM_RANGES_BY_WAVES 16384
+
+// The range of row block t, by a wavefront: both ends are first positions of the scan grid at which a condition holds (it
+// holds behind them too), and 64 positions of what is left are tried at a time: three trips to memory for 50000 columns
+// where halving takes sixteen for each end.  (Ends on any data: what is left shrinks.)
+__device__ __forceinline__ void wave_range(const RangeArgs& a, long long t) {
+    const int lane = threadIdx.x & 63;
+    const long long b = t / a.rows;
+    const long long i = t % a.rows;
+    const float* __restrict__ x1 = a.x1 + b * a.n1;
+    const float* __restrict__ x2 = a.x2 + b * a.n2;
+    const float first = x1[i * a.bs];
+    const float last = x1[min(i * a.bs + a.bs, a.n1) - 1];
+    const long long grid = (a.n2 + a.step - 1) / a.step;
+    long long lo[2] = {0, 0}, hi[2] = {grid, grid};
+    while (lo[0] < hi[0] || lo[1] < hi[1]) {
+        float x[2];
+        long long every[2], at[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            every[e] = (hi[e] - lo[e] + 63) / 64;
+            at[e] = lo[e] + lane * every[e];
+            x[e] = x2[min(max(min(at[e], hi[e] - 1), 0LL) * a.step, a.n2 - 1)];
+        }
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            if (lo[e] >= hi[e]) {
+                continue;
+            }
+            // start: first - x2[j] <= cutoff; end: x2[j] - last > cutoff
+            const bool holds = e == 0 ? first - x[e] <= a.cutoff : x[e] - last > a.cutoff;
+            const unsigned long long tried = __ballot(at[e] < hi[e]), found = __ballot(at[e] < hi[e] && holds);
+            const int place = found != 0 ? __builtin_ctzll(found) : 64 - __builtin_clzll(tried);
+            const long long from = lo[e];
+            hi[e] = found != 0 ? from + place * every[e] : hi[e];
+            lo[e] = place > 0 ? min(from + (place - 1) * every[e] + 1, hi[e]) : from;
+        }
+    }
+    if (lane == 0) {
+        const long long f = min(lo[0] * a.step, a.n2);
+        a.start[t] = (int)f;
+        a.end[t] = (int)max(f, min(lo[1] * a.step, a.n2));
+    }
+}
+
+__global__ void __launch_bounds__(256) ranges_asym_waves(const RangeArgs a) {
+    const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t < a.num_batch * a.rows) {
+        wave_range(a, t);
+    }
+}
+
 __global__ void __launch_bounds__(256) ranges_asym_kernel(const RangeArgs a) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.num_batch * a.rows) {
@@ -230,9 +283,8 @@ __global__ void __launch_bounds__(256) ranges_sym_start_kernel(const RangeArgs a
     a.start[t] = value;
 }
 
-hipError_t launch_make_ranges(const float* x1, const float* x2, int64_t num_batch, int64_t n1,
-                              int64_t n2, float cutoff, int block_size, int align, int32_t* start,
-                              int32_t* end, hipStream_t stream) {
+static RangeArgs range_args(const float* x1, const float* x2, int64_t num_batch, int64_t n1, int64_t n2, float cutoff,
+                            int block_size, int align, int32_t* start, int32_t* end) {
     RangeArgs a;
     a.x1 = x1;
     a.x2 = x2;
@@ -245,12 +297,24 @@ hipError_t launch_make_ranges(const float* x1, const float* x2, int64_t num_batc
     a.step = align ? block_size : 1;
     a.start = start;
     a.end = end;
+    return a;
+}
+
+// One wavefront per row block while the device holds them about at once, else one thread (which reads a sixty-fourth).
+hipError_t launch_make_ranges(const float* x1, const float* x2, int64_t num_batch, int64_t n1,
+                              int64_t n2, float cutoff, int block_size, int align, int32_t* start,
+                              int32_t* end, hipStream_t stream) {
+    const RangeArgs a = range_args(x1, x2, num_batch, n1, n2, cutoff, block_size, align, start, end);
     const long long total = a.num_batch * a.rows;
     if (total == 0) {
         return hipSuccess;
     }
-    hipLaunchKernelGGL(ranges_asym_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                       stream, a);
+    if (total <= KM_RANGES_BY_WAVES && n2 > 0) {
+        hipLaunchKernelGGL(ranges_asym_waves, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL(ranges_asym_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
+                           stream, a);
+    }
     return hipGetLastError();
 }
 
@@ -287,9 +351,9 @@ hipError_t launch_make_ranges_symmetric(const float* x, int64_t num_batch, int64
 // a word of its own, so that nothing has to be cleared first and the host reads one short array.  Bound
 // by latency.  Two arrays of 50000 and 9973 values, pattern and product: 133 -> 98 us a call against a
 // comparison, a reduction and a wait per array.
-__global__ void __launch_bounds__(1024) check_sorted_kernel(const float* __restrict__ x1, long long num1, long long n1,
-                                                            const float* __restrict__ x2, long long num2, long long n2,
-                                                            int* __restrict__ descents) {
+__device__ __forceinline__ void check_stripes(const float* __restrict__ x1, long long num1, long long n1,
+                                              const float* __restrict__ x2, long long num2, long long n2,
+                                              int* __restrict__ descents) {
     const long long first = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long step = (long long)gridDim.x * blockDim.x;
     bool descends = false;
@@ -315,6 +379,22 @@ __global__ void __launch_bounds__(1024) check_sorted_kernel(const float* __restr
     }
 }
 
+__global__ void __launch_bounds__(1024) check_sorted_kernel(const float* __restrict__ x1, long long num1, long long n1,
+                                                            const float* __restrict__ x2, long long num2, long long n2,
+                                                            int* __restrict__ descents) {
+    check_stripes(x1, num1, n1, x2, num2, n2, descents);
+}
+
+// The check and the builder's wavefronts in one launch (9973 against 50000 points: two launches of 4.3 and 6.4 us, the
+// second with one thread a row block, before).
+__global__ void __launch_bounds__(1024) ranges_checked_kernel(const RangeArgs a, int* __restrict__ descents) {
+    const long long waves = (long long)gridDim.x * (1024 / 64);
+    for (long long t = (long long)blockIdx.x * (1024 / 64) + (threadIdx.x >> 6); t < a.num_batch * a.rows; t += waves) {
+        wave_range(a, t);
+    }
+    check_stripes(a.x1, a.n1 > 1 ? a.num_batch : 0, a.n1, a.x2, a.n2 > 1 ? a.num_batch : 0, a.n2, descents);
+}
+
 hipError_t launch_check_sorted(const float* x1, int64_t num_batch1, int64_t n1, const float* x2, int64_t num_batch2,
                                int64_t n2, int32_t* descents, hipStream_t stream) {
     // (no rows, or rows of one value: nothing to compare)
@@ -323,6 +403,18 @@ hipError_t launch_check_sorted(const float* x1, int64_t num_batch1, int64_t n1, 
     hipLaunchKernelGGL(check_sorted_kernel, dim3(KM_SORTED_FLAGS), dim3(1024), 0, stream, x1, num1, (long long)n1, x2, num2,
                        (long long)n2, descents);
     return hipGetLastError();
+}
+
+hipError_t launch_make_ranges_checked(const float* x1, const float* x2, int64_t num_batch, int64_t n1, int64_t n2, float cutoff,
+                                      int block_size, int align, int32_t* start, int32_t* end, int32_t* descents,
+                                      hipStream_t stream) {
+    const RangeArgs a = range_args(x1, x2, num_batch, n1, n2, cutoff, block_size, align, start, end);
+    if (a.num_batch * a.rows <= KM_RANGES_BY_WAVES && n2 > 0) {
+        hipLaunchKernelGGL(ranges_checked_kernel, dim3(KM_SORTED_FLAGS), dim3(1024), 0, stream, a, descents);
+        return hipGetLastError();
+    }
+    const hipError_t err = launch_check_sorted(x1, num_batch, n1, x2, num_batch, n2, descents, stream);
+    return err != hipSuccess ? err : launch_make_ranges(x1, x2, num_batch, n1, n2, cutoff, block_size, align, start, end, stream);
 }
 
 }  // namespace km

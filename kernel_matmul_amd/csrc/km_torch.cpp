@@ -517,8 +517,8 @@ PyObject* py_views(PyObject*, PyObject* const* args, Py_ssize_t count) {
 }
 
 // make_ranges(cutoff, x1, x2 or None, block size, align) -> (start, end) of contiguous float32 device tensors [n] or
-// [batch, n] that ascend; None for all others.  Check and builder are enqueued together; the check's words are written to
-// host memory, and one wait covers both.
+// [batch, n] that ascend; None for all others.  The check's words are written to host memory, and one wait covers check
+// and builder.
 PyObject* py_make_ranges(PyObject*, PyObject* const* args, Py_ssize_t count) {
     HANDLE_TH_ERRORS
     if (count != 5 || !PyFloat_Check(args[0]) || !THPVariable_Check(args[1]) || !PyLong_Check(args[3]) || !PyBool_Check(args[4])) {
@@ -549,12 +549,14 @@ PyObject* py_make_ranges(PyObject*, PyObject* const* args, Py_ssize_t count) {
         Tensor words = at::empty({KM_SORTED_FLAGS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
         int32_t* descents = static_cast<int32_t*>(words.data_ptr());
         Launch on(x1.device());
-        check(km_check_sorted_device(data<float>(x1), batch, n1, symmetric ? nullptr : data<float>(x2), symmetric ? 0 : batch,
-                                     symmetric ? 0 : n2, descents, on.stream()));
         int32_t *s = static_cast<int32_t*>(start.data_ptr()), *e = static_cast<int32_t*>(end.data_ptr());
-        check(symmetric ? km_make_ranges_symmetric_device(data<float>(x1), batch, n1, cutoff, (int)block, s, e, on.stream())
-                        : km_make_ranges_device(data<float>(x1), data<float>(x2), batch, n1, n2, cutoff, (int)block, align, s, e,
-                                                on.stream()));
+        if (symmetric) {
+            check(km_check_sorted_device(data<float>(x1), batch, n1, nullptr, 0, 0, descents, on.stream()));
+            check(km_make_ranges_symmetric_device(data<float>(x1), batch, n1, cutoff, (int)block, s, e, on.stream()));
+        } else {
+            check(km_make_ranges_checked_device(data<float>(x1), data<float>(x2), batch, n1, n2, cutoff, (int)block, align, s, e,
+                                                descents, on.stream()));
+        }
         const hipError_t error = hipStreamSynchronize(static_cast<hipStream_t>(on.stream()));
         TORCH_CHECK(error == hipSuccess, "make_ranges: ", hipGetErrorString(error));
         for (int i = 0; i < KM_SORTED_FLAGS; i++) {

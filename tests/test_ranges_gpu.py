@@ -81,3 +81,17 @@ def test_unsorted_device_input_with_check(symmetric):
     a = make_ranges(1.0, xs.cuda())
     b = make_ranges(1.0, xs.cuda(), check_sorted=False)
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("n2", [1, 2, 63, 64, 65, 127, 4095, 4096, 4097, 70_001])
+@pytest.mark.parametrize("n1,block_size", [(1, 128), (129, 128), (4000, 1), (20_000, 1), (70_000, 3)])
+@pytest.mark.parametrize("align", [False, True])
+def test_searches_by_wavefronts_and_by_threads(n2, n1, block_size, align):
+    """On both sides of the number of row blocks up to which a wavefront searches for each, with and without the check."""
+    x1, x2 = _sorted(n1, scale=50.0), torch.sort((torch.rand(n2) * 200).round() / 4)[0]
+    for cutoff in (0.0, 0.75, 60.0):
+        s_ref, e_ref = oracle_ranges.make_ranges(cutoff, x1.numpy(), x2.numpy(), block_size=block_size, align=align)
+        for check in (True, False):
+            start, end = make_ranges(cutoff, x1.cuda(), x2.cuda(), block_size=block_size, align=align, check_sorted=check)
+            np.testing.assert_array_equal(start.cpu().numpy(), s_ref)
+            np.testing.assert_array_equal(end.cpu().numpy(), e_ref)
