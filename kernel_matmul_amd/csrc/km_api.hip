@@ -180,6 +180,42 @@ static bool periodic_plan(const MatmulProblem& p, const km_launch_options* opt, 
     return true;
 }
 
+// fp32 contraction without a decomposition asked for (fwd_grid_f32 of km_grid_f32.hip): wavefronts of a row block, more of them
+// where there are few items.  Measured, 1 / 2 / 4 / 8 against the kernels below, k = 16, cutoff of 6 lengthscales, us a call:
+// spectral 160 items at 10 points per unit 32 / 20 / 13.3 / 12.5 against 13.2, 314 items 34 / 26 / 17.2 / 22 against 20.1,
+// 1564 items 47 / 44 / 41 / 67 against 61, 3128 items 74 / 67 / 71 / 128 against 118, 6256 items 117 / 117 / 129 / 238 against 177; rbf
+// 314 items 26 / 20 / 13.5 / 17 against 18.1, 6256 items 80 / 83 / 94 / 173 against 146.  Below 120 items the smaller pieces of
+// those spread further (spectral 40 items 11.4 with 8 wavefronts against 7.3).  With four operand groups (spectral, more than
+// 16 columns) the sums of eight wavefronts do not fit into LDS and two wavefronts are resident where the others have three:
+// 314 items - / - / 31 against 27, 628 items 48 / 40 / 44 against 54, 3128 items 118 / 138 / 177 against 170.
+// Locally periodic, 2 / 4 / 8: 160 items 33 / 20.5 / 16.4 against 25.6, 1564 items 60 / 58 / 81 against 102, 6256 items
+// 169 / 173 / 285 against 246; one wavefront alone (180) adds up more products in a row than those did, and rounds more.
+static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
+    if (opt->rows_per_wave != 0 || opt->col_splits != 0 || opt->reserved != 0) {
+        return false;
+    }
+    const bool spectral = p.kernel_type == KM_KERNEL_SPECTRAL;
+    const int k_chunk = p.k <= 16 ? 16 : 32;
+    const long long items = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * p.num_batches * ((p.k + k_chunk - 1) / k_chunk);
+    const bool two_resident = spectral && k_chunk == 32;
+    if (items < (two_resident ? 400 : 120)) {
+        return false;
+    }
+    plan->variant = KM_VARIANT_GRID_F32;
+    plan->k_chunk = k_chunk;
+    plan->row_groups = 8;
+    plan->tail_balance = 0;
+    plan->group_tail_halves = 0;
+    if (two_resident) {
+        plan->col_splits = items < 700 ? 4 : 1;
+    } else if (p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
+        plan->col_splits = items < 250 ? 8 : (items < 5000 ? 4 : 2);
+    } else {
+        plan->col_splits = items < 250 ? 8 : (items < 2000 ? 4 : (items < 5000 ? 2 : 1));
+    }
+    return true;
+}
+
 static int make_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
     int variant = opt ? opt->variant : KM_VARIANT_AUTO;
     plan->phase_split = 0;
@@ -206,6 +242,9 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
         return KM_OK;
     }
     if (variant == KM_VARIANT_AUTO && periodic_plan(p, opt, plan)) {
+        return KM_OK;
+    }
+    if (variant == KM_VARIANT_MFMA_F32 && grid_f32_plan(p, opt, plan)) {
         return KM_OK;
     }
     if (variant == KM_VARIANT_AUTO) {
@@ -674,6 +713,10 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
         case KM_VARIANT_PERIODIC:
             snprintf(text, text_bytes, "km::fwd_block<%s, G=%d, R=%d, W=%d>: tabulated phases, %d wavefront(s) per %d rows", kt, G,
                      plan.row_groups, plan.col_splits, plan.col_splits, 16 * plan.row_groups);
+            break;
+        case KM_VARIANT_GRID_F32:
+            snprintf(text, text_bytes, "km::fwd_grid_f32<%s, G=%d, W=%d>: fp32 contraction %s, %d wavefront(s) per row block", kt, G,
+                     plan.col_splits, kernel_type == KM_KERNEL_LOCALLY_PERIODIC ? "by entries" : "through the grid", plan.col_splits);
             break;
         case KM_VARIANT_VALU:
             snprintf(text, text_bytes, "km::fwd_valu<%s, KC=%d>: 128 rows per workgroup, %lld workgroups", kt,

@@ -112,6 +112,32 @@ __device__ __forceinline__ float phase_rev(float f, float x, float c) {
     return __builtin_fmaf(f, lo, __builtin_fmaf(f, hi, -turns));
 }
 
+// Cosine and sine of the same phase with an error of about an fp32 ulp of 1 / 2 (v_cos_f32 and v_sin_f32 have one of 2^-22 and the
+// rounding of the phase adds as much): the phase beyond the next quarter turn, for which the Taylor polynomials of sin(2 pi t)
+// and cos(2 pi t) leave out less than 2e-9.
+__device__ __forceinline__ void phase_cos_sin(float f, float x, float c, float* cosine, float* sine) {
+    const float hi = x - c;
+    const float bb = hi - x;
+    const float lo = (x - (hi - bb)) - (c + bb);
+    const float quarters = __builtin_rintf(4.0f * f * hi);
+    const float t = __builtin_fmaf(f, lo, __builtin_fmaf(f, hi, -0.25f * quarters));
+    const float t2 = t * t;
+    // (2 pi)^n / n!
+    float s = __builtin_fmaf(t2, 42.0586939f, -76.7058598f);
+    s = __builtin_fmaf(t2, s, 81.6052493f);
+    s = __builtin_fmaf(t2, s, -41.3417022f);
+    s = __builtin_fmaf(t2 * t, s, t * -1.74845553e-7f) + t * 6.28318548f;
+    float q = __builtin_fmaf(t2, -26.4262568f, 60.2446414f);
+    q = __builtin_fmaf(t2, q, -85.4568172f);
+    q = __builtin_fmaf(t2, q, 64.9393940f);
+    q = __builtin_fmaf(t2, q, -19.7392088f);
+    q = __builtin_fmaf(t2, q, 1.0f);
+    const int k = (int)(quarters - 4.0f * __builtin_floorf(0.25f * quarters));
+    const float ca = (k & 1) != 0 ? s : q, sa = (k & 1) != 0 ? q : s;
+    *cosine = k == 1 || k == 2 ? -ca : ca;
+    *sine = k >= 2 ? -sa : sa;
+}
+
 // fp16 roundings of the residuals a0 * b0 - h[0], a1 * b1 - h[1] of two products against their
 // fp16 values h (the low halves of the hi + lo split).  Written as two fp32 results (one
 // v_fma_mix_f32 each, reading the fp16 operand directly) rounded together by one

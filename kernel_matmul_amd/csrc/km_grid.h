@@ -138,7 +138,8 @@ __device__ __forceinline__ void grid_load(const float* __restrict__ x2, long lon
 //         of the gap.  *fine is cleared when a coordinate lies beyond gw.first or gw.last or is NaN.
 //   else: the coordinates themselves (entry-wise evaluation).  *fine is cleared when a coordinate makes
 //         every entry of its column NaN: a NaN, or an infinity under an oscillating factor.
-template <bool GRID, bool PHASE, int N>
+//   EXACT_PHASE: cosines and sines to fp32's rounding (phase_cos_sin) instead of the hardware's.
+template <bool GRID, bool PHASE, int N, bool EXACT_PHASE = false>
 __device__ __forceinline__ unsigned grid_table(const float (&xv)[N], int first, int stride, int end,
                                                const GridWindow& gw, const KernelConsts& kc, float* __restrict__ tab,
                                                bool* fine) {
@@ -192,9 +193,16 @@ __device__ __forceinline__ unsigned grid_table(const float (&xv)[N], int first, 
         // (zero past the end of the range, where rhs values are those of the last row again)
         const bool inside = 32 * ((lane >> 5) + 2 * i) * stride + (lane & 31) <= last;
         if (PHASE) {
-            const float th = phase_rev(kc.f, xv[i], gw.x_ref);
-            tab[CH + q] = inside ? wgt * __builtin_amdgcn_cosf(th) : 0.0f;
-            tab[2 * CH + q] = inside ? wgt * __builtin_amdgcn_sinf(th) : 0.0f;
+            float cosine, sine;
+            if constexpr (EXACT_PHASE) {
+                phase_cos_sin(kc.f, xv[i], gw.x_ref, &cosine, &sine);
+            } else {
+                const float th = phase_rev(kc.f, xv[i], gw.x_ref);
+                cosine = __builtin_amdgcn_cosf(th);
+                sine = __builtin_amdgcn_sinf(th);
+            }
+            tab[CH + q] = inside ? wgt * cosine : 0.0f;
+            tab[2 * CH + q] = inside ? wgt * sine : 0.0f;
         } else {
             tab[CH + q] = inside ? wgt : 0.0f;
         }
@@ -722,6 +730,57 @@ __device__ __forceinline__ bool grid_columns(const GridVectors& a, float* __rest
         look_at_steps<G>(a, w, kbase, w.range_start + 32 * wave, 32 * W, beyond, rl, shift, scale);
     }
     return fine;
+}
+
+// A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the phase-split form
+// combined (with the cosines and sines of the rows' phases), and the masked store.
+template <int KT, int G>
+__device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, const float (&ca)[4], const float (&sa)[4],
+                                           const float4v* res, const float* down, int row, int kbase) {
+    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
+    const int lane = threadIdx.x & 63;
+    const int li = lane & 15;
+    const int kk = lane >> 4;
+    float* __restrict__ out = a.out + (w.b * (long long)a.m + row) * a.k + kbase;
+    auto value = [&](int g, int v) {
+        return PHASE ? ca[v] * (res[g][v] * down[g]) + sa[v] * (res[G + g][v] * down[G + g]) : res[g][v] * down[g];
+    };
+    // Whole groups of rows of moderate width: a scalar base and row offset (no address arithmetic per value).
+    if (row + 16 <= a.m && a.k <= (1 << 22)) {
+        const buffer_rsrc to = uniform_buffer(out);
+        const unsigned lane_bytes = 4u * (__umul24(4u * (unsigned)kk, (unsigned)a.k) + (unsigned)li);
+#pragma unroll
+        for (int g = 0; g < G; g++) {
+            if (kbase + 16 * g + li < a.k) {
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(value(g, v)), to, (int)(lane_bytes + 64u * g),
+                                                          (int)(4u * (unsigned)v * (unsigned)a.k), 0);
+                }
+            }
+        }
+        return;
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+        const int c = 16 * g + li;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            if (row + 4 * kk + v < a.m && kbase + c < a.k) {
+                out[(long long)(4 * kk + v) * a.k + c] = value(g, v);
+            }
+        }
+    }
+}
+
+// cos A / sin A of the rows, one held by each lane, in the accumulator layout.
+__device__ __forceinline__ void row_phases(float own_cos, float own_sin, int first, float (&ca)[4], float (&sa)[4]) {
+    const int kk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        ca[v] = __shfl(own_cos, first + 4 * kk + v, 64);
+        sa[v] = __shfl(own_sin, first + 4 * kk + v, 64);
+    }
 }
 
 }  // namespace km

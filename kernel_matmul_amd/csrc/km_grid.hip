@@ -37,57 +37,6 @@ __device__ __forceinline__ GridVectors vectors(const FwdArgs& a) {
     return {a.x2_s, a.rhs_s0, a.rhs_s1, a.k};
 }
 
-// A group of 16 rows from its accumulators (scaled back by down[]): the two parts of the phase-split form
-// combined (with the cosines and sines of the rows' phases), and the masked store.
-template <int KT, int G>
-__device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, const float (&ca)[4], const float (&sa)[4],
-                                           const float4v* res, const float* down, int row, int kbase) {
-    constexpr bool PHASE = KT == KM_KERNEL_SPECTRAL;
-    const int lane = threadIdx.x & 63;
-    const int li = lane & 15;
-    const int kk = lane >> 4;
-    float* __restrict__ out = a.out + (w.b * (long long)a.m + row) * a.k + kbase;
-    auto value = [&](int g, int v) {
-        return PHASE ? ca[v] * (res[g][v] * down[g]) + sa[v] * (res[G + g][v] * down[G + g]) : res[g][v] * down[g];
-    };
-    // Whole groups of rows of moderate width: a scalar base and row offset (no address arithmetic per value).
-    if (row + 16 <= a.m && a.k <= (1 << 22)) {
-        const buffer_rsrc to = uniform_buffer(out);
-        const unsigned lane_bytes = 4u * (__umul24(4u * (unsigned)kk, (unsigned)a.k) + (unsigned)li);
-#pragma unroll
-        for (int g = 0; g < G; g++) {
-            if (kbase + 16 * g + li < a.k) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(value(g, v)), to, (int)(lane_bytes + 64u * g),
-                                                          (int)(4u * (unsigned)v * (unsigned)a.k), 0);
-                }
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-        const int c = 16 * g + li;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            if (row + 4 * kk + v < a.m && kbase + c < a.k) {
-                out[(long long)(4 * kk + v) * a.k + c] = value(g, v);
-            }
-        }
-    }
-}
-
-// cos A / sin A of the rows, one held by each lane, in the accumulator layout.
-__device__ __forceinline__ void row_phases(float own_cos, float own_sin, int first, float (&ca)[4], float (&sa)[4]) {
-    const int kk = (threadIdx.x & 63) >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        ca[v] = __shfl(own_cos, first + 4 * kk + v, 64);
-        sa[v] = __shfl(own_sin, first + 4 * kk + v, 64);
-    }
-}
-
 // Rows whose values a wavefront holds, two per lane (the layout of BlockRows).
 struct HeldRows {
     float y[2], rest[2], cos[2], sin[2];

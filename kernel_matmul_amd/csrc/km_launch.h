@@ -16,7 +16,8 @@ enum {
     KM_VARIANT_BLOCK = 5,            // split-fp16 MFMA, rhs operand prepared once per workgroup of 4 row blocks
     KM_VARIANT_MFMA_F32_DIRECT = 6,  // fp32 MFMA with every entry evaluated directly, operands straight from memory
     KM_VARIANT_GRID = 7,             // split-fp16 MFMA, Gaussian factor through an equidistant grid (rbf and spectral)
-    KM_VARIANT_PERIODIC = 8          // split-fp16 MFMA, locally periodic entries from tabulated phases (the launch table's choice only)
+    KM_VARIANT_PERIODIC = 8,         // split-fp16 MFMA, locally periodic entries from tabulated phases (the launch table's choice only)
+    KM_VARIANT_GRID_F32 = 9          // fp32 MFMA, rbf and spectral through the grid, the rest by column tables (what KM_VARIANT_MFMA_F32 becomes)
 };
 
 struct MatmulProblem {
@@ -56,6 +57,7 @@ struct MatmulPlan {
 hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_periodic(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
+hipError_t launch_matmul_grid_f32(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_block(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 
 struct ParamGradProblem {

@@ -1401,6 +1401,9 @@ hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStre
     if (plan.variant == KM_VARIANT_PERIODIC) {
         return launch_matmul_periodic(p, plan, stream);
     }
+    if (plan.variant == KM_VARIANT_GRID_F32) {
+        return launch_matmul_grid_f32(p, plan, stream);
+    }
     FwdArgs a;
     fill_fwd_args(p, &a);
 
