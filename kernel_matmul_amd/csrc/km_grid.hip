@@ -619,6 +619,7 @@ __device__ __forceinline__ GridWindow group_window(const GridWindow& common, con
     gw.col_hi = uniform(lane_value(p.row_hi, lane) + cr);
     gw.first = lane_value(p.first, lane);
     gw.last = lane_value(p.last, lane);
+    grid_tiles(&gw, lane_value(p.row_lo, lane), lane_value(p.row_hi, lane), KM_GRID_MIDDLE / KM_GRID_REACH * gw.reach);
     return gw;
 }
 

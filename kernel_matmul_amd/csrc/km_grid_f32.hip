@@ -31,11 +31,9 @@
 
 namespace km {
 
-// V = 2^-z^2 down to 2^-125; K / sigma, at z apart in the coordinates of V 2^(-z^2 / 2), down to 2^-126; the terms of an
-// entry's sum down to 2^-28.9 of it.
+// V = 2^-z^2 down to 2^-125; K / sigma, at z apart in the coordinates of V 2^(-z^2 / 2), down to 2^-126.
 #define KM_GRID_F32_REACH 11.18f
 #define KM_GRID_F32_COLUMN_REACH 15.88f
-#define KM_GRID_F32_MIDDLE 3.8f
 // Columns in a row block's range from which the grid is taken.
 #define KM_GRID_F32_MIN_WIDTH 160
 // Magnitude of the sums over a grid point from which their products might leave fp32's range.
@@ -56,50 +54,40 @@ constexpr int grid_f32_exchange_floats() {
     return W * S::TABLE > (W > 1 ? W * S::MT * S::GE * 256 : 0) ? W * S::TABLE : W * S::MT * S::GE * 256;
 }
 
-// What the points of the row block's window follow from: relative to its origin, in units of length.
-struct GridF32Limits {
-    float row_lo, row_hi, first, last;  // of the rows, and of the columns of the range
-    float middle;                       // distance from a middle beyond which points do not count
-};
-
 // The window; ok only if the columns of the range lie between its first and last one's coordinates, which the table checks.
 template <int MT>
-__device__ __forceinline__ GridWindow grid_f32_window(const BlockRows& rows, const KernelConsts& kc, float x_first, float x_last,
-                                                      GridF32Limits* limits) {
+__device__ __forceinline__ GridWindow grid_f32_window(const BlockRows& rows, const KernelConsts& kc, float x_first, float x_last) {
     GridWindow gw;
-    GridF32Limits& l = *limits;
     gw.x_ref = uniform(rows.middle);
     const float ya = rows.xa - gw.x_ref, yb = rows.xb - gw.x_ref;
-    l.row_lo = fminf(ya, yb);
-    l.row_hi = fmaxf(ya, yb);
-    l.first = uniform(x_first - gw.x_ref);
-    l.last = uniform(x_last - gw.x_ref);
-    const bool finite = __all(fabsf(ya) + fabsf(yb) < 1e30f) && fabsf(l.first) + fabsf(l.last) < 1e30f && l.first <= l.last;
-    wave_min_max(&l.row_lo, &l.row_hi);
+    float row_lo = fminf(ya, yb), row_hi = fmaxf(ya, yb);
+    gw.first = uniform(x_first - gw.x_ref);
+    gw.last = uniform(x_last - gw.x_ref);
+    const bool finite = __all(fabsf(ya) + fabsf(yb) < 1e30f) && fabsf(gw.first) + fabsf(gw.last) < 1e30f && gw.first <= gw.last;
+    wave_min_max(&row_lo, &row_hi);
     gw.s2 = uniform(kc.s * 1.41421356237309504880f);
     const float inv = __builtin_amdgcn_rcpf(gw.s2);
     gw.h = uniform(__uint_as_float(__float_as_uint(KM_GRID_STEP * inv) & 0xfffff000u));
     const float inv_h = __builtin_amdgcn_rcpf(gw.h);
     gw.reach = uniform(KM_GRID_F32_REACH * inv);
-    l.middle = uniform(KM_GRID_F32_MIDDLE * inv);
-    const float lo = fmaxf(l.row_lo - gw.reach, 0.5f * (l.row_lo + l.first) - l.middle);
-    const float hi = fminf(l.row_hi + gw.reach, 0.5f * (l.row_hi + l.last) + l.middle);
+    const float middle = KM_GRID_MIDDLE * inv;
+    const float lo = fmaxf(row_lo - gw.reach, 0.5f * (row_lo + gw.first) - middle);
+    const float hi = fminf(row_hi + gw.reach, 0.5f * (row_hi + gw.last) + middle);
     gw.g_lo = uniform(floorf(lo * inv_h));
     const float count = ceilf(hi * inv_h) - gw.g_lo;
     gw.ok = finite && gw.h > 1e-30f && gw.h < 1e30f && count >= 0.0f && count < (float)(16 * MT) && fabsf(gw.g_lo) < 16000.0f;
     gw.tiles = __builtin_amdgcn_readfirstlane(gw.ok ? ((int)count + 16) / 16 : 0);
     const float cr = KM_GRID_F32_COLUMN_REACH * inv;
-    gw.col_lo = uniform(l.row_lo - cr);
-    gw.col_hi = uniform(l.row_hi + cr);
-    gw.first = l.first;
-    gw.last = l.last;
+    gw.col_lo = uniform(row_lo - cr);
+    gw.col_hi = uniform(row_hi + cr);
+    grid_tiles(&gw, row_lo, row_hi, middle);
     return gw;
 }
 
 // One step of 32 columns onto the grid.
 template <int KT, int G, int MT, int CH>
 __device__ __forceinline__ void grid_f32_step(const float* __restrict__ tab, int off, const float (&raw)[G][8], const GridWindow& gw,
-                                              const GridF32Limits& l, float t0, bool wide,
+                                              float t0, unsigned reached, bool wide,
                                               float4v (&acc)[MT][GridF32Shape<KT, G>::GE]) {
     constexpr int PARTS = GridF32Shape<KT, G>::PARTS;
     constexpr int GE = GridF32Shape<KT, G>::GE;
@@ -121,23 +109,16 @@ __device__ __forceinline__ void grid_f32_step(const float* __restrict__ tab, int
             }
         }
     }
-    const float lo = tab[3 * CH + (off >> 3)];
-    const float hi = tab[3 * CH + CH / 8 + (off >> 3)];
-    const float middle = 0.5f * (lo + hi);
-    const float t_lo = fmaxf(lo - gw.reach, 0.5f * (l.row_lo + lo) - l.middle);
-    const float t_hi = fminf(hi + gw.reach, 0.5f * (l.row_hi + hi) + l.middle);
+    const float middle = tab[3 * CH + (off >> 3)];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
-        if (mt >= gw.tiles) {
-            break;
-        }
-        const float t = __builtin_fmaf((float)(16 * mt), gw.h, t0);
-        if (!__any(!(t < t_lo || t > t_hi))) {
+        if ((reached >> mt & 1) == 0) {
             continue;
         }
+        const float t = __builtin_fmaf((float)(16 * mt), gw.h, t0);
         float v[8];
         if (!wide) {
-            const float av = (t - middle) * gw.s2;
+            const float av = __builtin_fmaf(t, gw.s2, -middle);
             const float rb = -av * av;
 #pragma unroll
             for (int u = 0; u < 8; u++) {
@@ -167,7 +148,7 @@ __device__ __forceinline__ void grid_f32_step(const float* __restrict__ tab, int
 // the form does not take.
 template <int KT, int G, int W>
 __device__ __forceinline__ bool grid_f32_columns(const FwdArgs& a, float* __restrict__ tab, const WaveView& w, int kbase, int wave,
-                                                 const GridWindow& gw, const GridF32Limits& l, const KernelConsts& kc,
+                                                 const GridWindow& gw, const KernelConsts& kc,
                                                  float (&xv)[GridF32Shape<KT, G>::CHUNK / 64],
                                                  float4v (&acc)[GridF32Shape<KT, G>::MT][GridF32Shape<KT, G>::GE]) {
     using S = GridF32Shape<KT, G>;
@@ -199,7 +180,8 @@ __device__ __forceinline__ bool grid_f32_columns(const FwdArgs& a, float* __rest
         const int first = (int)next_first;
         float next[G][8];
         grid_rhs<G>(vec, rhs, first, w.range_end, kk, rl, next);
-        const unsigned steps = grid_table<true, S::PARTS == 2, CH / 64, true>(xv, first, W, w.range_end, gw, kc, tab, &fine);
+        unsigned long long reached = 0;
+        const unsigned steps = grid_table<true, S::PARTS == 2, CH / 64, true>(xv, first, W, w.range_end, gw, kc, tab, &fine, &reached);
         if (next_first + CH * W < (unsigned)w.range_end) {
             grid_load(w.x2, a.x2_s, first + CH * W, W, w.range_end, xv);
         }
@@ -226,6 +208,7 @@ __device__ __forceinline__ bool grid_f32_columns(const FwdArgs& a, float* __rest
             }
             const int off = 32 * j + 8 * kk;
             const bool wide = (steps >> (16 + j) & 1) != 0;
+            const unsigned points = (unsigned)(reached >> (8 * j)) & 0xff;
             need &= need - 1;
             if (need != 0) {
                 j = __builtin_ctz(need);
@@ -239,7 +222,7 @@ __device__ __forceinline__ bool grid_f32_columns(const FwdArgs& a, float* __rest
                     asm volatile("" : "+v"(acc[m][g]));
                 }
             }
-            grid_f32_step<KT, G, S::MT, CH>(tab, off, raw, gw, l, t0, wide, acc);
+            grid_f32_step<KT, G, S::MT, CH>(tab, off, raw, gw, t0, points, wide, acc);
         } while (need != 0);
         // All reads of the table are done before the next chunk overwrites it.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -255,8 +238,7 @@ __device__ __forceinline__ bool grid_f32_columns(const FwdArgs& a, float* __rest
 
 // Grid -> rows: `groups` groups of 16 rows from row0 from the sums of their window.
 template <int KT, int G>
-__device__ __forceinline__ void grid_f32_rows(const FwdArgs& a, const WaveView& w, int row0, int groups, int kbase, const GridWindow& gw,
-                                              const GridF32Limits& l, const KernelConsts& kc,
+__device__ __forceinline__ void grid_f32_rows(const FwdArgs& a, const WaveView& w, int row0, int groups, int kbase, const GridWindow& gw, const KernelConsts& kc,
                                               const float4v (&acc)[GridF32Shape<KT, G>::MT][GridF32Shape<KT, G>::GE]) {
     using S = GridF32Shape<KT, G>;
     constexpr bool PHASE = S::PARTS == 2;
@@ -280,6 +262,7 @@ __device__ __forceinline__ void grid_f32_rows(const FwdArgs& a, const WaveView& 
     }
     const float mid0 = (gw.g_lo + (float)(4 * kk) + 1.5f) * gw.h;
     const float half = 1.5f * gw.h;
+    const float middle = uniform(KM_GRID_MIDDLE / KM_GRID_F32_REACH * gw.reach);
 #pragma unroll 1
     for (int r = 0; r < groups; r++) {
         const int row = row0 + 16 * r;
@@ -292,8 +275,8 @@ __device__ __forceinline__ void grid_f32_rows(const FwdArgs& a, const WaveView& 
             phase_cos_sin(kc.f, x, gw.x_ref, &cosine, &sine);
             row_phases(cosine, sine, 0, ca, sa);
         }
-        const float t_lo = fmaxf(y - gw.reach, 0.5f * (y + l.first) - l.middle) - half;
-        const float t_hi = fminf(y + gw.reach, 0.5f * (y + l.last) + l.middle) + half;
+        const float t_lo = fmaxf(y - gw.reach, 0.5f * (y + gw.first) - middle) - half;
+        const float t_hi = fminf(y + gw.reach, 0.5f * (y + gw.last) + middle) + half;
         float4v res[S::GE];
 #pragma unroll
         for (int g = 0; g < S::GE; g++) {
@@ -341,13 +324,12 @@ __device__ __forceinline__ bool grid_f32_item(const FwdArgs& a, float* lds, cons
     if (32 * wave < w.range_end - w.range_start) {
         grid_load(w.x2, a.x2_s, w.range_start + 32 * wave, W, w.range_end, xv);
     }
-    GridF32Limits l;
-    const GridWindow gw = grid_f32_window<S::MT>(rows, kc, x_first, x_last, &l);
+    const GridWindow gw = grid_f32_window<S::MT>(rows, kc, x_first, x_last);
     if (__builtin_amdgcn_readfirstlane(gw.ok) == 0) {
         return false;
     }
     float4v acc[S::MT][S::GE];
-    bool fine = grid_f32_columns<KT, G, W>(a, lds + wave * S::TABLE, w, kbase, wave, gw, l, kc, xv, acc);
+    bool fine = grid_f32_columns<KT, G, W>(a, lds + wave * S::TABLE, w, kbase, wave, gw, kc, xv, acc);
     if constexpr (W > 1) {
         float4v* const part = (float4v*)lds;
         unsigned* const words = (unsigned*)(lds + grid_f32_exchange_floats<KT, G, W>());
@@ -403,7 +385,7 @@ __device__ __forceinline__ bool grid_f32_item(const FwdArgs& a, float* lds, cons
     if (__builtin_amdgcn_readfirstlane(fine) == 0) {
         return false;
     }
-    grid_f32_rows<KT, G>(a, w, row0 + 16 * R * wave, R, kbase, gw, l, kc, acc);
+    grid_f32_rows<KT, G>(a, w, row0 + 16 * R * wave, R, kbase, gw, kc, acc);
     return true;
 }
 

@@ -982,7 +982,8 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
             }
         }
     }
-    const unsigned steps = grid_table<true, PHASE>(xv, g.row0, 1, row_end, gw, kc, tab, &fine);
+    unsigned long long reached = 0;
+    const unsigned steps = grid_table<true, PHASE>(xv, g.row0, 1, row_end, gw, kc, tab, &fine, &reached);
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < STEPS; j++) {
@@ -1038,22 +1039,18 @@ __device__ __forceinline__ bool grid_grad_pass(const GradArgs& a, const GradItem
         const float t = __builtin_fmaf((float)(16 * mt), gw.h, t0);
 #pragma unroll
         for (int j = 0; j < STEPS; j++) {
-            if ((steps >> j & 1) == 0) {
+            if ((steps >> j & 1) == 0 || (reached >> (8 * j + mt) & 1) == 0) {
                 continue;
             }
             int off = 32 * j + 8 * kk;
             asm volatile("" : "+v"(off));  // (read again for every tile, not kept over all of them: registers)
             const bool wide = (steps >> (16 + j) & 1) != 0;
-            const float lo_x = tab[3 * CH + (off >> 3)];
-            const float hi_x = tab[3 * CH + CH / 8 + (off >> 3)];
-            if (!__any(!(fmaxf(lo_x - t, t - hi_x) > gw.reach))) {
-                continue;
-            }
+            const float middle = tab[3 * CH + (off >> 3)];
             const float4v x0 = *(const float4v*)(tab + off);
             const float4v x1 = *(const float4v*)(tab + off + 4);
             float pr[8], arg[8];
             if (!wide) {
-                const float av = (t - 0.5f * (lo_x + hi_x)) * gw.s2;
+                const float av = __builtin_fmaf(t, gw.s2, -middle);
                 const float rb = __builtin_fmaf(-av, av, (float)KM_GRID_KS1);
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
@@ -1152,7 +1149,7 @@ __global__ void __launch_bounds__(64, KT == KM_KERNEL_SPECTRAL && !PACK ? 2 : 3)
     GridWindow gw;
     gw.ok = __builtin_amdgcn_readfirstlane(g.width >= a.grid_min_width) != 0;
     if (gw.ok) {
-        gw = grid_window<MT>(block_rows(g.x1, a.x1_s, g.row0, a.m), kc, KM_GG_STEP);
+        gw = grid_window<MT>(block_rows(g.x1, a.x1_s, g.row0, a.m), kc, KM_GG_STEP, __builtin_inff());
     }
     if (__builtin_amdgcn_readfirstlane(gw.ok) != 0) {
         // (fewer, longer shares than the pairwise form's: from the same split number)
