@@ -149,7 +149,22 @@ int km_matmul(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64
               const int64_t* start_strides, const int32_t* end, const int64_t* end_strides,
               float* out, const km_launch_options* options, void* stream);
 
-/* Which ahead-of-time kernel and decomposition km_matmul would pick for a problem of this
+/* The same with device scratch of km_matmul_workspace_size(...) bytes, whose contents on entry do not matter: few rows against
+ * many points (row blocks with long ranges that would leave most of the device idle) then have
+ * their ranges shared out, and the shares' sums are added in a fixed order.  The size is 0 for
+ * problems that gain nothing by it; with less (or none) the call does what km_matmul does. */
+size_t km_matmul_workspace_size(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m,
+                                int64_t n, int64_t k, const km_launch_options* options);
+
+int km_matmul_with_workspace(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m, int64_t n,
+                             int64_t k, const float* x1, const int64_t* x1_strides, const float* x2,
+                             const int64_t* x2_strides, const float* rhs, const int64_t* rhs_strides,
+                             const float* params, const int64_t* params_strides, const int32_t* start,
+                             const int64_t* start_strides, const int32_t* end, const int64_t* end_strides,
+                             float* out, const km_launch_options* options, void* workspace,
+                             size_t workspace_bytes, void* stream);
+
+/* Which ahead-of-time kernel and decomposition km_matmul_with_workspace would pick for a problem of this
  * size (host only; nothing is launched).  Writes a short description such as
  * "km::fwd_table_f16<spectral, G=1, R=8>: 128 rows per wavefront, ..." into `text`.
  * Stands in for the reference's autotune report (kernel_matmul/native_function.py:56-69,

@@ -92,6 +92,11 @@ def load_library():
         + tensor * 6
         + [_vp, ctypes.POINTER(LaunchOptions), _vp]
     )
+    lib.km_matmul_with_workspace.restype = ctypes.c_int
+    lib.km_matmul_with_workspace.argtypes = lib.km_matmul.argtypes[:-1] + [_vp, ctypes.c_size_t, _vp]
+    lib.km_matmul_workspace_size.restype = ctypes.c_size_t
+    lib.km_matmul_workspace_size.argtypes = [ctypes.c_int, ctypes.c_int, _i64p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+                                             ctypes.POINTER(LaunchOptions)]
     lib.km_param_grad_describe.restype = ctypes.c_int
     lib.km_param_grad_describe.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                            ctypes.c_char_p, ctypes.c_size_t]
@@ -287,7 +292,7 @@ def _check_matrix_inputs(kernel_type, x1, x2, params, start, end):
 
 def matmul(kernel_type: str, x1: Tensor, x2: Tensor, rhs: Tensor, params: Tensor, start: Tensor,
            end: Tensor, options: LaunchOptions | None = None, out: Tensor | None = None) -> Tensor:
-    """out[..., m, k] = K(x1, x2)[mask] @ rhs   (C ABI: km_matmul).
+    """out[..., m, k] = K(x1, x2)[mask] @ rhs   (C ABI: km_matmul_with_workspace).
 
     ``out`` (optional) is a contiguous fp32 tensor of the result's shape to write into."""
     result = torch_calls().matmul(KERNEL_TYPES.get(kernel_type), x1, x2, rhs, params, start, end,
@@ -305,9 +310,13 @@ def matmul(kernel_type: str, x1: Tensor, x2: Tensor, rhs: Tensor, params: Tensor
     device = x1.device
     out = _result((*batch_shape, m, k), device, out)
     lib = load_library()
+    options_ptr = ctypes.byref(options) if options is not None else None
+    head = (kid, len(batch_shape), _i64(batch_shape), m, n, k)
+    need = lib.km_matmul_workspace_size(*head, options_ptr)
+    workspace = torch.empty(need, dtype=torch.uint8, device=device) if need > 0 else None
     with _on_device(device):
-        status = lib.km_matmul(kid, len(batch_shape), _i64(batch_shape), m, n, k, *_tensors_args(x1, x2, rhs, params, start, end),
-                               _ptr(out), ctypes.byref(options) if options is not None else None, _stream(device))
+        status = lib.km_matmul_with_workspace(*head, *_tensors_args(x1, x2, rhs, params, start, end), _ptr(out), options_ptr,
+                                              workspace.data_ptr() if need > 0 else None, need, _stream(device))
     if status != 0:
         _raise(lib, status)
     return out

@@ -216,8 +216,52 @@ static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, 
     return true;
 }
 
-static int make_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
+// Few rows against many points (predictions): a row block's range spans the points between its rows, of which the columns per
+// row block are what the sizes tell.  A workgroup of eight wavefronts for each share of the ranges, then the sum of the shares;
+// the number of shares is the one for which rounds of 256 workgroups, each as long as its share and a start (what 1500 columns
+// out of reach take), are over first.  Measured, none (the forms below) against the shares taken, us a call, rbf: m = 100, n = 5000
+// 22.8 / 11.6, n = 20000 75 / 12.8, n = 1e6 4926 / 36, m = 1000, n = 30000 20.4 / 12.7 (4 sets), n = 1e5 59.7 / 23.1 (8 sets),
+// m = 3000, n = 1e5, 4 sets 26.1 / 19.4, n = 3e5, 16 sets 103 / 69, m = 300, n = 1e5, k = 32 178 / 17; spectral alike; locally
+// periodic m = 100, n = 1e6 3160 / 39, m = 3000, n = 1e5, 4 sets 21.3 / 20.8, n = 3e5, 16 sets 90 / 102 with two: not below three.
+// Fewer than 2048 columns a row block: n = 2000, m = 100 11.4 / 10.5 to 12.2, 1265 columns, 316 items 22.6 / 23.1.
+static bool shares_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
+    if (opt && (opt->variant != KM_VARIANT_AUTO || opt->rows_per_wave != 0 || opt->col_splits > 1 || opt->reserved != 0)) {
+        return false;
+    }
+    const int k_chunk = p.k <= 16 ? 16 : 32;
+    const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
+    const long long items = row_blocks * p.num_batches * ((p.k + k_chunk - 1) / k_chunk);
+    const long long columns = p.n / row_blocks;
+    if (columns < 2048 || items > 1024) {
+        return false;
+    }
+    const long long most = columns / 512 < 128 ? columns / 512 : 128;
+    long long shares = 1;
+    double best = 0.0;
+    for (long long s = 1; s <= most; s++) {
+        const double cost = (double)((items * s + 255) / 256) * (1.0 / (double)s + 1500.0 / (double)columns);
+        if (s == 1 || cost < 0.95 * best) {
+            best = cost;
+            shares = s;
+        }
+    }
+    if (shares < (p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC ? 3 : 2)) {
+        return false;
+    }
+    plan->variant = p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC ? KM_VARIANT_PERIODIC : KM_VARIANT_GRID;
+    plan->k_chunk = k_chunk;
+    plan->row_groups = 8;
+    plan->col_splits = 8;
+    plan->shares = (int)shares;
+    plan->tail_balance = 0;
+    plan->group_tail_halves = 0;
+    return true;
+}
+
+// shares: whether the caller has memory for them.
+static int make_plan(const MatmulProblem& p, const km_launch_options* opt, bool shares, MatmulPlan* plan) {
     int variant = opt ? opt->variant : KM_VARIANT_AUTO;
+    plan->shares = 1;
     plan->phase_split = 0;
     plan->group_tail = -1;
     plan->group_tail_halves = -1;
@@ -237,6 +281,9 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, Matmu
     }
     if (variant == KM_VARIANT_GRID && p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
         return fail(KM_ERR_INVALID_ARGUMENT, "km_matmul: the grid form takes rbf and spectral kernels only");
+    }
+    if (shares && shares_plan(p, opt, plan)) {
+        return KM_OK;
     }
     if (grid_plan(p, opt, variant, plan)) {
         return KM_OK;
@@ -587,12 +634,35 @@ int km_check_sorted_device(const float* x1, int64_t num_batch1, int64_t n1, cons
 // ---------------------------------------------------------------------------------------
 // matmul
 // ---------------------------------------------------------------------------------------
-int km_matmul(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m, int64_t n,
+static size_t shares_bytes(const MatmulProblem& p, const MatmulPlan& plan) {
+    return plan.shares > 1 ? sizeof(float) * (size_t)plan.shares * (size_t)p.num_batches * (size_t)p.m * (size_t)p.k : 0;
+}
+
+size_t km_matmul_workspace_size(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m, int64_t n, int64_t k,
+                                const km_launch_options* options) {
+    long long nb = 0;
+    if (check_common("km_matmul_workspace_size", kernel_type, batch_rank, batch_sizes, m, n, &nb) || nb == 0 || m == 0 || k <= 0 ||
+        k > INT_LIMIT || (long long)m * k > INT_LIMIT * 64LL) {
+        return 0;
+    }
+    MatmulProblem p;
+    memset(&p, 0, sizeof(p));
+    p.kernel_type = kernel_type;
+    p.num_batches = nb;
+    p.m = m;
+    p.n = n;
+    p.k = k;
+    MatmulPlan plan;
+    return shares_plan(p, options, &plan) ? shares_bytes(p, plan) : 0;
+}
+
+int km_matmul_with_workspace(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m, int64_t n,
               int64_t k, const float* x1, const int64_t* x1_strides, const float* x2,
               const int64_t* x2_strides, const float* rhs, const int64_t* rhs_strides,
               const float* params, const int64_t* params_strides, const int32_t* start,
               const int64_t* start_strides, const int32_t* end, const int64_t* end_strides,
-              float* out, const km_launch_options* options, void* stream) {
+              float* out, const km_launch_options* options, void* workspace,
+              size_t workspace_bytes, void* stream) {
     const char* op = "km_matmul";
     long long nb = 0;
     if (int rc = check_common(op, kernel_type, batch_rank, batch_sizes, m, n, &nb)) return rc;
@@ -654,9 +724,23 @@ int km_matmul(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64
     p.out = out;
 
     MatmulPlan plan;
-    if (int rc = make_plan(p, options, &plan)) return rc;
+    if (int rc = make_plan(p, options, workspace != nullptr, &plan)) return rc;
+    if (plan.shares > 1 && workspace_bytes < shares_bytes(p, plan)) {
+        if (int rc = make_plan(p, options, false, &plan)) return rc;
+    }
+    p.partials = (float*)workspace;
     hipError_t err = launch_matmul(p, plan, (hipStream_t)stream);
     return err == hipSuccess ? KM_OK : fail_hip(op, err);
+}
+
+int km_matmul(int kernel_type, int batch_rank, const int64_t* batch_sizes, int64_t m, int64_t n,
+              int64_t k, const float* x1, const int64_t* x1_strides, const float* x2,
+              const int64_t* x2_strides, const float* rhs, const int64_t* rhs_strides,
+              const float* params, const int64_t* params_strides, const int32_t* start,
+              const int64_t* start_strides, const int32_t* end, const int64_t* end_strides,
+              float* out, const km_launch_options* options, void* stream) {
+    return km_matmul_with_workspace(kernel_type, batch_rank, batch_sizes, m, n, k, x1, x1_strides, x2, x2_strides, rhs, rhs_strides,
+                                    params, params_strides, start, start_strides, end, end_strides, out, options, nullptr, 0, stream);
 }
 
 int km_param_grad_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t c, char* text,
@@ -689,7 +773,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
     p.n = n;
     p.k = k;
     MatmulPlan plan;
-    if (int rc = make_plan(p, options, &plan)) return rc;
+    if (int rc = make_plan(p, options, true, &plan)) return rc;
     static const char* const kernels[] = {"rbf", "spectral", "locally_periodic"};
     const char* kt = kernels[kernel_type];
     const long long row_blocks = (m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
@@ -697,7 +781,10 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
     const char* const halves = kernel_type == KM_KERNEL_SPECTRAL && G == 4 ? ", half of 64 columns each" : "";
     switch (plan.variant) {
         case KM_VARIANT_GRID:
-            if (plan.group_tail > 0) {
+            if (plan.shares > 1) {
+                snprintf(text, text_bytes, "km::fwd_grid_shares<%s, G=%d>: grid form, ranges in up to %d shares of 8 wavefronts, then their sums", kt,
+                         G, plan.shares);
+            } else if (plan.group_tail > 0) {
                 snprintf(text, text_bytes,
                          "km::fwd_grid_grouped<%s, G=%d>: grid form, 4 row blocks per workgroup of 4 wavefronts, "
                          "the last %lld row blocks of each XCD by a workgroup each%s",
@@ -711,6 +798,11 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
             }
             break;
         case KM_VARIANT_PERIODIC:
+            if (plan.shares > 1) {
+                snprintf(text, text_bytes, "km::fwd_block_shares<%s, G=%d>: ranges in up to %d shares of 8 wavefronts, then their sums", kt, G,
+                         plan.shares);
+                break;
+            }
             snprintf(text, text_bytes, "km::fwd_block<%s, G=%d, R=%d, W=%d>: tabulated phases, %d wavefront(s) per %d rows", kt, G,
                      plan.row_groups, plan.col_splits, plan.col_splits, 16 * plan.row_groups);
             break;

@@ -126,7 +126,7 @@ __device__ __forceinline__ unsigned entry_table(const float (&xv)[KM_ENTRY_CHUNK
         need |= bits(rel <= last && !(y < col_lo || y > col_hi), i);
         group8_min_max(y, &lo[i], &hi[i]);
         need |= (form.direct ? 3u << (2 * i) : bits(0.5f * (hi[i] - lo[i]) * kc.s > KM_ENTRY_SPAN, i)) << 16;
-        ok = ok && is_finite(xv[i]);
+        ok = ok && (!F32 && KT == KM_KERNEL_RBF ? xv[i] == xv[i] : is_finite(xv[i]));
     }
     need = __builtin_amdgcn_readfirstlane(need);
     *fine = *fine && __all(ok);
@@ -165,13 +165,12 @@ __device__ __forceinline__ unsigned entry_table(const float (&xv)[KM_ENTRY_CHUNK
     return need | (__all(exact) ? 0u : 1u << 31);
 }
 
-// Two entries from their exponents, split into fp16 halves, times 2^KM_F16_KSCALE_LOG2 (as entry_pair_f16).
-__device__ __forceinline__ void entry_exponents_f16(float a0, float a1, half2v* hi, half2v* lo) {
+// Two entries split into fp16 halves, times 2^KM_F16_KSCALE_LOG2 (as entry_pair_f16).
+__device__ __forceinline__ void entry_values_f16(float v0, float v1, half2v* hi, half2v* lo) {
     constexpr float S = (float)(1 << KM_F16_KSCALE_LOG2);
-    const float2v kv = {__builtin_amdgcn_exp2f(a0), __builtin_amdgcn_exp2f(a1)};
-    const half2v h = __builtin_convertvector(kv, half2v) * (half2v){(_Float16)S, (_Float16)S};
+    const half2v h = __builtin_convertvector((float2v){v0, v1}, half2v) * (half2v){(_Float16)S, (_Float16)S};
     *hi = h;
-    *lo = residual_f16x2(kv[0], S, kv[1], S, h);
+    *lo = residual_f16x2(v0, S, v1, S, h);
 }
 
 // One step of 32 columns against the row groups within reach.  F32: the products are fp32 MFMAs, of which number t
@@ -182,7 +181,6 @@ __device__ __forceinline__ void entry_step(const float* __restrict__ tab, int of
                                            const EntryForm& form, const KernelConsts& kc,
                                            const float (&scale)[G], float4v (&acc)[R][G]) {
     constexpr bool SPECTRAL = KT == KM_KERNEL_SPECTRAL, PERIODIC = KT == KM_KERNEL_LOCALLY_PERIODIC;
-    static_assert(F32 || PERIODIC, "the others' split-fp16 kernels are in km_grid.hip and km_matmul.hip");
     float xv[8], cb[8], sb[8];
     half8v bhi[F32 ? 1 : G], blo[F32 ? 1 : G];
     float bv[F32 ? G : 1][8];
@@ -273,7 +271,7 @@ __device__ __forceinline__ void entry_step(const float* __restrict__ tab, int of
             for (int t = 0; t < 8; t++) {
                 const float u = d[t] * kc.s;
                 arg[t] = -u * u;
-                // (F32: the phase rounded as what is left of it beyond whole turns)
+                // (the phase rounded as what is left of it beyond whole turns)
                 if constexpr (SPECTRAL) {
                     cosine[t] = __builtin_amdgcn_cosf(__builtin_fmaf(d[t], kc.f, -__builtin_rintf(d[t] * kc.f)));
                 } else if constexpr (PERIODIC) {
@@ -299,7 +297,12 @@ __device__ __forceinline__ void entry_step(const float* __restrict__ tab, int of
             half2v h2[4], l2[4];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                entry_exponents_f16(arg[2 * u], arg[2 * u + 1], &h2[u], &l2[u]);
+                float v0 = __builtin_amdgcn_exp2f(arg[2 * u]), v1 = __builtin_amdgcn_exp2f(arg[2 * u + 1]);
+                if (SPECTRAL) {
+                    v0 *= cosine[SPECTRAL ? 2 * u : 0];
+                    v1 *= cosine[SPECTRAL ? 2 * u + 1 : 0];
+                }
+                entry_values_f16(v0, v1, &h2[u], &l2[u]);
             }
             const half8v ahi = join_half2x4(h2);
             const half8v alo = join_half2x4(l2);

@@ -347,6 +347,24 @@ __device__ __forceinline__ WaveView wave_view(const FwdArgs& a, long long item, 
     return w;
 }
 
+// Launches of few row blocks with long ranges: a.chunks_per_block workgroups in a row take a piece of a range each, in whole
+// steps and no shorter than this, and write sums of their own, as a batch item further on.  (Neighbouring workgroups run on
+// different XCDs, and pieces have nothing in common.)
+#define KM_SHARE_COLUMNS 512
+__device__ __forceinline__ WaveView share_view(const FwdArgs& a) {
+    const unsigned shares = (unsigned)a.chunks_per_block;
+    const unsigned item = blockIdx.x / shares, share = blockIdx.x - item * shares;
+    int unused;
+    WaveView w = wave_view<true>(a, item, 1, &unused);
+    const int length = max(w.range_end - w.range_start, 0);
+    const int each = max((length / (int)shares + 256) & ~255, KM_SHARE_COLUMNS);
+    const long long first = min((long long)share * each, (long long)length);
+    w.range_end = w.range_start + (int)min(first + each, (long long)length);
+    w.range_start += (int)first;
+    w.b += (long long)share * a.num_batches;
+    return w;
+}
+
 // Work item of this workgroup.  Items are (row chunk, batch item) pairs, contiguous ranges of
 // which belong to one XCD (see xcd_item).  When the launch has a "tail" (only with 128 rows per
 // wavefront), the last `tail_items` items of every XCD are cut into 8 pieces of 16 rows that are

@@ -21,6 +21,7 @@
 #include "km_batch.h"
 #include "km_common.h"
 #include "km_fwd.h"
+#include "km_entries.h"
 #include "km_grid.h"
 #include "km_group_plan.h"
 #include "km_launch.h"
@@ -196,6 +197,25 @@ constexpr int grid_lds_floats() {
     return W == 1 ? KM_GRID_TABLE_FLOATS
                   : (W * KM_GRID_TABLE_FLOATS > W * MT * GE * 256 ? W * KM_GRID_TABLE_FLOATS : W * MT * GE * 256) +
                         W * (GE + 1);
+}
+
+// Whether the wavefronts of a workgroup share the steps of a range entry by entry as well (entry_item), for all rows each; else each
+// has rows of its own and takes all steps (grid_entrywise), as one wavefront alone does.  Rows that are far apart (predictions)
+// leave hardly any work but looking at the columns: rbf m = 9973, n = 50000, k = 3, 4 sets 27.1 -> 22.0 us.  With two groups of rhs
+// columns the sums of all rows are more than three resident wavefronts' registers hold.
+// Short ranges do not pay for the exchange of the sums: spectral n = 50000, k = 8, 2 sets at one point per unit (152 columns a row
+// block) with two wavefronts 13.8 -> 14.2, n = 8000, k = 16 with eight 9.3 -> 8.0.
+#define KM_SHARED_ENTRIES 1024 /* columns times wavefronts */
+template <int G, int W, bool SHARES>
+constexpr bool shares_entries() { return W > 1 && (G == 1 || SHARES); }
+
+// The LDS of both forms.
+template <int KT, int G, int W, bool SHARES = false>
+constexpr int item_lds_floats() {
+    using S = GridShape<KT, G>;
+    constexpr int grid = grid_lds_floats<S::GE, S::MT, W>();
+    constexpr int entries = shares_entries<G, W, SHARES>() ? entry_lds_floats(G, 8, W) : 0;
+    return grid > entries ? grid : entries;
 }
 
 // One item in the grid form for rhs columns [kbase, kbase + 16 G), by W wavefronts of which this is
@@ -405,11 +425,11 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
 
 // One item by W wavefronts (this one is number `wave`) for rhs columns [kbase, kbase + 16 G): the grid form, or
 // entry by entry.
-template <int KT, int G, int W>
+template <int KT, int G, int W, bool SHARES = false>
 __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int kbase, int wave) {
     using S = GridShape<KT, G>;
     int unused;
-    const WaveView w = wave_view<true>(a, item, 1, &unused);
+    const WaveView w = SHARES ? share_view(a) : wave_view<true>(a, item, 1, &unused);
     const int row0 = w.row_block * KM_BLOCK_SIZE;
     // The rows are requested first, then the first columns (which wait for the range), then the
     // window is computed.
@@ -427,7 +447,16 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
     // (always so; without the condition the kernel came out slower, rbf n = 65536, k = 64 21.9 against 21.6 us a call)
     if (kbase < a.k) {
         if (!grid || !grid_forward<KT, G, S::MT, W>(a, lds, w, row0, kbase, wave, gw, kc, xv)) {
-            grid_entrywise<KT, G, W>(a, lds, w, row0, kbase, wave, gw, kc);
+            if constexpr (shares_entries<G, W, SHARES>()) {
+                if (SHARES || w.range_end - w.range_start >= KM_SHARED_ENTRIES / W) {
+                    __syncthreads();  // (its tables lie elsewhere in LDS)
+                    entry_item<KT, false, G, 8, W>(a, lds, w, row0, kbase, wave);
+                    return;
+                }
+            }
+            if constexpr (!SHARES) {
+                grid_entrywise<KT, G, W>(a, lds, w, row0, kbase, wave, gw, kc);
+            }
         }
     }
 }
@@ -470,7 +499,7 @@ struct GroupShape {
     static constexpr int SUMS = KM_GROUP * TABLE;
     static constexpr int FLAGS = SUMS + QUADS * QUAD;
     static constexpr int FLOATS = FLAGS + 64;
-    static_assert(FLOATS >= grid_lds_floats<S::GE, S::MT, KM_GROUP>() && FLOATS >= KM_GROUP * KM_GRID_TABLE_FLOATS, "grid_item's LDS");
+    static_assert(FLOATS >= item_lds_floats<KT, G, KM_GROUP>() && FLOATS >= KM_GROUP * KM_GRID_TABLE_FLOATS, "grid_item's LDS");
     static_assert(KM_GROUP + (KM_GROUP_SEGMENTS + KM_GROUP) * G <= 64, "flags");
 };
 
@@ -919,9 +948,10 @@ struct GridColumns {
     }
 };
 
-// W: wavefronts per row block, or 1: fewer than one, the workgroup for several row blocks.
+// W: wavefronts per row block, or 1: fewer than one, the workgroup for several row blocks.  (Eight of one are launched where
+// there is a workgroup per compute unit at most.)
 template <int KT, int G, int W>
-__global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (GridColumns<KT, G>::RESIDENT)) fwd_grid(const FwdArgs a) {
+__global__ void __launch_bounds__(64 * (W == 1 ? KM_GROUP : W), (W == 8 ? 2 : GridColumns<KT, G>::RESIDENT)) fwd_grid(const FwdArgs a) {
     extern __shared__ float lds[];
     using C = GridColumns<KT, G>;
     const C c(a, a.items_per_xcd);
@@ -969,11 +999,28 @@ __global__ void __launch_bounds__(64 * KM_GROUP, (GridColumns<KT, G>::RESIDENT))
     }
 }
 
+// Few row blocks: their ranges in shares (launch_sum_shares adds up).
+template <int KT, int G>
+__global__ void __launch_bounds__(512, (G > 1 ? 2 : GridColumns<KT, G>::RESIDENT)) fwd_grid_shares(const FwdArgs a) {
+    extern __shared__ float lds[];
+    grid_item<KT, G, 8, true>(a, lds, 0, blockIdx.y * G * 16, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+}
+
+template <int KT, int G>
+static hipError_t launch_grid_shares(FwdArgs& a, const MatmulProblem& p, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
+    a.out = p.partials;
+    a.chunks_per_block = plan.shares;
+    a.total_items = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * a.num_batches;
+    hipLaunchKernelGGL((fwd_grid_shares<KT, G>), dim3((unsigned)(a.total_items * plan.shares), grid_y, 1), dim3(512, 1, 1),
+                       (sizeof(float) * item_lds_floats<KT, G, 8, true>()), stream, a);
+    const hipError_t err = hipGetLastError();
+    return err == hipSuccess ? launch_sum_shares(p, plan, stream) : err;
+}
+
 template <int KT, int G, int W>
 static hipError_t launch_grid_as(const FwdArgs& a, dim3 grid, hipStream_t stream) {
-    using S = typename GridColumns<KT, G>::Shape;
     hipLaunchKernelGGL((fwd_grid<KT, G, W>), grid, dim3(64 * W, 1, 1),
-                       (sizeof(float) * grid_lds_floats<S::GE, S::MT, W>()), stream, a);
+                       (sizeof(float) * item_lds_floats<KT, GridColumns<KT, G>::GROUPS, W>()), stream, a);
     return hipGetLastError();
 }
 
@@ -1021,6 +1068,14 @@ hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hi
     fill_fwd_args(p, &a);
     a.chunks_per_block = 1;
     const unsigned grid_y = (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk);
+    if (plan.shares > 1) {
+        if (p.kernel_type == KM_KERNEL_SPECTRAL) {
+            return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_SPECTRAL, 1>(a, p, plan, grid_y, stream)
+                                      : launch_grid_shares<KM_KERNEL_SPECTRAL, 2>(a, p, plan, grid_y, stream);
+        }
+        return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_RBF, 1>(a, p, plan, grid_y, stream)
+                                  : launch_grid_shares<KM_KERNEL_RBF, 2>(a, p, plan, grid_y, stream);
+    }
     if (p.kernel_type == KM_KERNEL_SPECTRAL) {
         return launch_grid_g<KM_KERNEL_SPECTRAL>(a, plan, grid_y, stream);
     }

@@ -39,6 +39,7 @@ struct MatmulProblem {
     const int32_t* end;
     const int64_t* end_strides;
     float* out;
+    float* partials;  // [shares][num_batches][m][k], if the plan has shares
 };
 
 // Which ahead-of-time instantiation runs and with what decomposition.
@@ -49,6 +50,7 @@ struct MatmulPlan {
     int col_splits;  // MFMA: wavefronts per workgroup sharing one column range (1, 2, 4, 8)
     int tail_balance;  // split-fp16 kernels: cut the uneven remainder into 16-row pieces
     int phase_split;   // KM_VARIANT_BLOCK: spectral kernel in phase-split form
+    int shares;        // workgroups that share each row block's range (1: none do)
     long long group_tail;  // table kernel: >= 0 selects the grouped launch (workgroups of 4 wavefronts) with
                            // this many items per XCD split by columns at the end; < 0: one wavefront per workgroup
     long long group_tail_halves;  // how many of those, the very last, also run as two halves of 64 rows
@@ -58,6 +60,7 @@ hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStre
 hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_periodic(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_grid_f32(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
+hipError_t launch_sum_shares(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_block(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 
 struct ParamGradProblem {

@@ -111,16 +111,19 @@ std::vector<int64_t> shape(c10::IntArrayRef batch, std::initializer_list<int64_t
 
 void check(int status) { TORCH_CHECK(status == KM_OK, km_last_error()); }
 
+Tensor workspace(size_t bytes, const Tensor& like) { return empty({(int64_t)(bytes > 0 ? bytes : 1)}, like, at::kByte); }
+
 Tensor matmul(const Matrix& a, const Tensor& rhs, const km_launch_options* options, const Tensor* into) {
     Tensor out = into ? *into : empty(shape(a.batch(), {a.m, rhs.size(-1)}), a.x1);
+    const size_t need = km_matmul_workspace_size(a.kernel, (int)a.rank, a.batch().data(), a.m, a.n, rhs.size(-1), options);
+    Tensor scratch = need > 0 ? workspace(need, a.x1) : Tensor();
     Launch on(a.device());
-    check(km_matmul(a.kernel, (int)a.rank, a.batch().data(), a.m, a.n, rhs.size(-1), data<float>(a.x1), strides(a.x1), data<float>(a.x2),
+    check(km_matmul_with_workspace(a.kernel, (int)a.rank, a.batch().data(), a.m, a.n, rhs.size(-1), data<float>(a.x1), strides(a.x1), data<float>(a.x2),
                     strides(a.x2), data<float>(rhs), strides(rhs), data<float>(a.params), strides(a.params), data<int32_t>(a.start),
-                    strides(a.start), data<int32_t>(a.end), strides(a.end), const_cast<float*>(data<float>(out)), options, on.stream()));
+                    strides(a.start), data<int32_t>(a.end), strides(a.end), const_cast<float*>(data<float>(out)), options,
+                                   need > 0 ? scratch.data_ptr() : nullptr, need, on.stream()));
     return out;
 }
-
-Tensor workspace(size_t bytes, const Tensor& like) { return empty({(int64_t)(bytes > 0 ? bytes : 1)}, like, at::kByte); }
 
 Tensor param_grad(const Matrix& a, const Tensor& left, const Tensor& right, const Tensor* into) {
     Tensor grad = into ? *into : empty(shape(a.batch(), {a.params.size(-1)}), a.x1);
