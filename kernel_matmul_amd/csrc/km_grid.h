@@ -20,6 +20,8 @@
 // make V(x, t) = 2^-(z_x - z_t)^2.
 #pragma once
 
+#include <type_traits>
+
 #include "km_common.h"
 #include "km_fwd.h"
 
@@ -798,15 +800,30 @@ __device__ __forceinline__ void grid_store(const FwdArgs& a, const WaveView& w, 
     if (row + 16 <= a.m && a.k <= (1 << 22)) {
         const buffer_rsrc to = uniform_buffer(out);
         const unsigned lane_bytes = 4u * (__umul24(4u * (unsigned)kk, (unsigned)a.k) + (unsigned)li);
+        float result[G][4];
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            if (kbase + 16 * g + li < a.k) {
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(value(g, v)), to, (int)(lane_bytes + 64u * g),
-                                                          (int)(4u * (unsigned)v * (unsigned)a.k), 0);
+            for (int v = 0; v < 4; v++) {
+                result[g][v] = value(g, v);
+            }
+        }
+        auto store = [&](auto streamed) {
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                if (kbase + 16 * g + li < a.k) {
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(result[g][v]), to, (int)(lane_bytes + 64u * g),
+                                                              (int)(4u * (unsigned)v * (unsigned)a.k), streamed ? 2 : 0);
+                    }
                 }
             }
+        };
+        if (a.stream_out != 0) {
+            store(std::true_type{});
+        } else {
+            store(std::false_type{});
         }
         return;
     }

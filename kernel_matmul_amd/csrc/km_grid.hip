@@ -1009,6 +1009,7 @@ __global__ void __launch_bounds__(512, (G > 1 ? 2 : GridColumns<KT, G>::RESIDENT
 template <int KT, int G>
 static hipError_t launch_grid_shares(FwdArgs& a, const MatmulProblem& p, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
     a.out = p.partials;
+    a.stream_out = 0;  // (read again)
     a.chunks_per_block = plan.shares;
     a.total_items = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * a.num_batches;
     hipLaunchKernelGGL((fwd_grid_shares<KT, G>), dim3((unsigned)(a.total_items * plan.shares), grid_y, 1), dim3(512, 1, 1),

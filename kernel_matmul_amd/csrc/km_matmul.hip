@@ -1359,6 +1359,12 @@ static hipError_t launch_valu(const FwdArgs& a, int KC, unsigned gx, unsigned gy
     return hipGetLastError();
 }
 
+// Results of up to this many values are stored past the caches (nontemporal): otherwise a launch ends with what the L2s still hold
+// of them being written back.  Measured, kept / past, us a call: rbf n = 65536, k = 64 21.8 / 20.0, spectral n = 1e5, 8 sets k = 16
+// 59.2 / 57.3, k = 32 101.2 / 97.8, n = 2e5 111.0 / 108.8, n = 20000, 4 sets 15.1 / 15.1 (14.8 / 14.4 with sets of their own).
+// Beyond half the last cache's size it depends on more than the size: n = 1e6, 8 sets, k = 32 869 / 837 with one result
+// written over and over, 782 / 817 with a new one for each call.
+#define KM_STREAM_OUT (32ll << 20)
 void fill_fwd_args(const MatmulProblem& p, FwdArgs* args) {
     FwdArgs& a = *args;
     const int r = p.batch_rank;
@@ -1389,6 +1395,7 @@ void fill_fwd_args(const MatmulProblem& p, FwdArgs* args) {
     a.chunks_per_block = 1;
     a.tail_items = 0;
     a.tail_half_items = 0;
+    a.stream_out = p.num_batches * p.m * p.k <= KM_STREAM_OUT;
 }
 
 hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream) {

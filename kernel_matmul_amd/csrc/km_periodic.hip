@@ -58,6 +58,7 @@ __global__ void __launch_bounds__(512, G == 1 ? 3 : 2) fwd_block_shares(const Fw
 template <int G>
 static hipError_t launch_periodic_shares(FwdArgs& a, const MatmulProblem& p, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
     a.out = p.partials;
+    a.stream_out = 0;  // (read again)
     a.chunks_per_block = plan.shares;
     a.total_items = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * a.num_batches;
     hipLaunchKernelGGL((fwd_block_shares<KM_KERNEL_LOCALLY_PERIODIC, G>), dim3((unsigned)(a.total_items * plan.shares), grid_y, 1), dim3(512, 1, 1), (sizeof(float) * entry_lds_floats(G, 8, 8)), stream, a);
