@@ -61,8 +61,8 @@ MEASURED_TRAFFIC_BYTES = {"headline": 60705292}
 # Share of the kernel's cycles in which the SIMDs' VALU is busy (SQ_ACTIVE_INST_VALU x 4 / SIMD
 # cycles), from the offline counter runs summarised under profiles/ (not measured by this script).
 VALU_BUSY = {
-    "headline": (0.54, "profiles/grid_form_kernels_profile.md"),
-    "headline_fp32": (0.46, "profiles/fwd_table_f32_grouped_headline_profile.md"),
+    "headline": (0.56, "profiles/operator_calls_profile.md"),
+    "headline_fp32": (0.34, "profiles/operator_calls_profile.md"),
     "c1": (0.11, "profiles/fwd_table_f16_midsize_c1_c2_c3_profile.md"),
     "c2": (0.29, "profiles/grid_form_kernels_profile.md"),
     "c3": (0.26, "profiles/param_grad_partial_c3_and_wide_vectors_profile.md"),
@@ -467,8 +467,8 @@ def main() -> int:
     }
 
     if default_run:
-        # The same workload with the contraction as a true fp32 MFMA (v_mfma_f32_16x16x4_f32): K
-        # evaluated in fp32 on the VALU, every product and sum of the contraction in fp32.
+        # The same workload with the contraction as a true fp32 MFMA (v_mfma_f32_16x16x4_f32): every
+        # factor evaluated in fp32 on the VALU, every product and sum of the contraction in fp32.
         f32_run = Prepared("headline", device, variant="mfma_f32")
         f32_timing = f32_run.measure(max(args.steps // 2, 5), 2)
         f32_ms, f32_out = f32_timing["kernel_ms"], f32_timing["out"]
@@ -476,9 +476,9 @@ def main() -> int:
             "kernel": f32_run.kernel,
             "pipe": pipe_of(f32_run.kernel),
             "valu_busy": VALU_BUSY["headline_fp32"][0],
-            "mfma_busy": 0.395,
+            "mfma_busy": 0.42,
             "busy_source": VALU_BUSY["headline_fp32"][1] + " (VALU and fp32-MFMA cycles are disjoint on gfx950: "
-                           "together 86 % of the kernel's cycles at batch 8, 95 % at batch 64)",
+                           "together 76 % of the kernel's cycles)",
             "kernel_ms": f32_ms,
             "frac": pairs * flops_per_pair / (f32_ms * 1e-3) / 1e12 / PEAK_FP32_TFLOPS,
             "back_to_back_kernel_ms": f32_timing["stream_ms"],
