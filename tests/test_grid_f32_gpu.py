@@ -121,7 +121,7 @@ def test_forms_of_coordinates_against_float64(kernel, form, density):
 
 
 @pytest.mark.parametrize("kernel", KERNELS)
-@pytest.mark.parametrize("m,n", [(1, 1), (128, 159), (128, 160), (129, 161), (385, 32)])
+@pytest.mark.parametrize("m,n", [(1, 1), (128, 95), (128, 96), (128, 159), (129, 161), (385, 32)])
 def test_ragged_and_short_ranges(kernel, m, n):
     batch = 130 // -(-m // 128) + 1
     args = _inputs(kernel, m, n, 5, batch)
