@@ -198,7 +198,11 @@ static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, 
     const int k_chunk = p.k <= 16 ? 16 : 32;
     const long long items = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * p.num_batches * ((p.k + k_chunk - 1) / k_chunk);
     const bool two_resident = spectral && k_chunk == 32;
-    if (items < (two_resident ? 400 : 120)) {
+    if (items < (two_resident ? 400 : 120) || p.k > 32LL * 65535) {  // (workgroups along y)
+        return false;
+    }
+    // (no more threads than a launch may have: two wavefronts a row block)
+    if (p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC && ((p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * p.num_batches + KM_NUM_XCD) * 128 > 0xffffffffLL) {
         return false;
     }
     plan->variant = KM_VARIANT_GRID_F32;
