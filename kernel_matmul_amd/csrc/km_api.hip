@@ -235,8 +235,11 @@ static bool shares_plan(const MatmulProblem& p, const km_launch_options* opt, Ma
     const int k_chunk = p.k <= 16 ? 16 : 32;
     const long long row_blocks = (p.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE;
     const long long items = row_blocks * p.num_batches * ((p.k + k_chunk - 1) / k_chunk);
+    if (items == 0 || items > 1024) {  // (descriptions are of empty problems too)
+        return false;
+    }
     const long long columns = p.n / row_blocks;
-    if (columns < 2048 || items > 1024) {
+    if (columns < 2048) {
         return false;
     }
     const long long most = columns / 512 < 128 ? columns / 512 : 128;

@@ -133,3 +133,12 @@ def test_launch_descriptions_without_a_gpu():
         _native.describe_param_grad("spectral", 1, -5, 4)
     with pytest.raises(RuntimeError, match="km_matmul_describe: invalid argument"):
         _native.describe_matmul("spectral", 1, -5, 10, 4)
+
+
+@pytest.mark.parametrize("kernel", ["rbf", "spectral", "locally_periodic"])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 5])
+@pytest.mark.parametrize("batches,m,n,k", [(0, 300, 9000, 4), (1, 0, 0, 1), (2, 0, 9000, 4), (1, 300, 0, 4), (1, 300, 9000, 0)])
+def test_descriptions_of_empty_problems(kernel, variant, batches, m, n, k):
+    """No rows, columns, right-hand sides or batch items: described, with nothing divided by their number."""
+    for options in (None, _native.LaunchOptions(variant=variant)):
+        assert "<" + kernel in _native.describe_matmul(kernel, batches, m, n, k, options)
