@@ -75,7 +75,7 @@ __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
     int row_block, split;
     const DenseView v = dense_view(a, item, a.col_splits, &row_block, &split);
     const int col_lo = split * a.cols_per_split;
-    const int col_hi = min(a.n, col_lo + a.cols_per_split);
+    const int col_hi = col_lo + min(a.n - col_lo, a.cols_per_split);
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int row_begin = row_block * KM_BLOCK_SIZE + wave * 32;
@@ -86,12 +86,13 @@ __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
     const KernelConsts kc = make_consts<KT>(v.params, a.params_s, true);
     float* __restrict__ out = a.out + v.b * (long long)a.m * a.n + (long long)row_begin * a.n;
     const int x1_bits = __float_as_int(v.x1[(long long)(row_begin + min(lane, rows - 1)) * a.x1_s]);
-    for (int col0 = col_lo; col0 < col_hi; col0 += 64 * V) {
-        const int col = col0 + V * lane;
-        const bool in_matrix = col < col_hi;  // (with all V: their number divides that of the columns)
+    // (compared by differences: what follows the last columns may lie past the largest int)
+    for (int col0 = col_lo;; col0 += 64 * V) {
+        const bool in_matrix = V * lane < col_hi - col0;  // (with all V: their number divides that of the columns)
+        const int col = in_matrix ? col0 + V * lane : col0;
         float* __restrict__ o = out + col;
         // Wave-uniform choice: column tiles fully outside the range are only cleared.
-        if (col0 < v.range_end && col0 + 64 * V > v.range_start) {
+        if (col0 < v.range_end && v.range_start - col0 < 64 * V) {
             float x2v[V];
             bool in_range[V];
 #pragma unroll
@@ -115,6 +116,9 @@ __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
             for (int r = 0; r < rows; r++) {
                 *(Vec*)(o + (long long)r * a.n) = (Vec)(0.0f);
             }
+        }
+        if (col_hi - col0 <= 64 * V) {
+            return;
         }
     }
 }

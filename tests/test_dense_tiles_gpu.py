@@ -59,3 +59,13 @@ def test_tiles(kernel, batch, m, n):
         size = abs(terms).max(axis=(1, 2)) * np.count_nonzero(terms, axis=(1, 2)) ** 0.5  # (of a sum of random signs)
         difference = abs(grads[0][b].cpu().double().numpy() - terms.sum(axis=(1, 2)))
         assert (difference <= RELATIVE * size + 1e-12).all()
+
+
+@pytest.mark.parametrize("n", [2 ** 31 - 132, 2 ** 31 - 129, 2 ** 31 - 256])
+def test_columns_up_to_the_largest_number(n):
+    """The columns behind the last ones of a matrix lie past the largest int.  Points in one place: every entry is one."""
+    x1, x2 = torch.zeros(1, device=DEVICE), torch.zeros(1, device=DEVICE).expand(n)
+    start, end = torch.tensor([5], dtype=torch.int32, device=DEVICE), torch.tensor([n - 3], dtype=torch.int32, device=DEVICE)
+    dense = _native.dense("rbf", x1, x2, torch.ones(2, device=DEVICE), start, end)[0]
+    assert not dense[:5].any() and not dense[-3:].any()
+    assert int((dense == 1).sum()) == n - 8
