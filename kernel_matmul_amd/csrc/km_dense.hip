@@ -144,8 +144,10 @@ __global__ void __launch_bounds__(64 * KM_DENSE_BWD_WAVES) dense_bwd_partial(con
 
     const int width = max(v.range_end - v.range_start, 0);
     const int per_split = ((width + a.col_splits - 1) / a.col_splits + 63) & ~63;
-    const int col_begin = v.range_start + split * per_split;
-    const int col_end = min(v.range_end, col_begin + per_split);
+    // (shares past the last column are empty, and may begin past the largest int)
+    const int range_end = max(v.range_end, v.range_start);
+    const int col_begin = (int)min(v.range_start + (long long)split * per_split, (long long)range_end);
+    const int col_end = col_begin + min(per_split, range_end - col_begin);
     const int row_begin = row_block * KM_BLOCK_SIZE + wave * KM_DENSE_BWD_ROWS;
     const int rows = min(KM_DENSE_BWD_ROWS, a.m - row_begin);
 

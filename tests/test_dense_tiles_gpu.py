@@ -69,3 +69,16 @@ def test_columns_up_to_the_largest_number(n):
     dense = _native.dense("rbf", x1, x2, torch.ones(2, device=DEVICE), start, end)[0]
     assert not dense[:5].any() and not dense[-3:].any()
     assert int((dense == 1).sum()) == n - 8
+
+
+def test_gradient_of_ranges_up_to_the_largest_number_of_columns():
+    """Shares of a short range that begin behind it lie past the largest int.  Points in one place: an entry's derivative
+    by the output scale is one, by the lengthscale zero."""
+    n = 2 ** 31 - 129
+    x1, x2 = torch.zeros(1, device=DEVICE), torch.zeros(1, device=DEVICE).expand(n)
+    weights = torch.ones(1, 1, device=DEVICE).expand(1, n)
+    for first in (n - 100, n - 1000, n - 2 ** 20):
+        start, end = (torch.tensor([i], dtype=torch.int32, device=DEVICE) for i in (first, n))
+        grad = _native.dense_bwd("rbf", x1, x2, torch.ones(2, device=DEVICE), start, end, weights)
+        # (whole numbers: exact)
+        assert grad.tolist() == [0.0, n - first]
