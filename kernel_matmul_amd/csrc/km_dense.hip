@@ -16,6 +16,7 @@ struct DenseArgs {
     BatchShape batch;
     long long num_batches;
     long long total_items;  // row blocks * col splits * batches
+    long long first_item, launch_items;  // of these, the ones of a launch (dense_bwd)
     long long items_per_xcd;
     int m, n;
     int col_splits;
@@ -129,15 +130,16 @@ __global__ void __launch_bounds__(256) dense_kernel(const DenseArgs a) {
 // 2500 columns a row block 17.0 -> 12.6 / 43.9 -> 24.3 us; n = 20000, all columns 385 -> 311 (5.2 TB/s).
 #define KM_DENSE_BWD_ROWS 16
 #define KM_DENSE_BWD_WAVES (KM_BLOCK_SIZE / KM_DENSE_BWD_ROWS)
+#define KM_DENSE_BWD_LAUNCH (1ll << 22) /* workgroups at a time: 2^31 threads */
 template <int KT>
 __global__ void __launch_bounds__(64 * KM_DENSE_BWD_WAVES) dense_bwd_partial(const DenseArgs a) {
     __shared__ float sums[KM_DENSE_BWD_WAVES][KM_MAX_PARAMS];
     const long long item = xcd_item(blockIdx.x, a.items_per_xcd);
-    if (item >= a.total_items) {
+    if (item >= a.launch_items) {
         return;
     }
     int row_block, split;
-    const DenseView v = dense_view(a, item, a.col_splits, &row_block, &split);
+    const DenseView v = dense_view(a, a.first_item + item, a.col_splits, &row_block, &split);
     const KernelConsts kc = make_consts<KT>(v.params, a.params_s, false);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -282,9 +284,11 @@ hipError_t launch_dense_bwd(const DenseProblem& p, hipStream_t stream) {
     if (a.col_splits > shares) a.col_splits = (int)shares;
     if (a.col_splits < 1) a.col_splits = 1;
     a.total_items = row_blocks * a.col_splits * p.num_batches;
-    a.items_per_xcd = (a.total_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
-    const unsigned grid = (unsigned)(a.items_per_xcd * KM_NUM_XCD);
-    if (grid > 0) {
+    // (a launch may have 2^32 - 1 threads)
+    for (a.first_item = 0; a.first_item < a.total_items; a.first_item += KM_DENSE_BWD_LAUNCH) {
+        a.launch_items = a.total_items - a.first_item < KM_DENSE_BWD_LAUNCH ? a.total_items - a.first_item : KM_DENSE_BWD_LAUNCH;
+        a.items_per_xcd = (a.launch_items + KM_NUM_XCD - 1) / KM_NUM_XCD;
+        const unsigned grid = (unsigned)(a.items_per_xcd * KM_NUM_XCD);
         switch (p.kernel_type) {
             case KM_KERNEL_RBF:
                 hipLaunchKernelGGL((dense_bwd_partial<KM_KERNEL_RBF>), dim3(grid), dim3(64 * KM_DENSE_BWD_WAVES), 0, stream, a);

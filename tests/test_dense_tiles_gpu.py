@@ -82,3 +82,12 @@ def test_gradient_of_ranges_up_to_the_largest_number_of_columns():
         grad = _native.dense_bwd("rbf", x1, x2, torch.ones(2, device=DEVICE), start, end, weights)
         # (whole numbers: exact)
         assert grad.tolist() == [0.0, n - first]
+
+
+def test_gradient_of_more_row_blocks_than_a_launch_takes():
+    """Eight wavefronts each for 2^23 row blocks and more are more threads than a launch may have.  Points in one place."""
+    m = 2 ** 30 + 1024
+    x1, x2 = torch.zeros(1, device=DEVICE).expand(m), torch.zeros(1, device=DEVICE)
+    start, end = (torch.full((1,), i, dtype=torch.int32, device=DEVICE).expand(m // 128) for i in (0, 1))
+    grad = _native.dense_bwd("rbf", x1, x2, torch.ones(2, device=DEVICE), start, end, torch.ones(1, 1, device=DEVICE).expand(m, 1))
+    assert grad.tolist() == [0.0, m]  # (whole numbers: exact)
