@@ -308,18 +308,23 @@ bool watched() {
     return (debug && std::strcmp(debug, "true") == 0) || (sizes && std::strcmp(sizes, "true") == 0);
 }
 
+// (all that is asked of the interpreter is asked here, while its lock is held)
 struct Arguments {
     PyObject* const* args;
-    Py_ssize_t count;
+    int64_t kernel;
     bool ok;
 
-    Arguments(PyObject* const* args_, Py_ssize_t count_, Py_ssize_t tensors, Py_ssize_t expected)
-        : args(args_), count(count_), ok(count_ == expected && PyLong_Check(args_[0])) {
+    Arguments(PyObject* const* args_, Py_ssize_t count, Py_ssize_t tensors, Py_ssize_t expected)
+        : args(args_), kernel(-1), ok(count == expected && PyLong_Check(args_[0])) {
+        if (ok) {
+            int overflow = 0;
+            kernel = PyLong_AsLongLongAndOverflow(args[0], &overflow);
+            ok = overflow == 0 && km_num_params((int)kernel) > 0 && kernel == (int)kernel;
+        }
         for (Py_ssize_t i = 1; ok && i <= tensors; i++) {
             ok = THPVariable_Check(args[i]);
         }
     }
-    int64_t kernel() const { return PyLong_AsLongLong(args[0]); }
     const Tensor& operator[](Py_ssize_t i) const { return THPVariable_Unpack(args[i]); }
 };
 
@@ -356,7 +361,7 @@ PyObject* py_matmul(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[4], t[5], t[6]);
+    Matrix a(t.kernel, t[1], t[2], t[4], t[5], t[6]);
     const Tensor& rhs = t[3];
     const Tensor* into;
     if (!a.fits() || !a.has_vectors(rhs, a.n) || !result_tensor(args[8], a, {a.m, rhs.size(-1)}, &into)) {
@@ -374,11 +379,11 @@ PyObject* py_matmul_recorded(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (!t.ok || watched()) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[4], t[5], t[6]);
+    Matrix a(t.kernel, t[1], t[2], t[4], t[5], t[6]);
     if (!a.fits() || !a.has_vectors(t[3], a.n)) {
         return none();
     }
-    return launched([&] { return MatmulNode::apply(t[1], t[2], t[3], t[4], t[5], t[6], t.kernel()); });
+    return launched([&] { return MatmulNode::apply(t[1], t[2], t[3], t[4], t[5], t[6], t.kernel); });
     END_HANDLE_TH_ERRORS
 }
 
@@ -389,7 +394,7 @@ PyObject* py_param_grad(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[5], t[6], t[7]);
+    Matrix a(t.kernel, t[1], t[2], t[5], t[6], t[7]);
     const Tensor &left = t[3], &right = t[4];
     const Tensor* into;
     if (!a.fits() || !a.has_vectors(left, a.m) || !a.has_vectors(right, a.n) || left.size(-1) != right.size(-1) ||
@@ -408,11 +413,11 @@ PyObject* py_dense(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok || (RECORD && watched())) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[3], t[4], t[5]);
+    Matrix a(t.kernel, t[1], t[2], t[3], t[4], t[5]);
     if (!a.fits()) {
         return none();
     }
-    return launched([&] { return RECORD ? DenseNode::apply(t[1], t[2], t[3], t[4], t[5], t.kernel()) : dense(a); });
+    return launched([&] { return RECORD ? DenseNode::apply(t[1], t[2], t[3], t[4], t[5], t.kernel) : dense(a); });
     END_HANDLE_TH_ERRORS
 }
 
@@ -423,7 +428,7 @@ PyObject* py_dense_bwd(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[3], t[4], t[5]);
+    Matrix a(t.kernel, t[1], t[2], t[3], t[4], t[5]);
     if (!a.fits() || !fits_matrix(a, t[6])) {
         return none();
     }
@@ -455,13 +460,13 @@ PyObject* py_index(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok || (RECORD && watched())) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[3], t[4], t[5]);
+    Matrix a(t.kernel, t[1], t[2], t[3], t[4], t[5]);
     Indices i;
     if (!a.fits() || !read_indices(args[8], t[6], t[7], &i) || !i.fit(a)) {
         return none();
     }
     return launched([&] {
-        return RECORD ? IndexNode::apply(t[1], t[2], t[3], t[4], t[5], t.kernel(), i.row, i.col, at::TensorList(i.batch)) : index(a, i);
+        return RECORD ? IndexNode::apply(t[1], t[2], t[3], t[4], t[5], t.kernel, i.row, i.col, at::TensorList(i.batch)) : index(a, i);
     });
     END_HANDLE_TH_ERRORS
 }
@@ -473,7 +478,7 @@ PyObject* py_index_bwd(PyObject*, PyObject* const* args, Py_ssize_t count) {
     if (!t.ok) {
         return none();
     }
-    Matrix a(t.kernel(), t[1], t[2], t[3], t[4], t[5]);
+    Matrix a(t.kernel, t[1], t[2], t[3], t[4], t[5]);
     Indices i;
     if (!a.fits() || !read_indices(args[9], t[6], t[7], &i) || !i.fit(a) || !fits_indices(a, i, t[8])) {
         return none();

@@ -49,3 +49,16 @@ def test_watched_calls_and_own_functions_take_the_general_path(monkeypatch):
         _native_dense = None
 
     assert make(Own)._calls("_native_dense") is None and make(Own)._calls("_native_matmul") is not None
+
+
+@pytest.mark.parametrize("number", [-1, 3, 2 ** 32 + 1, 2 ** 70, -2 ** 70])
+def test_numbers_that_are_no_kernels_are_handed_back(number):
+    calls = _native.torch_calls()
+    x1, x2, rhs, params, start, end = _args()
+    matrix = (number, x1, x2, params, start, end)
+    assert calls.matmul(number, x1, x2, rhs, params, start, end, None, None) is None
+    assert calls.matmul_recorded(number, x1, x2, rhs, params, start, end) is None
+    assert calls.param_grad(number, x1, x2, rhs, rhs, params, start, end, None) is None
+    assert calls.dense(*matrix) is None and calls.dense_recorded(*matrix) is None and calls.dense_bwd(*matrix, rhs) is None
+    assert calls.index(*matrix, start, start, ()) is None and calls.index_recorded(*matrix, start, start, ()) is None
+    assert calls.index_bwd(*matrix, start, start, x1, ()) is None
