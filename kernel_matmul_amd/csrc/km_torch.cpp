@@ -539,7 +539,8 @@ PyObject* py_make_ranges(PyObject*, PyObject* const* args, Py_ssize_t count) {
         return none();
     }
     const Tensor& x2 = symmetric ? x1 : THPVariable_Unpack(args[2]);
-    const int64_t block = PyLong_AsLongLong(args[3]);
+    int overflow = 0;
+    const int64_t block = PyLong_AsLongLongAndOverflow(args[3], &overflow);  // (-1 where it does not fit)
     const bool align = args[4] == Py_True;
     if (!x1.is_cuda() || !is_plain(x1, at::kFloat, x1.device()) || !is_plain(x2, at::kFloat, x1.device()) || !x1.is_contiguous() ||
         !x2.is_contiguous() || x1.dim() < 1 || x1.dim() > 2 || x2.dim() != x1.dim() || x1.numel() == 0 || x2.numel() == 0 ||

@@ -62,3 +62,10 @@ def test_numbers_that_are_no_kernels_are_handed_back(number):
     assert calls.dense(*matrix) is None and calls.dense_recorded(*matrix) is None and calls.dense_bwd(*matrix, rhs) is None
     assert calls.index(*matrix, start, start, ()) is None and calls.index_recorded(*matrix, start, start, ()) is None
     assert calls.index_bwd(*matrix, start, start, x1, ()) is None
+
+
+@pytest.mark.parametrize("block_size", [0, -1, 2 ** 31, 2 ** 70, -2 ** 70])
+def test_block_sizes_that_are_none_are_handed_back(block_size):
+    x = torch.arange(200.0)
+    assert _native.torch_calls().make_ranges(1.0, x, None, block_size, False) is None
+    assert _native.torch_calls().make_ranges(1.0, x, x, block_size, True) is None
