@@ -524,6 +524,25 @@ PyObject* py_views(PyObject*, PyObject* const* args, Py_ssize_t count) {
     END_HANDLE_TH_ERRORS
 }
 
+// Waits for what was launched, also where a later step throws: the host's memory that it writes is given back then.
+class Settled {
+  public:
+    explicit Settled(void* stream) : stream_(static_cast<hipStream_t>(stream)) {}
+    ~Settled() {
+        if (!done_) {
+            (void)hipStreamSynchronize(stream_);
+        }
+    }
+    hipError_t wait() {
+        done_ = true;
+        return hipStreamSynchronize(stream_);
+    }
+
+  private:
+    hipStream_t stream_;
+    bool done_ = false;
+};
+
 // make_ranges(cutoff, x1, x2 or None, block size, align) -> (start, end) of contiguous float32 device tensors [n] or
 // [batch, n] that ascend; None for all others.  The check's words are written to host memory, and one wait covers check
 // and builder.
@@ -558,6 +577,7 @@ PyObject* py_make_ranges(PyObject*, PyObject* const* args, Py_ssize_t count) {
         Tensor words = at::empty({KM_SORTED_FLAGS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
         int32_t* descents = static_cast<int32_t*>(words.data_ptr());
         Launch on(x1.device());
+        Settled settled(on.stream());
         int32_t *s = static_cast<int32_t*>(start.data_ptr()), *e = static_cast<int32_t*>(end.data_ptr());
         if (symmetric) {
             check(km_check_sorted_device(data<float>(x1), batch, n1, nullptr, 0, 0, descents, on.stream()));
@@ -566,7 +586,7 @@ PyObject* py_make_ranges(PyObject*, PyObject* const* args, Py_ssize_t count) {
             check(km_make_ranges_checked_device(data<float>(x1), data<float>(x2), batch, n1, n2, cutoff, (int)block, align, s, e,
                                                 descents, on.stream()));
         }
-        const hipError_t error = hipStreamSynchronize(static_cast<hipStream_t>(on.stream()));
+        const hipError_t error = settled.wait();
         TORCH_CHECK(error == hipSuccess, "make_ranges: ", hipGetErrorString(error));
         for (int i = 0; i < KM_SORTED_FLAGS; i++) {
             ascending = ascending && descents[i] == 0;

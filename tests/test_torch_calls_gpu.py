@@ -184,3 +184,14 @@ def test_ranges(two, batch, kind, align):
     for cutoff in (2.0, 2):
         got = make_ranges(cutoff, x1.to(DEVICE), x2.to(DEVICE) if two else None, align=align)
         assert all(torch.equal(a.cpu(), b) and a.is_cuda for a, b in zip(got, expected))
+
+
+def test_refused_ranges_leave_no_launch_behind():
+    """The order check writes to host memory that goes back to its pool: a builder that refuses the block size behind it
+    waits for it."""
+    x = torch.arange(200.0, device=DEVICE)
+    make_ranges(2.0, x)
+    torch.cuda._sleep(200_000_000)
+    with pytest.raises(RuntimeError, match="sizes out of range"):
+        make_ranges(2.0, x, block_size=2 ** 31 - 1)
+    assert torch.cuda.current_stream().query()
