@@ -240,7 +240,7 @@ class _Native:
             return self
         pool = {"compile_pool": operator._compile_pool} if self._autotuned else {}
         function = NativeFunction(self._op, self._configuration(operator._kernel_type), **pool)
-        operator.__dict__[self._name] = function
+        operator.__dict__[self._name] = operator._made[self._name] = function
         return function
 
 
@@ -302,6 +302,7 @@ class KernelMatmulLinearOperator(LinearOperator):
         self._ranges_t = None  # pattern of the transpose, built on first use
         self._diagonal_indices = None  # index tensors of the diagonal, built on first use
         self._native_args = None  # (batch shape, widened constructor tensors) of the last call
+        self._made = {}  # the native functions made so far (_Native)
 
     # -- helpers -------------------------------------------------------------------------
     # The constructor tensors as stride-0 views of the batch shape.
@@ -315,7 +316,8 @@ class KernelMatmulLinearOperator(LinearOperator):
         """The native module of calls on tensors, if nothing asks for the native functions of these names: they are
         the operator's own and nobody has taken them in hand, and their modules would watch no call."""
         for name in functions:
-            if name in self.__dict__ or getattr(type(self), name) is not KernelMatmulLinearOperator.__dict__[name]:
+            if (self.__dict__.get(name, self) is not self._made.get(name, self)
+                    or getattr(type(self), name) is not KernelMatmulLinearOperator.__dict__[name]):
                 return None
         calls = _native.torch_calls()
         return None if calls.watched() else calls

@@ -69,3 +69,14 @@ def test_block_sizes_that_are_none_are_handed_back(block_size):
     x = torch.arange(200.0)
     assert _native.torch_calls().make_ranges(1.0, x, None, block_size, False) is None
     assert _native.torch_calls().make_ranges(1.0, x, x, block_size, True) is None
+
+
+def test_native_functions_that_the_operator_made_itself_are_its_own():
+    x = torch.zeros(200, 1)
+    K = KernelMatmulLinearOperator(x, x, torch.ones(3), torch.zeros(2), torch.zeros(2), kernel_type="spectral", symmetric=True)
+    function = K._native_matmul
+    assert K._native_matmul is function and K._calls("_native_matmul", "_native_matmul_bwd") is not None
+    K._native_matmul = lambda *args: function(*args)
+    assert K._calls("_native_matmul") is None
+    K._native_matmul = function
+    assert K._calls("_native_matmul") is not None
