@@ -221,7 +221,12 @@ static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, 
 }
 
 // Few rows against many points (predictions): a row block's range spans the points between its rows, of which the columns per
-// row block are what the sizes tell.  A workgroup of eight wavefronts for each share of the ranges, then the sum of the shares;
+// row block are what the sizes tell.  Rows that are neighbours (forecasts) have short ranges all the same: the kernels find
+// one share in them, leave the other workgroups and the sums out and cost what is left of that, while ranges that are long
+// without shares leave most of the device idle for as long as one workgroup takes.  Near, none / shares, us a call, n = 1e6, 10 points
+// per unit, cutoff of 9 units: rbf m = 100, k = 1 5.0 / 9.2, m = 128, k = 16, 4 sets 5.3 / 10.8, m = 1000, k = 1 5.5 / 10.6 (with every
+// share writing its zeros, and all of them added, 14.3 / 14.5 / 12.3), spectral 5.4 / 9.3, 5.6 / 12.5, 5.9 / 11.9, locally
+// periodic 5.6 / 9.5, 5.8 / 10.6, 6.1 / 11.1.  A workgroup of eight wavefronts for each share of the ranges, then the sum of the shares;
 // the number of shares is the one for which rounds of 256 workgroups, each as long as its share and a start (what 1500 columns
 // out of reach take), are over first.  Measured, none (the forms below) against the shares taken, us a call, rbf: m = 100, n = 5000
 // 22.8 / 11.6, n = 20000 75 / 12.8, n = 1e6 4926 / 36, m = 1000, n = 30000 20.4 / 12.7 (4 sets), n = 1e5 59.7 / 23.1 (8 sets),

@@ -61,12 +61,15 @@ struct FwdArgs {
     float* out;
     BatchStrides x1_bs, x2_bs, rhs_bs, params_bs, start_bs, end_bs;
     long long x1_s, x2_s, rhs_s0, rhs_s1, params_s, start_s, end_s;
+    float* partials;         // sums of the shares of a range (share_view)
 };
 
 struct MatmulProblem;
 // Collapses the batch dimensions and copies pointers, sizes and strides (item counts are left
 // to the caller).
 void fill_fwd_args(const MatmulProblem& p, FwdArgs* args);
+// The sums of ranges in several shares (share_view), after the launch that made them.
+hipError_t launch_sum_shares(const FwdArgs& a, hipStream_t stream);
 
 // The split-fp16 kernels evaluate K / sigma scaled by 2^14 (folded into the exponent of the
 // base-2 exponential) so that its hi and lo halves stay inside the fp16 exponent range.
@@ -348,22 +351,38 @@ __device__ __forceinline__ WaveView wave_view(const FwdArgs& a, long long item, 
     return w;
 }
 
-// Launches of few row blocks with long ranges: a.chunks_per_block workgroups in a row take a piece of a range each, in whole
-// steps and no shorter than this, and write sums of their own, as a batch item further on.  (Neighbouring workgroups run on
-// different XCDs, and pieces have nothing in common.)
+// Launches of few row blocks whose ranges may be long: a.chunks_per_block workgroups in a row take a share of a range each, in
+// whole steps and no shorter than this, as many as there are; sum_shares adds up.  The sizes do not tell a long range from a short
+// one, which is one share, written to the result at once: the other workgroups return when they have read the range.
+// (Neighbouring workgroups run on different XCDs, and shares have nothing in common.)
 #define KM_SHARE_COLUMNS 512
-__device__ __forceinline__ WaveView share_view(const FwdArgs& a) {
-    const unsigned shares = (unsigned)a.chunks_per_block;
-    const unsigned item = blockIdx.x / shares, share = blockIdx.x - item * shares;
+struct ShareOf {
+    int each, present;  // columns of a share, shares
+};
+__device__ __forceinline__ ShareOf shares_of(int columns, int most) {
+    ShareOf s;
+    s.each = max((columns / most + 256) & ~255, KM_SHARE_COLUMNS);
+    s.present = columns > 0 ? (columns - 1) / s.each + 1 : 1;
+    return s;
+}
+
+// The share of this workgroup; false if there is none.  Sums of several go to partials, as a batch item further on each.
+__device__ __forceinline__ bool share_view(const FwdArgs& a, WaveView* w, float** out) {
+    const unsigned most = (unsigned)a.chunks_per_block;
+    const unsigned item = blockIdx.x / most, share = blockIdx.x - item * most;
     int unused;
-    WaveView w = wave_view<true>(a, item, 1, &unused);
-    const int length = max(w.range_end - w.range_start, 0);
-    const int each = max((length / (int)shares + 256) & ~255, KM_SHARE_COLUMNS);
-    const long long first = min((long long)share * each, (long long)length);
-    w.range_end = w.range_start + (int)min(first + each, (long long)length);
-    w.range_start += (int)first;
-    w.b += (long long)share * a.num_batches;
-    return w;
+    *w = wave_view<true>(a, item, 1, &unused);
+    const int columns = max(w->range_end - w->range_start, 0);
+    const ShareOf s = shares_of(columns, (int)most);
+    if ((int)share >= s.present) {
+        return false;
+    }
+    const int first = (int)share * s.each;
+    w->range_start += first;
+    w->range_end = w->range_start + min(s.each, columns - first);
+    w->b += (long long)share * a.num_batches;
+    *out = s.present > 1 ? a.partials : a.out;
+    return true;
 }
 
 // Work item of this workgroup.  Items are (row chunk, batch item) pairs, contiguous ranges of

@@ -426,10 +426,8 @@ __device__ __forceinline__ void grid_entrywise(const FwdArgs& a, float* lds, con
 // One item by W wavefronts (this one is number `wave`) for rhs columns [kbase, kbase + 16 G): the grid form, or
 // entry by entry.
 template <int KT, int G, int W, bool SHARES = false>
-__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int kbase, int wave) {
+__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, const WaveView& w, int kbase, int wave) {
     using S = GridShape<KT, G>;
-    int unused;
-    const WaveView w = SHARES ? share_view(a) : wave_view<true>(a, item, 1, &unused);
     const int row0 = w.row_block * KM_BLOCK_SIZE;
     // The rows are requested first, then the first columns (which wait for the range), then the
     // window is computed.
@@ -459,6 +457,12 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
             }
         }
     }
+}
+
+template <int KT, int G, int W>
+__device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long long item, int kbase, int wave) {
+    int unused;
+    grid_item<KT, G, W>(a, lds, wave_view<true>(a, item, 1, &unused), kbase, wave);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1003,19 +1007,23 @@ __global__ void __launch_bounds__(64 * KM_GROUP, (GridColumns<KT, G>::RESIDENT))
 template <int KT, int G>
 __global__ void __launch_bounds__(512, (G > 1 ? 2 : GridColumns<KT, G>::RESIDENT)) fwd_grid_shares(const FwdArgs a) {
     extern __shared__ float lds[];
-    grid_item<KT, G, 8, true>(a, lds, 0, blockIdx.y * G * 16, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    FwdArgs f = a;
+    WaveView w;
+    if (!share_view(a, &w, &f.out)) {
+        return;
+    }
+    grid_item<KT, G, 8, true>(f, lds, w, blockIdx.y * G * 16, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
 }
 
 template <int KT, int G>
-static hipError_t launch_grid_shares(FwdArgs& a, const MatmulProblem& p, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
-    a.out = p.partials;
+static hipError_t launch_grid_shares(FwdArgs& a, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
     a.stream_out = 0;  // (read again)
     a.chunks_per_block = plan.shares;
     a.total_items = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * a.num_batches;
     hipLaunchKernelGGL((fwd_grid_shares<KT, G>), dim3((unsigned)(a.total_items * plan.shares), grid_y, 1), dim3(512, 1, 1),
                        (sizeof(float) * item_lds_floats<KT, G, 8, true>()), stream, a);
     const hipError_t err = hipGetLastError();
-    return err == hipSuccess ? launch_sum_shares(p, plan, stream) : err;
+    return err == hipSuccess ? launch_sum_shares(a, stream) : err;
 }
 
 template <int KT, int G, int W>
@@ -1071,11 +1079,11 @@ hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hi
     const unsigned grid_y = (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk);
     if (plan.shares > 1) {
         if (p.kernel_type == KM_KERNEL_SPECTRAL) {
-            return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_SPECTRAL, 1>(a, p, plan, grid_y, stream)
-                                      : launch_grid_shares<KM_KERNEL_SPECTRAL, 2>(a, p, plan, grid_y, stream);
+            return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_SPECTRAL, 1>(a, plan, grid_y, stream)
+                                      : launch_grid_shares<KM_KERNEL_SPECTRAL, 2>(a, plan, grid_y, stream);
         }
-        return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_RBF, 1>(a, p, plan, grid_y, stream)
-                                  : launch_grid_shares<KM_KERNEL_RBF, 2>(a, p, plan, grid_y, stream);
+        return plan.k_chunk == 16 ? launch_grid_shares<KM_KERNEL_RBF, 1>(a, plan, grid_y, stream)
+                                  : launch_grid_shares<KM_KERNEL_RBF, 2>(a, plan, grid_y, stream);
     }
     if (p.kernel_type == KM_KERNEL_SPECTRAL) {
         return launch_grid_g<KM_KERNEL_SPECTRAL>(a, plan, grid_y, stream);

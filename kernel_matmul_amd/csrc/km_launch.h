@@ -60,7 +60,6 @@ hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStre
 hipError_t launch_matmul_grid(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_periodic(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_grid_f32(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
-hipError_t launch_sum_shares(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 hipError_t launch_matmul_block(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream);
 
 struct ParamGradProblem {

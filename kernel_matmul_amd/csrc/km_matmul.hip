@@ -1383,6 +1383,7 @@ void fill_fwd_args(const MatmulProblem& p, FwdArgs* args) {
     a.start = p.start;
     a.end = p.end;
     a.out = p.out;
+    a.partials = p.partials;
     a.x1_s = p.x1_strides[r];
     a.x2_s = p.x2_strides[r];
     a.rhs_s0 = p.rhs_strides[r];

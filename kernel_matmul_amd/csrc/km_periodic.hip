@@ -51,19 +51,21 @@ __global__ void __launch_bounds__(64 * W, G == 1 ? 3 : 2) fwd_block(const FwdArg
 template <int KT, int G>
 __global__ void __launch_bounds__(512, G == 1 ? 3 : 2) fwd_block_shares(const FwdArgs a) {
     extern __shared__ float lds[];
-    const WaveView w = share_view(a);
-    entry_item<KT, false, G, 8, 8>(a, lds, w, w.row_block * KM_BLOCK_SIZE, blockIdx.y * G * 16, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
+    FwdArgs f = a;
+    WaveView w;
+    if (!share_view(a, &w, &f.out)) {
+        return;
+    }
+    entry_item<KT, false, G, 8, 8>(f, lds, w, w.row_block * KM_BLOCK_SIZE, blockIdx.y * G * 16, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6));
 }
 
 template <int G>
-static hipError_t launch_periodic_shares(FwdArgs& a, const MatmulProblem& p, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
-    a.out = p.partials;
-    a.stream_out = 0;  // (read again)
+static hipError_t launch_periodic_shares(FwdArgs& a, const MatmulPlan& plan, unsigned grid_y, hipStream_t stream) {
     a.chunks_per_block = plan.shares;
     a.total_items = ((long long)a.m + KM_BLOCK_SIZE - 1) / KM_BLOCK_SIZE * a.num_batches;
     hipLaunchKernelGGL((fwd_block_shares<KM_KERNEL_LOCALLY_PERIODIC, G>), dim3((unsigned)(a.total_items * plan.shares), grid_y, 1), dim3(512, 1, 1), (sizeof(float) * entry_lds_floats(G, 8, 8)), stream, a);
     const hipError_t err = hipGetLastError();
-    return err == hipSuccess ? launch_sum_shares(p, plan, stream) : err;
+    return err == hipSuccess ? launch_sum_shares(a, stream) : err;
 }
 
 template <int G, int R, int W>
@@ -94,7 +96,7 @@ hipError_t launch_matmul_periodic(const MatmulProblem& p, const MatmulPlan& plan
     fill_fwd_args(p, &a);
     const unsigned grid_y = (unsigned)((p.k + plan.k_chunk - 1) / plan.k_chunk);
     if (plan.shares > 1) {
-        return plan.k_chunk == 16 ? launch_periodic_shares<1>(a, p, plan, grid_y, stream) : launch_periodic_shares<2>(a, p, plan, grid_y, stream);
+        return plan.k_chunk == 16 ? launch_periodic_shares<1>(a, plan, grid_y, stream) : launch_periodic_shares<2>(a, plan, grid_y, stream);
     }
     switch (plan.k_chunk / 16) {
         case 1: return plan.row_groups == 2 ? launch_periodic_as<1, 2, 8>(a, grid_y, stream) : launch_periodic_w<1, 8>(a, plan, grid_y, stream);

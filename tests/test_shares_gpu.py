@@ -150,3 +150,28 @@ def test_without_scratch_and_under_capture(kernel):
         torch.cuda.synchronize()
         assert torch.equal(captured, want)
         torch.randn(100000, device=DEVICE).sum().item()
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
+@pytest.mark.parametrize("columns", [0, 1, 31, 511, 512, 513, 1024, 5000])
+def test_short_ranges_are_one_share(kernel, columns):
+    """A range of up to 512 columns is written by one workgroup, and the scratch memory left alone; a longer one is not.
+    (Entries below 2^-24 of the output scale: their high half is within fp16's smallest step, 2^-24, their low half within
+    2^-11 of that, which shows where a range has hardly any columns.)"""
+    args = [t.clone() for t in _inputs(kernel, 200, 20000, 5, 2, local=True)]
+    args[4][:], args[5][:] = 37, 37 + columns
+    args[4][1, 1], args[5][1, 1] = 100, 300
+    lib, head = _native.load_library(), (_native._kernel_id(kernel), 1, _native._i64((2,)), 200, 20000, 5)
+    need = lib.km_matmul_workspace_size(*head, None)
+    assert need > 0
+    scratch = torch.full((need // 4,), float("nan"), device=DEVICE)
+    out = torch.full((2, 200, 5), float("nan"), device=DEVICE)
+    assert lib.km_matmul_with_workspace(*head, *_native._tensors_args(*args), out.data_ptr(), None, scratch.data_ptr(), need,
+                                        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    touched = ~scratch.isnan().view(-1, 2, 200, 5)
+    assert not touched[:, 1, 128:].any()
+    assert touched[:, 0].any() == (columns > 512) and touched[:, 1, :128].any() == (columns > 512)
+    for b in range(2):
+        exact, tolerance = _exact(kernel, args, b)
+        largest = args[2][b, 37:max(37 + columns, 300)].abs().sum(0).double()
+        assert ((out[b].double() - exact).abs() <= tolerance + 2.0 ** -35 * args[3][b, -1].abs() * largest).all()
