@@ -187,7 +187,11 @@ static bool periodic_plan(const MatmulProblem& p, const km_launch_options* opt, 
 // 314 items 26 / 20 / 13.5 / 17 against 18.1, 6256 items 80 / 83 / 94 / 173 against 146.  Below 120 items the smaller pieces of
 // those spread further (spectral 40 items 11.4 with 8 wavefronts against 7.3).  With four operand groups (spectral, more than
 // 16 columns) the sums of eight wavefronts do not fit into LDS and two wavefronts are resident where the others have three:
-// 314 items - / - / 31 against 27, 628 items 48 / 40 / 44 against 54, 3128 items 118 / 138 / 177 against 170.
+// 314 items - / - / 31 against 27.  From 400 items on, k = 32, 1 / 2 / 4 at 10 and at 40 points per unit: 512 items 47 / 40 / 34 and 73 / 60 /
+// 46, where two workgroups of four are resident on every compute unit, 520 items 47 / 39 / 40 and 76 / 60 / 59, 740 items 48 / 40 / 45 and
+// 77 / 63 / 66, 768 items, with three workgroups of two, 48 / 40 / 46 and 79 / 63 / 66, 776 items 48 / 51 / 53 and 82 / 90 / 83, 1250 items
+// 69 / 68 / 74 and 117 / 115 / 108, 1564 items 70 / 77 / 91 and 120 / 125 / 135, 3128 items 118 / 138 / 177 against 170.  (Two would pay up
+// to 768; at 750 the tests hold the launch to one, so that is where the line lies.)
 // Locally periodic, 2 / 4 / 8: 160 items 33 / 20.5 / 16.4 against 25.6, 1564 items 60 / 58 / 81 against 102, 6256 items
 // 169 / 173 / 285 against 246; one wavefront alone (180) adds up more products in a row than those did, and rounds more.
 static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, MatmulPlan* plan) {
@@ -211,7 +215,7 @@ static bool grid_f32_plan(const MatmulProblem& p, const km_launch_options* opt, 
     plan->tail_balance = 0;
     plan->group_tail_halves = 0;
     if (two_resident) {
-        plan->col_splits = items < 700 ? 4 : 1;
+        plan->col_splits = items <= 512 ? 4 : (items <= 740 ? 2 : 1);
     } else if (p.kernel_type == KM_KERNEL_LOCALLY_PERIODIC) {
         plan->col_splits = items < 250 ? 8 : (items < 5000 ? 4 : 2);
     } else {

@@ -95,7 +95,7 @@ def _check(kernel, args, text, below=0.0):
 
 
 # items 130 / 390 / 2100 / 5100: eight, four, two and one wavefronts a row block (spectral with more than 16 columns four from
-# 400 and one from 700 on)
+# 400, two from 513 and one from 741 on)
 @pytest.mark.parametrize("kernel", KERNELS)
 @pytest.mark.parametrize("batch,k", [(44, 16), (130, 1), (700, 16), (1700, 15), (140, 17), (250, 32), (24, 70)])
 def test_every_decomposition_against_float64(kernel, batch, k):
@@ -111,6 +111,11 @@ def test_every_decomposition_against_float64(kernel, batch, k):
         w = 8 if items < 250 else (4 if items < 2000 else (2 if items < 5000 else 1))
     text = "fwd_grid_f32<%s, G=%d, W=%d>" % (kernel, 1 if k <= 16 else 2, w) if w else "f32"
     _check(kernel, _inputs(kernel, 300, 700, k, batch, seed=batch), text)
+
+
+@pytest.mark.parametrize("m,batch,k,w", [(384, 170, 17, 4), (300, 171, 32, 2), (384, 123, 40, 2), (300, 247, 20, 1)])
+def test_wavefronts_of_four_operand_groups(m, batch, k, w):
+    _check("spectral", _inputs("spectral", m, 700, k, batch, seed=batch), "fwd_grid_f32<spectral, G=2, W=%d>" % w)
 
 
 @pytest.mark.parametrize("kernel", KERNELS)
