@@ -1363,7 +1363,13 @@ static hipError_t launch_valu(const FwdArgs& a, int KC, unsigned gx, unsigned gy
 // of them being written back.  Measured, kept / past, us a call: rbf n = 65536, k = 64 21.8 / 20.0, spectral n = 1e5, 8 sets k = 16
 // 59.2 / 57.3, k = 32 101.2 / 97.8, n = 2e5 111.0 / 108.8, n = 20000, 4 sets 15.1 / 15.1 (14.8 / 14.4 with sets of their own).
 // Beyond half the last cache's size it depends on more than the size: n = 1e6, 8 sets, k = 32 869 / 837 with one result
-// written over and over, 782 / 817 with a new one for each call.
+// written over and over, 782 / 817 with a new one for each call.  An operation that reads the result next takes back what
+// this gains and no more: with a sum of result and vectors behind it 5 MB (spectral n = 20000, 4 sets) 20.3 / 20.6, 17 MB (the rbf
+// above) 35.4 / 34.0, 51 MB 83.1 / 83.4, 102 MB 142.9 / 142.9, 128 MB 189.5 / 189.1.
+// Wide rows have to begin and end with 64 bytes that are written at once: others are read and written again in memory, rbf
+// n = 50021, 4 sets at one point per unit k = 32 28.7 / 27.9, k = 33 40.9 / 49.5, k = 48 41.7 / 40.4, k = 63 43.2 / 63.5, k = 64 43.3 /
+// 42.9, k = 100 83.3 / 99.3, k = 112 82.7 / 80.5; of up to 32 columns one wavefront writes neighbouring rows whole, k = 20 28.0 / 28.0,
+// k = 31 28.6 / 28.0.
 #define KM_STREAM_OUT (32ll << 20)
 void fill_fwd_args(const MatmulProblem& p, FwdArgs* args) {
     FwdArgs& a = *args;
@@ -1396,7 +1402,7 @@ void fill_fwd_args(const MatmulProblem& p, FwdArgs* args) {
     a.chunks_per_block = 1;
     a.tail_items = 0;
     a.tail_half_items = 0;
-    a.stream_out = p.num_batches * p.m * p.k <= KM_STREAM_OUT;
+    a.stream_out = p.num_batches * p.m * p.k <= KM_STREAM_OUT && (p.k <= 32 || (p.k % 16 == 0 && (uintptr_t)p.out % 64 == 0));
 }
 
 hipError_t launch_matmul(const MatmulProblem& p, const MatmulPlan& plan, hipStream_t stream) {

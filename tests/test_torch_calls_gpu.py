@@ -6,6 +6,7 @@ import pytest
 import torch
 from torch.utils.checkpoint import checkpoint
 
+from kernel_matmul_amd import _native
 from kernel_matmul_amd import linear_operator as lo
 from kernel_matmul_amd.linear_operator import KernelMatmulLinearOperator
 from kernel_matmul_amd.ranges import make_ranges
@@ -195,3 +196,19 @@ def test_refused_ranges_leave_no_launch_behind():
     with pytest.raises(RuntimeError, match="sizes out of range"):
         make_ranges(2.0, x, block_size=2 ** 31 - 1)
     assert torch.cuda.current_stream().query()
+
+
+@pytest.mark.parametrize("k", [5, 16, 31, 32, 33, 48, 63, 64, 65, 80])
+@pytest.mark.parametrize("offset", [0, 1, 16])
+def test_results_are_written_where_they_are_asked_for(k, offset):
+    """The way of the stores depends on the width of the rows and on where the result begins."""
+    K, _, g = _operator("rbf", (3,), n=3000, requires_grad=False)
+    x1, x2, params, start, end = K._get_args_for_native((3,))
+    args = (x1, x2, torch.randn(3, 3000, k, generator=g).to(DEVICE), params, start, end)
+    assert "fwd_grid" in _native.describe_matmul("rbf", 3, 3000, 3000, k)
+    memory = torch.full((offset + 3 * 3000 * k + 64,), float("nan"), device=DEVICE)
+    out = _native.matmul("rbf", *args, out=memory[offset:offset + 3 * 3000 * k].view(3, 3000, k))
+    assert torch.equal(out, _native.matmul("rbf", *args))
+    assert memory[:offset].isnan().all() and memory[offset + 3 * 3000 * k:].isnan().all()
+    exact = torch.stack([_native.dense("rbf", *(t[b] for t in (x1, x2, params, start, end))).double() @ args[2][b].double() for b in range(3)])
+    assert float((out.double() - exact).norm() / exact.norm()) < 4e-6  # (two fp16 halves of either factor, and the entries' own)
