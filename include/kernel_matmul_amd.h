@@ -52,10 +52,14 @@ extern "C" {
  * (kernel_matmul/configurations.py:84-118): nothing is compiled at run time, the values
  * only select among ahead-of-time instantiated kernels. */
 typedef struct km_launch_options {
-    int variant;          /* 0 = table, 1 = VALU FMA contraction, 2 = fp32 MFMA contraction (rbf and
+    int variant;          /* 0 = table, 1 = VALU FMA contraction, 2 = fp32 MFMA contraction: from 120
+                             row-block items on (spectral kernels with more than 16 rhs columns:
+                             400) rbf and spectral kernels through an equidistant grid as with 7,
+                             locally periodic ones by entries from column tables; below that, and
+                             wherever rows_per_wave, col_splits or reserved is set, rbf and
                              spectral kernels with at most 32 rhs columns through the same column
                              tables as 3, the cosine of the phase difference per entry from
-                             tabulated cosines and sines; others evaluated directly as with 6),
+                             tabulated cosines and sines, and others evaluated directly as with 6,
                              3 = split-fp16 (hi+lo) MFMA contraction with fp32 accumulation; rbf
                              and spectral kernels with at most 16 rhs columns go through
                              per-wavefront column tables (spectral in phase-split form), spectral
@@ -72,8 +76,11 @@ typedef struct km_launch_options {
                              coordinate that is not finite reaches every row whose range holds it,
                              as with the other variants.
                              The table picks 7 for rbf and spectral kernels from 48 row-block items
-                             on, 5 for large locally periodic problems with at most 16 rhs
-                             columns and 3 otherwise. */
+                             on, entries from tabulated phases (a kernel that no value here
+                             asks for) for locally periodic ones from 32 on, the same two with the
+                             ranges in shares for few rows against many points where there is
+                             scratch (km_matmul_workspace_size), and 3 otherwise.  A row-block item
+                             is a block of 128 rows of a batch item for 16, 32 or 64 rhs columns. */
     int rows_per_wave;    /* 0 = table; else 16, 32, 64 or 128 rows of x1 per wavefront */
     int col_splits;       /* 0 = table; else 1, 2, 4 or 8 wavefronts sharing one row range */
     int reserved;         /* tail handling, for measurements: 0 = table; 1 = no tail balancing (no

@@ -338,8 +338,9 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, bool 
         plan->tail_balance = 0;
         return KM_OK;
     }
-    // From here on for what the grid form does not take: fewer than 48 row-block items, locally periodic
-    // kernels, fp32 contractions, and decompositions asked for by an option.
+    // From here on for what none of the plans above takes: rbf and spectral kernels below 48 row-block items, locally
+    // periodic ones below 32, fp32 contractions below 120 (spectral with more than 16 columns: 400), and
+    // kernels and decompositions asked for by an option.
     // Table kernel (column tables in LDS, separable exponent): rbf and spectral kernels with up
     // to 16 rhs columns, the spectral one in phase-split form (two accumulator sets per rhs
     // column group); spectral kernels with 17 to 32 columns with the cosine per entry from
@@ -462,6 +463,7 @@ static int make_plan(const MatmulProblem& p, const km_launch_options* opt, bool 
         if (per_xcd >= 2 * 128) {
             plan->group_tail = per_xcd / 7 < 128 ? per_xcd / 7 : 128;
             if (variant == KM_VARIANT_MFMA_F32) {
+                // (rows_per_wave or a tail asked for: without options such sizes go through the grid)
                 // Four wavefronts per SIMD instead of three: the last resident round (512 per XCD)
                 // should consist of split pieces.  Measured at n = 1e5, k = 16, batch 8: 178 us
                 // with 111 split items, 164.5 with 160 of which 80 in halves, 166-167 up to 256.
@@ -832,7 +834,7 @@ int km_matmul_describe(int kernel_type, int64_t num_batches, int64_t m, int64_t 
             break;
         case KM_VARIANT_BLOCK:
             snprintf(text, text_bytes,
-                     "km::fwd_block<%s, phase_split=%d, G=%d>: 4 wavefronts per 4 row blocks, rhs operand shared in LDS",
+                     "km::fwd_shared_rhs<%s, phase_split=%d, G=%d>: 4 wavefronts per 4 row blocks, rhs operand shared in LDS",
                      kt, plan.phase_split, G);
             break;
         default: {

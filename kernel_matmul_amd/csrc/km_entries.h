@@ -1,4 +1,4 @@
-// Forward operator entry by entry from column tables, shared by the kernels of km_periodic.hip and km_grid_f32.hip.
+// Forward operator entry by entry from column tables, shared by the kernels of km_periodic.hip, km_grid_f32.hip and km_grid.hip.
 #pragma once
 
 #include "km_common.h"

@@ -38,8 +38,8 @@ namespace km {
 #define KM_GRID_SPAN 2.0f
 #define KM_GRID_KS2 10              /* ... and 2^10 (rows: reference within 3.5 h s2 = 2.24) */
 #define KM_GRID_NOT_FINITE 1000     /* in place of a rhs column's shift: it holds a value that is not finite */
-// Table of a chunk: coordinate, the two column factors, the smallest and largest coordinate of each 8
-// columns, and the remainder of the coordinate.
+// Table of a chunk: coordinate, the two column factors, for each 8 columns what is halfway between their ends (entry by entry:
+// the smallest and largest coordinate), and the remainder of the coordinate.
 constexpr int grid_table_rest(int chunk) { return 3 * chunk + 2 * chunk / 8; }
 constexpr int grid_table_floats(int chunk) { return grid_table_rest(chunk) + chunk; }
 #define KM_GRID_TABLE_FLOATS (grid_table_floats(KM_GRID_CHUNK))
@@ -155,7 +155,8 @@ __device__ __forceinline__ void grid_load(const float* __restrict__ x2, long lon
 //         column factors times 2^(-b^2).  *tiles: eight bits for each step, its groups of 16 grid points (made here, once
 //         for a group of 8 columns, with what bounds them about the middles: looked at tile by tile in grid_step, within reach
 //         alone, likelihood gradient n = 1e5, 16 sets 105.7 us instead of 104.1, forward n = 1e6, k = 32 781 instead of 776, fp32
-//         n = 1e5 119.0 instead of 118.0; other sizes 0 to 0.3 %).  Steps of which a group spreads further than KM_GRID_SPAN
+//         n = 1e5 119.0 instead of 118.0; other sizes 0 to 0.3 %; rbf gradients of one column at one point per unit, which
+//         reach one or two groups a step, the other way, n = 1e5, 8 sets 52.4 and 53.8).  Steps of which a group spreads further than KM_GRID_SPAN
 //         (a gap in the data) come back in the upper half of the mask: their factors lack 2^(-b^2)
 //         (it would leave the fp16 range) and their coordinates are y and its remainder, relative to
 //         the row block's origin: a reference in the middle of the gap would round them to a fraction

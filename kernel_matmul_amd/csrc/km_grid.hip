@@ -484,7 +484,7 @@ __device__ __forceinline__ void grid_item(const FwdArgs& a, float* lds, long lon
 // Measured (a call, queued), one row block per wavefront -> four per workgroup: spectral n = 1e5, k = 16, 8 sets
 // at 10 points per unit 64.5 -> 61 us (entry by entry 103.8), at 40 115 -> 70; 4 sets at 160 182 -> 86; n = 1e6,
 // k = 32, 8 sets 850 -> 778; rbf n = 1e5, k = 64, 8 sets 130 -> 114.  A row block of the first takes 3450 VALU
-// instructions instead of 4450 and the SIMDs' VALU is busy 54 % of the cycles instead of 66: with two wavefronts
+// instructions instead of 4450 and the SIMDs' VALU is busy 56 % of the cycles instead of 66: with two wavefronts
 // resident on average, what bounds the narrow ranges is the latency of a workgroup's start, windows and exchange.
 // Four: the sums of a group and their tables are then a third of the LDS for two operand groups, so that three
 // workgroups of four wavefronts are resident, as many as the registers allow; with three row blocks for three or

@@ -21,7 +21,7 @@
 //   fwd_valu      : one row per lane, contraction with v_fma_f32 on wave-uniform x2 / rhs
 //                   operands fetched through the scalar (read-only) path.
 //
-// (Locally periodic kernels from 32 row blocks on go through km_periodic.hip; the workgroup-shared fwd_block lives in
+// (Locally periodic kernels from 32 row blocks on go through km_periodic.hip; the workgroup-shared fwd_shared_rhs lives in
 // km_matmul_block.hip.)  LDS carries the column tables of fwd_table_f16 and the fixed-order
 // reduction when several wavefronts share a row range.
 #include "km_batch.h"

@@ -267,7 +267,7 @@ __device__ __forceinline__ void block_consume(
 }
 
 template <int KT, bool PHASE, int G>
-__global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs ba) {
+__global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_shared_rhs(const BlockArgs ba) {
     constexpr int GE = (PHASE ? 2 : 1) * G;
     constexpr int NB = KM_BLK_ROW_BLOCKS;
     constexpr bool TWO = KT != KM_KERNEL_RBF && !PHASE;
@@ -704,7 +704,7 @@ __global__ void __launch_bounds__(KM_BLK_THREADS, 3) fwd_block(const BlockArgs b
 template <int KT, bool PHASE, int G>
 static hipError_t launch_block_kernel(const BlockArgs& ba, unsigned gx, unsigned gy, hipStream_t stream) {
     constexpr int GE = (PHASE ? 2 : 1) * G;
-    hipLaunchKernelGGL((fwd_block<KT, PHASE, G>), dim3(gx, gy, 1), dim3(KM_BLK_THREADS, 1, 1),
+    hipLaunchKernelGGL((fwd_shared_rhs<KT, PHASE, G>), dim3(gx, gy, 1), dim3(KM_BLK_THREADS, 1, 1),
                        sizeof(BlockLds<GE>), stream, ba);
     return hipGetLastError();
 }

@@ -87,7 +87,13 @@ static hipError_t launch_periodic_w(FwdArgs& a, const MatmulPlan& plan, unsigned
         case 1: return launch_periodic_as<G, R, 1>(a, grid_y, stream);
         case 2: return launch_periodic_as<G, R, 2>(a, grid_y, stream);
         case 4: return launch_periodic_as<G, R, 4>(a, grid_y, stream);
-        default: return launch_periodic_as<G, R, 8>(a, grid_y, stream);
+        default:
+            // (up to 16 columns take eight wavefronts with fewer rows only: periodic_plan)
+            if constexpr (G == 1) {
+                return hipErrorInvalidValue;
+            } else {
+                return launch_periodic_as<G, R, 8>(a, grid_y, stream);
+            }
     }
 }
 
